@@ -16,7 +16,9 @@ from ._lib import HN_BATCH_ALL, hn_tune
 
 _CACHE: dict = {}
 
-BATCH_CANDIDATES = [(w, b) for w in (4, 8, 16, 32) for b in (256, 512, 1024)]
+# (0, 0) is the library's default path, a workgroup per region of a map; the
+# other shapes are those of the one-workgroup-per-map kernel.
+BATCH_CANDIDATES = [(0, 0)] + [(w, b) for w in (4, 8, 16, 32) for b in (256, 512, 1024)]
 
 
 def _time(fn, reps):

@@ -6,6 +6,20 @@
 // retrieve (retrieve_kernel 647-697), erase (delete_kernel 412-505), then
 // clean_tombstones (hashinator.h:1261-1315).
 //
+// The default (no launch tuning asked for): every map is cut into regions of
+// 64 KiB of slots (8,192 u32, 4,096 u64), and a workgroup runs a phase on one
+// region in LDS (k_region_insert, k_region_lookup, k_region_clean).  It reads
+// the map's whole key list and takes the keys whose home lies in its region;
+// what probes past the region's end is left to the kernels that follow
+// (k_boundary_insert, k_map_insert_end; k_map_clean_end) or, for lookups, goes
+// on in global memory.  One workgroup per map left the call waiting for the
+// largest maps' probe chains (1,024 u32 maps of 2^8..2^16 slots at load
+// factor 0.6, velocity-grid ids: 4.99 ms, two launches of 2.16 ms among them;
+// by regions 1.04 ms: insert 0.32 + 0.08, lookups 0.35, clean 0.15 + 0.05 ms.
+// 4,096 such maps: 10.3 -> 4.2 ms; one u64 map of 2^20 slots: 13.8 -> 1.3
+// ms).  Maps of more than kMaxRegions regions, maps that a call barely
+// touches, and calls with explicit tuning take the paths below:
+//
 // Insert, and erase + clean: one workgroup owns one map at a time and runs
 // the phases on it back to back, separated by workgroup barriers with
 // workgroup-scope fences (no other workgroup touches the map during the
@@ -16,6 +30,7 @@
 // (hn_probe.hpp), so a map's results are those of the plain calls.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "hn_device.hpp"
@@ -37,7 +52,36 @@ struct BatchArgs {
    const K* ers_keys;
    Slot<K>* clean_scratch;
    uint64_t* ticket;
+   uint32_t req;          // the call's phases (ops is the launch's)
+   const uint64_t* n_big; // if set, the launch serves only the maps without regions, this many
 };
+
+// ------------------------------------------------------------ regions
+//
+// A region is 64 KiB of slots: two workgroups share a CU's LDS.  128 KiB
+// regions (half the redundant key reads) would leave one.
+template <typename K>
+constexpr int kRegionLogB = sizeof(K) == 4 ? 13 : 12;
+constexpr uint64_t kMaxRegions = 1024;
+
+// Regions of a map, or 0 when it takes the one-workgroup path: a size power
+// out of range; more than kMaxRegions regions (every region reads the map's
+// whole key lists, so the reads grow with the square of the map: a u64 map of
+// 1,024 regions at load factor 0.6 takes 13.9 ms, one of 256 1.3 ms, against
+// 54 and 13.8 ms for one workgroup per map); lists
+// too long for 32-bit indices; or several regions and fewer keys than a
+// sixteenth of the slots, where loading the table costs more than probing it.
+template <typename K>
+__device__ __forceinline__ uint32_t batch_regions(const hn_batch_map& M, int sp, uint32_t ops) {
+   if (sp < 1 || sp > max_size_power<K>()) return 0;
+   const uint64_t n = 1ull << sp;
+   const uint64_t nreg = sp <= kRegionLogB<K> ? 1 : n >> kRegionLogB<K>;
+   const uint64_t ni = (ops & HN_BATCH_INSERT) ? M.ins_len : 0, nq = (ops & HN_BATCH_RETRIEVE) ? M.qry_len : 0,
+                  ne = (ops & HN_BATCH_ERASE) ? M.ers_len : 0;
+   if (nreg > kMaxRegions || ((ni | nq | ne) >> 31)) return 0;
+   if (nreg > 1 && !(ops & HN_BATCH_CLEAN) && (ni + nq + ne) * 16 < n) return 0;
+   return static_cast<uint32_t>(nreg);
+}
 
 __device__ __forceinline__ void phase_barrier() {
    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -53,6 +97,7 @@ __global__ __launch_bounds__(1024) void k_batch(BatchArgs<K> a) {
    const uint64_t groups = blockDim.x / G;
    const uint64_t g = threadIdx.x / G;
    const int lane = __lane_id();
+   if (a.n_big && *a.n_big == 0) return; // every map has regions
 
    auto reset_shared = [&]() {
       s_placed = 0;
@@ -86,6 +131,10 @@ __global__ __launch_bounds__(1024) void k_batch(BatchArgs<K> a) {
       const int sp = info->size_power;
       const bool sp_ok = sp >= 1 && sp <= max_size_power<K>();
       const uint64_t nsl = sp_ok ? (1ull << sp) : 0;
+      if (a.n_big && batch_regions<K>(M, sp, a.req)) {
+         __syncthreads(); // s_map is rewritten by thread 0 next
+         continue;
+      }
 
       if (a.ops & HN_BATCH_INSERT) {
          InsertCounters c;
@@ -214,49 +263,101 @@ struct BatchScratch {
    uint64_t ticket;     // map ticket of k_batch
    uint64_t qry_ticket; // unit ticket of the retrieve phase
    uint64_t units;      // units of all maps
-   uint64_t reserved[5];
-   // followed by unit_start[n_maps + 1]
+   uint64_t items;      // regions of all maps
+   uint64_t n_big;      // maps without regions
+   uint64_t pad[3];
+   // followed by unit_start[n_maps + 1], item_start[n_maps + 1], MapState[n_maps], kSpillCap indices per map
 };
 static_assert(sizeof(BatchScratch) == 64, "header of hn_batch_scratch_bytes");
 
+// What the region kernels leave for the per-map kernels.
+struct MapState {
+   uint32_t spilled;   // 1: an insert ran past its region's end; 2: k_boundary_insert left some keys
+   uint32_t n_spill;   // such keys; the first kSpillCap are listed by index
+   uint32_t listed;    // clean: keys in the map's scratch slice, to be placed by k_map_clean_end
+   uint32_t max_probe; // clean: longest probe of the keys placed by the regions
+   uint32_t displaced; // clean: a live key stood away from its home slot
+   uint32_t pad[3];
+};
+constexpr uint32_t kSpillCap = 248; // with the state, 1 KiB a map
+
 __host__ __device__ inline uint64_t* unit_start(BatchScratch* sc) { return reinterpret_cast<uint64_t*>(sc + 1); }
+__host__ __device__ inline uint64_t* item_start(BatchScratch* sc, uint32_t n_maps) {
+   return unit_start(sc) + n_maps + 1;
+}
+__host__ __device__ inline MapState* map_state(BatchScratch* sc, uint32_t n_maps) {
+   return reinterpret_cast<MapState*>(item_start(sc, n_maps) + n_maps + 1);
+}
+__host__ __device__ inline uint32_t* spill_list(BatchScratch* sc, uint32_t n_maps, uint64_t map) {
+   return reinterpret_cast<uint32_t*>(map_state(sc, n_maps) + n_maps) + map * kSpillCap;
+}
 
 size_t batch_scratch_bytes(uint32_t n_maps) {
-   const size_t b = sizeof(BatchScratch) + (static_cast<size_t>(n_maps) + 1) * sizeof(uint64_t);
+   const size_t b = sizeof(BatchScratch) + (static_cast<size_t>(n_maps) + 1) * 2 * sizeof(uint64_t) +
+                    static_cast<size_t>(n_maps) * (sizeof(MapState) + kSpillCap * sizeof(uint32_t));
    return (b + 255) & ~static_cast<size_t>(255);
 }
 
-// unit_start = exclusive prefix sum of ceil(qry_len / kBatchUnit) over the
-// maps, units = the total; the unit ticket starts at 0.  One workgroup of
-// 1024 threads, 1024 maps per step.
-__global__ __launch_bounds__(1024) void k_batch_prep(const hn_batch_map* maps, uint32_t n_maps, BatchScratch* sc) {
-   __shared__ uint64_t wsum[1024 / kWave];
-   __shared__ uint64_t carry;
-   const int lane = __lane_id();
-   const int w = threadIdx.x / kWave;
-   uint64_t* us = unit_start(sc);
-   if (threadIdx.x == 0) carry = 0;
+// Block-wide exclusive prefix of one value per thread (1,024 threads);
+// *total receives the sum.  wsum: one word per wave.
+__device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t* wsum, uint64_t* total) {
+   const int lane = __lane_id(), w = threadIdx.x / kWave;
+   uint64_t x = v;
+   for (int o = 1; o < kWave; o <<= 1) {
+      const uint64_t y = __shfl_up(x, o, kWave);
+      if (lane >= o) x += y;
+   }
+   if (lane == kWave - 1) wsum[w] = x;
    __syncthreads();
+   uint64_t off = 0, sum = 0;
+   for (int i = 0; i < 1024 / kWave; ++i) {
+      if (i < w) off += wsum[i];
+      sum += wsum[i];
+   }
+   __syncthreads();
+   *total = sum;
+   return off + x - v;
+}
+
+// Over the maps, exclusive prefix sums of the retrieve units (maps without
+// regions, or every map when `regions` is 0) and of the regions; the tickets
+// and the maps' states start at 0.  One workgroup of 1,024 threads, 1,024
+// maps per step.
+template <typename K>
+__global__ __launch_bounds__(1024) void k_batch_prep(const hn_batch_map* maps, uint32_t n_maps, uint32_t ops,
+                                                     int regions, BatchScratch* sc) {
+   __shared__ uint64_t wsum[1024 / kWave];
+   uint64_t* us = unit_start(sc);
+   uint64_t* is = item_start(sc, n_maps);
+   MapState* st = map_state(sc, n_maps);
+   uint64_t units = 0, items = 0, big = 0;
    for (uint64_t base = 0; base < n_maps; base += 1024) {
       const uint64_t m = base + threadIdx.x;
-      const uint64_t u = m < n_maps ? (maps[m].qry_len + kBatchUnit - 1) / kBatchUnit : 0;
-      uint64_t x = u; // inclusive scan over the wave
-      for (int o = 1; o < kWave; o <<= 1) {
-         const uint64_t y = __shfl_up(x, o, kWave);
-         if (lane >= o) x += y;
+      uint64_t u = 0, r = 0;
+      if (m < n_maps) {
+         const hn_batch_map M = maps[m];
+         r = regions ? batch_regions<K>(M, M.info->size_power, ops) : 0;
+         u = r ? 0 : (M.qry_len + kBatchUnit - 1) / kBatchUnit;
+         st[m] = MapState{};
       }
-      if (lane == kWave - 1) wsum[w] = x;
-      __syncthreads();
-      uint64_t off = carry;
-      for (int i = 0; i < w; ++i) off += wsum[i];
-      if (m < n_maps) us[m] = off + x - u;
-      __syncthreads();
-      if (threadIdx.x == 1023) carry = off + x;
-      __syncthreads();
+      uint64_t tu, ti, tb;
+      const uint64_t xu = block_excl_scan(u, wsum, &tu);
+      const uint64_t xi = block_excl_scan(r, wsum, &ti);
+      block_excl_scan(m < n_maps && r == 0 ? 1 : 0, wsum, &tb);
+      if (m < n_maps) {
+         us[m] = units + xu;
+         is[m] = items + xi;
+      }
+      units += tu;
+      items += ti;
+      big += tb;
    }
    if (threadIdx.x == 0) {
-      us[n_maps] = carry;
-      sc->units = carry;
+      us[n_maps] = units;
+      is[n_maps] = items;
+      sc->units = units;
+      sc->items = items;
+      sc->n_big = big;
       sc->qry_ticket = 0;
    }
 }
@@ -281,6 +382,7 @@ __global__ __launch_bounds__(kWave) void k_batch_retrieve_lane(BatchArgs<K> a, B
    __shared__ K ring_v[kLaneRing];
    __shared__ uint8_t ring_s[kLaneRing];
    const uint64_t units = sc->units;
+   if (units == 0) return; // every map has regions
    const uint64_t* us = unit_start(sc);
    for (;;) {
       const uint64_t u = next_unit(&sc->qry_ticket);
@@ -312,6 +414,958 @@ __global__ __launch_bounds__(kWave) void k_batch_retrieve_lane(BatchArgs<K> a, B
          }
          wave_lds_sync();
       }
+   }
+}
+
+// ------------------------------------------------------------ region kernels
+
+constexpr int kRgBS = 512; // threads per region; two regions share a CU
+constexpr int kRgWaves = kRgBS / kWave;
+constexpr uint32_t kRgQueue = 2 * kWave; // entries of a wave's queue
+constexpr uint32_t kRgRefill = 16;       // idle lanes before a wave takes more keys
+
+// Probe windows: four aligned slots, as the group insert's default
+// (hn_probe.hpp), whose rule an insert keeps: a copy of the key anywhere in
+// the window is updated before the window's EMPTY slots are looked at.
+constexpr uint32_t kRgWin = 4;
+
+template <typename K>
+struct RegionMem {
+   static constexpr uint32_t kSlots = 1u << kRegionLogB<K>;
+   __align__(16) K key[kSlots];
+   K val[kSlots]; // the value, or (insert, slots marked in `from`) its index in the list
+   uint32_t from[kSlots / 32];
+   K qkey[kRgWaves][kRgQueue];
+   uint32_t qidx[kRgWaves][kRgQueue];
+   unsigned long long n; // placed or erased
+   uint32_t max_probe, flag;
+};
+
+// The map of region `item`: the last one whose first region is <= item (it
+// has regions, since the next map's first is above).  A whole wave searches
+// 64 ways, so a batch of thousands of maps takes two or three loads.
+__device__ __forceinline__ uint64_t find_map(const uint64_t* start, uint32_t n_maps, uint64_t item) {
+   const int lane = __lane_id();
+   uint64_t lo = 0, hi = n_maps;
+   while (hi - lo > 1) {
+      const uint64_t step = (hi - lo + kWave - 1) / kWave;
+      const uint64_t i = lo + static_cast<uint64_t>(lane) * step;
+      const uint64_t m = __ballot(i < hi && start[i] <= item);
+      const uint64_t nlo = lo + static_cast<uint64_t>(__popcll(m) - 1) * step;
+      hi = nlo + step < hi ? nlo + step : hi;
+      lo = nlo;
+   }
+   return lo;
+}
+
+// The workgroup's next region, `item` and every gridDim.x-th after it: false
+// when there is none left.  The largest maps' regions come first and regions
+// of a map are alike, so dealing them out in turn balances the grid; a ticket
+// per region took 2,280 serial atomics per launch.
+template <typename Mem>
+__device__ __forceinline__ bool next_region(Mem& L, BatchScratch* sc, uint32_t n_maps, uint64_t* item, uint64_t* map,
+                                            uint64_t* region) {
+   const uint64_t it = *item;
+   if (it >= sc->items) return false;
+   *item = it + gridDim.x;
+   const uint64_t* is = item_start(sc, n_maps);
+   *map = find_map(is, n_maps, it);
+   *region = it - is[*map];
+   __syncthreads(); // the previous region's LDS is no longer read
+   if (threadIdx.x == 0) {
+      L.n = 0;
+      L.max_probe = 0;
+      L.flag = 0;
+   }
+   __syncthreads();
+   return true;
+}
+
+template <typename K>
+__device__ __forceinline__ K lds_cas(K* p, K expected, K desired) {
+   __hip_atomic_compare_exchange_strong(p, &expected, desired, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_WORKGROUP);
+   return expected;
+}
+
+// Match and EMPTY bits of the window that slot `pos` of an LDS key array lies
+// in, from pos on.  W slots (a power of two of at most kRgWin) per window.
+template <typename K>
+__device__ __forceinline__ void window_bits(const K* key_s, uint32_t pos, uint32_t W, K key, uint32_t* mm,
+                                            uint32_t* em) {
+   const uint32_t w = pos & ~(W - 1);
+   K k[kRgWin];
+   if constexpr (sizeof(K) == 4) {
+      // tiny regions (W < 4) start at slot 0 of the array: the load stays inside it
+      const uint4 v = *reinterpret_cast<const uint4*>(key_s + (w & ~3u));
+      k[0] = v.x, k[1] = v.y, k[2] = v.z, k[3] = v.w;
+   } else {
+      const ulonglong2 v0 = *reinterpret_cast<const ulonglong2*>(key_s + (w & ~3u));
+      const ulonglong2 v1 = *reinterpret_cast<const ulonglong2*>(key_s + (w & ~3u) + 2);
+      k[0] = v0.x, k[1] = v0.y, k[2] = v1.x, k[3] = v1.y;
+   }
+   uint32_t m = 0, e = 0;
+#pragma unroll
+   for (int j = 0; j < static_cast<int>(kRgWin); ++j) {
+      m |= (k[j] == key ? 1u : 0u) << j;
+      e |= (k[j] == empty_key<K>() ? 1u : 0u) << j;
+   }
+   const uint32_t valid = (W == kRgWin ? 15u : (1u << (w & 3u) << W) - 1u) & ~((1u << (pos & 3u)) - 1u);
+   *mm = m & valid;
+   *em = e & valid;
+}
+
+// The keys a workgroup runs through its LDS table: entries 4j..4j+3 in one
+// step, 16-byte loads where a list of keys allows (a group that lies wholly
+// inside [0, len) and starts on a 16-byte boundary).
+template <typename K>
+struct KeyList {
+   const K* list;
+   uint32_t len;
+   uint32_t lead; // entries of group 0 that lie before list[0], so that groups start on 16-byte boundaries
+   __device__ KeyList(const K* l, uint32_t n)
+       : list(l), len(n), lead(static_cast<uint32_t>((reinterpret_cast<uintptr_t>(l) / sizeof(K)) & (16 / sizeof(K) - 1))) {
+      if (reinterpret_cast<uintptr_t>(l) % sizeof(K)) lead = 0;
+   }
+   __device__ uint32_t entries() const { return len ? len + lead : 0; }
+   __device__ bool valid(uint32_t e) const { return e >= lead && e - lead < len; }
+   __device__ uint32_t index(uint32_t e) const { return e - lead; }
+   __device__ void load(uint32_t e, K k[4]) const {
+      if (e >= lead && e - lead + 4 <= len && (reinterpret_cast<uintptr_t>(list + (e - lead)) & 15u) == 0) {
+         if constexpr (sizeof(K) == 4) {
+            const uint4 v = *reinterpret_cast<const uint4*>(list + (e - lead));
+            k[0] = v.x, k[1] = v.y, k[2] = v.z, k[3] = v.w;
+         } else {
+            const ulonglong2 v0 = *reinterpret_cast<const ulonglong2*>(list + (e - lead));
+            const ulonglong2 v1 = *reinterpret_cast<const ulonglong2*>(list + (e - lead) + 2);
+            k[0] = v0.x, k[1] = v0.y, k[2] = v1.x, k[3] = v1.y;
+         }
+      } else {
+#pragma unroll
+         for (int j = 0; j < 4; ++j) k[j] = valid(e + j) ? list[e + j - lead] : K(0);
+      }
+   }
+};
+// The same over some of a list's keys, by index.
+template <typename K>
+struct PickedKeys {
+   const K* list;
+   const uint32_t* pick;
+   uint32_t len;
+   __device__ uint32_t entries() const { return len; }
+   __device__ bool valid(uint32_t e) const { return e < len; }
+   __device__ uint32_t index(uint32_t e) const { return e < len ? pick[e] : 0; }
+   __device__ void load(uint32_t e, K k[4]) const {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) k[j] = e + j < len ? list[pick[e + j]] : K(0);
+   }
+};
+// The same over the keys of a slot array.
+template <typename K>
+struct SlotKeys {
+   const Slot<K>* slots;
+   uint32_t len;
+   __device__ uint32_t entries() const { return len; }
+   __device__ bool valid(uint32_t e) const { return e < len; }
+   __device__ uint32_t index(uint32_t e) const { return e; }
+   __device__ void load(uint32_t e, K k[4]) const {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) k[j] = e + j < len ? slots[e + j].key : K(0);
+   }
+};
+
+// Runs the keys of `src` that `take` accepts through probes of the
+// workgroup's LDS table.  Every lane probes a key of its own; `step` looks at
+// one window (pos: the next slot to look at; off: its distance from the home
+// slot) and returns whether the key is finished, and a lane that finishes
+// takes the wave's next key, so a wave does not wait for its longest probe
+// (velocity-grid ids at load factor 0.6 in 2^15 slots: mean probe of an
+// absent key 54 slots, of the longest in 64 keys 198).  The waves take blocks
+// of 256 entries in turn, four per lane, loaded two blocks ahead (a region of
+// a map of eight reads eight times the keys it takes), and queue the ones
+// they keep.  Every lane of the workgroup calls.
+template <typename K, typename Src, typename Take, typename Home, typename Step>
+__device__ __forceinline__ void lds_probe(RegionMem<K>& L, const Src src, int sp, Take take, Home home_pos, Step step) {
+   const uint32_t lane = __lane_id();
+   const int wave = threadIdx.x / kWave;
+   K* const qk = L.qkey[wave];
+   uint32_t* const qi = L.qidx[wave];
+   const uint32_t len = src.entries();
+   uint32_t b = static_cast<uint32_t>(wave) * 4 * kWave; // the block in k0, `sub` of its four parts taken
+   uint32_t sub = 0;
+   K k0[4], k1[4], k2[4]; // blocks b, b + 4 * BS, b + 8 * BS
+   auto load = [&](uint32_t at, K k[4]) {
+      if (at < len) src.load(at + 4 * lane, k);
+   };
+   load(b, k0), load(b + 4 * kRgBS, k1), load(b + 8 * kRgBS, k2);
+   uint32_t head = 0, have = 0;
+   bool active = false;
+   K key = 0;
+   uint32_t idx = 0, pos = 0, off = 0;
+   for (;;) {
+      const uint64_t idle = __ballot(!active);
+      const uint32_t ni = static_cast<uint32_t>(__popcll(idle));
+      if (ni == kWave && b >= len && have == 0) break;
+      if (ni >= kRgRefill && (have || b < len)) {
+         while (have < ni && have <= kRgQueue - kWave && b < len) {
+            const uint32_t e = b + 4 * lane + sub;
+            const K k = k0[0];
+            const bool in = src.valid(e) && take(src.index(e), k, home_slot(k, sp));
+            k0[0] = k0[1], k0[1] = k0[2], k0[2] = k0[3];
+            if (++sub == 4) {
+               sub = 0;
+               b += 4 * kRgBS;
+#pragma unroll
+               for (int j = 0; j < 4; ++j) k0[j] = k1[j], k1[j] = k2[j];
+               load(b + 8 * kRgBS, k2);
+            }
+            const uint64_t m = __ballot(in);
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0));
+            if (in) {
+               const uint32_t q = (head + have + rank) & (kRgQueue - 1);
+               qk[q] = k;
+               qi[q] = src.index(e);
+            }
+            have += static_cast<uint32_t>(__popcll(m));
+         }
+         wave_lds_sync();
+         const uint32_t n = have < ni ? have : ni;
+         const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+             static_cast<uint32_t>(idle >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(idle), 0));
+         if (!active && rank < n) {
+            const uint32_t q = (head + rank) & (kRgQueue - 1);
+            key = qk[q];
+            idx = qi[q];
+            pos = home_pos(home_slot(key, sp));
+            off = 0;
+            active = true;
+         }
+         wave_lds_sync(); // entries read before they are written again
+         head += n;
+         have -= n;
+      }
+      if (active) active = !step(key, idx, pos, off);
+   }
+}
+
+// Insert phase on one region.  Bound by LDS probing and by the lists a region
+// has to read; the table passes through LDS once each way.  While keys are
+// placed a slot holds its value's index in the list, so that no probe waits
+// for a value; the values come in as the region is written back.
+template <typename K>
+__global__ __launch_bounds__(kRgBS) void k_region_insert(BatchArgs<K> a, BatchScratch* sc) {
+   __shared__ RegionMem<K> L;
+   constexpr K kEmpty = empty_key<K>();
+   uint64_t mi, r, item = blockIdx.x;
+   while (next_region(L, sc, a.n_maps, &item, &mi, &r)) {
+      const hn_batch_map M = a.maps[mi];
+      if (M.ins_len == 0) continue;
+      const int sp = M.info->size_power;
+      const int rlog = sp < kRegionLogB<K> ? sp : kRegionLogB<K>;
+      const uint32_t R = 1u << rlog, W = R < kRgWin ? R : kRgWin;
+      const uint64_t nreg = 1ull << (sp - rlog);
+      Slot<K>* b = static_cast<Slot<K>*>(M.buckets) + (r << rlog);
+      for (uint32_t i = threadIdx.x; i < R; i += kRgBS) {
+         const Slot<K> s = b[i];
+         L.key[i] = s.key;
+         L.val[i] = s.val;
+      }
+      for (uint32_t i = threadIdx.x; i < (R + 31) / 32; i += kRgBS) L.from[i] = 0;
+      __syncthreads();
+      uint32_t placed = 0, max_probe = 0;
+      bool spilled = false, failed = false;
+      auto put = [&](uint32_t at, uint32_t idx) {
+         L.val[at] = static_cast<K>(idx);
+         atomicOr(&L.from[at >> 5], 1u << (at & 31));
+      };
+      lds_probe<K>(
+          L, KeyList<K>(a.ins_keys + M.ins_off, static_cast<uint32_t>(M.ins_len)), sp,
+          [&](uint32_t, K, uint32_t home) { return (home >> rlog) == r; },
+          [&](uint32_t home) { return home & (R - 1); },
+          [&](K key, uint32_t idx, uint32_t& pos, uint32_t& off) -> bool {
+             uint32_t mm, em;
+             window_bits<K>(L.key, pos, W, key, &mm, &em);
+             const uint32_t w = pos & ~3u; // bit 0's slot
+             if (mm) {
+                put(w + __ffs(mm) - 1, idx);
+                return true;
+             }
+             if (em) {
+                const uint32_t at = w + __ffs(em) - 1;
+                const K old = lds_cas(&L.key[at], kEmpty, key);
+                if (old != kEmpty && old != key) return false; // another key took it: look at the window again
+                put(at, idx);
+                if (old == kEmpty) {
+                   ++placed;
+                   const uint32_t pr = off + (at - pos) + 1;
+                   max_probe = pr > max_probe ? pr : max_probe;
+                }
+                return true;
+             }
+             const uint32_t next = (pos & ~(W - 1)) + W;
+             off += next - pos;
+             pos = next;
+             if (pos == R) {
+                if (nreg > 1) { // k_boundary_insert's
+                   spilled = true;
+                   const uint32_t n = atomic_add_relaxed(&map_state(sc, a.n_maps)[mi].n_spill, 1u);
+                   if (n < kSpillCap) spill_list(sc, a.n_maps, mi)[n] = idx;
+                   return true;
+                }
+                pos = 0;
+             }
+             if (off >= R) {
+                failed = true;
+                return true;
+             }
+             return false;
+          });
+      placed = wave_sum(placed);
+      max_probe = wave_max(max_probe);
+      const bool ws = __ballot(spilled) != 0, wf = __ballot(failed) != 0;
+      if (__lane_id() == 0) {
+         if (placed) atomicAdd(&L.n, static_cast<unsigned long long>(placed));
+         if (max_probe) atomicMax(&L.max_probe, max_probe);
+         if (ws || wf) atomicOr(&L.flag, (ws ? 1u : 0u) | (wf ? 2u : 0u));
+      }
+      __syncthreads();
+      const K* vals = a.ins_vals + M.ins_off;
+      for (uint32_t i = threadIdx.x; i < R; i += kRgBS) {
+         Slot<K> s;
+         s.key = L.key[i];
+         s.val = L.val[i];
+         if ((L.from[i >> 5] >> (i & 31)) & 1u) s.val = vals[static_cast<uint32_t>(s.val)];
+         b[i] = s;
+      }
+      if (threadIdx.x == 0) {
+         if (L.n) atomic_add_relaxed(&M.info->fill, static_cast<uint64_t>(L.n));
+         if (L.max_probe)
+            atomic_max_relaxed(&M.info->current_max_bucket_overflow,
+                               next_overflow(L.max_probe, kBucketOverflow));
+         if (L.flag & 1u)
+            __hip_atomic_fetch_or(&map_state(sc, a.n_maps)[mi].spilled, 1u, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+         if (L.flag & 2u)
+            __hip_atomic_fetch_or(&M.info->reserved1, kInfoFail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+   }
+}
+
+// One key into a table in global memory by one lane (other lanes of the
+// workgroup insert into it too): insert_range's steps for a group of one,
+// with its window rule.
+template <typename K>
+__device__ __forceinline__ void insert_one(Slot<K>* b, int sp, K key, K val, InsertCounters& c) {
+   constexpr K kEmpty = empty_key<K>();
+   const uint64_t n = 1ull << sp, mask = n - 1;
+   const uint64_t W = n < kRgWin ? n : kRgWin;
+   const uint64_t home = fib_home(key, sp) & mask;
+   for (uint64_t off = 0; off < n; ++off) {
+      const uint64_t p = (home + off) & mask;
+      const K k = b[p].key;
+      if (k == key) {
+         b[p].val = val;
+         return;
+      }
+      if (k != kEmpty) continue;
+      for (uint64_t q = p + 1; q <= (p | (W - 1)); ++q) {
+         if (b[q].key == key) {
+            b[q].val = val;
+            return;
+         }
+      }
+      const K old = atomic_cas(&b[p].key, kEmpty, key);
+      if (old == kEmpty || old == key) {
+         b[p].val = val;
+         if (old == kEmpty) {
+            ++c.placed;
+            c.max_probe = off + 1 > c.max_probe ? off + 1 : c.max_probe;
+         }
+         return;
+      }
+   }
+   c.failed = 1;
+}
+
+// The keys that probe past the end of region r, tried in LDS over the kRgHalf
+// slots before the end and as many after it (the halves of neighbouring
+// regions do not meet).
+//
+// After k_region_insert (maps of several regions where a key did): the keys
+// that k_region_insert listed or, when it met more than the list holds, all
+// keys of the map that may be among them: such a key has every slot from its
+// home to the region's end occupied, so its home lies in the region's last
+// run of occupied slots.  After k_region_clean (CLEAN): the map's listed keys with a home
+// in the region.  A home further than kRgHalf before the end, or a key that
+// finds no slot in the window, is left to the per-map kernel that follows.
+constexpr uint32_t kRgHalf = 1024;
+template <typename K, bool CLEAN>
+__global__ __launch_bounds__(kRgBS) void k_boundary_insert(BatchArgs<K> a, BatchScratch* sc) {
+   __shared__ RegionMem<K> L;
+   constexpr K kEmpty = empty_key<K>();
+   constexpr uint32_t kSpan = 2 * kRgHalf;
+   static_assert(kSpan <= RegionMem<K>::kSlots, "the window fits a region's arrays; windows are disjoint");
+   uint64_t mi, r, item = blockIdx.x;
+   while (next_region(L, sc, a.n_maps, &item, &mi, &r)) {
+      MapState* const st = &map_state(sc, a.n_maps)[mi];
+      const hn_batch_map M = a.maps[mi];
+      const int sp = M.info->size_power;
+      if (CLEAN ? (st->listed == 0 || sp <= kRegionLogB<K>) : st->spilled == 0) continue;
+      const uint32_t mask = slot_mask32(sp);
+      Slot<K>* const b = static_cast<Slot<K>*>(M.buckets);
+      const uint32_t end = static_cast<uint32_t>((r + 1) << kRegionLogB<K>);
+      const uint32_t lo = end - kRgHalf; // slots [lo, lo + kSpan), taken mod 2^sp
+      uint32_t last = 0;                 // 1 + the last EMPTY slot of the first half
+      for (uint32_t i = threadIdx.x; i < kSpan; i += kRgBS) {
+         const Slot<K> s = b[(lo + i) & mask];
+         L.key[i] = s.key;
+         L.val[i] = s.val;
+         if (i < kRgHalf && s.key == kEmpty) last = i + 1;
+      }
+      for (uint32_t i = threadIdx.x; i < kSpan / 32; i += kRgBS) L.from[i] = 0;
+      last = wave_max(last);
+      if (__lane_id() == 0 && last) atomicMax(&L.max_probe, last);
+      __syncthreads();
+      uint32_t tail = L.max_probe; // the run starts at window slot `tail`
+      __syncthreads();
+      if (threadIdx.x == 0) L.max_probe = 0;
+      if (CLEAN) {
+         tail = 0;
+      } else {
+         if (tail == kRgHalf) continue; // the region's last slot is EMPTY
+         if (tail == 0) {               // the run may reach back further
+            if (threadIdx.x == 0) __hip_atomic_fetch_or(&st->spilled, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            continue;
+         }
+      }
+      __syncthreads();
+      uint32_t placed = 0, max_probe = 0;
+      bool left = false;
+      auto put = [&](uint32_t at, uint32_t idx) {
+         L.val[at] = static_cast<K>(idx);
+         atomicOr(&L.from[at >> 5], 1u << (at & 31));
+      };
+      auto take = [&](uint32_t, K, uint32_t home) {
+         if (CLEAN && home >> kRegionLogB<K> == r && home < lo) left = true;
+         return home - lo >= tail && home - lo < kRgHalf;
+      };
+      auto step = [&](K key, uint32_t idx, uint32_t& pos, uint32_t& off) -> bool {
+         uint32_t mm, em;
+         window_bits<K>(L.key, pos, kRgWin, key, &mm, &em);
+         const uint32_t w = pos & ~3u;
+         if (mm) {
+            if (pos >= kRgHalf) put(w + __ffs(mm) - 1, idx); // one before its region's end was set there
+            return true;
+         }
+         if (em) {
+            const uint32_t at = w + __ffs(em) - 1;
+            const K old = lds_cas(&L.key[at], kEmpty, key);
+            if (old != kEmpty && old != key) return false;
+            put(at, idx);
+            if (old == kEmpty) {
+               ++placed;
+               const uint32_t pr = off + (at - pos) + 1;
+               max_probe = pr > max_probe ? pr : max_probe;
+            }
+            return true;
+         }
+         const uint32_t next = w + kRgWin;
+         off += next - pos;
+         pos = next;
+         if (pos == kSpan) {
+            left = true;
+            return true;
+         }
+         return false;
+      };
+      auto place = [&](uint32_t home) { return home - lo; };
+      const Slot<K>* const list = CLEAN ? a.clean_scratch + M.scratch_off : nullptr;
+      if constexpr (CLEAN)
+         lds_probe<K>(L, SlotKeys<K>{list, st->listed}, sp, take, place, step);
+      else if (st->n_spill <= kSpillCap)
+         lds_probe<K>(L, PickedKeys<K>{a.ins_keys + M.ins_off, spill_list(sc, a.n_maps, mi), st->n_spill}, sp, take,
+                      place, step);
+      else
+         lds_probe<K>(L, KeyList<K>(a.ins_keys + M.ins_off, static_cast<uint32_t>(M.ins_len)), sp, take, place, step);
+      placed = wave_sum(placed);
+      max_probe = wave_max(max_probe);
+      const bool wl = __ballot(left) != 0;
+      if (__lane_id() == 0) {
+         if (placed) atomicAdd(&L.n, static_cast<unsigned long long>(placed));
+         if (max_probe) atomicMax(&L.max_probe, max_probe);
+         if (wl) L.flag = 1;
+      }
+      __syncthreads();
+      for (uint32_t i = threadIdx.x; i < kSpan; i += kRgBS) {
+         if (!((L.from[i >> 5] >> (i & 31)) & 1u)) continue;
+         const uint32_t at = static_cast<uint32_t>(L.val[i]);
+         Slot<K> s;
+         s.key = L.key[i];
+         s.val = CLEAN ? list[at].val : a.ins_vals[M.ins_off + at];
+         b[(lo + i) & mask] = s;
+      }
+      if (threadIdx.x == 0) {
+         if (L.flag) __hip_atomic_fetch_or(&st->spilled, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+         if constexpr (CLEAN) { // fill does not change
+            if (L.max_probe) atomic_max_relaxed(&st->max_probe, L.max_probe);
+         } else {
+            if (L.n) atomic_add_relaxed(&M.info->fill, static_cast<uint64_t>(L.n));
+            if (L.max_probe)
+               atomic_max_relaxed(&M.info->current_max_bucket_overflow, next_overflow(L.max_probe, kBucketOverflow));
+         }
+      }
+   }
+}
+
+// After k_region_insert and k_boundary_insert, one workgroup per map: the
+// keys that k_boundary_insert left (every key with a home in a region's last
+// run of occupied slots is tried in global memory), then err.
+template <typename K>
+__global__ __launch_bounds__(kRgBS) void k_map_insert_end(BatchArgs<K> a, BatchScratch* sc) {
+   __shared__ uint64_t tail[kMaxRegions]; // first slot of each region's last run of occupied slots
+   for (uint32_t m = blockIdx.x; m < a.n_maps; m += gridDim.x) {
+      const hn_batch_map M = a.maps[m];
+      hn_info* info = M.info;
+      const int sp = info->size_power;
+      const uint32_t nreg = batch_regions<K>(M, sp, a.req);
+      if (nreg == 0) continue;
+      if (map_state(sc, a.n_maps)[m].spilled & 2u) {
+         const int rlog = kRegionLogB<K>;
+         const uint64_t R = 1ull << rlog;
+         Slot<K>* b = static_cast<Slot<K>*>(M.buckets);
+         const int lane = __lane_id();
+         for (uint32_t r = threadIdx.x / kWave; r < nreg; r += kRgWaves) {
+            const uint64_t base = static_cast<uint64_t>(r) << rlog;
+            uint64_t first = base;
+            for (uint64_t o = R; o > 0; o -= kWave) {
+               const uint64_t e = __ballot(b[base + o - kWave + lane].key == empty_key<K>());
+               if (e) {
+                  first = base + o - __clzll(static_cast<long long>(e));
+                  break;
+               }
+            }
+            if (lane == 0) tail[r] = first;
+         }
+         __syncthreads();
+         InsertCounters c;
+         for (uint64_t i = threadIdx.x; i < M.ins_len; i += kRgBS) {
+            const K key = a.ins_keys[M.ins_off + i];
+            const uint64_t home = home_slot(key, sp);
+            if (home >= tail[home >> rlog]) insert_one<K>(b, sp, key, a.ins_vals[M.ins_off + i], c);
+         }
+         insert_fold(info, c.placed, c.max_probe, c.failed);
+         phase_barrier();
+      }
+      if (threadIdx.x == 0) {
+         const int32_t f = __hip_atomic_load(&info->reserved1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kInfoFail;
+         info->err = f ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
+         info->reserved1 = 0; // inserts do not keep Robin Hood order
+      }
+      __syncthreads(); // tail is rewritten for the next map
+   }
+}
+
+// Lookups on a region go through an index of it: its keys sorted by home slot
+// (a counting sort in LDS), so a query compares the keys of its own home slot
+// alone, however long the cluster it falls into.  kOver slots after the
+// region's end are held too, for the keys that probed past it.
+template <typename K>
+struct IndexMem {
+   static constexpr uint32_t kSlots = 1u << kRegionLogB<K>;
+   static constexpr uint32_t kOver = sizeof(K) == 4 ? 512 : 1024; // what the LDS of half a CU leaves
+   static constexpr uint32_t kHeld = kSlots + kOver;
+   K key[kHeld];                // by home slot
+   uint16_t slot[kHeld];        // and the held slot of each
+   uint32_t start[kSlots / 2 + 1]; // first key of each home slot, two 16-bit entries a word
+   uint32_t empty[kHeld / 32];  // EMPTY slots, one bit each
+   K qkey[kRgWaves][kRgQueue];
+   uint32_t qidx[kRgWaves][kRgQueue];
+   uint32_t wsum[kRgWaves];
+   unsigned long long n;
+   uint32_t max_probe, flag; // flag: held slots from there on hold no EMPTY one
+};
+
+// fn(i, key) for the keys of list[0, len) whose home lies in region r, a full
+// wave of them at a time while there are that many; lanes without one call
+// with on = false.  Every lane of the workgroup calls.
+template <typename K, typename Fn>
+__device__ __forceinline__ void region_keys(IndexMem<K>& L, const KeyList<K> src, int sp, int rlog, uint64_t nreg,
+                                            uint32_t r, Fn fn) {
+   const uint32_t lane = __lane_id();
+   const int wave = threadIdx.x / kWave;
+   const uint32_t len = src.entries();
+   K* const qk = L.qkey[wave];
+   uint32_t* const qi = L.qidx[wave];
+   uint32_t have = 0;
+   K k0[4], k1[4];
+   auto load = [&](uint32_t at, K k[4]) {
+      if (at < len) src.load(at + 4 * lane, k);
+   };
+   uint32_t b = static_cast<uint32_t>(wave) * 4 * kWave;
+   load(b, k0), load(b + 4 * kRgBS, k1);
+   for (; b < len; b += 4 * kRgBS) {
+      K k[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) k[j] = k0[j], k0[j] = k1[j];
+      load(b + 8 * kRgBS, k1);
+#pragma unroll 1
+      for (int j = 0; j < 4; ++j) {
+         const uint32_t e = b + 4 * lane + j;
+         K key = k[0];
+         k[0] = k[1], k[1] = k[2], k[2] = k[3];
+         uint32_t idx = src.index(e);
+         bool on = src.valid(e);
+         if (nreg > 1) {
+            const bool in = on && (home_slot(key, sp) >> rlog) == r;
+            const uint64_t m = __ballot(in);
+            const uint32_t at = have + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0));
+            if (in) {
+               qk[at] = key;
+               qi[at] = idx;
+            }
+            have += static_cast<uint32_t>(__popcll(m));
+            if (have < static_cast<uint32_t>(kWave)) continue;
+            wave_lds_sync(); // the first 64 out, the rest to the front
+            key = qk[lane];
+            idx = qi[lane];
+            const K mk = qk[kWave + lane];
+            const uint32_t mi = qi[kWave + lane];
+            wave_lds_sync();
+            have -= kWave;
+            if (lane < have) {
+               qk[lane] = mk;
+               qi[lane] = mi;
+            }
+            on = true;
+         }
+         fn(on, idx, key);
+      }
+   }
+   if (have) {
+      wave_lds_sync();
+      const bool on = lane < have;
+      fn(on, on ? qi[lane] : 0, on ? qk[lane] : K(0));
+   }
+}
+
+// Retrieve and erase on one region.  A query's key is the one that the plain
+// probe finds: within the bound, and with no EMPTY slot between its home and
+// its slot (a table with holes left by reset_to_empty may hold keys behind
+// one).  A probe that runs past the held slots goes on in global memory, slot
+// by slot.  A TOMBSTONE is stored to global memory slot by slot, never by
+// writing the region back, so another region's probe into these slots sees a
+// key or its TOMBSTONE, neither of which ends it; the keys of a region are
+// retrieved and erased by its workgroup alone, in that order.
+template <typename K>
+__global__ __launch_bounds__(kRgBS) __attribute__((amdgpu_waves_per_eu(4))) void k_region_lookup(BatchArgs<K> a, BatchScratch* sc) {
+   __shared__ IndexMem<K> L;
+   constexpr K kEmpty = empty_key<K>();
+   constexpr K kTomb = tomb_key<K>();
+   constexpr int E = static_cast<int>((IndexMem<K>::kHeld + kRgBS - 1) / kRgBS); // held slots per thread
+   const int lane = __lane_id(), wave = threadIdx.x / kWave;
+   uint64_t mi, r64, item = blockIdx.x;
+   while (next_region(L, sc, a.n_maps, &item, &mi, &r64)) {
+      const hn_batch_map M = a.maps[mi];
+      const uint32_t nq = (a.ops & HN_BATCH_RETRIEVE) ? static_cast<uint32_t>(M.qry_len) : 0;
+      const uint32_t ne = (a.ops & HN_BATCH_ERASE) ? static_cast<uint32_t>(M.ers_len) : 0;
+      if (nq == 0 && ne == 0) continue;
+      const int sp = M.info->size_power;
+      const int rlog = sp < kRegionLogB<K> ? sp : kRegionLogB<K>;
+      const uint32_t r = static_cast<uint32_t>(r64), R = 1u << rlog, mask = slot_mask32(sp), first = r << rlog;
+      const uint64_t nreg = 1ull << (sp - rlog);
+      const uint64_t ovf = M.info->current_max_bucket_overflow, nsl = static_cast<uint64_t>(mask) + 1;
+      const uint32_t bound = static_cast<uint32_t>(ovf < nsl ? ovf : nsl);
+      const uint32_t held = nreg > 1 ? IndexMem<K>::kHeld : R;
+      Slot<K>* const all = static_cast<Slot<K>*>(M.buckets);
+
+      // the index
+      const uint32_t words = R / 2 + 1; // of start
+      for (uint32_t i = threadIdx.x; i < words; i += kRgBS) L.start[i] = 0;
+      K key[E];
+      uint32_t hs[E]; // home slot in the region << 16 | rank among its keys by arrival
+      uint32_t clear_of = 0;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+         const uint32_t i = threadIdx.x + e * kRgBS;
+         key[e] = kTomb;
+         if (i < held) key[e] = all[(first + i) & mask].key;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+         const uint32_t i = threadIdx.x + e * kRgBS;
+         hs[e] = 0xFFFFFFFFu;
+         const uint64_t em = __ballot(key[e] == kEmpty);
+         if (i < held) {
+            if ((lane & 31) == 0) L.empty[i >> 5] = static_cast<uint32_t>(em >> (lane & 32));
+            if (key[e] == kEmpty) clear_of = i + 1;
+            if (key[e] != kEmpty && key[e] != kTomb) {
+               const uint32_t home = home_slot(key[e], sp);
+               if (home >> rlog == r) {
+                  const uint32_t h = home & (R - 1), sh = (h & 1) * 16;
+                  hs[e] = h << 16 | ((atomicAdd(&L.start[h >> 1], 1u << sh) >> sh) & 0xFFFFu);
+               }
+            }
+         }
+      }
+      clear_of = wave_max(clear_of);
+      if (lane == 0 && clear_of) atomicMax(&L.flag, clear_of);
+      __syncthreads();
+      { // exclusive scan of the 16-bit counts
+         const uint32_t per = (words + kRgBS - 1) / kRgBS;
+         const uint32_t c0 = std::min<uint32_t>(threadIdx.x * per, words), c1 = std::min<uint32_t>(c0 + per, words);
+         uint32_t acc = 0;
+         for (uint32_t i = c0; i < c1; ++i) acc += (L.start[i] & 0xFFFFu) + (L.start[i] >> 16);
+         uint32_t inc = acc;
+#pragma unroll
+         for (int o = 1; o < kWave; o <<= 1) {
+            const uint32_t y = __shfl_up(inc, o, kWave);
+            if (lane >= o) inc += y;
+         }
+         if (lane == kWave - 1) L.wsum[wave] = inc;
+         __syncthreads();
+         uint32_t run = inc - acc;
+         for (int w = 0; w < wave; ++w) run += L.wsum[w];
+         for (uint32_t i = c0; i < c1; ++i) {
+            const uint32_t c = L.start[i];
+            L.start[i] = run | (run + (c & 0xFFFFu)) << 16;
+            run += (c & 0xFFFFu) + (c >> 16);
+         }
+      }
+      __syncthreads();
+      auto start_of = [&](uint32_t h) { return (L.start[h >> 1] >> ((h & 1) * 16)) & 0xFFFFu; };
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+         if (hs[e] != 0xFFFFFFFFu) {
+            const uint32_t j = start_of(hs[e] >> 16) + (hs[e] & 0xFFFFu);
+            L.key[j] = key[e];
+            L.slot[j] = static_cast<uint16_t>(threadIdx.x + e * kRgBS);
+         }
+      }
+      const uint32_t run_from = L.flag; // held slots from here on are occupied
+      __syncthreads();
+
+      // EMPTY slots in [h, s) of the held slots?
+      auto gap = [&](uint32_t h, uint32_t s) {
+         uint32_t any = 0;
+         for (uint32_t w = h >> 5; w <= s >> 5 && h < s; ++w) {
+            uint32_t v = L.empty[w];
+            if (w == h >> 5) v &= ~0u << (h & 31);
+            if (w == s >> 5) v &= (1u << (s & 31)) - 1u;
+            any |= v;
+            if (any) break;
+         }
+         return any != 0;
+      };
+      // Where a lookup of key finds it: its place in the index (below kHeld),
+      // kHeld + its table slot, or kNone.
+      constexpr uint32_t kNone = 0xFFFFFFFFu;
+      auto walk = [&](K key, uint32_t off) -> uint32_t { // the probe in global memory from offset off on
+         const uint32_t home = home_slot(key, sp);
+         for (; off < bound; ++off) {
+            const uint32_t p = (home + off) & mask;
+            const K k = all[p].key;
+            if (k == kEmpty) return kNone;
+            if (k == key) return IndexMem<K>::kHeld + p;
+         }
+         return kNone;
+      };
+      auto find = [&](K key) -> uint32_t {
+         if (key == kTomb) return walk(key, 0); // TOMBSTONEs are not in the index
+         const uint32_t h = home_slot(key, sp) & (R - 1);
+         uint32_t at = kNone, off = bound; // the nearest copy within the bound
+         for (uint32_t j = start_of(h), j1 = start_of(h + 1); j < j1; ++j) {
+            if (L.key[j] == key) {
+               const uint32_t s = L.slot[j];
+               // A slot before h: round the table's end in a one-region map; a key that went
+               // round a larger one is left to the walk.
+               const uint32_t o = s >= h ? s - h : nreg > 1 ? bound : s + R - h;
+               if (o < off) {
+                  off = o;
+                  at = j;
+               }
+            }
+         }
+         if (at != kNone) {
+            const uint32_t s = h + off;
+            const bool g = s < R || nreg > 1 ? gap(h, s) : gap(h, R) || gap(0, s - R);
+            return g ? kNone : at;
+         }
+         // not held: the probe leaves the held slots if none from home on is EMPTY
+         if (nreg > 1 && h >= run_from) return walk(key, held - h);
+         return kNone;
+      };
+      auto slot_of = [&](uint32_t at) -> uint32_t {
+         return at < IndexMem<K>::kHeld ? (first + L.slot[at]) & mask : at - IndexMem<K>::kHeld;
+      };
+      if (nq) {
+         K* const qv = a.qry_vals + M.qry_off;
+         uint8_t* const qh = a.qry_hit ? a.qry_hit + M.qry_off : nullptr;
+         region_keys<K>(L, KeyList<K>(a.qry_keys + M.qry_off, nq), sp, rlog, nreg, r,
+                        [&](bool on, uint32_t idx, K k) {
+                           if (!on) return;
+                           const uint32_t at = find(k);
+                           if (at != kNone) qv[idx] = all[slot_of(at)].val;
+                           if (qh) qh[idx] = at != kNone ? 1 : 0;
+                        });
+      }
+      if (ne) {
+         if (nq) __syncthreads();
+         uint32_t erased = 0;
+         region_keys<K>(L, KeyList<K>(a.ers_keys + M.ers_off, ne), sp, rlog, nreg, r,
+                        [&](bool on, uint32_t, K k) {
+                           if (!on) return;
+                           const uint32_t at = find(k);
+                           if (at == kNone) return;
+                           if (at >= IndexMem<K>::kHeld) {
+                              if (atomic_cas(&all[slot_of(at)].key, k, kTomb) == k) ++erased;
+                           } else if (lds_cas(&L.key[at], k, kTomb) == k) {
+                              ++erased;
+                              all[slot_of(at)].key = kTomb;
+                           }
+                        });
+         erased = wave_sum(erased);
+         if (lane == 0 && erased) atomicAdd(&L.n, static_cast<unsigned long long>(erased));
+         __syncthreads();
+         if (threadIdx.x == 0 && L.n) {
+            atomic_add_relaxed(&M.info->tombstone_counter, static_cast<uint64_t>(L.n));
+            __hip_atomic_fetch_sub(&M.info->fill, static_cast<uint64_t>(L.n), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+         }
+      }
+   }
+}
+
+// Clean on one region: the live keys standing in it whose home lies in it are
+// placed again in an LDS image that starts empty (read from the table, which
+// does not change meanwhile), then the image is written over the region.
+// Keys of other regions standing here, and keys that run past the region's
+// end, go to the map's scratch slice (at most its live keys), from which
+// k_boundary_insert and k_map_clean_end place them.  The Info is not changed
+// here.
+template <typename K>
+__global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScratch* sc) {
+   __shared__ RegionMem<K> L;
+   constexpr K kEmpty = empty_key<K>();
+   constexpr int E = static_cast<int>(RegionMem<K>::kSlots / kRgBS); // slots per thread
+   uint64_t mi, r, item = blockIdx.x;
+   while (next_region(L, sc, a.n_maps, &item, &mi, &r)) {
+      const hn_batch_map M = a.maps[mi];
+      if (M.info->tombstone_counter == 0 || M.info->fill > M.scratch_cap) continue;
+      const int sp = M.info->size_power;
+      const int rlog = sp < kRegionLogB<K> ? sp : kRegionLogB<K>;
+      const uint32_t R = 1u << rlog, W = R < kRgWin ? R : kRgWin, first = static_cast<uint32_t>(r << rlog);
+      const uint64_t nreg = 1ull << (sp - rlog);
+      Slot<K>* const b = static_cast<Slot<K>*>(M.buckets) + first;
+      Slot<K>* const list = a.clean_scratch + M.scratch_off;
+      MapState* const st = &map_state(sc, a.n_maps)[mi];
+      for (uint32_t i = threadIdx.x; i < R; i += kRgBS) L.key[i] = kEmpty;
+      __syncthreads();
+      uint32_t max_probe = 0;
+      bool displaced = false;
+      lds_probe<K>(
+          L, SlotKeys<K>{b, R}, sp,
+          [&](uint32_t i, K key, uint32_t home) {
+             if (key == kEmpty || key == tomb_key<K>()) return false;
+             displaced = displaced || home != first + i;
+             const bool own = (home >> rlog) == r;
+             if (!own) list[atomic_add_relaxed(&st->listed, 1u)] = b[i];
+             return own;
+          },
+          [&](uint32_t home) { return home & (R - 1); },
+          [&](K key, uint32_t idx, uint32_t& pos, uint32_t& off) -> bool {
+             uint32_t mm, em;
+             window_bits<K>(L.key, pos, W, key, &mm, &em);
+             const uint32_t w = pos & ~3u;
+             if (em) {
+                const uint32_t at = w + __ffs(em) - 1;
+                if (lds_cas(&L.key[at], kEmpty, key) != kEmpty) return false;
+                L.val[at] = static_cast<K>(idx);
+                const uint32_t pr = off + (at - pos) + 1;
+                max_probe = pr > max_probe ? pr : max_probe;
+                return true;
+             }
+             const uint32_t next = (pos & ~(W - 1)) + W;
+             off += next - pos;
+             pos = next;
+             if (pos == R) {
+                if (nreg > 1) {
+                   list[atomic_add_relaxed(&st->listed, 1u)] = b[idx];
+                   return true;
+                }
+                pos = 0;
+             }
+             return false; // the region's keys fit: they came from its slots
+          });
+      max_probe = wave_max(max_probe);
+      const bool wd = __ballot(displaced) != 0;
+      if (__lane_id() == 0) {
+         if (max_probe) atomicMax(&L.max_probe, max_probe);
+         if (wd) L.flag = 1;
+      }
+      __syncthreads();
+      Slot<K> s[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+         const uint32_t i = threadIdx.x + e * kRgBS;
+         s[e].key = kEmpty;
+         s[e].val = 0;
+         if (i < R) {
+            s[e].key = L.key[i];
+            if (s[e].key != kEmpty) s[e].val = b[static_cast<uint32_t>(L.val[i])].val;
+         }
+      }
+      __syncthreads(); // every value is read before the region is written
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+         const uint32_t i = threadIdx.x + e * kRgBS;
+         if (i < R) b[i] = s[e];
+      }
+      if (threadIdx.x == 0) {
+         if (L.max_probe) atomic_max_relaxed(&st->max_probe, L.max_probe);
+         if (L.flag) __hip_atomic_store(&st->displaced, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+   }
+}
+
+// After k_region_clean and k_boundary_insert, one workgroup per map: the
+// listed keys, if some were left (those already placed find themselves),
+// then the Info.
+template <typename K>
+__global__ __launch_bounds__(kRgBS) void k_map_clean_end(BatchArgs<K> a, BatchScratch* sc) {
+   __shared__ uint32_t s_max, s_failed;
+   for (uint32_t m = blockIdx.x; m < a.n_maps; m += gridDim.x) {
+      const hn_batch_map M = a.maps[m];
+      hn_info* info = M.info;
+      const int sp = info->size_power;
+      if (batch_regions<K>(M, sp, a.req) == 0 || info->tombstone_counter == 0) continue;
+      if (info->fill > M.scratch_cap) { // not enough scratch: the map is left as it is
+         if (threadIdx.x == 0) info->err = HN_STATUS_FAIL;
+         continue;
+      }
+      const MapState st = map_state(sc, a.n_maps)[m];
+      if (threadIdx.x == 0) {
+         s_max = st.max_probe;
+         s_failed = 0;
+      }
+      __syncthreads();
+      InsertCounters c;
+      const Slot<K>* list = a.clean_scratch + M.scratch_off;
+      for (uint32_t i = threadIdx.x; (st.spilled & 2u) && i < st.listed; i += kRgBS)
+         insert_one<K>(static_cast<Slot<K>*>(M.buckets), sp, list[i].key, list[i].val, c);
+      if (c.max_probe) atomicMax(&s_max, static_cast<uint32_t>(c.max_probe));
+      if (c.failed) atomicOr(&s_failed, 1u);
+      __syncthreads();
+      if (threadIdx.x == 0) {
+         info->tombstone_counter = 0;
+         const uint64_t o = next_overflow(s_max, kBucketOverflow);
+         info->current_max_bucket_overflow = o > kBucketOverflow ? o : kBucketOverflow;
+         info->reserved1 = 0; // the keys are not placed in Robin Hood order
+         if (st.displaced) info->err = s_failed ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
+      }
+      __syncthreads(); // s_max is rewritten for the next map
    }
 }
 
@@ -376,25 +1430,46 @@ int batch_run(const hn_batch_map* maps, uint32_t n_maps, uint32_t ops, const K* 
    BatchKernel<K> k = pick_batch<K>(G);
    BatchScratch* sc = static_cast<BatchScratch*>(scratch);
    uint64_t* ticket = &sc->ticket;
-   BatchArgs<K> a{maps, n_maps, ops, ik, iv, qk, qv, qh, ek, static_cast<Slot<K>*>(clean_scratch), ticket};
+   // Launch tuning asks for the one-workgroup-per-map kernel at that shape.
+   const bool regions = !(t && (t->probe_width || t->block_size || t->grid_blocks));
+   BatchArgs<K> a{maps, n_maps, ops, ik, iv, qk, qv, qh, ek, static_cast<Slot<K>*>(clean_scratch), ticket, ops,
+                  regions ? &sc->n_big : nullptr};
+   const uint32_t rg_blocks = static_cast<uint32_t>(cu_count()) * 2; // two regions' LDS per CU
+   const uint32_t map_blocks = std::min<uint32_t>(n_maps, rg_blocks);
+   if (regions || (ops & HN_BATCH_RETRIEVE))
+      hipLaunchKernelGGL(k_batch_prep<K>, dim3(1), dim3(1024), 0, s, maps, n_maps, ops, regions ? 1 : 0, sc);
    // insert; retrieve (one key per lane, its own launch); erase and clean
    if (ops & HN_BATCH_INSERT) {
       a.ops = HN_BATCH_INSERT;
       hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, ticket);
       hipLaunchKernelGGL(k, dim3(blocks), dim3(bs), 0, s, a);
+      if (regions) {
+         hipLaunchKernelGGL(k_region_insert<K>, dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
+         hipLaunchKernelGGL((k_boundary_insert<K, false>), dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
+         hipLaunchKernelGGL(k_map_insert_end<K>, dim3(map_blocks), dim3(kRgBS), 0, s, a, sc);
+      }
    }
    if (ops & HN_BATCH_RETRIEVE) {
       static std::atomic<int> occ{0};
       const int per_cu = resident_blocks_per_cu(k_batch_retrieve_lane<K>, kWave, occ);
       a.ops = HN_BATCH_RETRIEVE;
-      hipLaunchKernelGGL(k_batch_prep, dim3(1), dim3(1024), 0, s, maps, n_maps, sc);
       hipLaunchKernelGGL(k_batch_retrieve_lane<K>, dim3(static_cast<uint32_t>(cu_count()) * per_cu), dim3(kWave), 0, s,
                          a, sc);
+   }
+   if (regions && (ops & (HN_BATCH_RETRIEVE | HN_BATCH_ERASE))) {
+      a.ops = ops & (HN_BATCH_RETRIEVE | HN_BATCH_ERASE);
+      hipLaunchKernelGGL(k_region_lookup<K>, dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
    }
    if (ops & (HN_BATCH_ERASE | HN_BATCH_CLEAN)) {
       a.ops = ops & (HN_BATCH_ERASE | HN_BATCH_CLEAN);
       hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, ticket);
       hipLaunchKernelGGL(k, dim3(blocks), dim3(bs), 0, s, a);
+   }
+   if (regions && (ops & HN_BATCH_CLEAN)) {
+      a.ops = HN_BATCH_CLEAN;
+      hipLaunchKernelGGL(k_region_clean<K>, dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
+      hipLaunchKernelGGL((k_boundary_insert<K, true>), dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
+      hipLaunchKernelGGL(k_map_clean_end<K>, dim3(map_blocks), dim3(kRgBS), 0, s, a, sc);
    }
    return static_cast<int>(hipGetLastError());
 }

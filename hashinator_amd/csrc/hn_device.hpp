@@ -75,6 +75,13 @@ __device__ __forceinline__ uint32_t fib_home32(uint32_t key, int sp) {
    const uint32_t plo = key * 2654435769u, phi = __umulhi(key, 2654435769u);
    return __builtin_amdgcn_alignbit(phi, plo, static_cast<uint32_t>(32 - sp));
 }
+// fib_home32 & (2^sp - 1), the home slot.  A 32-bit key's needs the low word
+// of the product only: its bits [32 - sp, 32).
+__device__ __forceinline__ uint32_t home_slot(uint64_t key, int sp) { return fib_home32(key, sp); }
+__device__ __forceinline__ uint32_t home_slot(uint32_t key, int sp) {
+   key ^= key >> (32 - sp);
+   return (key * 2654435769u) >> (32 - sp);
+}
 __device__ __forceinline__ uint32_t slot_mask32(int sp) { return sp >= 32 ? 0xFFFFFFFFu : ((1u << sp) - 1u); }
 
 // The G-lane slice of a wave-wide ballot in 32-bit arithmetic (G <= 32).

@@ -431,10 +431,12 @@ HN_API int hn_exclusive_scan_u64(const uint64_t* in, uint64_t* out, size_t n, vo
  * bucket array and Info, and slices of shared input/output arrays.  For every
  * map the requested phases run in the reference's order -- insert
  * (hashers.h:46-65), retrieve (111-119), erase (132-142), clean_tombstones
- * (hashinator.h:1261-1315) -- with the single-map semantics above; one
- * workgroup owns one map at a time for insert and for erase + clean, maps are
- * taken in array order (list the largest first); retrieve runs in between,
- * one key per lane over units of every map's queries.  Up to three persistent
+ * (hashinator.h:1261-1315) -- with the single-map semantics above; maps are
+ * taken in array order (list the largest first).  By default a workgroup runs
+ * a phase on one 64-KiB region of a map's slots in LDS; maps of more than 1,024
+ * regions, maps of several regions that a call without clean barely touches,
+ * and calls with launch tuning take one workgroup per map for insert and for
+ * erase + clean, and one key per lane for retrieve in between.  Persistent
  * launches plus small set-up kernels (graph-capturable: no host
  * synchronisation, no allocation, no memset). */
 typedef struct hn_batch_map {
@@ -448,8 +450,9 @@ typedef struct hn_batch_map {
 
 enum { HN_BATCH_INSERT = 1, HN_BATCH_RETRIEVE = 2, HN_BATCH_ERASE = 4, HN_BATCH_CLEAN = 8 };
 
-/* Device scratch of hn_batch_run for a batch of n_maps maps: the map and
- * unit tickets and each map's first retrieve unit (8 bytes per map). */
+/* Device scratch of hn_batch_run for a batch of n_maps maps: the tickets and,
+ * per map, its first retrieve unit, its first region and what its regions
+ * leave for the map (about 1 KiB per map). */
 HN_API size_t hn_batch_scratch_bytes(uint32_t n_maps);
 
 /* Fresh tables ({EMPTYBUCKET, 0}) and Info(sps[m]) for all maps, one launch.
@@ -460,8 +463,9 @@ HN_API int hn_batch_init_u64(const hn_batch_map* maps, uint32_t n_maps, const in
 /* Run the phases in `ops` (HN_BATCH_* bits) on every map.  `maps` is a device
  * array.  Unused input pointers may be NULL; qry_hit is optional.  A map
  * whose clean would need more than scratch_cap slots gets err = FAIL and is
- * left as it is.  tune: probe_width, block_size (threads per map), grid_blocks
- * (resident workgroups); NULL = defaults. */
+ * left as it is.  tune: probe_width, block_size (threads per map) and
+ * grid_blocks (resident workgroups) of the one-workgroup-per-map kernel; NULL
+ * or all zero = the default above. */
 HN_API int hn_batch_run_u32(const hn_batch_map* maps, uint32_t n_maps, uint32_t ops, const uint32_t* ins_keys,
                             const uint32_t* ins_vals, const uint32_t* qry_keys, uint32_t* qry_vals, uint8_t* qry_hit,
                             const uint32_t* ers_keys, void* clean_scratch, void* scratch, hn_stream_t s,

@@ -230,3 +230,95 @@ def test_batch_clean_without_enough_scratch_fails_cleanly(gpu):
     for m in range(4):
         if m != m0:
             assert bm.info(m).tombstone_counter == 0
+
+
+def region_batch(key_bits, lf, seed):
+    """Maps of one, two and several 64-KiB regions, most keys' homes spread, one map's crowded at region ends."""
+    one = 13 if key_bits == 32 else 12  # size power of a one-region map
+    sps = [one + 3, one + 2, one + 1, one + 1, one, one - 1, 2, 1, one + 4]
+    ins, vals, qry, ers = [], [], [], []
+    rng = np.random.default_rng(seed)
+    for m, sp in enumerate(sps):
+        n = max(1, int(lf * (1 << sp)))
+        if m == 3:  # homes near the end of a region and of the table: probes cross both ends
+            pool = W.unique_keys(1 << (sp + 3), key_bits, seed * 100 + m)
+            h = O.fibhash(pool, np.full(pool.size, sp), key_bits) & ((1 << sp) - 1)
+            near = pool[(h & ((1 << one) - 1)) >= (1 << one) - 700]
+            k = near[: min(near.size - 64, 2000)]
+            a = near[k.size:]
+        else:
+            if m == 8:
+                n = 1 << (sp - 5)  # a few keys in many regions
+            k = W.unique_keys(n, key_bits, seed * 100 + m)
+            a = W.unique_keys(max(1, n // 2), key_bits, seed * 100 + m, start=n + 2)
+        ins.append(k)
+        vals.append(W.values(k, m).astype(k.dtype))
+        qry.append(rng.permutation(np.concatenate([k, a])))
+        ers.append(rng.choice(k, max(1, k.size // 3), replace=False))
+    return np.array(sps), ins, vals, qry, ers
+
+
+@pytest.mark.parametrize("key_bits", [32, 64])
+@pytest.mark.parametrize("lf", [0.5, 0.9, 0.97])
+def test_batch_regions_vs_oracle(gpu, key_bits, lf):
+    wl = region_batch(key_bits, lf, seed=int(lf * 100))
+    bm = BatchedMaps(*wl, key_bits=key_bits)
+    bm.init()
+    bm.run()
+    torch.cuda.synchronize()
+    check_against_oracle(bm, wl, key_bits)
+
+
+@pytest.mark.parametrize("key_bits", [32, 64])
+def test_batch_regions_with_tombstones_between(gpu, key_bits):
+    """Erase, insert everything again over the TOMBSTONEs, retrieve, then clean: region probes over
+    tables that are neither empty nor free of TOMBSTONEs, phase by phase."""
+    wl = region_batch(key_bits, 0.7, seed=5)
+    sps, ins, vals, qry, ers = wl
+    bm = BatchedMaps(*wl, key_bits=key_bits)
+    bm.init()
+    steps = [_lib.HN_BATCH_INSERT, _lib.HN_BATCH_ERASE, _lib.HN_BATCH_INSERT, _lib.HN_BATCH_RETRIEVE,
+             _lib.HN_BATCH_ERASE | _lib.HN_BATCH_CLEAN, _lib.HN_BATCH_INSERT | _lib.HN_BATCH_RETRIEVE]
+    for ops in steps:
+        bm.run(ops)
+    torch.cuda.synchronize()
+    for m, sp in enumerate(sps):
+        model = O.GpuModel(int(sp), key_bits)
+        for ops in steps:
+            if ops & _lib.HN_BATCH_INSERT:
+                model.insert(ins[m], vals[m])
+            if ops & _lib.HN_BATCH_RETRIEVE:
+                ev, eh = model.retrieve(qry[m])
+            if ops & _lib.HN_BATCH_ERASE:
+                model.erase(ers[m])
+            if ops & _lib.HN_BATCH_CLEAN:
+                model.clean_tombstones()
+        v, h = bm.results(m)
+        assert np.array_equal(h, eh) and np.array_equal(v[h], ev[eh]), m
+        img, info = bm.buckets(m), bm.info(m)
+        assert np.array_equal(live_pairs(img, key_bits), live_pairs(model.b, key_bits)), m
+        assert info.fill == model.info.fill and info.tombstone_counter == model.info.tombstones, m
+        assert reachable_all(img, key_bits, int(sp)), m
+
+
+def test_batch_regions_full_and_short_scratch(gpu):
+    """A map that cannot take all its keys reports FAIL; a clean whose scratch is too small leaves its map."""
+    key_bits, sp = 32, 14
+    full = W.unique_keys((1 << sp) + 50, key_bits, 1)
+    some = W.unique_keys(9000, key_bits, 2)
+    wl = ([sp, sp], [full, some], [full, some], [full[:64], some], [full[:1], some[:4000]])
+    bm = BatchedMaps(*wl, key_bits=key_bits)
+    bm.init()
+    bm.run(_lib.HN_BATCH_INSERT | _lib.HN_BATCH_RETRIEVE)
+    torch.cuda.synchronize()
+    assert bm.info(0).err == 1 and bm.info(0).fill == 1 << sp
+    assert bm.info(1).err == 0 and bm.info(1).fill == 9000
+    assert bm.results(1)[1].all()
+    bm.descs.view(torch.int64).view(-1, 10)[:, 9] = 100  # scratch_cap
+    bm.run(_lib.HN_BATCH_ERASE)
+    torch.cuda.synchronize()
+    before = bm.buckets(1).copy()
+    bm.run(_lib.HN_BATCH_CLEAN)
+    torch.cuda.synchronize()
+    assert bm.info(1).err == 1 and bm.info(1).tombstone_counter == 4000
+    assert np.array_equal(before, bm.buckets(1))
