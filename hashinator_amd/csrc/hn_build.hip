@@ -58,17 +58,23 @@ namespace hn {
 
 constexpr int kRegionLog = 11;   // 2048 slots per region
 constexpr int kPartBS = 256;     // count workgroup
-constexpr int kPartBSS = 256, kPartRoundsS = 16;  // 4,096-pair scatter tiles: threads, pairs per thread
+constexpr int kPartBSS = 512, kPartRoundsS = 8;   // 4,096-pair scatter tiles: threads, pairs per thread
 constexpr int kPartBSL = 1024, kPartRoundsL = 8;  // 8,192-pair scatter tiles
-// Scatter tiles: 8,192 pairs (512 threads, 16-pair runs per 9-bit digit,
-// one block per CU) for inputs of at least kPartLargeMin pairs, 4,096 (256
-// threads, two blocks per CU) below, where the large tile would leave CUs
-// idle.  At 2^28 slots the large tile builds in 9.19 ms against 9.64 ms:
-// longer runs per digit, fewer partial lines; a 2,048-pair tile with three
-// blocks per CU took 10.7 ms.
+// Scatter tiles: 8,192 pairs (16-pair runs per 9-bit digit, one block per CU)
+// for inputs of at least kPartLargeMin pairs, 4,096 (two blocks per CU) below.
+// The scatter is bound by its scattered writes: longer runs per digit mean
+// fewer partial lines (2^28 u64 slots at LF 0.9, 242 M pairs: 7.97 ms against
+// 8.66 ms with the small tile; 2^26, 60 M: 2.01 against 2.07 ms), while the
+// small tile's two blocks keep a CU busy where the table stays in the caches
+// (2^24, 15 M pairs: 0.56 against 0.60 ms).  The small tile's 512 threads of
+// 8 pairs (88 VGPRs, four waves per SIMD) instead of 256 of 16 (151 VGPRs,
+// two) took the 2^20-slot build from 0.120 to 0.115 ms, 2^22 from 0.218 to
+// 0.202.  The next tile's loads issued a whole tile ahead, with nothing that
+// waits for a tile's stores, left the 2^28 scatters at 2.68 + 2.08 ms: the
+// memory, not the wait for it, is the bound.
 constexpr uint32_t kPartTileS = 4096;
 constexpr uint32_t kPartTileL = 8192;
-constexpr uint64_t kPartLargeMin = 1ull << 22;
+constexpr uint64_t kPartLargeMin = 1ull << 25;
 constexpr int kPartSub = 8;      // tiles per partition block at most (fewer for small inputs)
 constexpr int kMaxDigitBits = 9; // 512 digits per pass at most
 constexpr int kRegionBS = 512;
