@@ -287,8 +287,9 @@ int run_compact(const In* in, uint64_t n, Out* out, uint64_t* d_count, void* scr
    return static_cast<int>(sc::launch(in, n, out, d_count, scr, s, sel, proj));
 }
 
+// cleared: an earlier kernel has cleared the look-back words (scan_words_u32).
 template <typename T>
-int run_scan(const T* in, T* out, uint64_t n, void* scr, size_t bytes, hipStream_t s) {
+int run_scan(const T* in, T* out, uint64_t n, void* scr, size_t bytes, hipStream_t s, bool cleared = false) {
    if (n && (!in || !out)) return HN_EINVAL;
    if (n == 0) return 0;
    // Pointers not 16-byte aligned take element loads and a tile of
@@ -300,7 +301,7 @@ int run_scan(const T* in, T* out, uint64_t n, void* scr, size_t bytes, hipStream
    const uint64_t tiles = (n + TILE - 1) / TILE;
    if (!scr || bytes < lookback_bytes(tiles)) return HN_ESCRATCH;
    Lookback L = lookback_layout(scr, tiles);
-   hipLaunchKernelGGL(k_lookback_init, dim3(stream_blocks(tiles, 256)), dim3(256), 0, s, L, tiles);
+   if (!cleared) hipLaunchKernelGGL(k_lookback_init, dim3(stream_blocks(tiles, 256)), dim3(256), 0, s, L, tiles);
    if (vec)
       hipLaunchKernelGGL((k_scan<T, true, kRows>), dim3(static_cast<uint32_t>(tiles)), dim3(kBS), 0, s, in, out, n, L,
                          tiles);
@@ -308,6 +309,20 @@ int run_scan(const T* in, T* out, uint64_t n, void* scr, size_t bytes, hipStream
       hipLaunchKernelGGL((k_scan<T, false, kScanRowsScalar>), dim3(static_cast<uint32_t>(tiles)), dim3(kBS), 0, s, in,
                          out, n, L, tiles);
    return static_cast<int>(hipGetLastError());
+}
+
+// For the bulk build (hn_build.hip), whose count kernel clears the words of
+// the scan that follows it: the look-back words of a scan of n 32-bit
+// elements in place, which are 16-byte aligned, and the scan over them.
+uint64_t* scan_words_u32(void* scr, uint64_t n, uint32_t* count) {
+   const uint64_t TILE = static_cast<uint64_t>(kBS) * 4 * kRows;
+   const uint64_t tiles = (n + TILE - 1) / TILE;
+   *count = static_cast<uint32_t>((256 + tiles * 16) / sizeof(uint64_t));
+   return static_cast<uint64_t*>(scr);
+}
+int scan_u32_cleared(uint32_t* x, uint64_t n, void* scr, size_t bytes, hipStream_t s) {
+   if (reinterpret_cast<uintptr_t>(x) % 16) return HN_EINVAL; // the words were counted for 16-row tiles
+   return run_scan<uint32_t>(x, x, n, scr, bytes, s, true);
 }
 
 // ------------------------------------------------------------ compaction without allocation
