@@ -17,6 +17,7 @@
 #include "hn_device.hpp"
 #include "hn_host.hpp"
 #include "hn_probe.hpp"
+#include "hn_region.hpp"
 
 namespace hn {
 
@@ -38,6 +39,16 @@ template <typename K>
 int reorder_gated(void* buckets, hn_info* info, int sp, void* scratch, size_t bytes, const uint32_t* gate,
                   hipStream_t s);
 
+// Entries that a group takes at a time: one while there is a group for every
+// entry (a group resolves its entries one after another, so the others would
+// only wait: 8,000 u64 keys into 2^18 slots, a quarter of the groups at work,
+// 21.2 us, all of them 15.4; 10^3 into 2^14 at load .9 147 and 90).
+template <int G>
+__device__ __forceinline__ uint32_t entries_per_group(uint64_t len, uint64_t groups) {
+   const uint64_t per = (len + groups - 1) / groups;
+   return per < 1 ? 1 : per < G ? static_cast<uint32_t>(per) : G;
+}
+
 // insert_kernel / insert_index_kernel (kernels_AMD.h:136-405, 507-641)
 template <typename K, int G, int SRC>
 __global__ __launch_bounds__(1024) void k_insert(InsertArgs<K> a) {
@@ -48,19 +59,84 @@ __global__ __launch_bounds__(1024) void k_insert(InsertArgs<K> a) {
    const uint64_t blk = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G;
    InsertCounters c;
    c.failed = sp_ok ? 0 : 1;
-   if (sp_ok) insert_range<K, G, SRC>(a, sp, len, blk, gstride, c);
-   if (a.fail_sink) {
-      const uint64_t placed = wave_sum(c.placed);
-      const uint64_t max_probe = wave_max(c.max_probe);
-      const int failed = wave_max(c.failed);
-      if (__lane_id() == 0) {
-         if (placed) atomic_add_relaxed(&a.info->fill, placed);
-         if (max_probe)
-            atomic_max_relaxed(&a.info->current_max_bucket_overflow, next_overflow(max_probe, kBucketOverflow));
-         if (failed) __hip_atomic_fetch_or(a.fail_sink, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+   if (sp_ok) insert_range<K, G, SRC>(a, sp, len, blk, gstride, c, entries_per_group<G>(len, gstride));
+   insert_fold_block(a.info, a.fail_sink ? a.fail_sink : &a.info->reserved1, c.placed, c.max_probe, c.failed);
+}
+
+// A workgroup that ran a whole insert: err and the reserved words, as
+// k_insert_finish leaves them.  Thread 0 wrote the fold's atomics itself.
+__device__ __forceinline__ void insert_publish(hn_info* info) {
+   if (threadIdx.x != 0) return;
+   const int32_t f = __hip_atomic_load(&info->reserved1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kInfoFail;
+   info->err = f ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
+   info->reserved0 = 0;
+   info->reserved1 = 0;
+}
+
+// An insert of at most kSmallInsert keys.  Into a table of one region (64 KiB
+// of slots, known on the device only) and at least a 64th of its slots,
+// workgroup 0 runs it with the table in LDS, where a probe chain does not wait
+// for global memory at every step (900 u64 keys into 2^10 slots: k_insert
+// 32.8 us, here 21.6); otherwise as k_insert.  Up to kSoloInsert keys take one
+// workgroup, which finishes the Info too: a launch less (200 keys into 2^18
+// slots 19.1 -> 13.0 us; more keys want more CUs, whose address translations
+// run side by side: 10^3 keys on one workgroup took 21 us, on eight 14).
+constexpr uint64_t kSmallInsert = 8192, kSoloInsert = 256;
+template <typename K, int G, int SRC>
+__global__ __launch_bounds__(kRgBS) void k_insert_small(InsertArgs<K> a, int solo) {
+   __shared__ RegionMem<K> L;
+   const int sp = a.info->size_power;
+   const bool sp_ok = sp >= 1 && sp <= max_size_power<K>();
+   if (!(sp_ok && sp <= kRegionLogB<K> && a.len * 64 >= 1ull << sp)) {
+      InsertCounters c;
+      c.failed = sp_ok ? 0 : 1;
+      const uint64_t gstride = static_cast<uint64_t>(gridDim.x) * (blockDim.x / G);
+      if (sp_ok)
+         insert_range<K, G, SRC>(a, sp, a.len, (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G,
+                                 gstride, c, entries_per_group<G>(a.len, gstride));
+      insert_fold_block(a.info, &a.info->reserved1, c.placed, c.max_probe, c.failed);
+      if (solo) insert_publish(a.info);
+      return;
+   }
+   if (blockIdx.x > 0) return;
+   const uint32_t R = 1u << sp, W = R < kRgWin ? R : kRgWin;
+   for (uint32_t i = threadIdx.x; i < R; i += blockDim.x) {
+      const Slot<K> s = a.buckets[i];
+      L.key[i] = s.key;
+      L.val[i] = s.val;
+   }
+   for (uint32_t i = threadIdx.x; i < (R + 31) / 32; i += blockDim.x) L.from[i] = 0;
+   __syncthreads();
+   InsertCounters c;
+   auto step = [&](K key, uint32_t idx, uint32_t& pos, uint32_t& off) -> bool {
+      uint32_t at;
+      const InsertStep r = lds_insert_step<K>(L, R, W, key, idx, pos, off, &at);
+      if (r == STEP_PLACED) {
+         ++c.placed;
+         const uint64_t pr = off + (at - pos) + 1;
+         c.max_probe = pr > c.max_probe ? pr : c.max_probe;
       }
-   } else {
-      insert_fold(a.info, c.placed, c.max_probe, c.failed);
+      if (r != STEP_NEXT) return r != STEP_AGAIN;
+      if (pos == R) pos = 0;
+      if (off >= R) c.failed = 1;
+      return off >= R;
+   };
+   auto take = [](uint32_t, K, uint32_t) { return true; };
+   auto home = [](uint32_t h) { return h; };
+   const uint32_t len = static_cast<uint32_t>(a.len);
+   if constexpr (SRC == SRC_PAIRS)
+      lds_probe<K>(L, SlotKeys<K>{a.pairs, len}, sp, take, home, step);
+   else
+      lds_probe<K>(L, KeyList<K>(a.keys, len), sp, take, home, step);
+   insert_fold_block(a.info, &a.info->reserved1, c.placed, c.max_probe, c.failed); // and every key is placed
+   if (solo) insert_publish(a.info);
+   for (uint32_t i = threadIdx.x; i < R; i += blockDim.x) {
+      if (!((L.from[i >> 5] >> (i & 31)) & 1u)) continue; // as it was
+      const uint32_t q = static_cast<uint32_t>(L.val[i]);
+      Slot<K> s;
+      s.key = L.key[i];
+      s.val = SRC == SRC_PAIRS ? a.pairs[q].val : SRC == SRC_SOA ? a.vals[q] : static_cast<K>(q);
+      a.buckets[i] = s;
    }
 }
 
@@ -364,12 +440,35 @@ LookupKernel<K, PAIRS, MODE> pick_lookup(int G) {
 
 template <typename K, int SRC>
 int launch_insert(InsertArgs<K> a, uint64_t grid_len, hipStream_t s, const hn_tune* t, OpKind op) {
-   Launch L;
-   int rc = resolve_launch<K>(t, op, grid_len, &L);
-   if (rc) return rc;
-   InsertKernel<K, SRC> k = pick_insert<K, SRC>(L.probe_width);
-   if (!k) return HN_EINVAL;
-   hipLaunchKernelGGL(k, dim3(L.blocks), dim3(L.block_size), 0, s, a);
+   const bool tuned = t && (t->probe_width || t->block_size || t->grid_blocks);
+   bool small = false;
+   if constexpr (SRC != SRC_TABLE) small = !tuned && !a.d_len && !a.fail_sink && a.len <= kSmallInsert;
+   if (small) {
+      if constexpr (SRC != SRC_TABLE) {
+         constexpr int G = default_probe_width<K>(OP_INSERT);
+         if (a.len <= kSoloInsert) {
+            hipLaunchKernelGGL((k_insert_small<K, G, SRC>), dim3(1), dim3(kRgBS), 0, s, a, 1);
+            return static_cast<int>(hipGetLastError());
+         }
+         const uint32_t blocks = static_cast<uint32_t>((a.len + kRgBS / G - 1) / (kRgBS / G));
+         hipLaunchKernelGGL((k_insert_small<K, G, SRC>), dim3(blocks), dim3(kRgBS), 0, s, a, 0);
+      }
+   } else {
+      Launch L;
+      // Up to 2^23 entries 1,024 threads: the fold at a block's end costs about
+      // 16 ns on the Info's one line, one block after another (300,000 u64 keys
+      // into 2^20 slots: folded per wave 135 us, per 256 threads 70, per 512 58,
+      // per 1,024 45; 8 million into 2^24 768, 682, 650 and 634).  Beyond, the
+      // smaller blocks, whose CU takes no pause for its longest chain (16 million
+      // into 2^26, load .9: 2.42 ms at 256, 2.49 at 1,024).
+      hn_tune wide = t ? *t : hn_tune{};
+      if (!wide.block_size && grid_len <= 1ull << 23) wide.block_size = 1024;
+      int rc = resolve_launch<K>(&wide, op, grid_len, &L);
+      if (rc) return rc;
+      InsertKernel<K, SRC> k = pick_insert<K, SRC>(L.probe_width);
+      if (!k) return HN_EINVAL;
+      hipLaunchKernelGGL(k, dim3(L.blocks), dim3(L.block_size), 0, s, a);
+   }
    if (!a.fail_sink) hipLaunchKernelGGL(k_insert_finish, dim3(1), dim3(1), 0, s, a.info, a.expected_fill);
    return static_cast<int>(hipGetLastError());
 }
@@ -379,7 +478,10 @@ int launch_lookup(LookupArgs<K> a, hipStream_t s, const hn_tune* t, OpKind op) {
    if constexpr (MODE != LK_RESET) {
       if (!t || t->probe_width == 0) { // automatic: lane windows
          // block_size does not apply: the lane kernel runs one wave per block
-         uint64_t need = (a.len + 255) / 256; // at least 256 queries per wave
+         // One query per lane and up (at least 256 per wave left most of the
+         // device idle: 1,000 queries of a 2^20-slot table took 17.8 us on four
+         // waves, events included, and 10.5 us on 16).
+         uint64_t need = (a.len + kWave - 1) / kWave;
          if (need == 0) need = 1;
          // one resident wave per block slot: the waves split the queries
          // statically, so a block that waits for a free slot would finish late

@@ -50,10 +50,12 @@ struct InsertCounters {
 
 // insert_kernel / insert_index_kernel semantics (kernels_AMD.h:136-405, 507-641)
 // over input entries [0, len), starting at block `blk` and stepping `gstride`
-// blocks.  Must be called by whole waves (every lane of the wave).
+// blocks of `per` entries (G, or fewer where there are groups to spare: a
+// group resolves its block's entries one after another).  Must be called by
+// whole waves (every lane of the wave).
 template <typename K, int G, int SRC>
 __device__ __forceinline__ void insert_range(const InsertArgs<K>& a, const int sp, const uint64_t len, uint64_t blk,
-                                             const uint64_t gstride, InsertCounters& cnt) {
+                                             const uint64_t gstride, InsertCounters& cnt, const uint32_t per = G) {
    constexpr K kEmpty = empty_key<K>();
    constexpr K kTomb = tomb_key<K>();
    const int lane = __lane_id();
@@ -73,9 +75,9 @@ __device__ __forceinline__ void insert_range(const InsertArgs<K>& a, const int s
 
    auto load_block = [&]() {
       active = false;
-      while (blk * G < len) {
-         const uint64_t q = blk * G + static_cast<uint64_t>(gl);
-         bool ok = q < len;
+      while (blk * per < len) {
+         const uint64_t q = blk * per + static_cast<uint64_t>(gl);
+         bool ok = static_cast<uint32_t>(gl) < per && q < len;
          if (ok) {
             if constexpr (SRC == SRC_SOA) {
                my_key = a.keys[q];

@@ -470,3 +470,54 @@ def test_side_stream_growth_rehash_and_compaction(gpu, bits):
     out = tools.copy_if_flags(hm.buckets, flags, stream=s)
     snap = hm.host_buckets()
     assert np.array_equal(to_numpy(out, bits).reshape(-1, 2), snap[::3])
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("form", ["soa", "pairs", "index"])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_small_insert_sizes(gpu, bits, form, shift):
+    # One workgroup up to 256 keys, several beyond, the group kernel past 8,192;
+    # the table in LDS up to 64 KiB and from a 64th of its slots on.  Half of
+    # each batch is there already (other values), in a table with tombstones.
+    from hashinator_amd import _lib
+    L = _lib.load()
+    t = np.int32 if bits == 32 else np.int64
+    region = 13 if bits == 32 else 12
+    for sp, n in [(1, 1), (2, 3), (5, 20), (region, 63), (region, 64), (region, 257), (region, 1000),
+                  (region + 1, 256), (region + 1, 1000), (17, 8192), (17, 8193), (region, 2049)]:
+        slots = 1 << sp
+        old = keyset(min(int(0.6 * slots), 5000), bits, seed=sp)
+        model = fresh_model(sp, bits)
+        if old.size:
+            model.insert(old, old)
+            model.erase(old[::5])
+        hm = Hashmap(sp, bits, auto_reorder=0, auto_build=0)
+        upload(hm, model)
+        back = old[:min(n // 2, old.size)]
+        keys = np.concatenate([back, keyset(n - back.size, bits, seed=sp, start=6000)])[: slots - old.size]
+        n = keys.size
+        vals = np.arange(n).astype(NDT[bits]) if form == "index" else (keys ^ NDT[bits](0x3C3C)).astype(NDT[bits])
+        # a pointer that is aligned for one element (one pair) only
+        width = 2 if form == "pairs" else 1
+        dk = torch.zeros((n + shift) * width, dtype=torch.int32 if bits == 32 else torch.int64, device="cuda")
+        dv = torch.zeros_like(dk)
+        src = np.stack([keys, vals], axis=1).reshape(-1) if form == "pairs" else keys
+        dk[shift * width:] = torch.from_numpy(src.view(t)).cuda()
+        if form != "pairs":
+            dv[shift:] = torch.from_numpy(vals.view(t)).cuda()
+        at = C.c_void_p(dk.data_ptr() + shift * width * dk.element_size())
+        av = C.c_void_p(dv.data_ptr() + shift * dv.element_size())
+        b, i = C.c_void_p(hm.buckets.data_ptr()), C.c_void_p(hm._info.data_ptr())
+        if form == "soa":
+            rc = getattr(L, f"hn_insert_u{bits}")(at, av, b, i, n, None, None)
+            model.insert(keys, vals)
+        elif form == "pairs":
+            rc = getattr(L, f"hn_insert_pairs_u{bits}")(at, b, i, n, None, None)
+            model.insert_pairs(src)
+        else:
+            rc = getattr(L, f"hn_insert_index_u{bits}")(at, b, i, n, None, None)
+            model.insert_index(keys)
+        assert rc == 0
+        torch.cuda.synchronize()
+        check_insert_invariants(hm, model, bits)
+        assert hm.info().reserved0 == 0 and hm.info().reserved1 == 0
