@@ -374,10 +374,7 @@ __device__ __forceinline__ uint64_t next_unit(uint64_t* ticket) {
 
 template <typename K>
 __global__ __launch_bounds__(kWave) void k_batch_retrieve_lane(BatchArgs<K> a, BatchScratch* sc) {
-   __shared__ __align__(16) char win_s[kLaneWaveBytes];
-   __shared__ uint32_t wb_s[kWave];
-   __shared__ K ring_v[kLaneRing];
-   __shared__ uint8_t ring_s[kLaneRing];
+   __shared__ LaneLds<K, LK_RETRIEVE> L;
    const uint64_t units = sc->units;
    if (units == 0) return; // every map has regions
    const uint64_t* us = unit_start(sc);
@@ -405,7 +402,7 @@ __global__ __launch_bounds__(kWave) void k_batch_retrieve_lane(BatchArgs<K> a, B
                           a.qry_hit ? a.qry_hit + M.qry_off : nullptr, static_cast<Slot<K>*>(M.buckets), info,
                           M.qry_len};
          if (sp >= LaneWin<K>::kLog && ovf > 0) {
-            lane_lookup<K, false, LK_RETRIEVE>(la, sp, ovf, ordered, q0, q1, win_s, wb_s, ring_v, ring_s);
+            lane_lookup<K, false, LK_RETRIEVE>(la, sp, ovf, ordered, q0, q1, L);
          } else {
             lookup_range<K, 1, false, LK_RETRIEVE>(la, sp, ovf, q1, q0 + __lane_id(), kWave, ordered);
          }
@@ -463,7 +460,6 @@ __device__ __forceinline__ bool next_region(Mem& L, BatchScratch* sc, uint32_t n
 template <typename K>
 __global__ __launch_bounds__(kRgBS) void k_region_insert(BatchArgs<K> a, BatchScratch* sc) {
    __shared__ RegionMem<K> L;
-   constexpr K kEmpty = empty_key<K>();
    uint64_t mi, r, item = blockIdx.x;
    while (next_region(L, sc, a.n_maps, &item, &mi, &r)) {
       const hn_batch_map M = a.maps[mi];

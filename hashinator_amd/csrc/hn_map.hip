@@ -183,12 +183,7 @@ __global__ __launch_bounds__(1024) void k_lookup(LookupArgs<K> a) {
 constexpr int kLaneBlock = 64;
 template <typename K, bool PAIRS, int MODE>
 __global__ __launch_bounds__(kLaneBlock) void k_lookup_lane(LookupArgs<K> a) {
-   constexpr int kWaves = kLaneBlock / kWave;
-   constexpr int kRing = MODE == LK_RETRIEVE ? kLaneRing : 1;
-   __shared__ __align__(16) char win_s[kWaves][kLaneWaveBytes];
-   __shared__ uint32_t wb_s[kWaves][kWave];
-   __shared__ K ring_v[kWaves][kRing];
-   __shared__ uint8_t ring_s[kWaves][kRing];
+   __shared__ LaneLds<K, MODE> L[kLaneBlock / kWave];
    const int sp = a.info->size_power;
    const bool sp_ok = sp >= 1 && sp <= max_size_power<K>();
    const uint64_t ovf = a.info->current_max_bucket_overflow;
@@ -202,7 +197,7 @@ __global__ __launch_bounds__(kLaneBlock) void k_lookup_lane(LookupArgs<K> a) {
          const uint64_t per = a.len / nwaves, rem = a.len % nwaves;
          const uint64_t q0 = w * per + (w < rem ? w : rem);
          const uint64_t q1 = q0 + per + (w < rem ? 1 : 0);
-         erased = lane_lookup<K, PAIRS, MODE>(a, sp, ovf, ordered, q0, q1, win_s[wv], wb_s[wv], ring_v[wv], ring_s[wv]);
+         erased = lane_lookup<K, PAIRS, MODE>(a, sp, ovf, ordered, q0, q1, L[wv]);
       } else {
          const uint64_t gstride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
          const uint64_t blk = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;

@@ -381,16 +381,23 @@ __device__ __forceinline__ uint64_t lookup_range(const LookupArgs<K>& a, const i
 // VALU-bound.  Here each lane owns its key for the whole probe.  The reads
 // stay 128-byte coalesced: the 8 lanes of a group load the current window of
 // each of the group's 8 keys in turn (8 loads of 16 bytes per lane; lane j
-// reads chunk j of every window), stage them in LDS, and read back their own
-// window: lane j gets the 8 chunks of key j.  The scan then runs in the lane
-// with no cross-lane traffic.  A lane that finishes takes the next query of
-// its wave's range at once, so lanes never wait for slow probes of others.
+// reads chunk j of every window) and compare their chunk with that key, sent
+// to them from its lane by DPP.  That leaves lane j with bit t of "my chunk
+// holds key t" and "my chunk has an EMPTY": an 8x8 bit transposition (three
+// DPP exchanges) gives lane t the bits of its own window in slot order.  A
+// lane that finishes takes the next query of its wave's range at once, so
+// lanes never wait for slow probes of others.
 //
-// Staging layout (per wave): chunk p of key k of group g at byte
-// g*kLaneGroupBytes + k*kLaneRowBytes + p*16.  A row is padded to 144 bytes:
-// the 8 lanes of a group write 128 contiguous bytes, and reading their rows
-// they start 144 bytes apart, on 8 distinct bank groups; every address is a
-// lane base plus a constant.
+// What travels through LDS is one value per query (the chunk that holds the
+// key writes it for its lane) and, in ordered tables, the window's last key.
+// Staging whole windows instead (9 KiB a wave, 8 writes and 8 reads of 16
+// bytes per step) left 11 waves on a CU, waiting for LDS as much as for
+// memory.  Measured, 2^26 queries, half of them present, u64 and u32 at load
+// .9, staged -> here: 2^18 slots (in L2) 1.58 -> 1.03 ms and 1.93 -> 0.88;
+// 2^24 2.18 -> 2.20 and 2.40 -> 1.71; 2^28 2.97 -> 2.97 and 2.94 -> 2.12.
+// The bound is now the rate of 128-byte requests, 1.56 (u64) and 1.28 (u32)
+// a query here: random ones reach 98 G/s in L2 and 55 G/s beyond, and these
+// make 101 and 97 G/s in 2^18 slots, 48 and 50 in 2^24.
 //
 // The Robin Hood stop is tested on the window's LAST slot only: in an
 // ordered table the stop predicate is monotone along a cluster (homes never
@@ -405,15 +412,46 @@ struct LaneWin {
    static constexpr int kLog = kSlots == 8 ? 3 : 4;
    static constexpr int kPerChunk = 16 / kSlotBytes; // slots per 16-byte chunk
 };
-constexpr int kLaneGroup = 8;                             // lanes that load one window together
-constexpr int kLaneRowBytes = 144;                        // one staged window, padded
-constexpr int kLaneGroupBytes = kLaneRowBytes * kLaneGroup; // 1152
-constexpr int kLaneWaveBytes = kLaneGroupBytes * (kWave / kLaneGroup); // 9 KiB of staging per wave
+constexpr int kLaneGroup = 8; // lanes that load one window together
 
 __device__ __forceinline__ void wave_lds_sync() {
    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
    __builtin_amdgcn_wave_barrier();
    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Lane T of each group of 8 lanes to all lanes of its group.  DPP's
+// row_newbcast sends one lane of each row of 16 to the row; the second one
+// writes the row's upper half only.  All lanes active.
+template <int T>
+__device__ __forceinline__ uint32_t group8_bcast(uint32_t x) {
+   const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x150 + T, 0xF, 0xF, true);
+   return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(lo, static_cast<int>(x), 0x158 + T, 0xF, 0xC, false));
+}
+template <int T>
+__device__ __forceinline__ uint64_t group8_bcast(uint64_t x) {
+   return (static_cast<uint64_t>(group8_bcast<T>(static_cast<uint32_t>(x >> 32))) << 32) |
+          group8_bcast<T>(static_cast<uint32_t>(x));
+}
+
+// Transposes the 8x8 bit matrices that a group of 8 lanes holds, one in each
+// byte of x: afterwards bit j of a byte in lane t is what was bit t in lane
+// j.  All lanes active.
+__device__ __forceinline__ uint32_t group8_transpose(uint32_t x) {
+   const int lane = __lane_id();
+   // with lane ^ k: the bits whose index has bit k where the lane has it stay,
+   // the others come from the partner, k places over
+   auto step = [&](uint32_t y, int k, uint32_t m) { // m: bits whose index lacks bit k
+      const bool up = lane & k;
+      const uint32_t rot = __builtin_amdgcn_alignbit(y, y, static_cast<uint32_t>(up ? k : 32 - k));
+      const uint32_t keep = up ? ~m : m;
+      x = (x & keep) | (rot & ~keep);
+   };
+   step(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0xB1, 0xF, 0xF, true)), 1, 0x55555555u);
+   step(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x4E, 0xF, 0xF, true)), 2, 0x33333333u);
+   const int r = __builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x1B, 0xF, 0xF, true); // lane ^ 3, then ^ 7
+   step(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(r, 0x141, 0xF, 0xF, true)), 4, 0x0F0F0F0Fu);
+   return x;
 }
 
 // Results of a wave's queries are written back in query order through a
@@ -427,19 +465,28 @@ __device__ __forceinline__ void wave_lds_sync() {
 constexpr int kLaneRing = 512;
 constexpr uint8_t kRingPending = 2;
 
-// Queries [q_next, q_end) by one wave (every lane must call).  `win`: this
-// wave's kLaneWaveBytes of staging (16-byte aligned); `wbs`: 64 words; `ring_v`/`ring_s`:
-// kLaneRing result values and states (retrieve only).  Requires
+// LDS of one wave's lookups.
+template <typename K, int MODE>
+struct LaneLds {
+   static constexpr int kRing = MODE == LK_RETRIEVE ? kLaneRing : 1;
+   K val[MODE == LK_RETRIEVE ? kWave : 1]; // the value found for each lane
+   K last[kWave];                          // the last key of each lane's window
+   K ring_v[kRing];
+   uint8_t ring_s[kRing];
+};
+
+// Queries [q_next, q_end) by one wave (every lane must call).  Requires
 // sp >= LaneWin<K>::kLog (the table holds at least one window) and ovf >= 1.
 // Returns this lane's erase count.
 template <typename K, bool PAIRS, int MODE>
 __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const int sp, const uint64_t ovf,
-                                               const bool ordered, uint64_t q_next, const uint64_t q_end, char* win,
-                                               uint32_t* wbs, K* ring_v, uint8_t* ring_s) {
+                                               const bool ordered, uint64_t q_next, const uint64_t q_end,
+                                               LaneLds<K, MODE>& L) {
    static_assert(MODE == LK_RETRIEVE || MODE == LK_ERASE, "lane windows serve retrieve and erase");
    constexpr bool RING = MODE == LK_RETRIEVE;
    using LW = LaneWin<K>;
    constexpr int WS = LW::kSlots;
+   constexpr bool TWO = LW::kPerChunk == 2; // 32-bit keys: two slots per chunk
    constexpr K kEmpty = empty_key<K>();
    constexpr K kTomb = tomb_key<K>();
    constexpr uint64_t kRingMask = kLaneRing - 1;
@@ -450,9 +497,8 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
    const uint64_t nsl = static_cast<uint64_t>(mask) + 1;
    const uint64_t bound = ovf < nsl ? ovf : nsl;
 
-   // staging: I write chunk gl of the 8 windows of my group, and read my own window
-   char* const wr = win + g * kLaneGroupBytes + gl * 16;
-   const char* const rd = win + g * kLaneGroupBytes + gl * kLaneRowBytes;
+   // what lane t of group g receives through LDS stands at index 8t + g
+   const int at = gl * kLaneGroup + g;
    const char* const tbl = reinterpret_cast<const char*>(a.buckets) + gl * 16;
 
    K key = kEmpty;
@@ -478,9 +524,10 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
       nwin = static_cast<uint32_t>((span + WS - 1) >> LW::kLog);
       last_hi = static_cast<uint32_t>(span - (static_cast<uint64_t>(nwin - 1) << LW::kLog));
       active = true;
-      if constexpr (RING) ring_s[qq & kRingMask] = kRingPending;
+      if constexpr (RING) L.ring_s[qq & kRingMask] = kRingPending;
    };
-   uint64_t lo = q_next; // results of queries below lo are written out
+   uint64_t lo = q_next;  // results of queries below lo are written out
+   uint64_t chk = q_next; // and those below chk are complete
    {
       const uint64_t qq = q_next + static_cast<uint64_t>(lane);
       if (qq < q_end) start(qq, load_key(qq));
@@ -494,6 +541,16 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
       if (qq < q_end) pre = load_key(qq);
    }
 
+   // One look at the oldest 64 entries not yet known to be complete (a step
+   // completes fewer than that on average).
+   auto check = [&]() {
+      if constexpr (RING) {
+         const uint64_t run = q_end - chk < static_cast<uint64_t>(kWave) ? q_end - chk : kWave;
+         const uint64_t e = chk + static_cast<uint64_t>(lane);
+         const bool pend = static_cast<uint64_t>(lane) < run && (e >= q_next || L.ring_s[e & kRingMask] == kRingPending);
+         if (!__ballot(pend)) chk += run;
+      }
+   };
    // Write out complete 64-entry runs of results, oldest first.  A wave's
    // later loads wait for its earlier stores to complete, so the runs go out
    // in batches of kFlushRuns (or when the ring is nearly full, or at the end
@@ -501,27 +558,14 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
    constexpr int kFlushRuns = 4;
    auto flush = [&]() {
       if constexpr (RING) {
-         wave_lds_sync();
-         int ready = 0;
-         uint64_t l = lo;
-         for (int f = 0; f < kLaneRing / kWave; ++f) {
-            const uint64_t run = q_end - l < static_cast<uint64_t>(kWave) ? q_end - l : kWave;
-            if (run == 0) break;
-            const uint64_t e = l + static_cast<uint64_t>(lane);
-            const bool need = static_cast<uint64_t>(lane) < run;
-            const bool pend = need && (e >= q_next || ring_s[e & kRingMask] == kRingPending);
-            if (__ballot(pend)) break;
-            ++ready;
-            l += run;
-         }
-         if (ready > 0 && (ready >= kFlushRuns || q_next + kWave > lo + kLaneRing || l >= q_end)) {
-            for (int f = 0; f < ready; ++f) {
+         if (chk > lo && (chk >= lo + kFlushRuns * kWave || q_next + kWave > lo + kLaneRing || chk >= q_end)) {
+            while (lo < chk) {
                const uint64_t run = q_end - lo < static_cast<uint64_t>(kWave) ? q_end - lo : kWave;
                const uint64_t e = lo + static_cast<uint64_t>(lane);
                if (static_cast<uint64_t>(lane) < run) {
-                  const uint8_t st = ring_s[e & kRingMask];
+                  const uint8_t st = L.ring_s[e & kRingMask];
                   if (st == 1) {
-                     const K v = ring_v[e & kRingMask];
+                     const K v = L.ring_v[e & kRingMask];
                      if constexpr (PAIRS) {
                         a.pairs[e].val = v;
                      } else {
@@ -533,7 +577,6 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
                lo += run;
             }
          }
-         wave_lds_sync();
       }
    };
 
@@ -544,59 +587,73 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
       const bool any = __ballot(active) != 0;
       if (!any && q_next >= q_end && (!RING || lo >= q_end)) break;
       if (!any) {
+         check();
          flush();
       } else {
          const uint32_t wb = (base + (kw << LW::kLog)) & mask; // first slot of my window
-         wbs[lane] = wb;
-         wave_lds_sync();
-         const uint4 w0 = *reinterpret_cast<const uint4*>(wbs + g * 8);
-         const uint4 w1 = *reinterpret_cast<const uint4*>(wbs + g * 8 + 4);
-         const uint32_t bw[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-         auto ld = [&](int t) {
-            return *reinterpret_cast<const uint4*>(tbl + static_cast<uint64_t>(bw[t]) * LW::kSlotBytes);
+         auto ld = [&](uint32_t w) {
+            return *reinterpret_cast<const uint4*>(tbl + static_cast<uint64_t>(w) * LW::kSlotBytes);
          };
-         const uint4 c0 = ld(0), c1 = ld(1), c2 = ld(2), c3 = ld(3), c4 = ld(4), c5 = ld(5), c6 = ld(6), c7 = ld(7);
+         const uint4 c[8] = {ld(group8_bcast<0>(wb)), ld(group8_bcast<1>(wb)), ld(group8_bcast<2>(wb)),
+                             ld(group8_bcast<3>(wb)), ld(group8_bcast<4>(wb)), ld(group8_bcast<5>(wb)),
+                             ld(group8_bcast<6>(wb)), ld(group8_bcast<7>(wb))};
+         check();
          if constexpr (MODE == LK_ERASE) {
             if (cas_pending) erased += cas_old == cas_key ? 1 : 0;
             cas_pending = false;
          }
-         auto st = [&](int t, const uint4& v) { *reinterpret_cast<uint4*>(wr + t * kLaneRowBytes) = v; };
-         st(0, c0), st(1, c1), st(2, c2), st(3, c3), st(4, c4), st(5, c5), st(6, c6), st(7, c7);
+         // my chunk against each key of the group: bit t for key t
+         uint32_t m0 = 0, m1 = 0, e0 = 0, e1 = 0;
+         auto look = [&](const uint4& v, K kt, int t) {
+            if constexpr (TWO) {
+               const bool p0 = v.x == kt, p1 = v.z == kt;
+               m0 |= p0 ? 1u << t : 0u;
+               m1 |= p1 ? 1u << t : 0u;
+               e0 |= v.x == kEmpty ? 1u << t : 0u;
+               e1 |= v.z == kEmpty ? 1u << t : 0u;
+               if (RING && (p0 || p1)) L.val[t * kLaneGroup + g] = p0 ? v.y : v.w;
+               if (ordered && gl == kLaneGroup - 1) L.last[t * kLaneGroup + g] = v.z;
+            } else {
+               const uint64_t k0 = (static_cast<uint64_t>(v.y) << 32) | v.x;
+               const bool p0 = k0 == kt;
+               m0 |= p0 ? 1u << t : 0u;
+               e0 |= k0 == kEmpty ? 1u << t : 0u;
+               if (RING && p0) L.val[t * kLaneGroup + g] = (static_cast<uint64_t>(v.w) << 32) | v.z;
+               if (ordered && gl == kLaneGroup - 1) L.last[t * kLaneGroup + g] = k0;
+            }
+         };
+         look(c[0], group8_bcast<0>(key), 0), look(c[1], group8_bcast<1>(key), 1);
+         look(c[2], group8_bcast<2>(key), 2), look(c[3], group8_bcast<3>(key), 3);
+         look(c[4], group8_bcast<4>(key), 4), look(c[5], group8_bcast<5>(key), 5);
+         look(c[6], group8_bcast<6>(key), 6), look(c[7], group8_bcast<7>(key), 7);
          // Result stores go out here, a whole scan ahead of the next window
          // loads: the wait for those loads' data also waits for every store
          // issued before them.
          flush();
+         const uint32_t tr = group8_transpose(m0 | (e0 << 8) | (m1 << 16) | (e1 << 24));
          wave_lds_sync();
 
-         // scan my window: match / EMPTY bits in slot order
-         uint32_t mm = 0, em = 0;
-#pragma unroll
-         for (int t = 0; t < 8; ++t) {
-            if constexpr (LW::kPerChunk == 1) {
-               const K k0 = *reinterpret_cast<const K*>(rd + t * 16);
-               mm |= static_cast<uint32_t>(k0 == key) << t;
-               em |= static_cast<uint32_t>(k0 == kEmpty) << t;
-            } else {
-               const uint32_t* pc = reinterpret_cast<const uint32_t*>(rd + t * 16);
-               const K k0 = static_cast<K>(pc[0]), k1 = static_cast<K>(pc[2]);
-               mm |= (static_cast<uint32_t>(k0 == key) | (static_cast<uint32_t>(k1 == key) << 1)) << (2 * t);
-               em |= (static_cast<uint32_t>(k0 == kEmpty) | (static_cast<uint32_t>(k1 == kEmpty) << 1)) << (2 * t);
-            }
-         }
+         // my window: first match and first EMPTY at or after the home slot
          const uint32_t lo_s = kw == 0 ? d0 : 0u;
          const uint32_t hi_s = kw + 1 == nwin ? last_hi : static_cast<uint32_t>(WS);
-         const uint32_t vm = ((1u << hi_s) - 1u) & ~((1u << lo_s) - 1u);
-         mm &= vm;
-         em &= vm;
-         const uint32_t hm = mm & (em ? ((em & (0u - em)) - 1u) : ~0u); // matches before the first EMPTY
-         bool fin = hm != 0 || em != 0 || kw + 1 >= nwin;
+         uint32_t fm, fe, seen;
+         if constexpr (TWO) {
+            const uint32_t v0 = ~0u << ((lo_s + 1) >> 1), v1 = ~0u << (lo_s >> 1); // even and odd slots
+            const uint32_t a0 = tr & 0xFFu, a1 = (tr >> 16) & 0xFFu;
+            seen = a0 | (a1 << 8);
+            auto first = [](uint32_t b) { return static_cast<uint32_t>(__builtin_ctz(b | 0x100u)); };
+            fm = std::min(2 * first(a0 & v0), 2 * first(a1 & v1) + 1);
+            fe = std::min(2 * first((tr >> 8) & 0xFFu & v0), 2 * first((tr >> 24) & v1) + 1);
+         } else {
+            const uint32_t v0 = ~0u << lo_s;
+            seen = tr & 0xFFu;
+            fm = static_cast<uint32_t>(__builtin_ctz((seen & v0) | 0x100u));
+            fe = static_cast<uint32_t>(__builtin_ctz((((tr >> 8) & 0xFFu) & v0) | 0x100u));
+         }
+         const bool hit = fm < fe && fm < hi_s;
+         bool fin = hit || fe < hi_s || kw + 1 >= nwin;
          if (ordered && !fin) {
-            K kl;
-            if constexpr (LW::kPerChunk == 1) {
-               kl = *reinterpret_cast<const K*>(rd + 7 * 16);
-            } else {
-               kl = static_cast<K>(reinterpret_cast<const uint32_t*>(rd + 7 * 16)[2]);
-            }
+            const K kl = L.last[at];
             if (kl != kTomb) {
                const uint32_t slot_l = wb + (WS - 1);
                const uint32_t d_occ = (slot_l - fib_home32(kl, sp)) & mask;
@@ -606,22 +663,22 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
          }
          fin = fin && active;
          if (fin) {
-            const bool hit = hm != 0;
             if (hit) {
-               const uint32_t sl = static_cast<uint32_t>(__ffs(hm) - 1);
                if constexpr (MODE == LK_ERASE) {
                   // the CAS result is counted a step later, so the wave does
                   // not wait for the atomic here
-                  cas_old = atomic_cas(&a.buckets[wb + sl].key, key, kTomb);
+                  cas_old = atomic_cas(&a.buckets[wb + fm].key, key, kTomb);
                   cas_key = key;
                   cas_pending = true;
                } else {
-                  // the value sits next to the key in the staged window
-                  const K v = *reinterpret_cast<const K*>(rd + sl * LW::kSlotBytes + sizeof(K));
-                  ring_v[q & kRingMask] = v;
+                  K v = L.val[at];
+                  // several copies in the window (or one before the home
+                  // slot): any of their chunks may have written last
+                  if (seen & (seen - 1)) v = a.buckets[wb + fm].val;
+                  L.ring_v[q & kRingMask] = v;
                }
             }
-            if constexpr (RING) ring_s[q & kRingMask] = hit ? 1 : 0;
+            if constexpr (RING) L.ring_s[q & kRingMask] = hit ? 1 : 0;
             active = false;
          } else if (active) {
             ++kw;
@@ -649,7 +706,7 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
             if (pq < q_end) pre = load_key(pq);
          }
       }
-      wave_lds_sync(); // the next window's staging overwrites this one
+      wave_lds_sync(); // val, last and the ring are read before they are written again
    }
    if (cas_pending) erased += cas_old == cas_key ? 1 : 0;
    return erased;

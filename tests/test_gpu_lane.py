@@ -146,3 +146,35 @@ def test_lane_query_counts(gpu, bits, nq):
     hm.erase(q)
     model.erase(q)
     assert np.array_equal(hm.host_buckets().reshape(-1), model.b)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("sp", [4, 5, 7])
+@pytest.mark.parametrize("bound", [1, 7, 64])
+def test_lane_repeated_keys_in_windows(gpu, bits, sp, bound):
+    """Bucket images with several copies of a key in one window, copies before
+    the home slot and behind EMPTY and TOMBSTONE slots, and probe bounds that
+    end inside a window: the first copy in probe order answers."""
+    from tests.helpers import EMPTY, TOMB
+    rng = np.random.default_rng(sp * 10 + bits + bound)
+    N = 1 << sp
+    for density in (0.5, 0.95):
+        alphabet = keyset(max(4, N // 4), bits, seed=sp)
+        k = rng.choice(alphabet, N)
+        k[rng.random(N) > density] = EMPTY[bits]
+        k[rng.random(N) < 0.1] = TOMB[bits]
+        img = np.stack([k, np.arange(100, 100 + N).astype(NDT[bits])], axis=1).astype(NDT[bits])
+        fill = int(((k != EMPTY[bits]) & (k != TOMB[bits])).sum())
+        info = (sp, fill, bound, int((k == TOMB[bits]).sum()), 0)
+        model = model_from(img.copy(), info, bits)
+        hm = Hashmap(sp, bits, auto_reorder=0, auto_build=0)
+        from tests.test_gpu_map import upload
+        upload(hm, model)
+        q = rng.permutation(np.concatenate([np.repeat(alphabet, 5), keyset(70, bits, seed=sp, start=5000)]))
+        v, h = retrieve_np(hm, q, bits, NDT[bits](5))
+        ev, eh = model.retrieve(q, np.full(q.size, 5, dtype=NDT[bits]))
+        assert np.array_equal(h, eh) and np.array_equal(v, ev)
+        e = alphabet[::2]  # one erase call takes one copy of each
+        hm.erase(e)
+        model.erase(e)
+        assert np.array_equal(hm.host_buckets().reshape(-1), model.b)
