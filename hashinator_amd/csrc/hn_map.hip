@@ -481,7 +481,11 @@ int launch_lookup(LookupArgs<K> a, hipStream_t s, const hn_tune* t, OpKind op) {
          // one resident wave per block slot: the waves split the queries
          // statically, so a block that waits for a free slot would finish late
          static std::atomic<int> occ{0};
-         const int per_cu = resident_blocks_per_cu(k_lookup_lane<K, PAIRS, MODE>, kLaneBlock, occ);
+         // 16 waves on a CU: in L2 fewer are slower (2^26 u64 queries of 2^18
+         // slots: 12 waves 1.24 ms, 16 and 20 1.07), beyond it more only queue
+         // (2^24 slots: 16 waves 2.17 ms, 20 2.23; 2^28 2.93 and 2.97).
+         const int per_cu =
+             std::min(resident_blocks_per_cu(k_lookup_lane<K, PAIRS, MODE>, kLaneBlock, occ), 16);
          uint64_t cap = (t && t->grid_blocks > 0) ? static_cast<uint64_t>(t->grid_blocks)
                                                   : static_cast<uint64_t>(cu_count()) * per_cu;
          if (cap > (1u << 20)) cap = 1u << 20;
