@@ -600,17 +600,18 @@ __global__ __launch_bounds__(256) void k_region_starts(const Slot<K>* S, uint64_
 
 constexpr int kRegionNW = kRegionBS / kWave;
 constexpr uint32_t kRegionMax = 1u << kRegionLog;
-constexpr uint32_t kSpanMax = kRegionMax + kRegionCap; // slots one region writes at most
-constexpr uint32_t kSpanWords = (kSpanMax + 31) / 32;
 
-// LDS of one region: the sort tables are dead once each key knows its sorted
-// index, so the placement arrays reuse their space.
-template <typename K>
+// LDS of one region of at most IPT keys per thread: the sort tables are dead
+// once each key knows its sorted index, so the placement arrays reuse their
+// space.
+template <typename K, int IPT>
 struct RegionLds {
-   K key[kRegionCap];
-   uint16_t order[kRegionCap];
+   static constexpr uint32_t kCap = kRegionBS * IPT;
+   static constexpr uint32_t kSpanWords = (kRegionMax + kCap + 31) / 32; // a region writes at most kRegionMax + kCap slots
+   K key[kCap];
+   uint16_t order[kCap];
    union {
-      uint8_t dup[kRegionCap];
+      uint8_t dup[kCap];
       uint32_t occ[kSpanWords]; // slots of the write span holding a key
    } u1;
    union {
@@ -618,40 +619,24 @@ struct RegionLds {
          uint32_t cnt[kRegionMax + 1];  // keys per home offset, then their exclusive starts
          uint32_t scnt[kRegionMax + 1]; // the same over the surviving keys
       } c;
-      int32_t v[kRegionCap]; // by sorted index f: home offset - f, then its running max
+      int32_t v[kCap]; // by sorted index f: home offset - f, then its running max
    } u2;
+   static_assert(sizeof(uint32_t) * kSpanWords <= kCap, "occupancy bits fit the dup table");
+   static_assert(sizeof(int32_t) * kCap <= 2 * sizeof(uint32_t) * (kRegionMax + 1), "v fits the count tables");
    uint32_t wsum[kRegionNW];
    int32_t wmax[kRegionNW];
    uint32_t r;
    int64_t carry;
 };
-static_assert(sizeof(uint32_t) * kSpanWords <= kRegionCap, "occupancy bits fit the dup table");
-static_assert(sizeof(int32_t) * kRegionCap <= 2 * sizeof(uint32_t) * (kRegionMax + 1), "v fits the count tables");
-
-// Sort region keys S[lo, lo + m) in LDS by (home, key), keeping the last
-// occurrence of a repeated key.  Thread t owns keys t + k*kRegionBS; ff[k] =
-// its sorted index among the survivors, or -1.  Leaves v[f] = home offset - f.
-// Returns the number of survivors.  Called by the whole workgroup.
-//
-// A counting sort by home slot puts the keys, with their input indices, in
-// home order in LDS; a key's rank among its home's keys is then one pass over
-// that home's few entries (0.9 others on average at load factor 0.9), which
-// also spots repeated keys.  Without repeats in the region (the block agrees
-// with one __syncthreads_or) every key survives and the sorted index is
-// home start + rank; otherwise the survivors are counted per home and ranked
-// again among survivors.  PRE: kk/vv already hold the pairs (loaded ahead by
-// the caller), S is not read.
+// Pairs S[lo, lo + m) of a region: thread t owns keys t + k*kRegionBS, kk/vv
+// the pairs, uu[k] the key's home offset in the region.  PRE: kk
+// and vv hold the pairs (loaded ahead by the caller), S is not read.
 template <typename K, bool PRE = false>
-__device__ uint32_t region_sort(const Slot<K>* S, uint64_t lo, uint32_t m, int sp, uint64_t R, RegionLds<K>& L,
-                                K* kk, K* vv, uint32_t* uu, int32_t* ff) {
-   __syncthreads(); // the previous user of L is done
-   for (uint32_t i = threadIdx.x; i <= R; i += kRegionBS) L.u2.c.cnt[i] = 0;
-   __syncthreads();
-   uint32_t sub[kRegionIPT];
+__device__ __forceinline__ void region_pairs(const Slot<K>* S, uint64_t lo, uint32_t m, int sp, uint64_t R, K* kk,
+                                             K* vv, uint32_t* uu) {
 #pragma unroll
    for (int k = 0; k < kRegionIPT; ++k) {
       const uint32_t e = threadIdx.x + k * kRegionBS;
-      ff[k] = -1;
       if (e < m) {
          if (!PRE) {
             const Slot<K> s = S[lo + e];
@@ -659,16 +644,46 @@ __device__ uint32_t region_sort(const Slot<K>* S, uint64_t lo, uint32_t m, int s
             vv[k] = s.val;
          }
          uu[k] = static_cast<uint32_t>((fib_home(kk[k], sp) & ((1ull << sp) - 1)) & (R - 1));
-         sub[k] = atomicAdd(&L.u2.c.cnt[uu[k]], 1u);
       }
    }
+}
+
+// has() of region_sort where the first m elements are the keys.
+__device__ __forceinline__ auto in_first(uint32_t m) {
+   return [m](int k) { return threadIdx.x + k * kRegionBS < m; };
+}
+
+// Sort a region's keys in LDS by (home, key), keeping the last occurrence of
+// a repeated key.  Thread t owns the keys of input index t + k*kRegionBS for
+// which has(k); ff[k] = its sorted index among the survivors, or -1.
+// Leaves v[f] = home offset - f.  Returns the number of survivors.  Called by
+// the whole workgroup.
+//
+// A counting sort by home slot puts the keys, with their input indices, in
+// home order in LDS; a key's rank among its home's keys is then one pass over
+// that home's few entries (0.9 others on average at load factor 0.9), which
+// also spots repeated keys.  Without repeats in the region (the block agrees
+// with one __syncthreads_or) every key survives and the sorted index is
+// home start + rank; otherwise the survivors are counted per home and ranked
+// again among survivors.
+template <typename K, int IPT, typename F>
+__device__ uint32_t region_sort(uint64_t R, RegionLds<K, IPT>& L, F has, const K* kk, const uint32_t* uu, int32_t* ff) {
+   __syncthreads(); // the previous user of L is done
+   for (uint32_t i = threadIdx.x; i <= R; i += kRegionBS) L.u2.c.cnt[i] = 0;
    __syncthreads();
-   lds_exclusive_scan<kRegionBS>(L.u2.c.cnt, static_cast<uint32_t>(R) + 1, L.wsum);
+   uint32_t sub[IPT];
+#pragma unroll
+   for (int k = 0; k < IPT; ++k) {
+      ff[k] = -1;
+      if (has(k)) sub[k] = atomicAdd(&L.u2.c.cnt[uu[k]], 1u);
+   }
+   __syncthreads();
+   const uint32_t m = lds_exclusive_scan<kRegionBS>(L.u2.c.cnt, static_cast<uint32_t>(R) + 1, L.wsum);
    // keys and input indices in home order
 #pragma unroll
-   for (int k = 0; k < kRegionIPT; ++k) {
+   for (int k = 0; k < IPT; ++k) {
       const uint32_t e = threadIdx.x + k * kRegionBS;
-      if (e < m) {
+      if (has(k)) {
          const uint32_t pos = L.u2.c.cnt[uu[k]] + sub[k];
          L.key[pos] = kk[k];
          L.order[pos] = static_cast<uint16_t>(e);
@@ -679,9 +694,9 @@ __device__ uint32_t region_sort(const Slot<K>* S, uint64_t lo, uint32_t m, int s
    uint32_t dupm = 0; // bit k: key k is dropped
    int repeats = 0;
 #pragma unroll
-   for (int k = 0; k < kRegionIPT; ++k) {
+   for (int k = 0; k < IPT; ++k) {
       const uint32_t e = threadIdx.x + k * kRegionBS;
-      if (e < m) {
+      if (has(k)) {
          const uint32_t j0 = L.u2.c.cnt[uu[k]], j1 = L.u2.c.cnt[uu[k] + 1];
          int32_t rank = 0;
          for (uint32_t j = j0; j < j1; ++j) {
@@ -700,23 +715,23 @@ __device__ uint32_t region_sort(const Slot<K>* S, uint64_t lo, uint32_t m, int s
    if (!__syncthreads_or(repeats)) {
       ms = m;
 #pragma unroll
-      for (int k = 0; k < kRegionIPT; ++k)
+      for (int k = 0; k < IPT; ++k)
          if (ff[k] >= 0) ff[k] += static_cast<int32_t>(L.u2.c.cnt[uu[k]]);
    } else {
       for (uint32_t i = threadIdx.x; i <= R; i += kRegionBS) L.u2.c.scnt[i] = 0;
 #pragma unroll
-      for (int k = 0; k < kRegionIPT; ++k) {
+      for (int k = 0; k < IPT; ++k) {
          const uint32_t e = threadIdx.x + k * kRegionBS;
-         if (e < m) L.u1.dup[e] = (dupm >> k) & 1u;
+         if (has(k)) L.u1.dup[e] = (dupm >> k) & 1u;
       }
       __syncthreads();
 #pragma unroll
-      for (int k = 0; k < kRegionIPT; ++k)
+      for (int k = 0; k < IPT; ++k)
          if (ff[k] >= 0 && !((dupm >> k) & 1u)) atomicAdd(&L.u2.c.scnt[uu[k]], 1u);
       __syncthreads();
       ms = lds_exclusive_scan<kRegionBS>(L.u2.c.scnt, static_cast<uint32_t>(R) + 1, L.wsum);
 #pragma unroll
-      for (int k = 0; k < kRegionIPT; ++k) {
+      for (int k = 0; k < IPT; ++k) {
          if (ff[k] < 0) continue;
          if ((dupm >> k) & 1u) {
             ff[k] = -1;
@@ -730,17 +745,17 @@ __device__ uint32_t region_sort(const Slot<K>* S, uint64_t lo, uint32_t m, int s
    }
    __syncthreads(); // count tables dead from here; v takes their place
 #pragma unroll
-   for (int k = 0; k < kRegionIPT; ++k)
+   for (int k = 0; k < IPT; ++k)
       if (ff[k] >= 0) L.u2.v[ff[k]] = static_cast<int32_t>(uu[k]) - ff[k];
    __syncthreads();
    return ms;
 }
 
-template <typename K>
-__device__ RegionSum region_summary(RegionLds<K>& L, uint32_t ms, uint64_t R, const int32_t* ff) {
+template <typename K, int IPT>
+__device__ RegionSum region_summary(RegionLds<K, IPT>& L, uint32_t ms, uint64_t R, const int32_t* ff) {
    int32_t M = INT32_MIN;
 #pragma unroll
-   for (int k = 0; k < kRegionIPT; ++k)
+   for (int k = 0; k < IPT; ++k)
       if (ff[k] >= 0) M = std::max(M, L.u2.v[ff[k]]);
    M = wave_max(M);
    if (__lane_id() == 0) L.wmax[threadIdx.x / kWave] = M;
@@ -759,8 +774,8 @@ __device__ RegionSum region_summary(RegionLds<K>& L, uint32_t ms, uint64_t R, co
 // and write the span [c, max(R, last p + 1)) of slots (keys and EMPTY) at
 // base + offset.  `keep` picks by unwrapped position: 0 = below N only, 1 =
 // all, 2 = N and above only.  Returns this thread's longest probe.
-template <typename K>
-__device__ uint32_t region_place(RegionLds<K>& L, uint32_t ms, int64_t c, uint64_t base, int sp, uint64_t R,
+template <typename K, int IPT>
+__device__ uint32_t region_place(RegionLds<K, IPT>& L, uint32_t ms, int64_t c, uint64_t base, int sp, uint64_t R,
                                  int keep, const K* kk, const K* vv, const uint32_t* uu, const int32_t* ff,
                                  Slot<K>* b) {
    const int lane = __lane_id(), wave = threadIdx.x / kWave;
@@ -796,7 +811,7 @@ __device__ uint32_t region_place(RegionLds<K>& L, uint32_t ms, int64_t c, uint64
    auto kept = [&](uint64_t pos) { return keep == 1 || (keep == 0 ? pos < N : pos >= N); };
    uint32_t probe = 0;
 #pragma unroll
-   for (int k = 0; k < kRegionIPT; ++k) {
+   for (int k = 0; k < IPT; ++k) {
       if (ff[k] >= 0) {
          const int64_t p = ff[k] + std::max<int64_t>(L.u2.v[ff[k]], c);
          const int64_t q = p - c;
@@ -826,8 +841,8 @@ __device__ uint32_t region_place(RegionLds<K>& L, uint32_t ms, int64_t c, uint64
    return probe;
 }
 
-template <typename K>
-__device__ void probe_to_header(RegionLds<K>& L, uint32_t probe, BuildHeader* h) {
+template <typename K, int IPT>
+__device__ void probe_to_header(RegionLds<K, IPT>& L, uint32_t probe, BuildHeader* h) {
    probe = wave_max(probe);
    __syncthreads();
    if (__lane_id() == 0) L.wmax[threadIdx.x / kWave] = static_cast<int32_t>(probe);
@@ -868,7 +883,7 @@ template <typename K>
 __global__ __launch_bounds__(kRegionBS) __attribute__((amdgpu_waves_per_eu(4))) void k_region_build(
     const Slot<K>* S, const uint64_t* start, RegionLB lb, Slot<K>* b, int sp, int rlog, uint64_t NR, uint32_t chunk,
     BuildHeader* h) {
-   __shared__ RegionLds<K> L;
+   __shared__ RegionLds<K, kRegionIPT> L;
    if (!h->go) return;
    const uint64_t R = 1ull << rlog;
    const int64_t Ri = static_cast<int64_t>(R);
@@ -898,8 +913,9 @@ __global__ __launch_bounds__(kRegionBS) __attribute__((amdgpu_waves_per_eu(4))) 
       // region taken with no carry in: exact unless a spill crosses it whole.
       const uint64_t lo = start[r0 - 1], m = start[r0] - lo;
       if (m <= static_cast<uint64_t>(kRegionCap)) {
-         const uint32_t ms = region_sort<K>(S, lo, static_cast<uint32_t>(m), sp, R, L, kk, vv, uu, ff);
-         const RegionSum g = region_summary<K>(L, ms, R, ff);
+         region_pairs<K>(S, lo, static_cast<uint32_t>(m), sp, R, kk, vv, uu);
+         const uint32_t ms = region_sort(R, L, in_first(static_cast<uint32_t>(m)), kk, uu, ff);
+         const RegionSum g = region_summary(L, ms, R, ff);
          c = std::max(g.a, g.b);
       }
    }
@@ -914,9 +930,10 @@ __global__ __launch_bounds__(kRegionBS) __attribute__((amdgpu_waves_per_eu(4))) 
          kk[k] = nk[k];
          vv[k] = nv[k];
       }
-      const uint32_t ms = region_sort<K, true>(S, lo, static_cast<uint32_t>(m), sp, R, L, kk, vv, uu, ff);
+      region_pairs<K, true>(S, lo, static_cast<uint32_t>(m), sp, R, kk, vv, uu);
+      const uint32_t ms = region_sort(R, L, in_first(static_cast<uint32_t>(m)), kk, uu, ff);
       if (r + 1 < r1) prefetch(r + 1);
-      probe = std::max(probe, region_place<K>(L, ms, c, r * R, sp, R, 0, kk, vv, uu, ff, b));
+      probe = std::max(probe, region_place(L, ms, c, r * R, sp, R, 0, kk, vv, uu, ff, b));
       // The region's summary from the prefix max the placement left in v:
       // v[ms - 1] = max over its keys of (home offset - sorted index).
       RegionSum g;
@@ -928,7 +945,7 @@ __global__ __launch_bounds__(kRegionBS) __attribute__((amdgpu_waves_per_eu(4))) 
       }
       c = std::max(g.a, c + g.b);
    }
-   probe_to_header<K>(L, probe, h);
+   probe_to_header(L, probe, h);
 }
 
 // True carries.  The carry into region 0 is the least fixed point of the
@@ -996,6 +1013,7 @@ __global__ __launch_bounds__(1024) void k_carry_top(RegionSum* blk, uint64_t nbl
    if (threadIdx.x == 0) {
       h->c0 = c0;
       h->n_distinct = static_cast<uint64_t>(T.b + static_cast<int64_t>(N));
+      if (T.b >= 0) h->fail = 1; // a merge's union would fill the table: there is no carry to place it with
    }
 }
 
@@ -1088,7 +1106,9 @@ __global__ __launch_bounds__(1024) void k_carry_small(RegionLB lb, uint64_t NR, 
    if (threadIdx.x == 0) {
       h->c0 = c0;
       h->n_distinct = static_cast<uint64_t>(T.b + static_cast<int64_t>(N));
+      if (T.b >= 0) h->fail = 1; // as in k_carry_top
    }
+   if (T.b >= 0) return;
    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
    __syncthreads();
    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -1119,7 +1139,7 @@ __device__ void build_fallback_prep(Slot<K>* b, uint64_t N, hn_info* info, Build
 template <typename K>
 __global__ __launch_bounds__(kRegionBS) void k_region_fix(const Slot<K>* S, const uint64_t* start, RegionLB lb,
                                                          Slot<K>* b, int sp, int rlog, hn_info* info, BuildHeader* h) {
-   __shared__ RegionLds<K> L;
+   __shared__ RegionLds<K, kRegionIPT> L;
    if (!h->go) return;
    if (h->fail) {
       build_fallback_prep<K>(b, 1ull << sp, info, h);
@@ -1134,24 +1154,28 @@ __global__ __launch_bounds__(kRegionBS) void k_region_fix(const Slot<K>* S, cons
    for (uint32_t i = blockIdx.x; i < nfix; i += gridDim.x) {
       const uint32_t r = lb.list[i];
       const uint64_t lo = start[r];
-      const uint32_t ms = region_sort<K>(S, lo, static_cast<uint32_t>(start[r + 1] - lo), sp, R, L, kk, vv, uu, ff);
-      probe = std::max(probe, region_place<K>(L, ms, lb.carry[r], static_cast<uint64_t>(r) * R, sp, R, 1, kk, vv,
+      const uint32_t m = static_cast<uint32_t>(start[r + 1] - lo);
+      region_pairs<K>(S, lo, m, sp, R, kk, vv, uu);
+      const uint32_t ms = region_sort(R, L, in_first(m), kk, uu, ff);
+      probe = std::max(probe, region_place(L, ms, lb.carry[r], static_cast<uint64_t>(r) * R, sp, R, 1, kk, vv,
                                               uu, ff, b));
    }
-   probe_to_header<K>(L, probe, h);
+   probe_to_header(L, probe, h);
 }
 
 // Finish the Info.  Not run (go = 0): an empty-table build reports
-// err = INVALID with the table untouched.  Placed: fill, overflow of the layout, ordered.  Fallback: the
-// insert has set fill and overflow.
+// err = INVALID with the table untouched (so does a merge whose size power is
+// not the table's).  Placed: fill, overflow of the layout, ordered.
+// Fallback: the insert has set fill and overflow; a merge's keeps the old
+// table's TOMBSTONEs.
 __global__ void k_build_end(hn_info* info, const BuildHeader* h, int mode) {
    if (threadIdx.x != 0) return;
    if (!h->go) {
-      if (mode == BUILD_EMPTY) info->err = HN_STATUS_INVALID;
+      if (mode != BUILD_REHASH) info->err = HN_STATUS_INVALID;
       return;
    }
    info->reserved0 = 0;
-   info->tombstone_counter = 0;
+   if (!(mode == BUILD_MERGE && h->fail)) info->tombstone_counter = 0;
    if (h->fail) {
       info->err = h->fb_fail ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
       info->reserved1 = 0;
@@ -1234,6 +1258,16 @@ template <typename K>
 int launch_insert_pairs_dlen(const Slot<K>* pairs, Slot<K>* buckets, hn_info* info, uint64_t max_len,
                              const uint64_t* d_len, int32_t* fail_sink, hipStream_t s);
 
+inline RegionLB region_lb(const BuildPlan& P, char* base) {
+   RegionLB lb;
+   lb.word = reinterpret_cast<uint64_t*>(base + P.off_word);
+   lb.spec = reinterpret_cast<int64_t*>(base + P.off_spec);
+   lb.carry = reinterpret_cast<int64_t*>(base + P.off_carry);
+   lb.mark = reinterpret_cast<uint32_t*>(base + P.off_mark);
+   lb.list = reinterpret_cast<uint32_t*>(base + P.off_list);
+   return lb;
+}
+
 // The partition passes and the region starts: the input pairs end in S,
 // stably partitioned by region, with start[r] the first of region r.  src0
 // picks the first pass's input kind; n_in is its element count (the old
@@ -1252,12 +1286,7 @@ int partition_regions(const BuildPlan& P, int mode, const hn_info* info, int src
    const size_t scan_bytes = P.off_start - P.off_scan;
    uint64_t* start = reinterpret_cast<uint64_t*>(base + P.off_start);
    uint8_t* dig = reinterpret_cast<uint8_t*>(base + P.off_dig);
-   RegionLB lb;
-   lb.word = reinterpret_cast<uint64_t*>(base + P.off_word);
-   lb.spec = reinterpret_cast<int64_t*>(base + P.off_spec);
-   lb.carry = reinterpret_cast<int64_t*>(base + P.off_carry);
-   lb.mark = reinterpret_cast<uint32_t*>(base + P.off_mark);
-   lb.list = reinterpret_cast<uint32_t*>(base + P.off_list);
+   const RegionLB lb = region_lb(P, base);
    BuildBegin bg{};
    if (mode == BUILD_REHASH)
       hipLaunchKernelGGL(k_build_begin, dim3(1), dim3(64), 0, s, info, h, P.sp, mode);
@@ -1300,28 +1329,8 @@ int partition_regions(const BuildPlan& P, int mode, const hn_info* info, int src
    return static_cast<int>(hipGetLastError());
 }
 
-// Everything after the first partition pass's input is chosen (see
-// partition_regions for src0 and n_in).
-template <typename K>
-int build_core(const BuildPlan& P, int mode, int src0, PartIn<K> in0, uint64_t n_in, void* buckets, hn_info* info,
-               void* scratch, hipStream_t s) {
-   char* base = static_cast<char*>(scratch);
-   BuildHeader* h = reinterpret_cast<BuildHeader*>(base);
-   Slot<K>* S = reinterpret_cast<Slot<K>*>(base + P.off_pairs);
-   uint64_t* start = reinterpret_cast<uint64_t*>(base + P.off_start);
-   RegionLB lb;
-   lb.word = reinterpret_cast<uint64_t*>(base + P.off_word);
-   lb.spec = reinterpret_cast<int64_t*>(base + P.off_spec);
-   lb.carry = reinterpret_cast<int64_t*>(base + P.off_carry);
-   lb.mark = reinterpret_cast<uint32_t*>(base + P.off_mark);
-   lb.list = reinterpret_cast<uint32_t*>(base + P.off_list);
-   Slot<K>* T = static_cast<Slot<K>*>(buckets);
-
-   int rc = partition_regions<K>(P, mode, info, src0, in0, n_in, T, scratch, s);
-   if (rc) return rc;
-   const uint32_t chunk = region_chunk(P.NR);
-   hipLaunchKernelGGL(k_region_build<K>, dim3(static_cast<uint32_t>((P.NR + chunk - 1) / chunk)), dim3(kRegionBS), 0,
-                      s, S, start, lb, T, P.sp, P.rlog, P.NR, chunk, h);
+// True carries, and the regions to place again.
+inline void launch_carry(const BuildPlan& P, RegionLB lb, char* base, BuildHeader* h, hipStream_t s) {
    RegionSum* blk = reinterpret_cast<RegionSum*>(base + P.off_blk);
    const uint64_t nblk = (P.NR + kCarryTile - 1) / kCarryTile;
    const int64_t Ri = static_cast<int64_t>(P.R), Ni = static_cast<int64_t>(P.N);
@@ -1333,6 +1342,26 @@ int build_core(const BuildPlan& P, int mode, int src0, PartIn<K> in0, uint64_t n
       hipLaunchKernelGGL(k_carry_apply, dim3(static_cast<uint32_t>(nblk)), dim3(kCarryBS), 0, s, lb, blk, P.NR, Ri, h);
       hipLaunchKernelGGL(k_carry_mark, dim3(stream_blocks(P.NR, 256)), dim3(256), 0, s, lb, P.NR, Ri, Ni, h);
    }
+}
+
+// Everything after the first partition pass's input is chosen (see
+// partition_regions for src0 and n_in).
+template <typename K>
+int build_core(const BuildPlan& P, int mode, int src0, PartIn<K> in0, uint64_t n_in, void* buckets, hn_info* info,
+               void* scratch, hipStream_t s) {
+   char* base = static_cast<char*>(scratch);
+   BuildHeader* h = reinterpret_cast<BuildHeader*>(base);
+   Slot<K>* S = reinterpret_cast<Slot<K>*>(base + P.off_pairs);
+   uint64_t* start = reinterpret_cast<uint64_t*>(base + P.off_start);
+   const RegionLB lb = region_lb(P, base);
+   Slot<K>* T = static_cast<Slot<K>*>(buckets);
+
+   int rc = partition_regions<K>(P, mode, info, src0, in0, n_in, T, scratch, s);
+   if (rc) return rc;
+   const uint32_t chunk = region_chunk(P.NR);
+   hipLaunchKernelGGL(k_region_build<K>, dim3(static_cast<uint32_t>((P.NR + chunk - 1) / chunk)), dim3(kRegionBS), 0,
+                      s, S, start, lb, T, P.sp, P.rlog, P.NR, chunk, h);
+   launch_carry(P, lb, base, h, s);
    const uint32_t gfix = static_cast<uint32_t>(std::min<uint64_t>(P.NR, static_cast<uint64_t>(cu_count()) * 2));
    hipLaunchKernelGGL(k_region_fix<K>, dim3(gfix), dim3(kRegionBS), 0, s, S, start, lb, T, P.sp, P.rlog, info, h);
    rc = launch_insert_pairs_dlen<K>(S, T, info, P.n, &h->fb_len, &h->fb_fail, s);
@@ -1407,95 +1436,36 @@ int rehash_build(const void* old_b, int old_sp, void* new_b, int new_sp, hn_info
 // slot, and the keys whose home lies in region r fill one run of slots
 // [s_r, s_{r+1}): s_r is the first slot at or after rR that is EMPTY or holds
 // a key whose home is at or after rR (k_merge_bounds).  The new pairs take
-// the build's partition passes.  Then one workgroup per region, in ticket
-// order (k_merge_region), loads both, sorts the union by (home offset, key)
-// with a home histogram in LDS, keeps only the newest copy of a key (old
-// before new, new in batch order: an insert of a present key overwrites its
-// value, a key repeated in the batch keeps its last value) and places it:
-// p_j = j + max(v_j, carry), v the prefix max of (home offset - j) and carry
-// the slots the earlier regions spill into this one, passed along by a
-// decoupled look-back over the maps x -> max(A, x + C) (a region: A the
-// position of its last key with no carry, C its key count).  A region
-// writes its span [carry, max(R, last + 1)) of the output, keys and EMPTY
-// slots, so the spans tile the table, and positions past the end wrap into
-// region 0's carry-in slots, which region 0 does not write.  Region 0's
-// carry comes from that wrap, known only at the end, so region 0 is parked in
-// scratch and placed by k_merge_end.  When the table has TOMBSTONEs or no
-// order flag, a region exceeds its LDS capacity (3,072 old slots or 1,536 new
-// pairs), the old table is not in order after all (a key outside its
-// region's run), the wrap would change what region 0 spills into region 1,
-// or the union would fill the table, the output is made the other way, on
-// the device: the old table copied, then the probing insert of the
-// partitioned batch (the partition keeps the batch order of equal keys), so
-// the output is hn_insert_*'s result and the order flag is cleared.
-constexpr int kMergeBS = 512;
+// the build's partition passes.  Then the build's walk over regions, its
+// carries and its second placement, with a region's keys taken from both: the
+// old run first, the new pairs in batch order behind it, so that the last
+// copy of a key, which the sort keeps, is the newest (an insert of a present
+// key overwrites its value, a key repeated in the batch keeps its last
+// value).  When the table has TOMBSTONEs or no order flag, a region exceeds
+// its capacity (2,560 old slots or 1,536 new pairs), the old table is not in
+// order after all (a key outside its region's run), or the union would fill
+// the table, the output is made the other way, on the device: the old table
+// copied, then the probing insert of the partitioned batch (the partition
+// keeps the batch order of equal keys), so the output is hn_insert_*'s result
+// and the order flag is cleared.
+//
 // 2,560 old slots per 2,048-slot region: a region's run is its 2,048 slots
 // plus the difference of the spills across its two ends (tens of slots at
-// load factor 0.9); a run longer than that sends the call to the fallback.
-// Six per thread (3,072) cost 11 spilled VGPRs and took 8.99 ms instead of
-// 8.50 ms for 120 M keys into a half-full 2^28 table.
-constexpr int kMergeEO = 5; // old slots per thread
-constexpr int kMergeEN = 3; // new pairs per thread
-constexpr uint32_t kMergeCapO = kMergeBS * kMergeEO;
-constexpr uint32_t kMergeCapN = kMergeBS * kMergeEN;
-constexpr uint32_t kMergeCap = kMergeCapO + kMergeCapN;
-constexpr uint32_t kMergeSpanWords = (kRegionMax + kMergeCap + 31) / 32;
-constexpr uint32_t kMgBias = 1u << 16; // keeps home offset - sorted index non-negative
-static_assert(kMergeCap < 0x8000, "element ids leave the top bit of a 16-bit order entry free");
+// load factor 0.9).
+constexpr uint32_t kMergeCapO = 2560, kMergeCapN = 1536;
+constexpr uint32_t kAbsent = 0xFFFFFFFFu;
+constexpr int kMergeIPT = static_cast<int>((kMergeCapO + kMergeCapN) / kRegionBS);
 
-struct MergeHeader {
-   uint32_t ticket;     // next region
-   uint32_t fail;       // a region gave up, or a bound was not found
-   uint32_t max_probe;  // longest probe of the keys placed by the regions
-   uint32_t n0;         // keys of region 0, parked
-   uint32_t ineligible; // TOMBSTONEs or no order flag: the regions do not run
-   int32_t fb_fail;     // the fallback insert found no slot for a key
-   uint64_t fb_len;     // pairs the fallback insert takes (0: the merge stands)
-   uint32_t pad[56];
-};
-static_assert(sizeof(MergeHeader) == 256, "header is one 256-byte line");
-
-// A parked key of region 0: its prefix-max term and home offset.
+// sb[r] = s_r (unwrapped, < rR + kMergeCapO), sb[NR] = N + s_0.  One wave per
+// region.
 template <typename K>
-struct MergePark {
-   K key, val;
-   int32_t v;
-   uint32_t hr;
-};
-
-// Region state for the look-back: 2 state bits, A + 1 and C in 31 bits each
-// (table size power at most 30).
-constexpr uint64_t kMgAgg = 1ull << 62, kMgInc = 2ull << 62;
-__device__ __forceinline__ uint64_t mg_pack(uint64_t st, RegionSum g) {
-   return st | (static_cast<uint64_t>(g.a + 1) << 31) | static_cast<uint64_t>(g.b);
-}
-__device__ __forceinline__ RegionSum mg_unpack(uint64_t w) {
-   RegionSum g;
-   g.a = static_cast<int64_t>((w >> 31) & 0x7FFFFFFFull) - 1;
-   g.b = static_cast<int64_t>(w & 0x7FFFFFFFull);
-   return g;
-}
-// No keys: (A, C) = (-1, 0) acts as the identity for region maps (A >= C - 1).
-constexpr RegionSum kMgNone = {-1, 0};
-
-__global__ void k_merge_begin(const hn_info* info, MergeHeader* mh) {
-   if (threadIdx.x == 0) {
-      mh->ticket = 0;
-      mh->fail = 0;
-      mh->max_probe = 0;
-      mh->n0 = 0;
-      mh->ineligible = (info->tombstone_counter != 0 || !(info->reserved1 & kInfoOrdered)) ? 1u : 0u;
-      mh->fb_fail = 0;
-      mh->fb_len = 0;
+__global__ __launch_bounds__(256) void k_merge_bounds(const Slot<K>* ob, const hn_info* info, int sp, int rlog,
+                                                      uint64_t NR, uint64_t* sb, BuildHeader* h) {
+   if (!h->go) return;
+   if (info->tombstone_counter != 0 || !(info->reserved1 & kInfoOrdered)) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) h->fail = 1;
+      return;
    }
-}
-
-// sb[r] = s_r (unwrapped, < rR + kMergeCapO), sb[NR] = N + s_0; clears the
-// region states.  One wave per region.
-template <typename K>
-__global__ __launch_bounds__(256) void k_merge_bounds(const Slot<K>* ob, int sp, int rlog, uint64_t NR, uint64_t* sb,
-                                                      uint64_t* status, MergeHeader* mh, const BuildHeader* h) {
-   if (!h->go || mh->ineligible) return;
    const int lane = __lane_id();
    const uint64_t N = 1ull << sp, mask = N - 1;
    const uint64_t waves = static_cast<uint64_t>(gridDim.x) * (blockDim.x / kWave);
@@ -1519,445 +1489,171 @@ __global__ __launch_bounds__(256) void k_merge_bounds(const Slot<K>* ob, int sp,
       }
       if (lane == 0) {
          if (found < 0) {
-            __hip_atomic_store(&mh->fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&h->fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             found = lo;
          }
          sb[r] = static_cast<uint64_t>(found);
          if (r == 0) sb[NR] = N + static_cast<uint64_t>(found);
-         status[r] = 0;
       }
    }
 }
 
-// Inclusive prefix max of x[0, m) in place by the whole workgroup.
-template <int BS>
-__device__ void lds_incl_max16(int16_t* x, uint32_t m, int32_t* wmax) {
-   const int lane = __lane_id(), wave = threadIdx.x / kWave;
-   const uint32_t per = (m + BS - 1) / BS;
-   const uint32_t c0 = std::min<uint32_t>(threadIdx.x * per, m), c1 = std::min<uint32_t>(c0 + per, m);
-   int32_t acc = INT32_MIN;
-   for (uint32_t i = c0; i < c1; ++i) acc = std::max<int32_t>(acc, x[i]);
-   int32_t inc = acc;
-#pragma unroll
-   for (int o = 1; o < kWave; o <<= 1) {
-      const int32_t y = __shfl_up(inc, o, kWave);
-      if (lane >= o) inc = std::max(inc, y);
-   }
-   if (lane == kWave - 1) wmax[wave] = inc;
-   __syncthreads();
-   int32_t run = __shfl_up(inc, 1, kWave);
-   if (lane == 0) run = INT32_MIN;
-   for (int w = 0; w < wave; ++w) run = std::max(run, wmax[w]);
-   for (uint32_t i = c0; i < c1; ++i) {
-      run = std::max<int32_t>(run, x[i]);
-      x[i] = static_cast<int16_t>(run);
-   }
-   __syncthreads();
-}
-
+// A region's two inputs: Lo old slots from o0 (EMPTY ones among them), then
+// Ln new pairs from n0.  Element e < Lo + Ln.
 template <typename K>
-struct MergeLds {
-   K key[kMergeCap];        // by element id: old slot offset, or kMergeCapO + new index
-   uint16_t order[kMergeCap]; // ids by home offset (top bit: a dropped copy)
-   int16_t v[kMergeCap];    // prefix-max terms by sorted index
-   uint32_t cnt[kRegionMax + 1];
-   // With repeats: the group starts over all copies, kept for the re-ranking
-   // of the survivors (in LDS rather than per-element registers: with them in
-   // registers the u64 kernel spilled 28 VGPRs and merged 10.18 ms, not 8.99).
-   uint32_t cnt0[kRegionMax + 1];
-   uint32_t occ[kMergeSpanWords];
-   uint32_t wsum[kMergeBS / kWave];
-   int32_t wmax[kMergeBS / kWave];
-   uint32_t wa[kMergeBS / kWave];  // per wave: max of (home offset - sorted index) + kMgBias
-   int64_t lb_a[kMergeBS / kWave]; // look-back: each wave's composed window
-   int64_t lb_b[kMergeBS / kWave];
-   int32_t lb_inc[kMergeBS / kWave];
-   uint32_t ticket;
-   uint32_t probe;
-   int64_t xin;
+struct MergeRegion {
+   uint64_t o0, n0;
+   uint32_t Lo, m; // m = Lo + Ln; both 0 when the region is over capacity
+   bool fits;
+   __device__ MergeRegion(const uint64_t* sb, const uint64_t* start, uint64_t r) : o0(sb[r]), n0(start[r]) {
+      const uint64_t lo = sb[r + 1] - o0, ln = start[r + 1] - n0;
+      fits = lo <= kMergeCapO && ln <= kMergeCapN;
+      Lo = fits ? static_cast<uint32_t>(lo) : 0;
+      m = fits ? static_cast<uint32_t>(lo + ln) : 0;
+   }
+   // Thread t owns elements t + k * kRegionBS: their keys, and their values.
+   __device__ __forceinline__ void keys(const Slot<K>* ob, const Slot<K>* S, uint64_t mask, K* kk) const {
+#pragma unroll
+      for (int k = 0; k < kMergeIPT; ++k) {
+         const uint32_t e = threadIdx.x + k * kRegionBS;
+         if (e < m) kk[k] = e < Lo ? ob[(o0 + e) & mask].key : S[n0 + (e - Lo)].key;
+      }
+   }
+   __device__ __forceinline__ void vals(const Slot<K>* ob, const Slot<K>* S, uint64_t mask, K* vv) const {
+#pragma unroll
+      for (int k = 0; k < kMergeIPT; ++k) {
+         const uint32_t e = threadIdx.x + k * kRegionBS;
+         if (e < m) vv[k] = e < Lo ? ob[(o0 + e) & mask].val : S[n0 + (e - Lo)].val;
+      }
+   }
+   // Home offsets of the loaded keys; false in a thread whose old key does
+   // not belong to the region.
+   __device__ __forceinline__ bool homes(const K* kk, uint64_t rb, int sp, uint64_t R, uint32_t* uu) const {
+      const uint64_t mask = (1ull << sp) - 1;
+      bool ok = true;
+#pragma unroll
+      for (int k = 0; k < kMergeIPT; ++k) {
+         const uint32_t e = threadIdx.x + k * kRegionBS;
+         uu[k] = kAbsent;
+         if (e < m && (e >= Lo || kk[k] != empty_key<K>())) {
+            const uint64_t hr = (fib_home(kk[k], sp) - rb) & mask;
+            if (hr >= R || (e < Lo && kk[k] == tomb_key<K>()))
+               ok = false;
+            else
+               uu[k] = static_cast<uint32_t>(hr);
+         }
+      }
+      return ok;
+   }
 };
 
-// Rank of one element in its home group order[g0, g1): keys below it, and
-// whether a newer copy of its key (a larger id) drops it.
+// k_region_build over both inputs.  Only the next region's keys are held in
+// registers ahead (with the values the u64 kernel spilled 88 VGPRs); the values
+// come from L2, where the keys' lines already are.  A workgroup per region in
+// ticket order, each waiting for its carry by a look-back over the regions in
+// flight, took 20.7 us a region where the walk takes 11: 2^24 keys into 2^26
+// u64 slots up to load .9 the whole merge 1.71 -> 1.36 ms, 2^22 up to load .5
+// 1.31 -> 0.96, u32 1.42 -> 1.12 and 1.13 -> 0.84.
 template <typename K>
-__device__ __forceinline__ uint32_t merge_rank(const MergeLds<K>& L, uint32_t id, uint32_t g0, uint32_t g1, bool& drop,
-                                               bool& rep) {
-   const K key = L.key[id];
-   uint32_t rank = 0;
-   for (uint32_t k = g0; k < g1; ++k) {
-      const uint32_t id2 = L.order[k];
-      const K k2 = L.key[id2];
-      rank += k2 < key ? 1u : 0u;
-      if (k2 == key && id2 != id) {
-         rep = true;
-         drop = drop || id2 > id;
-      }
-   }
-   return rank;
-}
-// The same over the copies that stay (dropped ones carry the top bit).
-template <typename K>
-__device__ __forceinline__ uint32_t merge_rank_kept(const MergeLds<K>& L, uint32_t id, uint32_t g0, uint32_t g1) {
-   const K key = L.key[id];
-   uint32_t rank = 0;
-   for (uint32_t k = g0; k < g1; ++k) {
-      const uint32_t e = L.order[k];
-      if (!(e & 0x8000u)) rank += L.key[e] < key ? 1u : 0u;
-   }
-   return rank;
-}
-
-// A thread holds kMergeEO old slots (ids threadIdx.x + e * kMergeBS) and
-// kMergeEN new pairs (ids kMergeCapO + threadIdx.x + e * kMergeBS); element
-// state is packed to keep registers low: hs = home offset << 16 | arrival
-// rank within the home (kNoElem: no element), g = group start | end << 16,
-// j = sorted index, one drop bit per element.  Keys stay in LDS; values are
-// read again from memory when written.
-constexpr int kMergeE = kMergeEO + kMergeEN;
-constexpr uint32_t kNoElem = 0xFFFFFFFFu;
-
-template <typename K>
-__global__ __launch_bounds__(kMergeBS) __attribute__((amdgpu_waves_per_eu(4))) void k_merge_region(const Slot<K>* ob, const Slot<K>* S, const uint64_t* start,
-                                                          const uint64_t* sb, uint64_t* status, Slot<K>* nb,
-                                                          MergePark<K>* park, MergeHeader* mh, const BuildHeader* h,
-                                                          int sp, int rlog, uint64_t NR) {
-   __shared__ MergeLds<K> L;
-   if (!h->go || mh->ineligible) return; // the same for every workgroup: no look-back waits on a skipped region
-   const uint64_t N = 1ull << sp, mask = N - 1, R = 1ull << rlog;
-   const int lane = __lane_id(), wave = threadIdx.x / kWave;
-   if (threadIdx.x == 0) L.probe = 0;
-   uint32_t max_probe = 0;
-   auto elem_id = [&](int e) -> uint32_t {
-      return e < kMergeEO ? threadIdx.x + e * kMergeBS : kMergeCapO + threadIdx.x + (e - kMergeEO) * kMergeBS;
-   };
-   for (;;) {
-      __syncthreads(); // LDS of the previous region is no longer read
-      if (threadIdx.x == 0) L.ticket = atomic_add_relaxed(&mh->ticket, 1u);
-      __syncthreads();
-      const uint64_t r = L.ticket;
-      if (r >= NR) break;
-      const uint64_t rb = r << rlog;
-      const uint64_t o0 = sb[r], n0 = start[r];
-      const uint64_t Lo = sb[r + 1] - o0, Ln = start[r + 1] - n0;
-      auto give_up = [&]() { // the call fails; successors still get a state
-         if (threadIdx.x == 0) {
-            __hip_atomic_store(&mh->fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&status[r], mg_pack(kMgInc, kMgNone), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-         }
-      };
-      if (Lo > kMergeCapO || Ln > kMergeCapN) {
-         give_up();
-         continue;
-      }
-      for (uint32_t i = threadIdx.x; i <= R; i += kMergeBS) L.cnt[i] = 0;
-      __syncthreads();
-      // the value of element e, read again at write time
-      auto value = [&](int e) -> K {
-         return e < kMergeEO ? ob[(o0 + threadIdx.x + e * kMergeBS) & mask].val
-                             : S[n0 + threadIdx.x + (e - kMergeEO) * kMergeBS].val;
-      };
-      uint32_t hs[kMergeE], jj[kMergeE];
-      bool bad = false;
-#pragma unroll
-      for (int e = 0; e < kMergeE; ++e) {
-         hs[e] = kNoElem;
-         const uint32_t x = e < kMergeEO ? threadIdx.x + e * kMergeBS : threadIdx.x + (e - kMergeEO) * kMergeBS;
-         if (e < kMergeEO ? x < Lo : x < Ln) {
-            const K key = e < kMergeEO ? ob[(o0 + x) & mask].key : S[n0 + x].key;
-            if (e >= kMergeEO || key != empty_key<K>()) {
-               const uint64_t hr = (fib_home(key, sp) - rb) & mask;
-               if (hr >= R || (e < kMergeEO && key == tomb_key<K>())) {
-                  bad = true;
-               } else {
-                  L.key[elem_id(e)] = key;
-                  hs[e] = static_cast<uint32_t>(hr << 16) | atomicAdd(&L.cnt[hr], 1u);
-               }
-            }
-         }
-      }
-      if (__syncthreads_or(bad)) {
-         give_up();
-         continue;
-      }
-      lds_exclusive_scan<kMergeBS>(L.cnt, static_cast<uint32_t>(R) + 1, L.wsum);
-#pragma unroll
-      for (int e = 0; e < kMergeE; ++e)
-         if (hs[e] != kNoElem) L.order[L.cnt[hs[e] >> 16] + (hs[e] & 0xFFFFu)] = static_cast<uint16_t>(elem_id(e));
-      __syncthreads();
-      // sorted index: group start + rank by key; a newer copy drops an element
-      uint32_t drop = 0;
-      bool rep = false;
-      uint32_t dmax = 0; // max of (home offset - sorted index) + kMgBias over this thread's elements
-#pragma unroll
-      for (int e = 0; e < kMergeE; ++e) {
-         if (hs[e] != kNoElem) {
-            const uint32_t g0 = L.cnt[hs[e] >> 16], g1 = L.cnt[(hs[e] >> 16) + 1];
-            bool d = false;
-            jj[e] = g0 + merge_rank(L, elem_id(e), g0, g1, d, rep);
-            drop |= d ? (1u << e) : 0u;
-            dmax = std::max<uint32_t>(dmax, (hs[e] >> 16) + kMgBias - jj[e]);
-         }
-      }
-      dmax = wave_max(dmax);
-      if (lane == 0) L.wa[wave] = dmax;
-      uint32_t ms;
-      bool published = false;
-      if (!__syncthreads_or(rep)) {
-         ms = L.cnt[R];
-         // Every element stays, so the region's map x -> max(A, x + C) is
-         // known now: C = ms, A = rb + ms - 1 + max(home offset - sorted
-         // index), the last key's position with no carry.  Published before
-         // the prefix max, it holds up the regions behind it for less time
-         // (10.34 -> 10.15 ms for 120 M keys into a half-full 2^28 table).
-         if (threadIdx.x == 0) {
-            RegionSum ea = kMgNone;
-            if (ms) {
-               uint32_t m = 0;
-               for (int w = 0; w < kMergeBS / kWave; ++w) m = std::max(m, L.wa[w]);
-               ea.a = static_cast<int64_t>(rb) + static_cast<int64_t>(ms - 1) + static_cast<int64_t>(m) - kMgBias;
-               ea.b = ms;
-            }
-            __hip_atomic_store(&status[r], mg_pack(r == 0 ? kMgInc : kMgAgg, ea), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-         }
-         published = true;
-      } else {
-         // mark the dropped copies, then count and rank the kept ones
-#pragma unroll
-         for (int e = 0; e < kMergeE; ++e)
-            if (hs[e] != kNoElem && ((drop >> e) & 1u)) L.order[L.cnt[hs[e] >> 16] + (hs[e] & 0xFFFFu)] |= 0x8000u;
-         for (uint32_t i = threadIdx.x; i <= R; i += kMergeBS) L.cnt0[i] = L.cnt[i];
-         __syncthreads();
-         for (uint32_t i = threadIdx.x; i <= R; i += kMergeBS) L.cnt[i] = 0;
-         __syncthreads();
-#pragma unroll
-         for (int e = 0; e < kMergeE; ++e)
-            if (hs[e] != kNoElem && !((drop >> e) & 1u)) atomicAdd(&L.cnt[hs[e] >> 16], 1u);
-         __syncthreads();
-         ms = lds_exclusive_scan<kMergeBS>(L.cnt, static_cast<uint32_t>(R) + 1, L.wsum);
-#pragma unroll
-         for (int e = 0; e < kMergeE; ++e)
-            if (hs[e] != kNoElem && !((drop >> e) & 1u))
-               jj[e] = L.cnt[hs[e] >> 16] +
-                       merge_rank_kept(L, elem_id(e), L.cnt0[hs[e] >> 16], L.cnt0[(hs[e] >> 16) + 1]);
-      }
-#pragma unroll
-      for (int e = 0; e < kMergeE; ++e)
-         if (hs[e] != kNoElem && !((drop >> e) & 1u))
-            L.v[jj[e]] = static_cast<int16_t>(static_cast<int32_t>(hs[e] >> 16) - static_cast<int32_t>(jj[e]));
-      __syncthreads();
-      lds_incl_max16<kMergeBS>(L.v, ms, L.wmax);
-      RegionSum agg = kMgNone;
-      if (ms) {
-         agg.a = static_cast<int64_t>(rb) + static_cast<int64_t>(ms - 1) + L.v[ms - 1];
-         agg.b = ms;
-      }
-      // look-back: the carry is the position of the last key of regions < r.
-      // Every wave reads 64 predecessors, so one round of loads covers the
-      // kMergeBS regions in flight (lane i of wave w: region top - 64w - i).
-      if (threadIdx.x == 0 && !published)
-         __hip_atomic_store(&status[r], mg_pack(r == 0 ? kMgInc : kMgAgg, agg), __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT);
-      RegionSum excl = kMgNone;
-      if (r > 0) {
-         int64_t top = static_cast<int64_t>(r) - 1;
-         for (;;) {
-            const int64_t q = top - static_cast<int64_t>(threadIdx.x);
-            uint64_t w = kMgInc;
-            if (q >= 0) w = __hip_atomic_load(&status[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            while (__ballot((w >> 62) == 0)) {
-               if ((w >> 62) == 0) w = __hip_atomic_load(&status[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            const uint64_t incm = __ballot((w >> 62) == 2);
-            const int k = incm ? first_bit(incm) : kWave - 1;
-            RegionSum gs = lane <= k ? mg_unpack(w) : kMgNone;
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1) { // lane i + d holds earlier regions than lane i
-               RegionSum y;
-               y.a = __shfl_down(gs.a, d, kWave);
-               y.b = __shfl_down(gs.b, d, kWave);
-               if (lane + d < kWave) gs = compose(y, gs);
-            }
-            if (lane == 0) {
-               L.lb_a[wave] = gs.a;
-               L.lb_b[wave] = gs.b;
-               L.lb_inc[wave] = incm ? 1 : 0;
-            }
-            __syncthreads();
-            // waves in order from the nearest; stop at the first holding an inclusive state
-            bool found = false;
-            RegionSum win = kMgNone;
-            for (int v = 0; v < kMergeBS / kWave && !found; ++v) {
-               RegionSum gv;
-               gv.a = L.lb_a[v];
-               gv.b = L.lb_b[v];
-               win = compose(gv, win);
-               found = L.lb_inc[v] != 0;
-            }
-            excl = compose(win, excl);
-            __syncthreads();
-            if (found) break;
-            top -= kMergeBS;
-         }
-         if (threadIdx.x == 0)
-            __hip_atomic_store(&status[r], mg_pack(kMgInc, compose(excl, agg)), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-      }
-      if (threadIdx.x == 0) L.xin = excl.a;
-      __syncthreads();
-      const int64_t carry = L.xin + 1 - static_cast<int64_t>(rb);
-      if (r == 0) { // parked until the wrap is known
-#pragma unroll
-         for (int e = 0; e < kMergeE; ++e)
-            if (hs[e] != kNoElem && !((drop >> e) & 1u))
-               park[jj[e]] = MergePark<K>{L.key[elem_id(e)], value(e), L.v[jj[e]], hs[e] >> 16};
-         if (threadIdx.x == 0) mh->n0 = ms;
-         continue;
-      }
-      const int64_t last = ms ? static_cast<int64_t>(ms - 1) + std::max<int64_t>(L.v[ms - 1], carry) : -1;
-      const int64_t c0 = std::max<int64_t>(carry, 0);
-      const int64_t span = std::max<int64_t>(static_cast<int64_t>(R), last + 1) - c0;
-      const int64_t words = span > 0 ? (span + 31) / 32 : 0;
-      for (int64_t w = threadIdx.x; w < words; w += kMergeBS) L.occ[w] = 0;
-      __syncthreads();
-#pragma unroll
-      for (int e = 0; e < kMergeE; ++e) {
-         if (hs[e] != kNoElem && !((drop >> e) & 1u)) {
-            const int64_t p = static_cast<int64_t>(jj[e]) + std::max<int64_t>(L.v[jj[e]], carry);
-            const int64_t q = p - c0;
-            atomicOr(&L.occ[q >> 5], 1u << (q & 31));
-            Slot<K> sl;
-            sl.key = L.key[elem_id(e)];
-            sl.val = value(e);
-            nb[(rb + static_cast<uint64_t>(p)) & mask] = sl;
-            max_probe = std::max<uint32_t>(max_probe, static_cast<uint32_t>(p - static_cast<int64_t>(hs[e] >> 16) + 1));
-         }
-      }
-      __syncthreads();
-      for (int64_t q = threadIdx.x; q < span; q += kMergeBS) {
-         if (!((L.occ[q >> 5] >> (q & 31)) & 1u)) {
-            Slot<K> sl;
-            sl.key = empty_key<K>();
-            sl.val = 0;
-            nb[(rb + static_cast<uint64_t>(c0 + q)) & mask] = sl;
-         }
-      }
-   }
-   max_probe = wave_max(max_probe);
-   if (lane == 0 && max_probe) atomicMax(&L.probe, max_probe);
-   __syncthreads();
-   if (threadIdx.x == 0 && L.probe > __hip_atomic_load(&mh->max_probe, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      atomic_max_relaxed(&mh->max_probe, L.probe);
-}
-
-// Region 0 with its carry from the wrap, then the Info; or, when the merge
-// does not stand, the fallback's length.  One workgroup.
-template <typename K>
-__global__ __launch_bounds__(kMergeBS) void k_merge_end(const MergePark<K>* park, const uint64_t* status, Slot<K>* nb,
-                                                       hn_info* info, MergeHeader* mh, const BuildHeader* h,
-                                                       int sp, int rlog, uint64_t NR) {
-   __shared__ uint32_t occ[kMergeSpanWords];
-   __shared__ uint32_t probe_s;
-   const uint64_t N = 1ull << sp, mask = N - 1, R = 1ull << rlog;
-   if (!h->go) { // a size power that is not the table's
-      if (threadIdx.x == 0) info->err = HN_STATUS_INVALID;
-      return;
-   }
-   bool fail = mh->ineligible || mh->fail;
-   const RegionSum tot = fail ? kMgNone : mg_unpack(status[NR - 1]);
-   fail = fail || tot.b >= static_cast<int64_t>(N);
-   const uint32_t n0 = fail ? 0 : mh->n0;
-   const int64_t c0 = std::max<int64_t>(tot.a + 1 - static_cast<int64_t>(N), 0); // slots the wrap fills in region 0
-   const int64_t vlast = n0 ? park[n0 - 1].v : 0;
-   const int64_t last = n0 ? static_cast<int64_t>(n0 - 1) + std::max<int64_t>(vlast, c0) : c0 - 1;
-   const int64_t spec = n0 ? static_cast<int64_t>(n0 - 1) + vlast : -1; // what region 1 was placed after
-   if (NR > 1 && std::max<int64_t>(last + 1 - static_cast<int64_t>(R), 0) !=
-                     std::max<int64_t>(spec + 1 - static_cast<int64_t>(R), 0))
-      fail = true;
-   if (fail) {
-      if (threadIdx.x == 0) mh->fb_len = h->n;
-      return;
-   }
-   const int64_t span = std::max<int64_t>(static_cast<int64_t>(R), last + 1) - c0;
-   for (int64_t w = threadIdx.x; w < (span + 31) / 32; w += kMergeBS) occ[w] = 0;
-   if (threadIdx.x == 0) probe_s = 0;
-   __syncthreads();
+__global__ __launch_bounds__(kRegionBS) __attribute__((amdgpu_waves_per_eu(4))) void k_merge_build(
+    const Slot<K>* ob, const uint64_t* sb, const Slot<K>* S, const uint64_t* start, RegionLB lb, Slot<K>* b, int sp,
+    int rlog, uint64_t NR, uint32_t chunk, BuildHeader* h) {
+   __shared__ RegionLds<K, kMergeIPT> L;
+   if (__syncthreads_or(!h->go || h->fail)) return; // a workgroup may see another's failure: all its threads do
+   const uint64_t R = 1ull << rlog, mask = (1ull << sp) - 1;
+   const int64_t Ri = static_cast<int64_t>(R);
+   const uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * chunk;
+   const uint64_t r1 = std::min<uint64_t>(r0 + chunk, NR);
+   K kk[kMergeIPT], vv[kMergeIPT];
+   K nk[kMergeIPT]; // the next region's keys, loaded while this one is placed; the values then come from L2
+   uint32_t uu[kMergeIPT];
+   int32_t ff[kMergeIPT];
    uint32_t probe = 0;
-   for (uint32_t j = threadIdx.x; j < n0; j += kMergeBS) {
-      const MergePark<K> e = park[j];
-      const int64_t p = static_cast<int64_t>(j) + std::max<int64_t>(e.v, c0);
-      const int64_t q = p - c0;
-      atomicOr(&occ[q >> 5], 1u << (q & 31));
-      Slot<K> sl;
-      sl.key = e.key;
-      sl.val = e.val;
-      nb[static_cast<uint64_t>(p) & mask] = sl;
-      probe = std::max<uint32_t>(probe, static_cast<uint32_t>(p - static_cast<int64_t>(e.hr) + 1));
-   }
-   __syncthreads();
-   for (int64_t q = threadIdx.x; q < span; q += kMergeBS) {
-      if (!((occ[q >> 5] >> (q & 31)) & 1u)) {
-         Slot<K> sl;
-         sl.key = empty_key<K>();
-         sl.val = 0;
-         nb[static_cast<uint64_t>(c0 + q) & mask] = sl;
+   int64_t c = 0;
+   if (r0 < r1) MergeRegion<K>(sb, start, r0).keys(ob, S, mask, nk);
+   if (r0 > 0) { // the carry out of the region before, as in k_region_build
+      const MergeRegion<K> g(sb, start, r0 - 1);
+      if (g.fits) {
+         g.keys(ob, S, mask, kk);
+         g.homes(kk, (r0 - 1) << rlog, sp, R, uu); // its own walk reports a key out of place
+         const uint32_t ms = region_sort(R, L, [&](int k) { return uu[k] != kAbsent; }, kk, uu, ff);
+         const RegionSum gs = region_summary(L, ms, R, ff);
+         c = std::max(gs.a, gs.b);
       }
    }
-   probe = wave_max(probe);
-   if (__lane_id() == 0 && probe) atomicMax(&probe_s, probe);
-   __syncthreads();
-   if (threadIdx.x == 0) {
-      const uint64_t mp = std::max<uint32_t>(probe_s, mh->max_probe);
-      info->fill = static_cast<uint64_t>(tot.b);
-      info->tombstone_counter = 0;
-      info->current_max_bucket_overflow = std::max<uint64_t>(kBucketOverflow, next_overflow(mp, kBucketOverflow));
-      info->reserved0 = 0;
-      info->reserved1 = kInfoOrdered;
-      info->err = HN_STATUS_SUCCESS;
+   for (uint64_t r = r0; r < r1; ++r) {
+      const MergeRegion<K> g(sb, start, r);
+#pragma unroll
+      for (int k = 0; k < kMergeIPT; ++k) kk[k] = nk[k];
+      g.vals(ob, S, mask, vv);
+      if (__syncthreads_or(!g.fits || !g.homes(kk, r << rlog, sp, R, uu))) { // abandon the merge
+         if (threadIdx.x == 0) __hip_atomic_store(&h->fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+         return;
+      }
+      const uint32_t ms = region_sort(R, L, [&](int k) { return uu[k] != kAbsent; }, kk, uu, ff);
+      if (r + 1 < r1) MergeRegion<K>(sb, start, r + 1).keys(ob, S, mask, nk);
+      probe = std::max(probe, region_place(L, ms, c, r * R, sp, R, 0, kk, vv, uu, ff, b));
+      RegionSum gs;
+      gs.b = static_cast<int64_t>(ms) - Ri;
+      gs.a = ms > 0 ? std::max<int64_t>(0, static_cast<int64_t>(ms) - Ri + L.u2.v[ms - 1]) : 0;
+      if (threadIdx.x == 0) {
+         lb.word[r] = pack_sum(gs, Ri);
+         lb.spec[r] = c;
+      }
+      c = std::max(gs.a, c + gs.b);
    }
+   probe_to_header(L, probe, h);
 }
 
-// Fallback: the old table into the output, then (the probing insert of the
-// partitioned batch runs between) err and the flags.
+// The listed regions again with their true carries; or, where the merge does
+// not stand, the old table copied for the probing insert of the batch.
 template <typename K>
-__global__ __launch_bounds__(256) void k_merge_copy(const Slot<K>* ob, Slot<K>* nb, uint64_t N, const MergeHeader* mh) {
-   if (!mh->fb_len) return;
-   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < N; i += stride) nb[i] = ob[i];
-}
-__global__ void k_merge_fin(hn_info* info, const MergeHeader* mh) {
-   if (threadIdx.x != 0 || !mh->fb_len) return;
-   info->err = mh->fb_fail ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
-   info->reserved0 = 0;
-   info->reserved1 = 0;
+__global__ __launch_bounds__(kRegionBS) void k_merge_fix(const Slot<K>* ob, const uint64_t* sb, const Slot<K>* S,
+                                                         const uint64_t* start, RegionLB lb, Slot<K>* b, int sp,
+                                                         int rlog, BuildHeader* h) {
+   __shared__ RegionLds<K, kMergeIPT> L;
+   if (!h->go) return;
+   const uint64_t R = 1ull << rlog, N = 1ull << sp;
+   if (h->fail) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) h->fb_len = h->n;
+      const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kRegionBS;
+      for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kRegionBS + threadIdx.x; i < N; i += stride) b[i] = ob[i];
+      return;
+   }
+   K kk[kMergeIPT], vv[kMergeIPT];
+   uint32_t uu[kMergeIPT];
+   int32_t ff[kMergeIPT];
+   uint32_t probe = 0;
+   const uint32_t nfix = h->n_fix;
+   for (uint32_t i = blockIdx.x; i < nfix; i += gridDim.x) {
+      const uint64_t r = lb.list[i];
+      const MergeRegion<K> g(sb, start, r);
+      g.keys(ob, S, N - 1, kk);
+      g.vals(ob, S, N - 1, vv);
+      g.homes(kk, r << rlog, sp, R, uu);
+      const uint32_t ms = region_sort(R, L, [&](int k) { return uu[k] != kAbsent; }, kk, uu, ff);
+      probe = std::max(probe, region_place(L, ms, lb.carry[r], r * R, sp, R, 1, kk, vv, uu, ff, b));
+   }
+   probe_to_header(L, probe, h);
 }
 
-template <typename K>
 struct MergePlan {
    BuildPlan P;
-   size_t off_mh, off_sb, off_status, off_park, total;
+   size_t off_sb, total;
 };
 
 template <typename K>
-bool merge_plan(int sp, uint64_t len, MergePlan<K>* M) {
+bool merge_plan(int sp, uint64_t len, MergePlan* M) {
    if (sp < 1 || sp > 30 || len == 0) return false;
    if (!build_plan<K>(sp, len, kMaxDigitBits, &M->P)) return false;
-   size_t o = align256(M->P.total);
-   M->off_mh = o;
-   o = align256(o + sizeof(MergeHeader));
-   M->off_sb = o;
-   o = align256(o + (M->P.NR + 1) * sizeof(uint64_t));
-   M->off_status = o;
-   o = align256(o + M->P.NR * sizeof(uint64_t));
-   M->off_park = o;
-   o = align256(o + kMergeCap * sizeof(MergePark<K>));
-   M->total = o;
+   M->off_sb = align256(M->P.total);
+   M->total = align256(M->off_sb + (M->P.NR + 1) * sizeof(uint64_t));
    return true;
 }
 
 template <typename K>
 size_t merge_scratch_bytes(int sp, size_t len) {
-   MergePlan<K> M;
+   MergePlan M;
    return merge_plan<K>(sp, len, &M) ? M.total : 0;
 }
 
@@ -1973,7 +1669,7 @@ int merge(const void* keys, const void* vals, const void* pairs, const void* old
    if (o0 < n0 + N * sizeof(Slot<K>) && n0 < o0 + N * sizeof(Slot<K>)) return HN_EINVAL;
    if (len == 0) // nothing to merge: the output is the table
       return static_cast<int>(hipMemcpyAsync(new_b, old_b, N * sizeof(Slot<K>), hipMemcpyDeviceToDevice, s));
-   MergePlan<K> M;
+   MergePlan M;
    if (!merge_plan<K>(sp, len, &M)) return HN_EINVAL;
    if (!scratch || bytes < M.total) return HN_ESCRATCH;
    if (!scratch_aligned(scratch)) return HN_EINVAL;
@@ -1982,31 +1678,26 @@ int merge(const void* keys, const void* vals, const void* pairs, const void* old
    BuildHeader* h = reinterpret_cast<BuildHeader*>(base);
    const Slot<K>* S = reinterpret_cast<const Slot<K>*>(base + P.off_pairs);
    const uint64_t* start = reinterpret_cast<const uint64_t*>(base + P.off_start);
-   MergeHeader* mh = reinterpret_cast<MergeHeader*>(base + M.off_mh);
    uint64_t* sb = reinterpret_cast<uint64_t*>(base + M.off_sb);
-   uint64_t* status = reinterpret_cast<uint64_t*>(base + M.off_status);
-   MergePark<K>* park = reinterpret_cast<MergePark<K>*>(base + M.off_park);
+   const RegionLB lb = region_lb(P, base);
    const Slot<K>* ob = static_cast<const Slot<K>*>(old_b);
    Slot<K>* nb = static_cast<Slot<K>*>(new_b);
 
-   hipLaunchKernelGGL(k_merge_begin, dim3(1), dim3(64), 0, s, info, mh);
    PartIn<K> in{static_cast<const K*>(keys), static_cast<const K*>(vals), static_cast<const Slot<K>*>(pairs)};
    const int src0 = pairs ? SRC_PAIRS : (vals ? SRC_SOA : SRC_INDEX);
    int rc = partition_regions<K>(P, BUILD_MERGE, info, src0, in, len, nb, scratch, s);
    if (rc) return rc;
    hipLaunchKernelGGL(k_merge_bounds<K>, dim3(static_cast<uint32_t>(std::min<uint64_t>((P.NR + 3) / 4, 65536))),
-                      dim3(256), 0, s, ob, sp, P.rlog, P.NR, sb, status, mh, h);
-   static std::atomic<int> occ{0};
-   const int per_cu = resident_blocks_per_cu(k_merge_region<K>, kMergeBS, occ);
-   const uint32_t grid =
-       static_cast<uint32_t>(std::min<uint64_t>(P.NR, static_cast<uint64_t>(cu_count()) * static_cast<uint64_t>(per_cu)));
-   hipLaunchKernelGGL(k_merge_region<K>, dim3(grid), dim3(kMergeBS), 0, s, ob, S, start, sb, status, nb, park, mh, h,
-                      sp, P.rlog, P.NR);
-   hipLaunchKernelGGL(k_merge_end<K>, dim3(1), dim3(kMergeBS), 0, s, park, status, nb, info, mh, h, sp, P.rlog, P.NR);
-   hipLaunchKernelGGL(k_merge_copy<K>, dim3(stream_blocks(N, 256)), dim3(256), 0, s, ob, nb, N, mh);
-   rc = launch_insert_pairs_dlen<K>(S, nb, info, len, &mh->fb_len, &mh->fb_fail, s);
+                      dim3(256), 0, s, ob, info, sp, P.rlog, P.NR, sb, h);
+   const uint32_t chunk = region_chunk(P.NR);
+   hipLaunchKernelGGL(k_merge_build<K>, dim3(static_cast<uint32_t>((P.NR + chunk - 1) / chunk)), dim3(kRegionBS), 0, s,
+                      ob, sb, S, start, lb, nb, sp, P.rlog, P.NR, chunk, h);
+   launch_carry(P, lb, base, h, s);
+   const uint32_t gfix = static_cast<uint32_t>(std::min<uint64_t>(P.NR, static_cast<uint64_t>(cu_count()) * 2));
+   hipLaunchKernelGGL(k_merge_fix<K>, dim3(gfix), dim3(kRegionBS), 0, s, ob, sb, S, start, lb, nb, sp, P.rlog, h);
+   rc = launch_insert_pairs_dlen<K>(S, nb, info, len, &h->fb_len, &h->fb_fail, s);
    if (rc) return rc;
-   hipLaunchKernelGGL(k_merge_fin, dim3(1), dim3(64), 0, s, info, mh);
+   hipLaunchKernelGGL(k_build_end, dim3(1), dim3(64), 0, s, info, h, BUILD_MERGE);
    return static_cast<int>(hipGetLastError());
 }
 

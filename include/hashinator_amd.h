@@ -312,14 +312,13 @@ HN_API int hn_build_pairs_u64(const void* pairs, void* buckets, hn_info* info, s
  * batch takes the bulk build's partition passes, then each 2048-slot region
  * merges its run of the old table (in Robin Hood order the keys of a region
  * stand together) with its share of the batch in LDS and places the union,
- * regions chained by a decoupled look-back.  Needs size_power <= 30 (the
+ * as the bulk build places its regions.  Needs size_power <= 30 (the
  * table's; otherwise err = INVALID and nothing else changes), len <
  * 2^size_power, buffers that do not overlap, and `scratch` of
  * hn_merge_scratch_bytes_*(size_power, len) bytes.  The merge runs on a
  * table with HN_INFO_ORDERED and no TOMBSTONEs; when the table is not such,
  * a region holds more than 2,560 old slots or 1,536 batch pairs (skewed
- * keys), the wrap past the table's end would move region 0's spill, or the
- * union would fill the table, new_buckets receives instead, on the device,
+ * keys), or the union would fill the table, new_buckets receives instead, on the device,
  * the old table with the batch inserted by probing: hn_insert_*'s result
  * (its live set, arrival order, err = SUCCESS or FAIL, HN_INFO_ORDERED
  * cleared; of a key repeated in the batch one of its values, as there).  Either way the result is in new_buckets and

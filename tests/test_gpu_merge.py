@@ -277,3 +277,53 @@ def test_map_grow_then_merge(gpu, bits):
     hm.insert(keys, vals, targetLF=0.9)  # grows to 2^13: the batch is over a quarter of it
     assert hm.getSizePower() == sp + 1 and hm.ordered()
     _check_map(hm, bits, _final(old_keys, old_keys, keys, vals))
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_merge_wrap_moves_the_spill(gpu, bits):
+    """The batch fills the table's end until the wrap pushes region 0's keys
+    on into region 1 (and a cluster of its own runs across a whole region), so
+    that regions placed without that carry are placed again."""
+    sp = 13
+    N, R = 1 << sp, 2048
+    cand = keyset(60 * N, bits, seed=17)
+    home = O.fibhash(cand, sp, bits).astype(np.int64) & (N - 1)
+
+    def pick(lo, hi, n):
+        return cand[(home >= lo) & (home < hi)][:n]
+
+    old_keys = np.concatenate([pick(0, R, 2000), pick(R, 2 * R, 1500), pick(3 * R, N, 1800)])
+    old, inf = ordered_table(bits, sp, old_keys, old_keys)
+    old_img = to_numpy(old, bits).reshape(-1, 2).copy()
+    more = np.setdiff1d(np.concatenate([pick(N - 200, N, 700), pick(2 * R, 3 * R, 1200)]), old_keys)
+    keys = np.random.default_rng(3).permutation(more)
+    vals = (keys + NDT[bits](5)).astype(NDT[bits])
+    m = expected(bits, sp, old_img, inf.cpu().numpy(), keys, vals)
+    rc, img, inf1 = run_merge(bits, sp, old, inf, keys, vals)
+    assert rc == 0
+    check_merge(bits, img, inf1, m)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("sp", [3, 11, 13])
+@pytest.mark.parametrize("over", [-1, 0, 1])
+def test_merge_up_to_a_full_table(gpu, bits, sp, over):
+    """A union of N - 1 keys is merged; one of N fills the table by probing,
+    one of N + 1 fills it and reports FAIL."""
+    N = 1 << sp
+    allk = keyset(N + over, bits, seed=sp + 40)
+    old_keys, keys = allk[: (5 * N) // 8], allk[(5 * N) // 8:]
+    old, inf = ordered_table(bits, sp, old_keys, old_keys)
+    old_img = to_numpy(old, bits).reshape(-1, 2).copy()
+    vals = (keys + NDT[bits](9)).astype(NDT[bits])
+    if over < 0:
+        m = expected(bits, sp, old_img, inf.cpu().numpy(), keys, vals)
+        rc, img, inf1 = run_merge(bits, sp, old, inf, keys, vals)
+        assert rc == 0
+        check_merge(bits, img, inf1, m)
+        return
+    rc, img, inf1 = run_merge(bits, sp, old, inf, keys, vals)
+    assert rc == 0
+    assert int(inf1[1]) == N and (int(inf1[4]) & 0xFFFFFFFF) == (0 if over == 0 else 1) and (int(inf1[4]) >> 32) == 0
+    rows = live_pairs(img, bits)
+    assert rows.shape[0] == N and np.all(np.isin(old_keys, rows[:, 0])) and np.all(np.isin(rows[:, 0], allk))
