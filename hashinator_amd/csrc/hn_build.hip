@@ -101,7 +101,9 @@ struct BuildHeader {
    uint64_t n;         // pairs after the first partition pass (the live slots when the input is a table)
    uint64_t fb_len;    // pairs the fallback insert takes from the partitioned array (0: none)
    uint64_t prior_fill; // rehash: the old table's fill, which the new one must hold
-   uint32_t pad[48];
+   uint64_t grow_old, grow_new; // rehash with a batch: the old table's slots, the batch's length (else 0)
+   uint64_t fb_new;     // its fallback: pairs taken from the batch (fb_len then counts old slots)
+   uint32_t pad[42];
 };
 static_assert(sizeof(BuildHeader) == 256, "header is one 256-byte line");
 
@@ -203,14 +205,22 @@ struct PartIn {
    const K* keys;        // SRC_SOA / SRC_INDEX
    const K* vals;        // SRC_SOA
    const Slot<K>* pairs; // SRC_PAIRS / SRC_TABLE (a pair array)
+   // SRC_GROW: the n_table slots of `table`, then the batch in one of the forms above
+   const Slot<K>* table;
+   uint64_t n_table;
 };
+constexpr int SRC_GROW = SRC_TABLE + 1;
 
 template <typename K, int SRC>
 __device__ __forceinline__ K part_key(const PartIn<K>& in, uint64_t e) {
-   if constexpr (SRC == SRC_SOA || SRC == SRC_INDEX)
+   if constexpr (SRC == SRC_SOA || SRC == SRC_INDEX) {
       return in.keys[e];
-   else
+   } else if constexpr (SRC == SRC_GROW) {
+      if (e < in.n_table) return in.table[e].key;
+      return in.pairs ? in.pairs[e - in.n_table].key : in.keys[e - in.n_table];
+   } else {
       return in.pairs[e].key;
+   }
 }
 
 template <typename K, int SRC>
@@ -222,10 +232,26 @@ __device__ __forceinline__ Slot<K> part_pair(const PartIn<K>& in, uint64_t e) {
    } else if constexpr (SRC == SRC_INDEX) {
       s.key = in.keys[e];
       s.val = static_cast<K>(e);
+   } else if constexpr (SRC == SRC_GROW) {
+      const uint64_t q = e - in.n_table;
+      if (e < in.n_table) {
+         s = in.table[e];
+      } else if (in.pairs) {
+         s = in.pairs[q];
+      } else {
+         s.key = in.keys[q];
+         s.val = in.vals ? in.vals[q] : static_cast<K>(q);
+      }
    } else {
       s = in.pairs[e];
    }
    return s;
+}
+
+// A table's EMPTY and TOMBSTONE slots are left out; a batch's keys are not looked at.
+template <typename K, int SRC>
+__device__ __forceinline__ bool part_live(const PartIn<K>& in, uint64_t e, K key) {
+   return (SRC == SRC_GROW && e >= in.n_table) || (key != empty_key<K>() && key != tomb_key<K>());
 }
 
 template <typename K>
@@ -235,9 +261,10 @@ __device__ __forceinline__ uint32_t region_of(K key, int sp, int rlog) {
 }
 
 // Build from caller arrays into an empty table, (rehash) from the live
-// slots of another, smaller table into a new one, or (merge) from caller
-// arrays and an ordered table into a second array of the table's size.
-enum BuildMode { BUILD_EMPTY = 0, BUILD_REHASH = 2, BUILD_MERGE = 3 };
+// slots of another, smaller table into a new one, (grow) from those and
+// caller arrays, or (merge) from caller arrays and an ordered table into a
+// second array of the table's size.
+enum BuildMode { BUILD_EMPTY = 0, BUILD_REHASH = 2, BUILD_MERGE = 3, BUILD_GROW = 4 };
 
 // What the first kernel of a build does besides its own work: with `info`
 // set, decide whether the build runs and set up its header (a launch of its
@@ -252,12 +279,13 @@ struct BuildBegin {
 };
 
 __device__ __forceinline__ bool build_go(const hn_info* info, int sp, int mode) {
-   if (mode == BUILD_REHASH) return true; // k_rehash_info has just set the Info up for the new table
+   if (mode == BUILD_REHASH || mode == BUILD_GROW) return true; // k_rehash_info has just set the Info up for the new table
    const bool sp_ok = info->size_power == sp;
    // a merge's batch is partitioned whether the merge or its fallback runs
    return sp_ok && (mode == BUILD_MERGE || (info->fill == 0 && info->tombstone_counter == 0));
 }
-__device__ __forceinline__ void build_header(BuildHeader* h, bool go, uint64_t n) {
+__device__ __forceinline__ void build_header(BuildHeader* h, bool go, uint64_t n, uint64_t grow_old = 0,
+                                             uint64_t grow_new = 0) {
    h->go = go ? 1u : 0u;
    h->fail = 0;
    h->max_probe = 0;
@@ -266,18 +294,17 @@ __device__ __forceinline__ void build_header(BuildHeader* h, bool go, uint64_t n
    h->n_fix = 0;
    h->fb_fail = 0;
    h->fb_len = 0;
+   h->fb_new = 0;
+   h->grow_old = grow_old;
+   h->grow_new = grow_new;
    h->n = n;
 }
 
 // A rehash counts the live slots in its first pass, so its header is set up
 // before that.
-__global__ void k_build_begin(const hn_info* info, BuildHeader* h, int sp, int mode) {
-   if (threadIdx.x == 0) build_header(h, build_go(info, sp, mode), 0);
-}
-
-template <typename K>
-__device__ __forceinline__ bool live_key(K k) {
-   return k != empty_key<K>() && k != tomb_key<K>();
+__global__ void k_build_begin(const hn_info* info, BuildHeader* h, int sp, int mode, uint64_t grow_old,
+                              uint64_t grow_new) {
+   if (threadIdx.x == 0) build_header(h, build_go(info, sp, mode), 0, grow_old, grow_new);
 }
 
 // Per-block digit counts, written digit-major: mat[d * nblocks + block].  A
@@ -338,7 +365,7 @@ __global__ __launch_bounds__(kPartBS) void k_part_count(PartIn<K> in, uint64_t n
 #pragma unroll
          for (int u = 0; u < U; ++u) {
             const uint64_t e = e0 + static_cast<uint64_t>(u) * kPartBS;
-            if (e >= t1 || (FILTER && !live_key(key[u]))) continue;
+            if (e >= t1 || (FILTER && !part_live<K, SRC>(in, e, key[u]))) continue;
             atomicAdd(&hist[(region_of(key[u], sp, rlog) >> dshift) & dmask], 1u);
             ++live;
          }
@@ -436,7 +463,7 @@ __global__ __launch_bounds__(BS) void k_part_scatter(PartIn<K> in, uint64_t n_in
          dg[r] = 0;
          ok[r] = false;
          if (e < n) {
-            ok[r] = !FILTER || live_key(el[r].key);
+            ok[r] = !FILTER || part_live<K, SRC>(in, e, el[r].key);
             dg[r] = (region_of(el[r].key, sp, rlog) >> dshift) & dmask;
          }
       }
@@ -1116,11 +1143,14 @@ __global__ __launch_bounds__(1024) void k_carry_small(RegionLB lb, uint64_t NR, 
 }
 
 // A region over capacity abandons the placement: the table is emptied and
-// the probing insert takes the partitioned pairs (all of them, in S).
+// the probing insert takes the partitioned pairs (all of them, in S); a
+// rehash with a batch inserts the old table and then the batch, whose values
+// win.
 template <typename K>
 __device__ void build_fallback_prep(Slot<K>* b, uint64_t N, hn_info* info, BuildHeader* h) {
    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      h->fb_len = h->n;
+      h->fb_len = h->grow_old ? h->grow_old : h->n;
+      h->fb_new = h->grow_new;
       info->fill = 0;
       info->current_max_bucket_overflow = kBucketOverflow;
    }
@@ -1171,7 +1201,7 @@ __global__ __launch_bounds__(kRegionBS) void k_region_fix(const Slot<K>* S, cons
 __global__ void k_build_end(hn_info* info, const BuildHeader* h, int mode) {
    if (threadIdx.x != 0) return;
    if (!h->go) {
-      if (mode != BUILD_REHASH) info->err = HN_STATUS_INVALID;
+      info->err = HN_STATUS_INVALID; // (a rehash always goes)
       return;
    }
    info->reserved0 = 0;
@@ -1257,6 +1287,13 @@ int launch_part(const BuildPlan& P, int pass, PartIn<K> in, uint64_t n_in, const
 template <typename K>
 int launch_insert_pairs_dlen(const Slot<K>* pairs, Slot<K>* buckets, hn_info* info, uint64_t max_len,
                              const uint64_t* d_len, int32_t* fail_sink, hipStream_t s);
+// The same from a table's slots, and from a batch in any of its forms.
+template <typename K>
+int launch_insert_table_dlen(const Slot<K>* table, Slot<K>* buckets, hn_info* info, uint64_t max_len,
+                             const uint64_t* d_len, int32_t* fail_sink, hipStream_t s);
+template <typename K>
+int launch_insert_batch_dlen(const K* keys, const K* vals, const Slot<K>* pairs, Slot<K>* buckets, hn_info* info,
+                             uint64_t max_len, const uint64_t* d_len, int32_t* fail_sink, hipStream_t s);
 
 inline RegionLB region_lb(const BuildPlan& P, char* base) {
    RegionLB lb;
@@ -1288,8 +1325,9 @@ int partition_regions(const BuildPlan& P, int mode, const hn_info* info, int src
    uint8_t* dig = reinterpret_cast<uint8_t*>(base + P.off_dig);
    const RegionLB lb = region_lb(P, base);
    BuildBegin bg{};
-   if (mode == BUILD_REHASH)
-      hipLaunchKernelGGL(k_build_begin, dim3(1), dim3(64), 0, s, info, h, P.sp, mode);
+   if (mode == BUILD_REHASH || mode == BUILD_GROW)
+      hipLaunchKernelGGL(k_build_begin, dim3(1), dim3(64), 0, s, info, h, P.sp, mode, in0.n_table,
+                         mode == BUILD_GROW ? n_in - in0.n_table : 0);
    else
       bg = BuildBegin{info, P.sp, mode, P.n, nullptr, 0};
    const Slot<K>* src = nullptr;
@@ -1310,13 +1348,17 @@ int partition_regions(const BuildPlan& P, int mode, const hn_info* info, int src
             rc = launch_part<K, SRC_INDEX, false>(P, 0, in0, n_in, nullptr, dst, mat, scan_scratch, scan_bytes, h, dig, bg,
                                                   start, lb, s);
             break;
+         case SRC_GROW:
+            rc = launch_part<K, SRC_GROW, true>(P, 0, in0, n_in, nullptr, dst, mat, scan_scratch, scan_bytes, h, dig, bg,
+                                                start, lb, s);
+            break;
          default:
             rc = launch_part<K, SRC_TABLE, true>(P, 0, in0, n_in, nullptr, dst, mat, scan_scratch, scan_bytes, h, dig, bg,
                                                  start, lb, s);
             break;
          }
       } else {
-         PartIn<K> in{nullptr, nullptr, src};
+         PartIn<K> in{nullptr, nullptr, src, nullptr, 0};
          rc = launch_part<K, SRC_TABLE, false>(P, pass, in, 0, &h->n, dst, mat, scan_scratch, scan_bytes, h, dig,
                                                BuildBegin{}, start, lb, s);
       }
@@ -1364,7 +1406,14 @@ int build_core(const BuildPlan& P, int mode, int src0, PartIn<K> in0, uint64_t n
    launch_carry(P, lb, base, h, s);
    const uint32_t gfix = static_cast<uint32_t>(std::min<uint64_t>(P.NR, static_cast<uint64_t>(cu_count()) * 2));
    hipLaunchKernelGGL(k_region_fix<K>, dim3(gfix), dim3(kRegionBS), 0, s, S, start, lb, T, P.sp, P.rlog, info, h);
-   rc = launch_insert_pairs_dlen<K>(S, T, info, P.n, &h->fb_len, &h->fb_fail, s);
+   if (mode == BUILD_GROW) {
+      rc = launch_insert_table_dlen<K>(in0.table, T, info, in0.n_table, &h->fb_len, &h->fb_fail, s);
+      if (!rc)
+         rc = launch_insert_batch_dlen<K>(in0.keys, in0.vals, in0.pairs, T, info, n_in - in0.n_table, &h->fb_new,
+                                          &h->fb_fail, s);
+   } else {
+      rc = launch_insert_pairs_dlen<K>(S, T, info, P.n, &h->fb_len, &h->fb_fail, s);
+   }
    if (rc) return rc;
    hipLaunchKernelGGL(k_build_end, dim3(1), dim3(64), 0, s, info, h, mode);
    return static_cast<int>(hipGetLastError());
@@ -1381,7 +1430,7 @@ int build(const void* keys, const void* vals, const void* pairs, void* buckets, 
    if (!build_plan<K>(sp, len, dcap, &P)) return HN_EINVAL;
    if (!scratch || bytes < P.total) return HN_ESCRATCH;
    if (!scratch_aligned(scratch)) return HN_EINVAL;
-   PartIn<K> in{static_cast<const K*>(keys), static_cast<const K*>(vals), static_cast<const Slot<K>*>(pairs)};
+   PartIn<K> in{static_cast<const K*>(keys), static_cast<const K*>(vals), static_cast<const Slot<K>*>(pairs), nullptr, 0};
    const int src0 = pairs ? SRC_PAIRS : (vals ? SRC_SOA : SRC_INDEX);
    return build_core<K>(P, BUILD_EMPTY, src0, in, len, buckets, info, scratch, s);
 }
@@ -1421,8 +1470,45 @@ int rehash_build(const void* old_b, int old_sp, void* new_b, int new_sp, hn_info
    if (!scratch || bytes < P.total) return HN_ESCRATCH;
    if (!scratch_aligned(scratch)) return HN_EINVAL;
    hipLaunchKernelGGL(k_rehash_info, dim3(1), dim3(64), 0, s, info, new_sp, static_cast<BuildHeader*>(scratch));
-   PartIn<K> in{nullptr, nullptr, static_cast<const Slot<K>*>(old_b)};
+   PartIn<K> in{nullptr, nullptr, static_cast<const Slot<K>*>(old_b), nullptr, 0};
    return build_core<K>(P, BUILD_REHASH, SRC_TABLE, in, 1ull << old_sp, new_b, info, scratch, s);
+}
+
+// An insert that grows the table (hashinator.h:1329-1335: resize, then
+// insert) as one build: the first partition pass reads the old table's live
+// slots and then the batch, so the sort's last copy of a key is the newest.
+// A rehash, the probing insert and the reorder go through the new table twice
+// more: 3 million u64 keys to 3 million of 2^23 slots 0.73 ms, here 0.43; 1.1
+// million 0.59 and 0.39; 60,000 to 60,000 of 2^17 0.098 and 0.074.
+template <typename K>
+bool grow_plan(int old_sp, int new_sp, uint64_t len, BuildPlan* P) {
+   if (old_sp < 1 || new_sp <= old_sp || new_sp > std::min(max_size_power<K>(), 32)) return false;
+   if (len == 0 || len >= 1ull << new_sp) return false;
+   return build_plan<K>(new_sp, (1ull << old_sp) + len, kMaxDigitBits, P);
+}
+
+template <typename K>
+size_t grow_scratch_bytes(int old_sp, int new_sp, size_t len) {
+   BuildPlan P;
+   return grow_plan<K>(old_sp, new_sp, len, &P) ? P.total : 0;
+}
+
+template <typename K>
+int grow(const void* keys, const void* vals, const void* pairs, const void* old_b, int old_sp, void* new_b, int new_sp,
+         hn_info* info, size_t len, void* scratch, size_t bytes, hipStream_t s) {
+   if (!old_b || !new_b || !info || (!keys && !pairs)) return HN_EINVAL;
+   BuildPlan P;
+   if (!grow_plan<K>(old_sp, new_sp, len, &P)) return HN_EINVAL;
+   const char* o0 = static_cast<const char*>(old_b);
+   const char* n0 = static_cast<const char*>(new_b);
+   if (o0 < n0 + P.N * sizeof(Slot<K>) && n0 < o0 + (1ull << old_sp) * sizeof(Slot<K>)) return HN_EINVAL;
+   if (!scratch || bytes < P.total) return HN_ESCRATCH;
+   if (!scratch_aligned(scratch)) return HN_EINVAL;
+   const uint64_t nt = 1ull << old_sp;
+   hipLaunchKernelGGL(k_rehash_info, dim3(1), dim3(64), 0, s, info, new_sp, static_cast<BuildHeader*>(scratch));
+   PartIn<K> in{static_cast<const K*>(keys), static_cast<const K*>(vals), static_cast<const Slot<K>*>(pairs),
+                static_cast<const Slot<K>*>(old_b), nt};
+   return build_core<K>(P, BUILD_GROW, SRC_GROW, in, nt + len, new_b, info, scratch, s);
 }
 
 
@@ -1683,7 +1769,7 @@ int merge(const void* keys, const void* vals, const void* pairs, const void* old
    const Slot<K>* ob = static_cast<const Slot<K>*>(old_b);
    Slot<K>* nb = static_cast<Slot<K>*>(new_b);
 
-   PartIn<K> in{static_cast<const K*>(keys), static_cast<const K*>(vals), static_cast<const Slot<K>*>(pairs)};
+   PartIn<K> in{static_cast<const K*>(keys), static_cast<const K*>(vals), static_cast<const Slot<K>*>(pairs), nullptr, 0};
    const int src0 = pairs ? SRC_PAIRS : (vals ? SRC_SOA : SRC_INDEX);
    int rc = partition_regions<K>(P, BUILD_MERGE, info, src0, in, len, nb, scratch, s);
    if (rc) return rc;
@@ -1734,6 +1820,24 @@ int hn_build_pairs_u32(const void* p, void* b, hn_info* i, size_t n, int sp, voi
 int hn_build_pairs_u64(const void* p, void* b, hn_info* i, size_t n, int sp, void* sc, size_t sb, hn_stream_t s,
                        const hn_tune* t) {
    return build<uint64_t>(nullptr, nullptr, p, b, i, n, sp, sc, sb, s, t);
+}
+size_t hn_grow_scratch_bytes_u32(int osp, int nsp, size_t len) { return grow_scratch_bytes<uint32_t>(osp, nsp, len); }
+size_t hn_grow_scratch_bytes_u64(int osp, int nsp, size_t len) { return grow_scratch_bytes<uint64_t>(osp, nsp, len); }
+int hn_grow_u32(const void* k, const void* v, const void* ob, int osp, void* nb, int nsp, hn_info* i, size_t n,
+                void* sc, size_t sb, hn_stream_t s) {
+   return grow<uint32_t>(k, v, nullptr, ob, osp, nb, nsp, i, n, sc, sb, s);
+}
+int hn_grow_u64(const void* k, const void* v, const void* ob, int osp, void* nb, int nsp, hn_info* i, size_t n,
+                void* sc, size_t sb, hn_stream_t s) {
+   return grow<uint64_t>(k, v, nullptr, ob, osp, nb, nsp, i, n, sc, sb, s);
+}
+int hn_grow_pairs_u32(const void* p, const void* ob, int osp, void* nb, int nsp, hn_info* i, size_t n, void* sc,
+                      size_t sb, hn_stream_t s) {
+   return grow<uint32_t>(nullptr, nullptr, p, ob, osp, nb, nsp, i, n, sc, sb, s);
+}
+int hn_grow_pairs_u64(const void* p, const void* ob, int osp, void* nb, int nsp, hn_info* i, size_t n, void* sc,
+                      size_t sb, hn_stream_t s) {
+   return grow<uint64_t>(nullptr, nullptr, p, ob, osp, nb, nsp, i, n, sc, sb, s);
 }
 size_t hn_merge_scratch_bytes_u32(int sp, size_t len) { return merge_scratch_bytes<uint32_t>(sp, len); }
 size_t hn_merge_scratch_bytes_u64(int sp, size_t len) { return merge_scratch_bytes<uint64_t>(sp, len); }

@@ -640,6 +640,28 @@ int launch_insert_pairs_dlen(const Slot<K>* pairs, Slot<K>* buckets, hn_info* in
    InsertArgs<K> a{nullptr, nullptr, pairs, buckets, info, max_len, d_len, nullptr, fail_sink};
    return launch_insert<K, SRC_PAIRS>(a, max_len, s, nullptr, OP_REINSERT);
 }
+template <typename K>
+int launch_insert_table_dlen(const Slot<K>* table, Slot<K>* buckets, hn_info* info, uint64_t max_len,
+                             const uint64_t* d_len, int32_t* fail_sink, hipStream_t s) {
+   InsertArgs<K> a{nullptr, nullptr, table, buckets, info, max_len, d_len, nullptr, fail_sink};
+   return launch_insert<K, SRC_TABLE>(a, max_len, s, nullptr, OP_REINSERT);
+}
+template <typename K>
+int launch_insert_batch_dlen(const K* keys, const K* vals, const Slot<K>* pairs, Slot<K>* buckets, hn_info* info,
+                             uint64_t max_len, const uint64_t* d_len, int32_t* fail_sink, hipStream_t s) {
+   InsertArgs<K> a{keys, vals, pairs, buckets, info, max_len, d_len, nullptr, fail_sink};
+   if (pairs) return launch_insert<K, SRC_PAIRS>(a, max_len, s, nullptr, OP_INSERT);
+   if (vals) return launch_insert<K, SRC_SOA>(a, max_len, s, nullptr, OP_INSERT);
+   return launch_insert<K, SRC_INDEX>(a, max_len, s, nullptr, OP_INSERT);
+}
+#define HN_DLEN(K)                                                                                                    \
+   template int launch_insert_table_dlen<K>(const Slot<K>*, Slot<K>*, hn_info*, uint64_t, const uint64_t*, int32_t*,  \
+                                            hipStream_t);                                                             \
+   template int launch_insert_batch_dlen<K>(const K*, const K*, const Slot<K>*, Slot<K>*, hn_info*, uint64_t,         \
+                                            const uint64_t*, int32_t*, hipStream_t);
+HN_DLEN(uint32_t)
+HN_DLEN(uint64_t)
+#undef HN_DLEN
 template int launch_insert_pairs_dlen<uint32_t>(const Slot<uint32_t>*, Slot<uint32_t>*, hn_info*, uint64_t,
                                                 const uint64_t*, int32_t*, hipStream_t);
 template int launch_insert_pairs_dlen<uint64_t>(const Slot<uint64_t>*, Slot<uint64_t>*, hn_info*, uint64_t,

@@ -144,10 +144,11 @@ class Hashmap:
         (and of ``build_min_keys``) into a table that holds keys and no
         tombstones takes the merge (hn_merge_*), which writes the insert +
         reorder image into a fresh bucket array; the merge reads and writes
-        the whole table (about 7 ms at 2^28 u64 slots, against 0.18 ns per
-        key for the probing insert there), so it pays from about a quarter of
-        the table.  A table not in Robin Hood order is reordered first when
-        the batch is at least 4/3 of this fraction.  0 turns it off."""
+        the whole table, so it pays from about a quarter of the table (one
+        MI355X, a quarter of 2^26 u64 slots up to load 0.5: 1.26 ms against
+        1.77), sooner only where the table is nearly full (see _try_merge).
+        A table not in Robin Hood order is reordered first when the batch is
+        at least 4/3 of this fraction.  0 turns it off."""
         if key_bits not in (32, 64):
             raise ValueError("key_bits must be 32 or 64")
         self.kb = key_bits
@@ -240,12 +241,60 @@ class Hashmap:
         return to_numpy(self.buckets, self.kb).reshape(-1, 2)
 
     # ----------------------------------------------------------- accelerated API
-    def _grow_for(self, n, targetLF, stream):
-        """Auto-grow before an insert (hashinator.h:1329-1332)."""
-        fill = self.size()
+    def _grow_for(self, k, v, n, pairs, targetLF, stream) -> bool:
+        """Auto-grow before an insert (hashinator.h:1329-1332).  True when the
+        batch is in the table already: growing a map of many keys by a batch
+        that the reorder pass would follow is one build of both (hn_grow_*).
+        An empty map that the build will fill is not rehashed."""
+        i = self.info()
+        fill = i.fill
         needed = math.ceil(math.log2((fill + n) * (1.0 / targetLF)))
-        if needed > self._sp:
-            self.resize(needed, targets.device, stream)
+        if needed <= self._sp:
+            return False
+        N = 1 << needed
+        if fill == 0 and needed <= 32 and self._builds(n, N) and \
+                getattr(self._L, f"hn_build_scratch_bytes_{self._sfx}")(needed, n):
+            self.buckets = self._new_table(needed, init=False)  # the build writes every slot
+            self._sp = needed
+            check(self._L.hn_info_init(_ptr(self._info), needed, _stream(stream)), "hn_info_init")
+            built = False
+            try:
+                built = self._try_build(k, v, n, pairs, stream)
+            finally:
+                if not built:  # no memory for its scratch, say
+                    check(self._fn("table_init")(_ptr(self.buckets), N, _stream(stream)), "hn_table_init")
+            return built
+        if self.auto_build and self.auto_reorder and fill >= self.build_min_keys and n >= self.auto_reorder * N:
+            if self._grow(k, v, n, pairs, needed, stream):
+                return True
+        self.resize(needed, targets.device, stream)
+        return False
+
+    def _grow(self, k, v, n, pairs, new_sp, stream) -> bool:
+        sb = 0 if new_sp > 32 else getattr(self._L, f"hn_grow_scratch_bytes_{self._sfx}")(self._sp, new_sp, n)
+        if sb == 0:
+            return False
+        try:
+            scratch = torch.empty(sb, dtype=torch.uint8, device=self.device)
+            nb = self._new_table(new_sp, init=False)
+        except torch.OutOfMemoryError:
+            return False  # the rehash needs less
+        old, head = self.buckets, (_ptr(k),) if pairs else (_ptr(k), _ptr(v) if v is not None else None)
+        check(self._fn("grow_pairs" if pairs else "grow")(*head, _ptr(old), self._sp, _ptr(nb), new_sp,
+                                                          _ptr(self._info), n, _ptr(scratch), sb, _stream(stream)),
+              "insert")
+        self.buckets = nb
+        self._sp = new_sp
+        self._sync(stream)
+        del old, scratch
+        if not self.ordered():
+            self._reorder(stream)  # skewed keys: inserted in arrival order
+            self._sync(stream)
+        return True
+
+    def _builds(self, n, N) -> bool:
+        """Whether n keys into an empty table of N slots take the bulk build."""
+        return bool(self.auto_build) and n >= self.auto_build * N and n >= self.build_min_keys and n < N
 
     @on_stream
     def insert(self, keys, vals=None, targetLF: float = 0.5, stream=None):
@@ -264,7 +313,8 @@ class Hashmap:
         if n == 0:
             self._info.view(torch.int32)[8] = status.success
             return
-        self._grow_for(n, targetLF, stream)
+        if self._grow_for(k, None if vals is None else v, n, vals is None, targetLF, stream):
+            return
         if self._try_build(k, None if vals is None else v, n, vals is None, stream):
             return
         if self._try_merge(k, None if vals is None else v, n, vals is None, stream):
@@ -283,8 +333,7 @@ class Hashmap:
         not empty and is untouched; the probing insert runs instead).  Strongly
         skewed keys are placed by the device's own probing fallback inside the
         same call (err = SUCCESS, table not marked ordered)."""
-        N = self.bucket_count()
-        if not self.auto_build or n < self.auto_build * N or n < self.build_min_keys or n >= N:
+        if not self._builds(n, self.bucket_count()):
             return False
         i = self.info()
         if i.fill != 0 or i.tombstone_counter != 0:
@@ -309,22 +358,41 @@ class Hashmap:
         insert + reorder image into a fresh bucket array, which then replaces
         the old one.  Where the merge itself declines (keys crowding one
         region, say), the device writes the probing insert's result into the
-        new array instead, so the insert is complete either way."""
+        new array instead, so the insert is complete either way.
+
+        Smaller inserts that the reorder pass would follow take it too where
+        the map ends at least 85% full and is ordered already: the probing
+        insert's chains grow with the load, the merge does not (one MI355X,
+        insert + reorder against merge + copy, a sixteenth of the slots
+        inserted up to load 0.9: 2^26 u64 slots 2.00 and 1.46 ms, 2^22 0.24
+        and 0.18; up to 0.8: 1.27 and 1.45, 0.13 and 0.17).  The image is
+        copied back, so that the bucket array stays the one that it was."""
         N = self.bucket_count()
-        if not self.merge_min or n < self.merge_min * N or n < self.build_min_keys or n >= N or self._sp > 30:
+        if not self.merge_min or n < self.build_min_keys or n >= N or self._sp > 30:
+            return False
+        small = n < self.merge_min * N
+        if small and not (self.auto_reorder and n >= self.auto_reorder * N):
             return False
         i = self.info()
         if i.fill == 0 or i.tombstone_counter != 0:
             return False
-        if not (i.reserved1 & _lib.HN_INFO_ORDERED):
+        ordered = bool(i.reserved1 & _lib.HN_INFO_ORDERED)
+        if small and not (ordered and i.fill + n >= 0.85 * N):
+            return False
+        if not ordered:
             if n < self.merge_min * N * 4 / 3:
                 return False
             self._reorder(stream)
         sb = getattr(self._L, f"hn_merge_scratch_bytes_{self._sfx}")(self._sp, n)
         if sb == 0:
             return False
-        scratch = torch.empty(sb, dtype=torch.uint8, device=self.device)
-        nb = self._new_table(self._sp, init=False)  # the merge (or its fallback) writes every slot
+        try:
+            scratch = torch.empty(sb, dtype=torch.uint8, device=self.device)
+            nb = self._new_table(self._sp, init=False)  # the merge (or its fallback) writes every slot
+        except torch.OutOfMemoryError:
+            if small:
+                return False  # the probing insert needs no memory
+            raise
         if pairs:
             rc = self._fn("merge_pairs")(_ptr(k), _ptr(self.buckets), _ptr(nb), _ptr(self._info), n, self._sp,
                                          _ptr(scratch), sb, _stream(stream))
@@ -333,9 +401,12 @@ class Hashmap:
                                    _ptr(self._info), n, self._sp, _ptr(scratch), sb, _stream(stream))
         check(rc, "merge")
         old = self.buckets  # read by the merge until the stream is synchronised
-        self.buckets = nb
+        if small:
+            old.copy_(nb)
+        else:
+            self.buckets = nb
         self._sync(stream)
-        del old, scratch
+        del old, nb, scratch
         if self.auto_reorder and not self.ordered() and n >= self.auto_reorder * N:
             self._reorder(stream)  # the fallback inserted in arrival order
             self._sync(stream)
@@ -375,7 +446,8 @@ class Hashmap:
         if n == 0:
             self._info.view(torch.int32)[8] = status.success
             return
-        self._grow_for(n, targetLF, stream)
+        if self._grow_for(k, None, n, False, targetLF, stream):
+            return
         if self._try_build(k, None, n, False, stream):
             return
         if self._try_merge(k, None, n, False, stream):

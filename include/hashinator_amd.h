@@ -354,6 +354,27 @@ HN_API int hn_rehash_build_u32(const void* old_buckets, int old_sp, void* new_bu
 HN_API int hn_rehash_build_u64(const void* old_buckets, int old_sp, void* new_buckets, int new_sp, hn_info* info,
                                void* scratch, size_t scratch_bytes, hn_stream_t s);
 
+/* An insert that grows the table (hashinator.h:1329-1335: resize(), then
+ * insert) as one bulk build: new_buckets receives the union of old_buckets'
+ * live set and the batch, as hn_rehash_build_* followed by hn_merge_* gives
+ * it (a present key takes the batch's value, a repeated key its last one),
+ * and *info becomes that table's; err = SUCCESS, or FAIL where a key found no
+ * slot.  Needs old_sp < new_sp <= 32, 0 < len < 2^new_sp, 2^old_sp + len <
+ * 2^new_sp, buffers that do not overlap, and `scratch` of
+ * hn_grow_scratch_bytes_*(old_sp, new_sp, len) bytes (0: not possible).
+ * Strongly skewed keys are placed by probing instead, the old table's first.
+ * `vals` NULL stores each key's index in the batch. */
+HN_API size_t hn_grow_scratch_bytes_u32(int old_sp, int new_sp, size_t len);
+HN_API size_t hn_grow_scratch_bytes_u64(int old_sp, int new_sp, size_t len);
+HN_API int hn_grow_u32(const void* keys, const void* vals, const void* old_buckets, int old_sp, void* new_buckets,
+                       int new_sp, hn_info* info, size_t len, void* scratch, size_t scratch_bytes, hn_stream_t s);
+HN_API int hn_grow_u64(const void* keys, const void* vals, const void* old_buckets, int old_sp, void* new_buckets,
+                       int new_sp, hn_info* info, size_t len, void* scratch, size_t scratch_bytes, hn_stream_t s);
+HN_API int hn_grow_pairs_u32(const void* pairs, const void* old_buckets, int old_sp, void* new_buckets, int new_sp,
+                             hn_info* info, size_t len, void* scratch, size_t scratch_bytes, hn_stream_t s);
+HN_API int hn_grow_pairs_u64(const void* pairs, const void* old_buckets, int old_sp, void* new_buckets, int new_sp,
+                             hn_info* info, size_t len, void* scratch, size_t scratch_bytes, hn_stream_t s);
+
 /* ---------------------------------------------------------------- compaction and scan */
 
 /* Scratch for one compaction or scan of n elements

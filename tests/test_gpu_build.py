@@ -448,3 +448,28 @@ def test_build_rejects_misaligned_scratch(gpu):
                         ms.data_ptr() + 64, msb, None)
     torch.cuda.synchronize()
     assert rc == _lib.HN_EINVAL and torch.equal(b, img1) and torch.equal(inf, inf1)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("byte", [0x00, 0x01, 0xA5])
+def test_fallback_reads_nothing_from_old_scratch(gpu, bits, byte):
+    """The probing fallback of an over-full region takes its lengths from what
+    the call itself wrote, whatever the scratch memory held before."""
+    sp = 14
+    keys = concentrated_keys(bits, sp, 3000, 2048, seed=6)
+    vals = (keys ^ NDT[bits](3)).astype(NDT[bits])
+    L, sfx = _lib.load(), f"u{bits}"
+    b = torch.empty((1 << sp, 2), dtype=TDT[bits], device="cuda")
+    inf = torch.zeros(5, dtype=torch.int64, device="cuda")
+    _lib.check(L.hn_info_init(inf.data_ptr(), sp, None), "info")
+    sb = getattr(L, f"hn_build_scratch_bytes_{sfx}")(sp, keys.size)
+    sc = torch.full((sb,), byte, dtype=torch.uint8, device="cuda")
+    dk, dv = dev(keys, bits), dev(vals, bits)
+    rc = getattr(L, f"hn_build_{sfx}")(dk.data_ptr(), dv.data_ptr(), b.data_ptr(), inf.data_ptr(), keys.size, sp,
+                                       sc.data_ptr(), sb, None, None)
+    torch.cuda.synchronize()
+    after = inf.cpu().numpy()
+    assert rc == 0 and (int(after[1]), int(after[3]), int(after[4])) == (keys.size, 0, 0)
+    rows = live_pairs(to_numpy(b, bits), bits)
+    order = np.argsort(keys)
+    assert np.array_equal(rows, np.stack([keys[order], vals[order]], axis=1))

@@ -11,7 +11,7 @@ import torch
 import oracle as O
 from hashinator_amd import Hashmap, to_numpy
 from hashinator_amd import _lib
-from tests.helpers import NDT, keyset, live_pairs, occupancy, reachable_all
+from tests.helpers import EMPTY, NDT, TOMB, fresh_model, keyset, live_pairs, occupancy, reachable_all
 from tests.test_gpu_build import concentrated_keys
 
 pytestmark = pytest.mark.gpu
@@ -135,3 +135,105 @@ def test_rehash_build_invalid_args(gpu):
     assert f(hm.bucket_ptr(), 10, b2.data_ptr(), 11, None, sc.data_ptr(), sb, None) == _lib.HN_EINVAL
     torch.cuda.synchronize()
     assert hm.getSizePower() == 10 and hm.info().size_power == 10  # nothing ran
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("form", ["soa", "pairs", "index"])
+@pytest.mark.parametrize("old_sp,new_sp,n", [(1, 2, 1), (3, 5, 20), (6, 7, 60), (10, 11, 1000), (10, 14, 4096),
+                                             (12, 13, 3900), (13, 15, 1), (14, 16, 30000), (17, 19, 200003)])
+def test_grow_is_rehash_and_insert(gpu, bits, form, old_sp, new_sp, n):
+    """hn_grow_*: the old table's live slots (tombstones among them) and a
+    batch of new keys, keys of the table and keys of its own, in one build;
+    the image and Info are the oracle's insert of both and reorder."""
+    from tests.test_gpu_merge import batch, check_merge
+    from tests.test_gpu_build import dev
+    from hashinator_amd import _lib, to_numpy
+    L, sfx = _lib.load(), f"u{bits}"
+    N0, N1 = 1 << old_sp, 1 << new_sp
+    old = fresh_model(old_sp, bits)
+    ok = keyset(max(1, int(0.6 * N0)), bits, seed=old_sp + bits)
+    old.insert(ok, (ok ^ NDT[bits](0x77)).astype(NDT[bits]))
+    old.erase(ok[::4])
+    img = old.b.reshape(-1, 2)
+    live = img[(img[:, 0] != EMPTY[bits]) & (img[:, 0] != TOMB[bits])]
+    keys, vals = batch(bits, ok, max(1, int(n / 1.2)), seed=new_sp)
+    keys, vals = keys[:n], vals[:n]
+    if form == "index":
+        vals = np.arange(keys.size).astype(NDT[bits])
+    m = fresh_model(new_sp, bits)
+    m.insert_pairs(live.reshape(-1).copy())
+    assert m.insert(keys, vals) == 0
+    assert m.reorder() == 1
+    ob = dev(img.copy(), bits)
+    inf = torch.from_numpy(np.frombuffer(bytes(old.info), dtype=np.int64).copy()).cuda()
+    nb = torch.full((N1, 2), 0x5A5A, dtype=ob.dtype, device="cuda")
+    sb = getattr(L, f"hn_grow_scratch_bytes_{sfx}")(old_sp, new_sp, keys.size)
+    assert sb > 0
+    sc = torch.empty(sb, dtype=torch.uint8, device="cuda")
+    tail = (ob.data_ptr(), old_sp, nb.data_ptr(), new_sp, inf.data_ptr(), keys.size, sc.data_ptr(), sb, None)
+    if form == "pairs":
+        dp = dev(np.stack([keys, vals], axis=1), bits)
+        rc = getattr(L, f"hn_grow_pairs_{sfx}")(dp.data_ptr(), *tail)
+    else:
+        dk, dv = dev(keys, bits), dev(vals, bits)
+        rc = getattr(L, f"hn_grow_{sfx}")(dk.data_ptr(), None if form == "index" else dv.data_ptr(), *tail)
+    torch.cuda.synchronize()
+    assert rc == 0 and int(inf[0]) == new_sp
+    check_merge(bits, to_numpy(nb, bits).reshape(-1, 2), inf.cpu().numpy(), m)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_grow_declines_and_falls_back(gpu, bits):
+    """Sizes that do not fit are refused; keys that crowd one region are
+    placed by probing, the old table's first: the batch's values win."""
+    from tests.test_gpu_build import dev
+    from hashinator_amd import _lib, to_numpy
+    L, sfx = _lib.load(), f"u{bits}"
+    scratch = getattr(L, f"hn_grow_scratch_bytes_{sfx}")
+    assert scratch(10, 10, 5) == 0 and scratch(10, 11, 1024) == 0 and scratch(10, 11, 0) == 0 and scratch(10, 33, 5) == 0
+    old_sp, new_sp = 12, 14
+    cand = keyset(60 * 4096, bits, seed=5)
+    home = O.fibhash(cand, new_sp, bits).astype(np.int64) & ((1 << new_sp) - 1)
+    crowd = cand[(home >= 2048) & (home < 4096)][:2900]
+    ok = crowd[:2000]
+    old = fresh_model(old_sp, bits)
+    old.insert(ok, ok)
+    keys = np.concatenate([crowd[1000:2900], cand[home >= 8192][:3000]])
+    vals = (keys ^ NDT[bits](0x11)).astype(NDT[bits])
+    m = fresh_model(new_sp, bits)
+    m.insert(ok, ok)
+    m.insert(keys, vals)
+    ob, dk, dv = dev(old.b.reshape(-1, 2).copy(), bits), dev(keys, bits), dev(vals, bits)
+    inf = torch.from_numpy(np.frombuffer(bytes(old.info), dtype=np.int64).copy()).cuda()
+    nb = torch.empty((1 << new_sp, 2), dtype=ob.dtype, device="cuda")
+    sb = scratch(old_sp, new_sp, keys.size)
+    sc = torch.empty(sb, dtype=torch.uint8, device="cuda")
+    assert getattr(L, f"hn_grow_{sfx}")(dk.data_ptr(), dv.data_ptr(), ob.data_ptr(), old_sp, nb.data_ptr(), new_sp,
+                                        inf.data_ptr(), keys.size, sc.data_ptr(), sb, None) == 0
+    torch.cuda.synchronize()
+    img, after = to_numpy(nb, bits).reshape(-1, 2), inf.cpu().numpy()
+    assert np.array_equal(live_pairs(img, bits), live_pairs(m.b, bits)) and reachable_all(img, bits, new_sp)
+    assert (int(after[1]), int(after[3]), int(after[4])) == (m.info.fill, 0, 0)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("lf,frac", [(0.9, 1 / 8), (0.9, 1 / 20), (0.8, 1 / 8)])
+def test_map_insert_near_full(gpu, bits, lf, frac):
+    """Inserts below the merge's share of the table: merged into a map that
+    ends at least 85% full, probed otherwise; the bucket array stays."""
+    sp = 18
+    N = 1 << sp
+    n, tot = int(frac * N), int(lf * N)
+    keys = keyset(tot, bits, seed=77)
+    hm = Hashmap(sp, bits, build_min_keys=1)
+    hm.insert(keys[n:], keys[n:], targetLF=1.0)
+    at = hm.bucket_ptr()
+    again = np.concatenate([keys[:n], keys[n:n + 500]])
+    vals = (again + NDT[bits](3)).astype(NDT[bits])
+    hm.insert(again, vals, targetLF=1.0)
+    assert hm.bucket_ptr() == at and hm.size() == tot and hm.peek_status() == 0
+    assert hm.ordered() == (n >= N // 16)
+    exp = dict(zip(keys.tolist(), keys.tolist()))
+    exp.update(zip(again.tolist(), vals.tolist()))
+    rows = live_pairs(hm.host_buckets(), bits)
+    assert np.array_equal(rows, np.array(sorted(exp.items()), dtype=NDT[bits]))
