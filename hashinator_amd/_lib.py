@@ -90,6 +90,8 @@ SIGNATURES = {
     "hn_insert_pairs_u64": (I, [P, P, P, S, P, TUNE]),
     "hn_retrieve_u32": (I, [P, P, P, P, P, S, P, TUNE]),
     "hn_retrieve_u64": (I, [P, P, P, P, P, S, P, TUNE]),
+    "hn_retrieve_zero_u32": (I, [P, P, P, P, P, S, P, TUNE]),
+    "hn_retrieve_zero_u64": (I, [P, P, P, P, P, S, P, TUNE]),
     "hn_retrieve_pairs_u32": (I, [P, P, P, P, S, P, TUNE]),
     "hn_retrieve_pairs_u64": (I, [P, P, P, P, S, P, TUNE]),
     "hn_erase_u32": (I, [P, P, P, S, P, TUNE]),

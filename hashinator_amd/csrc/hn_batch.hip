@@ -158,13 +158,13 @@ __global__ __launch_bounds__(1024) void k_batch(BatchArgs<K> a) {
       }
       if ((a.ops & HN_BATCH_RETRIEVE) && sp_ok) {
          LookupArgs<K> la{a.qry_keys + M.qry_off, a.qry_vals + M.qry_off, nullptr,
-                          a.qry_hit ? a.qry_hit + M.qry_off : nullptr, b, info, M.qry_len};
+                          a.qry_hit ? a.qry_hit + M.qry_off : nullptr, b, info, M.qry_len, false};
          lookup_range<K, G, false, LK_RETRIEVE>(la, sp, info->current_max_bucket_overflow, M.qry_len, g, groups,
                                                 (info->reserved1 & kInfoOrdered) != 0);
          phase_barrier();
       }
       if ((a.ops & HN_BATCH_ERASE) && sp_ok) {
-         LookupArgs<K> la{a.ers_keys + M.ers_off, nullptr, nullptr, nullptr, b, info, M.ers_len};
+         LookupArgs<K> la{a.ers_keys + M.ers_off, nullptr, nullptr, nullptr, b, info, M.ers_len, false};
          const uint64_t e =
              wave_sum(lookup_range<K, G, false, LK_ERASE>(la, sp, info->current_max_bucket_overflow, M.ers_len, g, groups,
                                                           (info->reserved1 & kInfoOrdered) != 0));
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(kWave) void k_batch_retrieve_lane(BatchArgs<K> a, B
          const bool ordered = (info->reserved1 & kInfoOrdered) != 0;
          LookupArgs<K> la{a.qry_keys + M.qry_off, a.qry_vals + M.qry_off, nullptr,
                           a.qry_hit ? a.qry_hit + M.qry_off : nullptr, static_cast<Slot<K>*>(M.buckets), info,
-                          M.qry_len};
+                          M.qry_len, false};
          if (sp >= LaneWin<K>::kLog && ovf > 0) {
             lane_lookup<K, false, LK_RETRIEVE>(la, sp, ovf, ordered, q0, q1, L);
          } else {

@@ -151,6 +151,18 @@ __global__ void k_insert_finish(hn_info* info, const uint64_t* expected_fill) {
    info->reserved1 = 0;
 }
 
+// A size power that no table has: nothing is found, and a caller that left its
+// values to the kernel gets its zeros all the same.
+template <typename K, bool PAIRS, int MODE>
+__device__ __forceinline__ void zero_vals(const LookupArgs<K>& a) {
+   if constexpr (MODE == LK_RETRIEVE && !PAIRS) {
+      if (!a.zero) return;
+      const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+      for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < a.len; i += stride)
+         a.vals[i] = 0;
+   }
+}
+
 // retrieve_kernel (kernels_AMD.h:647-752), delete_kernel (412-505), reset_to_empty (65-134)
 template <typename K, int G, bool PAIRS, int MODE>
 __global__ __launch_bounds__(1024) void k_lookup(LookupArgs<K> a) {
@@ -162,6 +174,8 @@ __global__ __launch_bounds__(1024) void k_lookup(LookupArgs<K> a) {
    if (sp_ok)
       erased = lookup_range<K, G, PAIRS, MODE>(a, sp, a.info->current_max_bucket_overflow, a.len, blk, gstride,
                                                (a.info->reserved1 & kInfoOrdered) != 0);
+   else
+      zero_vals<K, PAIRS, MODE>(a);
    if constexpr (MODE == LK_ERASE) {
       erased = wave_sum(erased);
       if (__lane_id() == 0 && erased) {
@@ -203,6 +217,8 @@ __global__ __launch_bounds__(kLaneBlock) void k_lookup_lane(LookupArgs<K> a) {
          const uint64_t blk = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
          erased = lookup_range<K, 1, PAIRS, MODE>(a, sp, ovf, a.len, blk, gstride, ordered);
       }
+   } else {
+      zero_vals<K, PAIRS, MODE>(a);
    }
    if constexpr (MODE == LK_ERASE) {
       erased = wave_sum(erased);
@@ -528,11 +544,11 @@ int insert_pairs(const void* pairs, void* buckets, hn_info* info, size_t len, hi
 
 template <typename K>
 int retrieve_soa(const K* keys, K* vals, uint8_t* hit, const void* buckets, const hn_info* info, size_t len,
-                 hipStream_t s, const hn_tune* t) {
+                 hipStream_t s, const hn_tune* t, bool zero) {
    if (!buckets || !info || (len && (!keys || !vals))) return HN_EINVAL;
    if (len == 0) return 0;
    LookupArgs<K> a{keys, vals, nullptr, hit, const_cast<Slot<K>*>(static_cast<const Slot<K>*>(buckets)),
-                   const_cast<hn_info*>(info), len};
+                   const_cast<hn_info*>(info), len, zero};
    return launch_lookup<K, false, LK_RETRIEVE>(a, s, t, OP_RETRIEVE);
 }
 
@@ -542,7 +558,7 @@ int retrieve_pairs(void* pairs, uint8_t* hit, const void* buckets, const hn_info
    if (!buckets || !info || (len && !pairs)) return HN_EINVAL;
    if (len == 0) return 0;
    LookupArgs<K> a{nullptr, nullptr, static_cast<Slot<K>*>(pairs), hit,
-                   const_cast<Slot<K>*>(static_cast<const Slot<K>*>(buckets)), const_cast<hn_info*>(info), len};
+                   const_cast<Slot<K>*>(static_cast<const Slot<K>*>(buckets)), const_cast<hn_info*>(info), len, false};
    return launch_lookup<K, true, LK_RETRIEVE>(a, s, t, OP_RETRIEVE);
 }
 
@@ -550,7 +566,7 @@ template <typename K>
 int erase_keys(const K* keys, void* buckets, hn_info* info, size_t len, hipStream_t s, const hn_tune* t) {
    if (!buckets || !info || (len && !keys)) return HN_EINVAL;
    if (len == 0) return 0;
-   LookupArgs<K> a{keys, nullptr, nullptr, nullptr, static_cast<Slot<K>*>(buckets), info, len};
+   LookupArgs<K> a{keys, nullptr, nullptr, nullptr, static_cast<Slot<K>*>(buckets), info, len, false};
    return launch_lookup<K, false, LK_ERASE>(a, s, t, OP_ERASE);
 }
 
@@ -559,7 +575,7 @@ int reset_keys(const void* pairs, void* buckets, hn_info* info, size_t len, hipS
    if (!buckets || !info || (len && !pairs)) return HN_EINVAL;
    if (len == 0) return 0;
    LookupArgs<K> a{nullptr, nullptr, const_cast<Slot<K>*>(static_cast<const Slot<K>*>(pairs)), nullptr,
-                   static_cast<Slot<K>*>(buckets), info, len};
+                   static_cast<Slot<K>*>(buckets), info, len, false};
    return launch_lookup<K, true, LK_RESET>(a, s, nullptr, OP_ERASE);
 }
 
@@ -771,11 +787,19 @@ int hn_insert_pairs_u64(const void* p, void* b, hn_info* i, size_t n, hn_stream_
 }
 int hn_retrieve_u32(const uint32_t* k, uint32_t* v, uint8_t* h, const void* b, const hn_info* i, size_t n,
                     hn_stream_t s, const hn_tune* t) {
-   return retrieve_soa<uint32_t>(k, v, h, b, i, n, s, t);
+   return retrieve_soa<uint32_t>(k, v, h, b, i, n, s, t, false);
 }
 int hn_retrieve_u64(const uint64_t* k, uint64_t* v, uint8_t* h, const void* b, const hn_info* i, size_t n,
                     hn_stream_t s, const hn_tune* t) {
-   return retrieve_soa<uint64_t>(k, v, h, b, i, n, s, t);
+   return retrieve_soa<uint64_t>(k, v, h, b, i, n, s, t, false);
+}
+int hn_retrieve_zero_u32(const uint32_t* k, uint32_t* v, uint8_t* h, const void* b, const hn_info* i, size_t n,
+                         hn_stream_t s, const hn_tune* t) {
+   return retrieve_soa<uint32_t>(k, v, h, b, i, n, s, t, true);
+}
+int hn_retrieve_zero_u64(const uint64_t* k, uint64_t* v, uint8_t* h, const void* b, const hn_info* i, size_t n,
+                         hn_stream_t s, const hn_tune* t) {
+   return retrieve_soa<uint64_t>(k, v, h, b, i, n, s, t, true);
 }
 int hn_retrieve_pairs_u32(void* p, uint8_t* h, const void* b, const hn_info* i, size_t n, hn_stream_t s,
                           const hn_tune* t) {

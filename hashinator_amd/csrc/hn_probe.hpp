@@ -211,6 +211,7 @@ struct LookupArgs {
    Slot<K>* buckets;
    hn_info* info;
    uint64_t len;
+   bool zero; // SoA retrieve: vals[i] = 0 on a miss, instead of untouched
 };
 
 enum LookupMode { LK_RETRIEVE = 0, LK_ERASE = 1, LK_RESET = 2 };
@@ -299,12 +300,10 @@ __device__ __forceinline__ uint64_t lookup_range(const LookupArgs<K>& a, const i
       if constexpr (MODE == LK_RETRIEVE) {
          const uint64_t q = blk * G + static_cast<uint64_t>(gl);
          if (q < len) {
-            if (res_hit) {
-               if constexpr (PAIRS) {
-                  a.pairs[q].val = res_val;
-               } else {
-                  a.vals[q] = res_val;
-               }
+            if constexpr (PAIRS) {
+               if (res_hit) a.pairs[q].val = res_val;
+            } else {
+               if (res_hit || a.zero) a.vals[q] = res_hit ? res_val : 0;
             }
             if (a.hit) a.hit[q] = res_hit ? 1 : 0;
          }
@@ -564,8 +563,8 @@ __device__ __forceinline__ uint64_t lane_lookup(const LookupArgs<K>& a, const in
                const uint64_t e = lo + static_cast<uint64_t>(lane);
                if (static_cast<uint64_t>(lane) < run) {
                   const uint8_t st = L.ring_s[e & kRingMask];
-                  if (st == 1) {
-                     const K v = L.ring_v[e & kRingMask];
+                  if (st == 1 || (!PAIRS && a.zero)) {
+                     const K v = st == 1 ? L.ring_v[e & kRingMask] : 0;
                      if constexpr (PAIRS) {
                         a.pairs[e].val = v;
                      } else {

@@ -478,10 +478,12 @@ class Hashmap:
             vals = out_tensor(vals, n, _TDT[self.kb], self.device, "vals")
         if hit is not None:
             hit = out_tensor(hit, n, torch.uint8, self.device, "hit")
-        v = vals if vals is not None else torch.zeros(n, dtype=_TDT[self.kb], device=self.device)
+        # values of its own: the kernel writes the misses' zeros too
+        v = vals if vals is not None else torch.empty(n, dtype=_TDT[self.kb], device=self.device)
         h = hit if hit is not None else torch.empty(n, dtype=torch.uint8, device=self.device)
-        check(self._fn("retrieve")(_ptr(k), _ptr(v), _ptr(h), _ptr(self.buckets), _ptr(self._info), n,
-                                   _stream(stream), self._tune()), "retrieve")
+        fn = self._fn("retrieve_zero" if vals is None else "retrieve")
+        check(fn(_ptr(k), _ptr(v), _ptr(h), _ptr(self.buckets), _ptr(self._info), n, _stream(stream), self._tune()),
+              "retrieve")
         self._sync(stream)
         return k, v, h
 

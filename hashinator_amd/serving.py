@@ -312,11 +312,11 @@ class ServingEngine:
                                                           m.info.data_ptr(), n, s.cuda_stream, self.tune), "insert")
                 m.fill_upper += n
             elif kind == RETRIEVE:
-                dv = torch.zeros(n, dtype=_TDT[self.kb], device=self.dev)
+                dv = torch.empty(n, dtype=_TDT[self.kb], device=self.dev)
                 dh = torch.empty(n, dtype=torch.uint8, device=self.dev)
-                check(getattr(L, f"hn_retrieve_{sfx}")(dk.data_ptr(), dv.data_ptr(), dh.data_ptr(),
-                                                        m.buckets.data_ptr(), m.info.data_ptr(), n, s.cuda_stream,
-                                                        self.tune), "retrieve")
+                check(getattr(L, f"hn_retrieve_zero_{sfx}")(dk.data_ptr(), dv.data_ptr(), dh.data_ptr(),
+                                                             m.buckets.data_ptr(), m.info.data_ptr(), n,
+                                                             s.cuda_stream, self.tune), "retrieve")
                 hv = torch.empty(n, dtype=_TDT[self.kb], pin_memory=True)
                 hh = torch.empty(n, dtype=torch.uint8, pin_memory=True)
                 hv.copy_(dv, non_blocking=True)

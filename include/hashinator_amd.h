@@ -157,6 +157,12 @@ HN_API int hn_retrieve_u32(const uint32_t* keys, uint32_t* vals, uint8_t* hit, c
                     const hn_info* info, size_t len, hn_stream_t s, const hn_tune* t);
 HN_API int hn_retrieve_u64(const uint64_t* keys, uint64_t* vals, uint8_t* hit, const void* buckets,
                     const hn_info* info, size_t len, hn_stream_t s, const hn_tune* t);
+/* The same with vals[i] = 0 on a miss: vals need not be initialised, and the
+ * values of a run of queries leave in whole lines. */
+HN_API int hn_retrieve_zero_u32(const uint32_t* keys, uint32_t* vals, uint8_t* hit, const void* buckets,
+                                const hn_info* info, size_t len, hn_stream_t s, const hn_tune* t);
+HN_API int hn_retrieve_zero_u64(const uint64_t* keys, uint64_t* vals, uint8_t* hit, const void* buckets,
+                                const hn_info* info, size_t len, hn_stream_t s, const hn_tune* t);
 
 /* Hasher::retrieve(src pairs, ...) (hashers.h:121-129) -> retrieve_kernel over
  * hash_pair (kernels_AMD.h:703-752): src[i].second is written on a hit. */

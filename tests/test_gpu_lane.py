@@ -178,3 +178,27 @@ def test_lane_repeated_keys_in_windows(gpu, bits, sp, bound):
         hm.erase(e)
         model.erase(e)
         assert np.array_equal(hm.host_buckets().reshape(-1), model.b)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("width", [0, 1, 4])
+@pytest.mark.parametrize("sp", [1, 3, 10, 33])
+def test_retrieve_zero_fills_misses(gpu, bits, width, sp):
+    """hn_retrieve_zero_*: the hits' values and zeros, whatever was there
+    before; zeros throughout for an Info whose size power is no table's."""
+    import ctypes as C
+    L, bad = _lib.load(), sp == 33
+    hm, model, keys = make(bits, min(sp, 10), 0.7, seed=sp + bits, ordered=True)
+    q = queries(keys, bits, seed=sp)[:777]
+    dq = torch.from_numpy(q.view(TD[bits])).cuda()
+    v = torch.full((q.size,), 0x5A, dtype=dq.dtype, device="cuda")
+    h = torch.zeros(q.size, dtype=torch.uint8, device="cuda")
+    if bad:
+        hm._info.view(torch.int32)[0] = 33
+    t = hn_tune(width, 256, 0, 0) if width else None
+    rc = getattr(L, f"hn_retrieve_zero_u{bits}")(dq.data_ptr(), v.data_ptr(), h.data_ptr(), hm.bucket_ptr(),
+                                                 hm.info_ptr(), q.size, None, C.byref(t) if t else None)
+    torch.cuda.synchronize()
+    ev, eh = model.retrieve(q, np.zeros(q.size, dtype=NDT[bits]))
+    assert rc == 0 and np.array_equal(to_numpy(v, bits), np.zeros_like(ev) if bad else ev)
+    assert np.array_equal(h.cpu().numpy().astype(bool), np.zeros_like(eh) if bad else eh)
