@@ -1,7 +1,7 @@
 /* split_compact.h -- single-pass stable stream compaction for gfx950, as a
  * template over the element type, the selector and the projection.
  *
- * One kernel over tiles of 8,192 elements (1,024 threads, 8 each) with
+ * One kernel over tiles of 8,192 or 16,384 elements (1,024 threads) with
  * decoupled look-back: a tile takes a ticket (so every tile it waits on has
  * already started), counts its selected elements with wave ballots,
  * publishes that aggregate, folds its predecessors' published values 64 at
@@ -38,13 +38,23 @@ namespace compact {
 
 // Large tiles because every tile pays a serial cost, its ticket and its step
 // in the look-back chain: at 2^28 elements, 256-thread tiles ran copy_if in
-// 2.0 ms; 1,024 threads with 8 elements each take 1.23 ms (4 or 16 elements
-// per thread were slower).
+// 2.0 ms; 1,024 threads with 8 elements each take 1.23 ms.  16 each where a
+// thread keeps at most 8 bytes of an element between its count and its write
+// (small elements, and pairs of which the keys are taken): 2^27 pairs, 30%
+// kept, u64 keys 0.58 -> 0.52 ms, u32 pairs 0.47 -> 0.39, u32 keys 0.44 ->
+// 0.35; whole u64 pairs 0.63 -> 0.67, their registers leaving one workgroup
+// on a CU (in the caches they gain too: 2^23 pairs 48 -> 43 us, 2^24
+// 93 -> 94).  From kLargeMin elements on: below, the larger tiles are too few
+// for the CUs (u32 pairs: 2^21 18.0 -> 20.0 us, 2^22 24.5 -> 23.2).  (Workgroups that take tile after tile, with the next tile's
+// elements loaded or not while the current one waits for its prefix, were
+// slower than one workgroup per tile, two on a CU: 0.65 to 0.72 ms and 0.57
+// at best for the u64 keys.)
 constexpr int kThreads = 1024;
 constexpr int kWaveSize = 64;
 constexpr int kWaves = kThreads / kWaveSize;
-constexpr int kPerThread = 8;
-constexpr uint64_t kTile = static_cast<uint64_t>(kThreads) * kPerThread;
+constexpr int kPerThread = 8, kPerThreadLarge = 16;
+constexpr uint64_t kTile = static_cast<uint64_t>(kThreads) * kPerThread; // the smaller tile: scratch is sized by it
+constexpr uint64_t kLargeMin = 1ull << 22, kLargeMax = 1ull << 24;
 
 // A tile's look-back word: state in the top two bits (0 not yet published,
 // 1 aggregate, 2 inclusive prefix), the element count below.  Words are
@@ -158,25 +168,25 @@ __global__ __launch_bounds__(256) void k_prepare(TileState st, uint64_t tiles, C
 // element leaves the edit in the input, as a rule run on the element in
 // place does; for a rule that edits nothing the check folds away at compile
 // time.
-template <typename In, typename Out, class Sel, class Proj>
+template <int PER_THREAD, typename In, typename Out, class Sel, class Proj>
 __global__ __launch_bounds__(kThreads) void k_compact(In* __restrict__ in, uint64_t n, Out* __restrict__ out,
                                                       uint64_t* count, TileState st, uint64_t tiles, Sel sel,
                                                       Proj proj) {
    using T = typename std::remove_cv<In>::type;
    __shared__ uint32_t s_tile;
-   __shared__ uint32_t s_cnt[kPerThread][kWaves];
+   __shared__ uint32_t s_cnt[PER_THREAD][kWaves];
    __shared__ uint64_t s_prefix;
    const int lane = __lane_id();
    const int wave = threadIdx.x / kWaveSize;
    if (threadIdx.x == 0) s_tile = __hip_atomic_fetch_add(st.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
    __syncthreads();
    const uint32_t tile = s_tile;
-   const uint64_t base = static_cast<uint64_t>(tile) * kTile;
+   const uint64_t base = static_cast<uint64_t>(tile) * kThreads * PER_THREAD;
 
-   T v[kPerThread];
-   uint64_t bal[kPerThread];
+   T v[PER_THREAD];
+   uint64_t bal[PER_THREAD];
 #pragma unroll
-   for (int j = 0; j < kPerThread; ++j) {
+   for (int j = 0; j < PER_THREAD; ++j) {
       const uint64_t i = base + static_cast<uint64_t>(j) * kThreads + threadIdx.x;
       bool keep = false;
       if (i < n) {
@@ -196,7 +206,7 @@ __global__ __launch_bounds__(kThreads) void k_compact(In* __restrict__ in, uint6
    if (wave == 0) {
       // Exclusive prefix of the counts, j-major and wave-minor (= input
       // order), by one wave: each lane scans PER consecutive counts.
-      constexpr int E = kPerThread * kWaves;
+      constexpr int E = PER_THREAD * kWaves;
       constexpr int PER = (E + kWaveSize - 1) / kWaveSize;
       uint32_t* flat = &s_cnt[0][0];
       uint32_t c[PER];
@@ -226,7 +236,7 @@ __global__ __launch_bounds__(kThreads) void k_compact(In* __restrict__ in, uint6
    const uint64_t pre = s_prefix;
    const uint64_t below = (1ull << lane) - 1ull;
 #pragma unroll
-   for (int j = 0; j < kPerThread; ++j) {
+   for (int j = 0; j < PER_THREAD; ++j) {
       if ((bal[j] >> lane) & 1ull) {
          const uint64_t r = pre + s_cnt[j][wave] + static_cast<uint64_t>(__popcll(bal[j] & below));
          out[r] = proj(v[j]);
@@ -258,14 +268,22 @@ struct RuleSel {
 // number.  scratch: scratch_bytes(n) bytes of device memory.
 template <typename In, typename Out, class Sel, class Proj>
 hipError_t launch(In* in, uint64_t n, Out* out, uint64_t* count, void* scratch, hipStream_t s, Sel sel, Proj proj) {
-   const uint64_t tiles = tiles_for(n);
+   constexpr bool kFits = sizeof(In) <= 16, kKeepsLittle = kFits && (sizeof(In) <= 8 || sizeof(Out) <= 8);
+   const bool large = kFits && n >= kLargeMin && (kKeepsLittle || n < kLargeMax);
+   const uint64_t per = static_cast<uint64_t>(kThreads) * (large ? kPerThreadLarge : kPerThread);
+   const uint64_t tiles = (n + per - 1) / per;
    const TileState st = state_at(scratch);
    const uint64_t want = (tiles + 255) / 256;
    const unsigned blocks = want == 0 ? 1u : static_cast<unsigned>(want < 2048 ? want : 2048);
    hipLaunchKernelGGL(k_prepare<uint64_t>, dim3(blocks), dim3(256), 0, s, st, tiles, count);
-   if (tiles)
-      hipLaunchKernelGGL((k_compact<In, Out, Sel, Proj>), dim3(static_cast<uint32_t>(tiles)), dim3(kThreads), 0, s,
-                         in, n, out, count, st, tiles, sel, proj);
+   const dim3 grid(static_cast<uint32_t>(tiles));
+   if constexpr (kFits)
+      if (large)
+         hipLaunchKernelGGL((k_compact<kPerThreadLarge, In, Out, Sel, Proj>), grid, dim3(kThreads), 0, s, in, n, out,
+                            count, st, tiles, sel, proj);
+   if (tiles && !large)
+      hipLaunchKernelGGL((k_compact<kPerThread, In, Out, Sel, Proj>), grid, dim3(kThreads), 0, s, in, n, out, count, st,
+                         tiles, sel, proj);
    return hipGetLastError();
 }
 

@@ -116,3 +116,38 @@ def test_extract_pattern_on_map_snapshot(gpu, bits):
     assert np.array_equal(to_numpy(hm.extractPatternLoop(), bits).reshape(-1, 2), exp)
     assert np.array_equal(to_numpy(hm.extractAllKeysLoop(), bits), exp[:, 0])
     assert np.array_equal(to_numpy(hm.extractKeysByPatternLoop(lt), bits), got)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("n", [(1 << 22) - 1, 1 << 22, (1 << 22) + 16385, (1 << 24) - 1, 1 << 24])
+def test_compaction_tile_sizes(gpu, bits, n):
+    """Around the element counts at which the tile changes: pairs and keys by
+    a rule, elements by flags, against torch's own mask selection."""
+    import ctypes as C
+    from hashinator_amd import _lib
+    L = _lib.load()
+    dt = torch.int32 if bits == 32 else torch.int64
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + bits)
+    x = torch.randint(0, 1 << 30, (n, 2), dtype=dt, device="cuda", generator=g)
+    lim = 3 << 28
+    pr = _lib.hn_pred()
+    pr.kind, pr.field, pr.value = _lib.HN_PRED_LT, 0, lim
+    sb = int(L.hn_compact_scratch_bytes(n))
+    sc = torch.empty(sb, dtype=torch.uint8, device="cuda")
+    cnt = torch.zeros(1, dtype=torch.int64, device="cuda")
+    out, keys = torch.full_like(x, -1), torch.full((n,), -1, dtype=dt, device="cuda")
+    keep = x[:, 0] < lim
+    m = int(keep.sum())
+    u = f"u{bits}"
+    assert getattr(L, f"hn_copy_if_pairs_{u}")(x.data_ptr(), n, C.byref(pr), out.data_ptr(), cnt.data_ptr(),
+                                               sc.data_ptr(), sb, None) == 0
+    assert int(cnt) == m and torch.equal(out[:m], x[keep]) and bool((out[m:] == -1).all())
+    assert getattr(L, f"hn_copy_keys_if_pairs_{u}")(x.data_ptr(), n, C.byref(pr), keys.data_ptr(), cnt.data_ptr(),
+                                                    sc.data_ptr(), sb, None) == 0
+    assert int(cnt) == m and torch.equal(keys[:m], x[:, 0][keep]) and bool((keys[m:] == -1).all())
+    flags = keep.to(torch.uint8)
+    out.fill_(-1)
+    assert L.hn_copy_if_flags(x.data_ptr(), flags.data_ptr(), n, bits // 4, out.data_ptr(), cnt.data_ptr(),
+                              sc.data_ptr(), sb, None) == 0
+    assert int(cnt) == m and torch.equal(out[:m], x[keep])
