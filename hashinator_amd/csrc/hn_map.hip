@@ -54,6 +54,7 @@ template <typename K, int G, int SRC>
 __global__ __launch_bounds__(1024) void k_insert(InsertArgs<K> a) {
    const int sp = a.info->size_power;
    const bool sp_ok = sp >= 1 && sp <= max_size_power<K>();
+   if (a.d_len && *a.d_len == 0) return; // a build's fallback that is not needed
    const uint64_t len = !sp_ok ? 0 : (a.d_len ? *a.d_len : a.len);
    const uint64_t gstride = static_cast<uint64_t>(gridDim.x) * (blockDim.x / G);
    const uint64_t blk = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G;
@@ -189,15 +190,17 @@ __global__ __launch_bounds__(1024) void k_lookup(LookupArgs<K> a) {
    }
 }
 
-// Lane-window lookups (one key per lane, see lane_lookup): one wave per
-// block (no block-level cooperation; single-wave blocks pack the LDS of a CU
-// best), each with its own staging and its own contiguous share of the
-// queries.  Tables smaller than one 128-byte window (and a zero probe bound)
-// take the group loop with one lane per key.
-constexpr int kLaneBlock = 64;
+// Lane-window lookups (one key per lane, see lane_lookup): each wave with its
+// own LDS and its own contiguous share of the queries.  Tables smaller than
+// one 128-byte window (and a zero probe bound) take the group loop with one
+// lane per key.  One wave per block, four for an erase, which adds its count
+// to the Info once per block (two atomics, some 16 ns each one after another:
+// 2^24 u64 erases in 2^26 slots 0.89 -> 0.85 ms).
+constexpr int lane_block(int mode) { return mode == LK_ERASE ? 256 : kWave; }
 template <typename K, bool PAIRS, int MODE>
-__global__ __launch_bounds__(kLaneBlock) void k_lookup_lane(LookupArgs<K> a) {
-   __shared__ LaneLds<K, MODE> L[kLaneBlock / kWave];
+__global__ __launch_bounds__(lane_block(MODE)) void k_lookup_lane(LookupArgs<K> a) {
+   constexpr int kWaves = lane_block(MODE) / kWave;
+   __shared__ LaneLds<K, MODE> L[kWaves];
    const int sp = a.info->size_power;
    const bool sp_ok = sp >= 1 && sp <= max_size_power<K>();
    const uint64_t ovf = a.info->current_max_bucket_overflow;
@@ -206,8 +209,8 @@ __global__ __launch_bounds__(kLaneBlock) void k_lookup_lane(LookupArgs<K> a) {
    if (sp_ok) {
       if (sp >= LaneWin<K>::kLog && ovf > 0) {
          const int wv = threadIdx.x / kWave;
-         const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * (kLaneBlock / kWave);
-         const uint64_t w = static_cast<uint64_t>(blockIdx.x) * (kLaneBlock / kWave) + wv;
+         const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * kWaves;
+         const uint64_t w = static_cast<uint64_t>(blockIdx.x) * kWaves + wv;
          const uint64_t per = a.len / nwaves, rem = a.len % nwaves;
          const uint64_t q0 = w * per + (w < rem ? w : rem);
          const uint64_t q1 = q0 + per + (w < rem ? 1 : 0);
@@ -221,10 +224,16 @@ __global__ __launch_bounds__(kLaneBlock) void k_lookup_lane(LookupArgs<K> a) {
       zero_vals<K, PAIRS, MODE>(a);
    }
    if constexpr (MODE == LK_ERASE) {
+      __shared__ unsigned long long erased_s;
+      if (threadIdx.x == 0) erased_s = 0;
+      __syncthreads();
       erased = wave_sum(erased);
-      if (__lane_id() == 0 && erased) {
-         atomic_add_relaxed(&a.info->tombstone_counter, erased);
-         __hip_atomic_fetch_sub(&a.info->fill, erased, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__lane_id() == 0 && erased) atomicAdd(&erased_s, static_cast<unsigned long long>(erased));
+      __syncthreads();
+      if (threadIdx.x == 0 && erased_s) {
+         const uint64_t e = erased_s;
+         atomic_add_relaxed(&a.info->tombstone_counter, e);
+         __hip_atomic_fetch_sub(&a.info->fill, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
    }
 }
@@ -492,7 +501,8 @@ int launch_lookup(LookupArgs<K> a, hipStream_t s, const hn_tune* t, OpKind op) {
          // One query per lane and up (at least 256 per wave left most of the
          // device idle: 1,000 queries of a 2^20-slot table took 17.8 us on four
          // waves, events included, and 10.5 us on 16).
-         uint64_t need = (a.len + kWave - 1) / kWave;
+         constexpr int kBlock = lane_block(MODE);
+         uint64_t need = (a.len + kBlock - 1) / kBlock;
          if (need == 0) need = 1;
          // one resident wave per block slot: the waves split the queries
          // statically, so a block that waits for a free slot would finish late
@@ -501,12 +511,12 @@ int launch_lookup(LookupArgs<K> a, hipStream_t s, const hn_tune* t, OpKind op) {
          // slots: 12 waves 1.24 ms, 16 and 20 1.07), beyond it more only queue
          // (2^24 slots: 16 waves 2.17 ms, 20 2.23; 2^28 2.93 and 2.97).
          const int per_cu =
-             std::min(resident_blocks_per_cu(k_lookup_lane<K, PAIRS, MODE>, kLaneBlock, occ), 16);
+             std::min(resident_blocks_per_cu(k_lookup_lane<K, PAIRS, MODE>, kBlock, occ), 16 * kWave / kBlock);
          uint64_t cap = (t && t->grid_blocks > 0) ? static_cast<uint64_t>(t->grid_blocks)
                                                   : static_cast<uint64_t>(cu_count()) * per_cu;
          if (cap > (1u << 20)) cap = 1u << 20;
          const uint32_t blocks = static_cast<uint32_t>(need < cap ? need : cap);
-         hipLaunchKernelGGL((k_lookup_lane<K, PAIRS, MODE>), dim3(blocks), dim3(kLaneBlock), 0, s, a);
+         hipLaunchKernelGGL((k_lookup_lane<K, PAIRS, MODE>), dim3(blocks), dim3(kBlock), 0, s, a);
          return static_cast<int>(hipGetLastError());
       }
    }
