@@ -544,6 +544,28 @@ __global__ __launch_bounds__(BS) void k_part_scatter(PartIn<K> in, uint64_t n_in
    }
 }
 
+// Inclusive sum and maximum over the wave: DPP row shifts inside 16-lane
+// rows, then row broadcasts across rows.
+__device__ __forceinline__ uint32_t wave_incl_add(uint32_t x) {
+   int v = static_cast<int>(x);
+   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false); // row_shr:1
+   v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false); // row_shr:2
+   v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false); // row_shr:4
+   v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false); // row_shr:8
+   v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15 -> rows 1, 3
+   v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31 -> rows 2, 3
+   return static_cast<uint32_t>(v);
+}
+__device__ __forceinline__ int32_t wave_incl_max(int32_t v) {
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x111, 0xf, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x112, 0xf, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x114, 0xf, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x118, 0xf, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x142, 0xa, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x143, 0xc, 0xf, false));
+   return v;
+}
+
 // Exclusive scan of x[0..m) in LDS by a whole workgroup; returns the total.
 template <int BS>
 __device__ uint32_t lds_exclusive_scan(uint32_t* x, uint32_t m, uint32_t* wsum) {
@@ -552,18 +574,15 @@ __device__ uint32_t lds_exclusive_scan(uint32_t* x, uint32_t m, uint32_t* wsum) 
    const uint32_t c0 = std::min<uint32_t>(threadIdx.x * per, m), c1 = std::min<uint32_t>(c0 + per, m);
    uint32_t acc = 0;
    for (uint32_t i = c0; i < c1; ++i) acc += x[i];
-   uint32_t inc = acc;
-#pragma unroll
-   for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t y = __shfl_up(inc, o, kWave);
-      if (lane >= o) inc += y;
-   }
+   const uint32_t inc = wave_incl_add(acc);
    if (lane == kWave - 1) wsum[wave] = inc;
    __syncthreads();
    uint32_t run = inc - acc, total = 0;
+#pragma unroll
    for (int w = 0; w < BS / kWave; ++w) {
-      if (w < wave) run += wsum[w];
-      total += wsum[w];
+      const uint32_t c = wsum[w];
+      run += w < wave ? c : 0u;
+      total += c;
    }
    for (uint32_t i = c0; i < c1; ++i) {
       const uint32_t v = x[i];
@@ -631,15 +650,17 @@ constexpr uint32_t kRegionMax = 1u << kRegionLog;
 // LDS of one region of at most IPT keys per thread: the sort tables are dead
 // once each key knows its sorted index, so the placement arrays reuse their
 // space.
+constexpr uint32_t kStage = kRegionMax + 512; // slots of a region's write span held at a time
 template <typename K, int IPT>
 struct RegionLds {
    static constexpr uint32_t kCap = kRegionBS * IPT;
-   static constexpr uint32_t kSpanWords = (kRegionMax + kCap + 31) / 32; // a region writes at most kRegionMax + kCap slots
-   K key[kCap];
-   uint16_t order[kCap];
    union {
-      uint8_t dup[kCap];
-      uint32_t occ[kSpanWords]; // slots of the write span holding a key
+      struct {
+         K key[kCap];
+         uint16_t order[kCap];
+         uint8_t dup[kCap];
+      } s;
+      Slot<K> out[kStage];
    } u1;
    union {
       struct {
@@ -648,7 +669,6 @@ struct RegionLds {
       } c;
       int32_t v[kCap]; // by sorted index f: home offset - f, then its running max
    } u2;
-   static_assert(sizeof(uint32_t) * kSpanWords <= kCap, "occupancy bits fit the dup table");
    static_assert(sizeof(int32_t) * kCap <= 2 * sizeof(uint32_t) * (kRegionMax + 1), "v fits the count tables");
    uint32_t wsum[kRegionNW];
    int32_t wmax[kRegionNW];
@@ -712,44 +732,63 @@ __device__ uint32_t region_sort(uint64_t R, RegionLds<K, IPT>& L, F has, const K
       const uint32_t e = threadIdx.x + k * kRegionBS;
       if (has(k)) {
          const uint32_t pos = L.u2.c.cnt[uu[k]] + sub[k];
-         L.key[pos] = kk[k];
-         L.order[pos] = static_cast<uint16_t>(e);
+         L.u1.s.key[pos] = kk[k];
+         L.u1.s.order[pos] = static_cast<uint16_t>(e);
       }
    }
    __syncthreads();
-   // rank among the home's keys; a later copy of the same key drops this one
-   uint32_t dupm = 0; // bit k: key k is dropped
-   int repeats = 0;
+   // Rank among the home's keys, several of a thread's keys side by side: the
+   // homes' entries are read one round after another, one wait each (a loop
+   // per key waited for each key's entries in turn; absent keys read entry 0).
+   // Two where there are eight, most of whose last rows are empty.
+   constexpr int SIDE = IPT <= 5 ? IPT : 2;
+   uint32_t twice = 0; // bit k: key k's home holds it more than once
 #pragma unroll
-   for (int k = 0; k < IPT; ++k) {
-      const uint32_t e = threadIdx.x + k * kRegionBS;
-      if (has(k)) {
-         const uint32_t j0 = L.u2.c.cnt[uu[k]], j1 = L.u2.c.cnt[uu[k] + 1];
-         int32_t rank = 0;
-         for (uint32_t j = j0; j < j1; ++j) {
-            const K kj = L.key[j];
-            const uint32_t oj = L.order[j];
-            rank += kj < kk[k] ? 1 : 0;
-            if (kj == kk[k] && oj != e) {
-               repeats = 1;
-               if (oj > e) dupm |= 1u << k;
-            }
-         }
-         ff[k] = rank;
+   for (int b = 0; b < IPT; b += SIDE) {
+      uint32_t j0[SIDE], jn[SIDE], eq[SIDE];
+#pragma unroll
+      for (int i = 0; i < SIDE; ++i) {
+         const bool h = b + i < IPT && has(b + i);
+         j0[i] = h ? L.u2.c.cnt[uu[b + i]] : 0;
+         jn[i] = h ? L.u2.c.cnt[uu[b + i] + 1] - j0[i] : 0;
+         eq[i] = 0;
+         if (b + i < IPT) ff[b + i] = h ? static_cast<int32_t>(j0[i]) : -1;
       }
+      for (uint32_t r = 0;; ++r) {
+         bool any = false;
+#pragma unroll
+         for (int i = 0; i < SIDE; ++i) any = any || r < jn[i];
+         if (!__ballot(any)) break;
+         K kj[SIDE];
+#pragma unroll
+         for (int i = 0; i < SIDE; ++i) kj[i] = L.u1.s.key[j0[i] + (r < jn[i] ? r : 0)];
+#pragma unroll
+         for (int i = 0; i < SIDE; ++i) {
+            if (b + i >= IPT) continue;
+            ff[b + i] += r < jn[i] && kj[i] < kk[b + i] ? 1 : 0;
+            eq[i] += r < jn[i] && kj[i] == kk[b + i] ? 1 : 0;
+         }
+      }
+#pragma unroll
+      for (int i = 0; i < SIDE; ++i) twice |= eq[i] > 1 ? 1u << (b + i) : 0u;
    }
    uint32_t ms;
-   if (!__syncthreads_or(repeats)) {
+   if (!__syncthreads_or(twice != 0)) {
       ms = m;
-#pragma unroll
-      for (int k = 0; k < IPT; ++k)
-         if (ff[k] >= 0) ff[k] += static_cast<int32_t>(L.u2.c.cnt[uu[k]]);
    } else {
+      uint32_t dupm = 0; // bit k: a later copy of key k drops it
+#pragma unroll
+      for (int k = 0; k < IPT; ++k) {
+         const uint32_t e = threadIdx.x + k * kRegionBS;
+         if ((twice >> k) & 1u)
+            for (uint32_t j = L.u2.c.cnt[uu[k]]; j < L.u2.c.cnt[uu[k] + 1]; ++j)
+               if (L.u1.s.key[j] == kk[k] && L.u1.s.order[j] > e) dupm |= 1u << k;
+      }
       for (uint32_t i = threadIdx.x; i <= R; i += kRegionBS) L.u2.c.scnt[i] = 0;
 #pragma unroll
       for (int k = 0; k < IPT; ++k) {
          const uint32_t e = threadIdx.x + k * kRegionBS;
-         if (has(k)) L.u1.dup[e] = (dupm >> k) & 1u;
+         if (has(k)) L.u1.s.dup[e] = (dupm >> k) & 1u;
       }
       __syncthreads();
 #pragma unroll
@@ -766,7 +805,7 @@ __device__ uint32_t region_sort(uint64_t R, RegionLds<K, IPT>& L, F has, const K
          }
          int32_t rank = 0;
          for (uint32_t j = L.u2.c.cnt[uu[k]]; j < L.u2.c.cnt[uu[k] + 1]; ++j)
-            rank += (!L.u1.dup[L.order[j]] && L.key[j] < kk[k]) ? 1 : 0;
+            rank += (!L.u1.s.dup[L.u1.s.order[j]] && L.u1.s.key[j] < kk[k]) ? 1 : 0;
          ff[k] = static_cast<int32_t>(L.u2.c.scnt[uu[k]]) + rank;
       }
    }
@@ -812,17 +851,16 @@ __device__ uint32_t region_place(RegionLds<K, IPT>& L, uint32_t ms, int64_t c, u
       const uint32_t j0 = std::min<uint32_t>(threadIdx.x * per, ms), j1 = std::min<uint32_t>(j0 + per, ms);
       int32_t acc = INT32_MIN;
       for (uint32_t j = j0; j < j1; ++j) acc = std::max(acc, L.u2.v[j]);
-      int32_t inc = acc;
-#pragma unroll
-      for (int o = 1; o < kWave; o <<= 1) {
-         const int32_t y = __shfl_up(inc, o, kWave);
-         if (lane >= o) inc = std::max(inc, y);
-      }
+      const int32_t inc = wave_incl_max(acc);
       if (lane == kWave - 1) L.wmax[wave] = inc;
       __syncthreads();
       int32_t run = __shfl_up(inc, 1, kWave);
       if (lane == 0) run = INT32_MIN;
-      for (int w = 0; w < wave; ++w) run = std::max(run, L.wmax[w]);
+#pragma unroll
+      for (int w = 0; w < kRegionNW; ++w) {
+         const int32_t c = L.wmax[w];
+         run = std::max(run, w < wave ? c : INT32_MIN);
+      }
       for (uint32_t j = j0; j < j1; ++j) {
          run = std::max(run, L.u2.v[j]);
          L.u2.v[j] = run;
@@ -832,37 +870,37 @@ __device__ uint32_t region_place(RegionLds<K, IPT>& L, uint32_t ms, int64_t c, u
    const int64_t last = ms ? static_cast<int64_t>(ms - 1) + std::max<int64_t>(L.u2.v[ms - 1], c) : -1;
    const int64_t end = std::max<int64_t>(static_cast<int64_t>(R), last + 1);
    const int64_t span = end - c;
-   const int64_t words = span > 0 ? (span + 31) / 32 : 0;
-   for (int64_t w = threadIdx.x; w < words; w += kRegionBS) L.u1.occ[w] = 0;
-   __syncthreads();
    auto kept = [&](uint64_t pos) { return keep == 1 || (keep == 0 ? pos < N : pos >= N); };
    uint32_t probe = 0;
-#pragma unroll
-   for (int k = 0; k < IPT; ++k) {
-      if (ff[k] >= 0) {
-         const int64_t p = ff[k] + std::max<int64_t>(L.u2.v[ff[k]], c);
-         const int64_t q = p - c;
-         atomicOr(&L.u1.occ[q >> 5], 1u << (q & 31));
-         const uint64_t pos = base + static_cast<uint64_t>(p);
-         if (kept(pos)) {
-            Slot<K> s;
-            s.key = kk[k];
-            s.val = vv[k];
-            b[pos & mask] = s;
-         }
-         probe = std::max<uint32_t>(probe, static_cast<uint32_t>(p - static_cast<int64_t>(uu[k]) + 1));
+   // The span leaves in slot order from LDS: stored from the threads that
+   // sorted them, a wave's 64 slots went to as many lines.  With the ranks
+   // side by side (region_sort) the builds of 2^28 slots at load .9 went from
+   // 7.94 to 7.67 ms (u64) and 5.82 to 5.56 (u32), a merge of 2^22 keys into
+   // 2^26 u32 slots from 0.93 to 0.83, into u64 slots 1.07 to 1.04.
+   for (int64_t s0 = 0; s0 < span; s0 += kStage) {
+      const uint32_t m = static_cast<uint32_t>(std::min<int64_t>(span - s0, kStage));
+      if (s0) __syncthreads(); // the pass before has been written out
+      for (uint32_t q = threadIdx.x; q < m; q += kRegionBS) {
+         L.u1.out[q].key = empty_key<K>();
+         L.u1.out[q].val = 0;
       }
-   }
-   __syncthreads();
-   for (int64_t q = threadIdx.x; q < span; q += kRegionBS) {
-      if (!((L.u1.occ[q >> 5] >> (q & 31)) & 1u)) {
-         const uint64_t pos = base + static_cast<uint64_t>(c + q);
-         if (kept(pos)) {
-            Slot<K> s;
-            s.key = empty_key<K>();
-            s.val = 0;
-            b[pos & mask] = s;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < IPT; ++k) {
+         if (ff[k] >= 0) {
+            const int64_t p = ff[k] + std::max<int64_t>(L.u2.v[ff[k]], c);
+            const int64_t q = p - c - s0;
+            if (q >= 0 && q < m) {
+               L.u1.out[q].key = kk[k];
+               L.u1.out[q].val = vv[k];
+               probe = std::max<uint32_t>(probe, static_cast<uint32_t>(p - static_cast<int64_t>(uu[k]) + 1));
+            }
          }
+      }
+      __syncthreads();
+      for (uint32_t q = threadIdx.x; q < m; q += kRegionBS) {
+         const uint64_t pos = base + static_cast<uint64_t>(c + s0 + q);
+         if (kept(pos)) b[pos & mask] = L.u1.out[q];
       }
    }
    return probe;
@@ -1597,20 +1635,32 @@ struct MergeRegion {
       Lo = fits ? static_cast<uint32_t>(lo) : 0;
       m = fits ? static_cast<uint32_t>(lo + ln) : 0;
    }
-   // Thread t owns elements t + k * kRegionBS: their keys, and their values.
-   __device__ __forceinline__ void keys(const Slot<K>* ob, const Slot<K>* S, uint64_t mask, K* kk) const {
+   // Thread t owns elements t + k * kRegionBS: f(k, element).  Three bases that
+   // are the same for every lane and a 32-bit index (one address per element
+   // and lane took the u64 kernel over its registers).
+   template <typename F>
+   __device__ __forceinline__ void each(const Slot<K>* ob, const Slot<K>* S, uint64_t mask, F f) const {
+      const uint64_t first = o0 & mask;
+      const uint32_t turn = static_cast<uint32_t>(std::min<uint64_t>(mask + 1 - first, Lo)); // old slots before the wrap
+      const Slot<K>* const p0 = ob + first;
+      const Slot<K>* const p1 = ob - turn;
+      const Slot<K>* const p2 = S + n0 - Lo;
 #pragma unroll
       for (int k = 0; k < kMergeIPT; ++k) {
          const uint32_t e = threadIdx.x + k * kRegionBS;
-         if (e < m) kk[k] = e < Lo ? ob[(o0 + e) & mask].key : S[n0 + (e - Lo)].key;
+         if (e < turn)
+            f(k, p0[e]);
+         else if (e < Lo)
+            f(k, p1[e]);
+         else if (e < m)
+            f(k, p2[e]);
       }
    }
+   __device__ __forceinline__ void keys(const Slot<K>* ob, const Slot<K>* S, uint64_t mask, K* kk) const {
+      each(ob, S, mask, [&](int k, const Slot<K>& s) { kk[k] = s.key; });
+   }
    __device__ __forceinline__ void vals(const Slot<K>* ob, const Slot<K>* S, uint64_t mask, K* vv) const {
-#pragma unroll
-      for (int k = 0; k < kMergeIPT; ++k) {
-         const uint32_t e = threadIdx.x + k * kRegionBS;
-         if (e < m) vv[k] = e < Lo ? ob[(o0 + e) & mask].val : S[n0 + (e - Lo)].val;
-      }
+      each(ob, S, mask, [&](int k, const Slot<K>& s) { vv[k] = s.val; });
    }
    // Home offsets of the loaded keys; false in a thread whose old key does
    // not belong to the region.
