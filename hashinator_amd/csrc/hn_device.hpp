@@ -144,6 +144,28 @@ __device__ __forceinline__ T atomic_cas(T* p, T expected, T desired) {
    return expected;
 }
 
+// Inclusive sum and maximum over the wave: DPP row shifts inside 16-lane
+// rows, then row broadcasts across rows.
+__device__ __forceinline__ uint32_t wave_incl_add(uint32_t x) {
+   int v = static_cast<int>(x);
+   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false); // row_shr:1
+   v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false); // row_shr:2
+   v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false); // row_shr:4
+   v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false); // row_shr:8
+   v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15 -> rows 1, 3
+   v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31 -> rows 2, 3
+   return static_cast<uint32_t>(v);
+}
+__device__ __forceinline__ int32_t wave_incl_max(int32_t v) {
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x111, 0xf, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x112, 0xf, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x114, 0xf, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x118, 0xf, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x142, 0xa, 0xf, false));
+   v = std::max(v, __builtin_amdgcn_update_dpp(INT32_MIN, v, 0x143, 0xc, 0xf, false));
+   return v;
+}
+
 // Per-wave epilogue of the insert kernels: fold the wave's counters into the
 // map's Info with relaxed device-scope atomics (a failure sets bit 0 of
 // reserved1).  `err` is published by a one-thread kernel launched after the

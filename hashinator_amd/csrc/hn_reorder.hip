@@ -85,11 +85,17 @@ __device__ uint64_t first_empty(const Slot<K>* b, uint64_t mask, uint64_t from, 
    return kNoPos;
 }
 
-// One workgroup per segment.  LDS per slot of capacity: the key, a packed
-// (histogram << 16 | occupied) scan word, and two 16-bit index tables.
+// One workgroup per segment.  LDS per slot of capacity: a key (in home
+// order), a packed (histogram << 16 | occupied) scan word, and the slot of
+// each occupied rank.  Bound by its LDS latencies, one after another, so the
+// scan runs on DPP and the ranks of four keys side by side.  AHEAD (the first
+// pass): the tile's keys are loaded at once and the segment's bounds found in
+// them, instead of the bounds first; the values of the keys that move (few, in
+// a sparse table) follow when that is known.  2^26 slots, before -> here: u64
+// at load .36 686 -> 467 us, at .9 891 -> 586; u32 507 -> 448 and 630 -> 537.
 // SOLO: the launch is one workgroup over the whole table, its begin and its
 // end among the rest.
-template <typename K, int BS, int E, bool SOLO = false>
+template <typename K, int BS, int E, bool AHEAD, bool SOLO = false>
 __global__ __launch_bounds__(BS) void k_reorder(Slot<K>* b, int sp, hn_info* info, ReorderHeader* h,
                                                 uint32_t* over, uint64_t tile, uint32_t n_tiles, int second,
                                                 const uint32_t* gate) {
@@ -97,9 +103,9 @@ __global__ __launch_bounds__(BS) void k_reorder(Slot<K>* b, int sp, hn_info* inf
    static_assert(CAP < 65536, "16-bit LDS indices and packed scan halves");
    __shared__ K key_s[CAP];
    __shared__ uint32_t pre_s[CAP + 1];
-   __shared__ uint16_t order_s[CAP];
    __shared__ uint16_t slot_of_s[CAP];
    __shared__ uint64_t bounds_s[2];
+   __shared__ uint32_t rel_s[2];
    __shared__ uint32_t wsum_s[BS / kWave];
    __shared__ uint32_t probe_s;
    if constexpr (SOLO) {
@@ -119,12 +125,46 @@ __global__ __launch_bounds__(BS) void k_reorder(Slot<K>* b, int sp, hn_info* inf
       __syncthreads(); // LDS of the previous segment is no longer read
       const uint64_t t = second ? over[it] : it;
       const uint64_t lo = t * tile;
-      if (wave < 2) {
-         const uint64_t r = wave == 0 ? first_empty<K>(b, mask, lo, tile) : first_empty<K>(b, mask, lo + tile, CAP);
-         if (lane == 0) bounds_s[wave] = r;
+      K kk[E];
+      uint64_t b0, b1;
+      // the slot of a thread's element e, from b0
+      auto at = [&](int e) -> uint32_t {
+         const uint32_t x = threadIdx.x + e * BS;
+         return AHEAD ? x - static_cast<uint32_t>(b0 - lo) : x; // before b0: past len
+      };
+      if constexpr (AHEAD) {
+         if (threadIdx.x < 2) rel_s[threadIdx.x] = ~0u;
+#pragma unroll
+         for (int e = 0; e < E; ++e) {
+            const uint32_t x = threadIdx.x + e * BS;
+            if (x < tile) kk[e] = b[(lo + x) & mask].key;
+         }
+         K next = empty_key<K>(); // wave 0 looks behind the tile
+         if (wave == 0) next = b[(lo + tile + lane) & mask].key;
+         __syncthreads();
+#pragma unroll
+         for (int e = 0; e < E; ++e) {
+            const uint32_t x = threadIdx.x + e * BS;
+            const uint64_t m = __ballot(x < tile && kk[e] == empty_key<K>());
+            if (m && lane == 0) atomicMin(&rel_s[0], x + static_cast<uint32_t>(first_bit(m)));
+         }
+         if (wave == 0) {
+            const uint64_t m = __ballot(next == empty_key<K>());
+            uint64_t r = m ? lo + tile + first_bit(m) : first_empty<K>(b, mask, lo + tile + kWave, CAP);
+            if (lane == 0 && r != kNoPos) rel_s[1] = static_cast<uint32_t>(r - lo);
+         }
+         __syncthreads();
+         b0 = rel_s[0] == ~0u ? kNoPos : lo + rel_s[0];
+         b1 = rel_s[1] > CAP ? kNoPos : lo + rel_s[1];
+      } else {
+         if (wave < 2) {
+            const uint64_t r = wave == 0 ? first_empty<K>(b, mask, lo, tile) : first_empty<K>(b, mask, lo + tile, CAP);
+            if (lane == 0) bounds_s[wave] = r;
+         }
+         __syncthreads();
+         b0 = bounds_s[0];
+         b1 = bounds_s[1];
       }
-      __syncthreads();
-      const uint64_t b0 = bounds_s[0], b1 = bounds_s[1];
       // No EMPTY slot in this tile: the segment is empty (b_t == b_{t+1}).
       if (b0 == kNoPos || b0 >= lo + tile) continue;
       if (b1 == kNoPos || b1 - b0 > CAP) {
@@ -140,26 +180,21 @@ __global__ __launch_bounds__(BS) void k_reorder(Slot<K>* b, int sp, hn_info* inf
       }
       const uint32_t len = static_cast<uint32_t>(b1 - b0);
       for (uint32_t i = threadIdx.x; i <= len; i += BS) pre_s[i] = 0;
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+         if (at(e) < len && (!AHEAD || threadIdx.x + e * BS >= tile)) kk[e] = b[(b0 + at(e)) & mask].key;
       __syncthreads();
 
-      K kk[E], vv[E];
-      uint32_t rr[E], sub[E];
+      uint32_t rs[E]; // home from the segment's start << 16 | rank among its arrivals; 0: no key
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-         const uint32_t i = threadIdx.x + e * BS;
-         kk[e] = empty_key<K>();
-         if (i < len) {
-            const Slot<K> s = b[(b0 + i) & mask];
-            kk[e] = s.key;
-            vv[e] = s.val;
-            key_s[i] = s.key;
-            if (s.key != empty_key<K>()) {
-               // Home relative to the segment start; a valid table has 1 <= r <= i.
-               uint32_t r = static_cast<uint32_t>(std::min<uint64_t>((fib_home(s.key, sp) - b0) & mask, i));
-               rr[e] = r;
-               sub[e] = atomicAdd(&pre_s[r], 1u << 16) >> 16;
-               atomicAdd(&pre_s[i], 1u);
-            }
+         const uint32_t i = at(e);
+         rs[e] = 0;
+         if (i < len && kk[e] != empty_key<K>()) {
+            // A valid table has 1 <= r <= i.
+            const uint32_t r = static_cast<uint32_t>(std::min<uint64_t>((fib_home(kk[e], sp) - b0) & mask, i));
+            rs[e] = (r << 16) | (atomicAdd(&pre_s[r], 1u << 16) >> 16);
+            atomicAdd(&pre_s[i], 1u);
          }
       }
       __syncthreads();
@@ -172,16 +207,15 @@ __global__ __launch_bounds__(BS) void k_reorder(Slot<K>* b, int sp, hn_info* inf
          const uint32_t c0 = std::min<uint32_t>(threadIdx.x * per, m), c1 = std::min<uint32_t>(c0 + per, m);
          uint32_t acc = 0;
          for (uint32_t x = c0; x < c1; ++x) acc += pre_s[x];
-         uint32_t inc = acc;
-#pragma unroll
-         for (int d = 1; d < kWave; d <<= 1) {
-            const uint32_t y = __shfl_up(inc, d, kWave);
-            if (lane >= d) inc += y;
-         }
+         const uint32_t inc = wave_incl_add(acc);
          if (lane == kWave - 1) wsum_s[wave] = inc;
          __syncthreads();
          uint32_t run = inc - acc;
-         for (int w = 0; w < wave; ++w) run += wsum_s[w];
+#pragma unroll
+         for (int w = 0; w < BS / kWave; ++w) {
+            const uint32_t c = wsum_s[w];
+            run += w < wave ? c : 0u;
+         }
          for (uint32_t x = c0; x < c1; ++x) {
             const uint32_t v = pre_s[x];
             pre_s[x] = run;
@@ -190,32 +224,61 @@ __global__ __launch_bounds__(BS) void k_reorder(Slot<K>* b, int sp, hn_info* inf
       }
       __syncthreads();
 
+      auto has = [&](int e) { return at(e) < len && kk[e] != empty_key<K>(); };
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-         const uint32_t i = threadIdx.x + e * BS;
-         if (i < len && kk[e] != empty_key<K>()) {
-            slot_of_s[pre_s[i] & 0xFFFFu] = static_cast<uint16_t>(i);
-            order_s[(pre_s[rr[e]] >> 16) + sub[e]] = static_cast<uint16_t>(i);
+         if (has(e)) {
+            slot_of_s[pre_s[at(e)] & 0xFFFFu] = static_cast<uint16_t>(at(e));
+            key_s[(pre_s[rs[e] >> 16] >> 16) + (rs[e] & 0xFFFFu)] = kk[e];
          }
       }
       __syncthreads();
 
+      uint32_t dest[E];
+      constexpr int SIDE = E < 4 ? E : 4;
+#pragma unroll
+      for (int b4 = 0; b4 < E; b4 += SIDE) {
+         uint32_t s0[SIDE], sn[SIDE], tie[SIDE];
+#pragma unroll
+         for (int x = 0; x < SIDE; ++x) {
+            const bool h4 = b4 + x < E && has(b4 + x);
+            s0[x] = h4 ? pre_s[rs[b4 + x] >> 16] >> 16 : 0;
+            sn[x] = h4 ? (pre_s[(rs[b4 + x] >> 16) + 1] >> 16) - s0[x] : 0;
+            tie[x] = 0;
+         }
+         for (uint32_t r = 0;; ++r) {
+            bool any = false;
+#pragma unroll
+            for (int x = 0; x < SIDE; ++x) any = any || r < sn[x];
+            if (!__ballot(any)) break;
+            K kj[SIDE];
+#pragma unroll
+            for (int x = 0; x < SIDE; ++x) kj[x] = key_s[s0[x] + (r < sn[x] ? r : 0)];
+#pragma unroll
+            for (int x = 0; x < SIDE; ++x)
+               if (b4 + x < E) tie[x] += r < sn[x] && kj[x] < kk[b4 + x] ? 1u : 0u;
+         }
+#pragma unroll
+         for (int x = 0; x < SIDE; ++x)
+            if (b4 + x < E) dest[b4 + x] = sn[x] ? slot_of_s[s0[x] + tie[x]] : at(b4 + x);
+      }
+      // The values of the keys that move, all read before a slot is written.
+      K vv[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) vv[e] = dest[e] != at(e) ? b[(b0 + at(e)) & mask].val : 0;
+#pragma unroll
+      for (int e = 0; e < E; ++e) asm volatile("" ::"v"(vv[e]) : "memory"); // they have arrived
+      __syncthreads();
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-         const uint32_t i = threadIdx.x + e * BS;
-         if (i < len && kk[e] != empty_key<K>()) {
-            const uint32_t s0 = pre_s[rr[e]] >> 16, s1 = pre_s[rr[e] + 1] >> 16;
-            uint32_t tie = 0;
-            for (uint32_t j = s0; j < s1; ++j) tie += key_s[order_s[j]] < kk[e] ? 1u : 0u;
-            const uint32_t dest = slot_of_s[s0 + tie];
-            if (dest != i) {
-               Slot<K> s;
-               s.key = kk[e];
-               s.val = vv[e];
-               b[(b0 + dest) & mask] = s;
-            }
-            if (dest >= rr[e]) max_probe = std::max<uint32_t>(max_probe, dest - rr[e] + 1);
+         const uint32_t r = rs[e] >> 16;
+         if (dest[e] != at(e)) {
+            Slot<K> s;
+            s.key = kk[e];
+            s.val = vv[e];
+            b[(b0 + dest[e]) & mask] = s;
          }
+         if (has(e) && dest[e] >= r) max_probe = std::max<uint32_t>(max_probe, dest[e] - r + 1);
       }
    }
    // One atomic per block at most, and only while the running maximum grows.
@@ -257,15 +320,15 @@ int reorder(void* buckets, hn_info* info, int sp, void* scratch, size_t bytes, h
    uint32_t* over = reinterpret_cast<uint32_t*>(h + 1);
    Slot<K>* b = static_cast<Slot<K>*>(buckets);
    if (sp <= kReorderSolo) {
-      hipLaunchKernelGGL((k_reorder<K, kReorderBS2, kReorderE, true>), dim3(1), dim3(kReorderBS2), 0, s, b, sp, info, h,
+      hipLaunchKernelGGL((k_reorder<K, kReorderBS2, kReorderE, false, true>), dim3(1), dim3(kReorderBS2), 0, s, b, sp, info, h,
                          over, n, 1u, 0, gate);
       return static_cast<int>(hipGetLastError());
    }
    hipLaunchKernelGGL(k_reorder_begin, dim3(1), dim3(64), 0, s, info, h, n, gate);
-   hipLaunchKernelGGL((k_reorder<K, kReorderBS1, kReorderE>), dim3(static_cast<uint32_t>(tiles)), dim3(kReorderBS1), 0,
+   hipLaunchKernelGGL((k_reorder<K, kReorderBS1, kReorderE, true>), dim3(static_cast<uint32_t>(tiles)), dim3(kReorderBS1), 0,
                       s, b, sp, info, h, over, tile, static_cast<uint32_t>(tiles), 0, nullptr);
    const uint32_t grid2 = static_cast<uint32_t>(std::min<uint64_t>(tiles, static_cast<uint64_t>(cu_count())));
-   hipLaunchKernelGGL((k_reorder<K, kReorderBS2, kReorderE>), dim3(grid2), dim3(kReorderBS2), 0, s, b, sp, info, h,
+   hipLaunchKernelGGL((k_reorder<K, kReorderBS2, kReorderE, false>), dim3(grid2), dim3(kReorderBS2), 0, s, b, sp, info, h,
                       over, tile, static_cast<uint32_t>(tiles), 1, nullptr);
    hipLaunchKernelGGL(k_reorder_end, dim3(1), dim3(64), 0, s, info, h);
    return static_cast<int>(hipGetLastError());
