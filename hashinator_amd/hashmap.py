@@ -145,8 +145,8 @@ class Hashmap:
         tombstones takes the merge (hn_merge_*), which writes the insert +
         reorder image into a fresh bucket array; the merge reads and writes
         the whole table, so it pays from about a quarter of the table (one
-        MI355X, a quarter of 2^26 u64 slots up to load 0.5: 1.26 ms against
-        1.77), sooner only where the table is nearly full (see _try_merge).
+        MI355X, a quarter of 2^26 u64 slots up to load 0.5: 1.32 ms against
+        1.54), sooner only where the table is nearly full (see _try_merge).
         A table not in Robin Hood order is reordered first when the batch is
         at least 4/3 of this fraction.  0 turns it off."""
         if key_bits not in (32, 64):
@@ -361,11 +361,11 @@ class Hashmap:
         new array instead, so the insert is complete either way.
 
         Smaller inserts that the reorder pass would follow take it too where
-        the map ends at least 85% full and is ordered already: the probing
+        the map ends at least 87% full and is ordered already: the probing
         insert's chains grow with the load, the merge does not (one MI355X,
         insert + reorder against merge + copy, a sixteenth of the slots
-        inserted up to load 0.9: 2^26 u64 slots 2.00 and 1.46 ms, 2^22 0.24
-        and 0.18; up to 0.8: 1.27 and 1.45, 0.13 and 0.17).  The image is
+        inserted up to load 0.9: 2^26 u64 slots 1.73 and 1.44 ms, 2^22 0.23
+        and 0.17; up to 0.85: 1.26 and 1.44, 0.15 and 0.17).  The image is
         copied back, so that the bucket array stays the one that it was."""
         N = self.bucket_count()
         if not self.merge_min or n < self.build_min_keys or n >= N or self._sp > 30:
@@ -377,7 +377,7 @@ class Hashmap:
         if i.fill == 0 or i.tombstone_counter != 0:
             return False
         ordered = bool(i.reserved1 & _lib.HN_INFO_ORDERED)
-        if small and not (ordered and i.fill + n >= 0.85 * N):
+        if small and not (ordered and i.fill + n >= 0.87 * N):
             return False
         if not ordered:
             if n < self.merge_min * N * 4 / 3:

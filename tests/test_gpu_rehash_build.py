@@ -220,7 +220,7 @@ def test_grow_declines_and_falls_back(gpu, bits):
 @pytest.mark.parametrize("lf,frac", [(0.9, 1 / 8), (0.9, 1 / 20), (0.8, 1 / 8)])
 def test_map_insert_near_full(gpu, bits, lf, frac):
     """Inserts below the merge's share of the table: merged into a map that
-    ends at least 85% full, probed otherwise; the bucket array stays."""
+    ends at least 87% full, probed otherwise; the bucket array stays."""
     sp = 18
     N = 1 << sp
     n, tot = int(frac * N), int(lf * N)
