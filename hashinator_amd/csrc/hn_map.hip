@@ -198,7 +198,7 @@ __global__ __launch_bounds__(1024) void k_lookup(LookupArgs<K> a) {
 // 2^24 u64 erases in 2^26 slots 0.89 -> 0.85 ms).
 constexpr int lane_block(int mode) { return mode == LK_ERASE ? 256 : kWave; }
 template <typename K, bool PAIRS, int MODE>
-__global__ __launch_bounds__(lane_block(MODE)) void k_lookup_lane(LookupArgs<K> a) {
+__global__ __launch_bounds__(lane_block(MODE)) void k_lookup_lane(LookupArgs<K> a, uint32_t cus) {
    constexpr int kWaves = lane_block(MODE) / kWave;
    __shared__ LaneLds<K, MODE> L[kWaves];
    const int sp = a.info->size_power;
@@ -209,12 +209,21 @@ __global__ __launch_bounds__(lane_block(MODE)) void k_lookup_lane(LookupArgs<K> 
    if (sp_ok) {
       if (sp >= LaneWin<K>::kLog && ovf > 0) {
          const int wv = threadIdx.x / kWave;
-         const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * kWaves;
+         // Waves on a CU, where the grid is the automatic one: 16 for a table in
+         // the L2s, 8 for one in the last-level cache, 12 beyond, where more only
+         // queue for the memory (u64 queries, 8 / 12 / 16 / 20 waves: 2^26 of 2^18
+         // slots 1.66 / 1.24 / 1.07 / 1.06 ms; 12 million of 2^24 319 / 326 / 331 /
+         // 333 us; 30 million of 2^26 1.195 / 1.126 / 1.122 / 1.133 ms).  The size
+         // is known on the device only: the waves over that number end at once.
+         const uint64_t bytes = sizeof(Slot<K>) << sp;
+         const uint64_t per_cu = bytes <= 1ull << 25 ? 16 : bytes <= 1ull << 28 ? 8 : 12;
+         uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * kWaves;
+         if (cus) nwaves = std::min<uint64_t>(nwaves, cus * per_cu);
          const uint64_t w = static_cast<uint64_t>(blockIdx.x) * kWaves + wv;
          const uint64_t per = a.len / nwaves, rem = a.len % nwaves;
          const uint64_t q0 = w * per + (w < rem ? w : rem);
          const uint64_t q1 = q0 + per + (w < rem ? 1 : 0);
-         erased = lane_lookup<K, PAIRS, MODE>(a, sp, ovf, ordered, q0, q1, L[wv]);
+         if (w < nwaves) erased = lane_lookup<K, PAIRS, MODE>(a, sp, ovf, ordered, q0, q1, L[wv]);
       } else {
          const uint64_t gstride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
          const uint64_t blk = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -507,16 +516,15 @@ int launch_lookup(LookupArgs<K> a, hipStream_t s, const hn_tune* t, OpKind op) {
          // one resident wave per block slot: the waves split the queries
          // statically, so a block that waits for a free slot would finish late
          static std::atomic<int> occ{0};
-         // 16 waves on a CU: in L2 fewer are slower (2^26 u64 queries of 2^18
-         // slots: 12 waves 1.24 ms, 16 and 20 1.07), beyond it more only queue
-         // (2^24 slots: 16 waves 2.17 ms, 20 2.23; 2^28 2.93 and 2.97).
+         // at most 16 waves on a CU; the kernel may use fewer (see there)
          const int per_cu =
              std::min(resident_blocks_per_cu(k_lookup_lane<K, PAIRS, MODE>, kBlock, occ), 16 * kWave / kBlock);
          uint64_t cap = (t && t->grid_blocks > 0) ? static_cast<uint64_t>(t->grid_blocks)
                                                   : static_cast<uint64_t>(cu_count()) * per_cu;
          if (cap > (1u << 20)) cap = 1u << 20;
          const uint32_t blocks = static_cast<uint32_t>(need < cap ? need : cap);
-         hipLaunchKernelGGL((k_lookup_lane<K, PAIRS, MODE>), dim3(blocks), dim3(kBlock), 0, s, a);
+         hipLaunchKernelGGL((k_lookup_lane<K, PAIRS, MODE>), dim3(blocks), dim3(kBlock), 0, s, a,
+                            t && t->grid_blocks > 0 ? 0u : static_cast<uint32_t>(cu_count()));
          return static_cast<int>(hipGetLastError());
       }
    }
