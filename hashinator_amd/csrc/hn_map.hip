@@ -506,7 +506,7 @@ template <typename K, bool PAIRS, int MODE>
 int launch_lookup(LookupArgs<K> a, hipStream_t s, const hn_tune* t, OpKind op) {
    if constexpr (MODE != LK_RESET) {
       if (!t || t->probe_width == 0) { // automatic: lane windows
-         // block_size does not apply: the lane kernel runs one wave per block
+         // block_size does not apply: the lane kernel's blocks are lane_block()
          // One query per lane and up (at least 256 per wave left most of the
          // device idle: 1,000 queries of a 2^20-slot table took 17.8 us on four
          // waves, events included, and 10.5 us on 16).
