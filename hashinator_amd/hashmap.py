@@ -162,7 +162,7 @@ class Hashmap:
         self._sfx = "u32" if key_bits == 32 else "u64"
         self._sp = int(sizePower)
         self.buckets = self._new_table(self._sp)
-        self._info = torch.zeros(5, dtype=torch.int64, device=self.device)  # 40 bytes == Info
+        self._info = torch.empty(5, dtype=torch.int64, device=self.device)  # 40 bytes == Info; hn_info_init writes it
         check(self._L.hn_info_init(_ptr(self._info), self._sp, _stream()), "hn_info_init")
         self._sync()
 
