@@ -287,6 +287,17 @@ int run_compact(const In* in, uint64_t n, Out* out, uint64_t* d_count, void* scr
    return static_cast<int>(sc::launch(in, n, out, d_count, scr, s, sel, proj));
 }
 
+// Rows of a tile: 4 for inputs up to 8 MiB, which a few 16-row tiles would
+// leave to a few CUs, one long tile after another (whole call, 16 rows and 4:
+// 2^16 u32 13.1 and 10.4 us, 2^20 u64 22.9 and 15.7, 2^21 u32 15.7 and 13.3;
+// 2^22 u32 17.2 and 17.0, 2^24 30.8 and 43.9, where the tiles' tickets count).
+constexpr int kRowsSmall = 4;
+constexpr uint64_t kSmallScan = 8ull << 20;
+template <typename T>
+constexpr int scan_rows(uint64_t n) {
+   return n * sizeof(T) <= kSmallScan ? kRowsSmall : kRows;
+}
+
 // cleared: an earlier kernel has cleared the look-back words (scan_words_u32).
 template <typename T>
 int run_scan(const T* in, T* out, uint64_t n, void* scr, size_t bytes, hipStream_t s, bool cleared = false) {
@@ -297,14 +308,18 @@ int run_scan(const T* in, T* out, uint64_t n, void* scr, size_t bytes, hipStream
    // either tile holds at least a compaction tile, so the scratch sized by
    // hn_compact_scratch_bytes covers its look-back words.
    const bool vec = (reinterpret_cast<uintptr_t>(in) % 16 == 0) && (reinterpret_cast<uintptr_t>(out) % 16 == 0);
-   const uint64_t TILE = static_cast<uint64_t>(kBS) * (16 / sizeof(T)) * (vec ? kRows : kScanRowsScalar);
+   const int rows = vec ? scan_rows<T>(n) : kScanRowsScalar;
+   const uint64_t TILE = static_cast<uint64_t>(kBS) * (16 / sizeof(T)) * rows;
    const uint64_t tiles = (n + TILE - 1) / TILE;
    if (!scr || bytes < lookback_bytes(tiles)) return HN_ESCRATCH;
    Lookback L = lookback_layout(scr, tiles);
    if (!cleared) hipLaunchKernelGGL(k_lookback_init, dim3(stream_blocks(tiles, 256)), dim3(256), 0, s, L, tiles);
-   if (vec)
+   if (vec && rows == kRows)
       hipLaunchKernelGGL((k_scan<T, true, kRows>), dim3(static_cast<uint32_t>(tiles)), dim3(kBS), 0, s, in, out, n, L,
                          tiles);
+   else if (vec)
+      hipLaunchKernelGGL((k_scan<T, true, kRowsSmall>), dim3(static_cast<uint32_t>(tiles)), dim3(kBS), 0, s, in, out,
+                         n, L, tiles);
    else
       hipLaunchKernelGGL((k_scan<T, false, kScanRowsScalar>), dim3(static_cast<uint32_t>(tiles)), dim3(kBS), 0, s, in,
                          out, n, L, tiles);
@@ -315,13 +330,13 @@ int run_scan(const T* in, T* out, uint64_t n, void* scr, size_t bytes, hipStream
 // the scan that follows it: the look-back words of a scan of n 32-bit
 // elements in place, which are 16-byte aligned, and the scan over them.
 uint64_t* scan_words_u32(void* scr, uint64_t n, uint32_t* count) {
-   const uint64_t TILE = static_cast<uint64_t>(kBS) * 4 * kRows;
+   const uint64_t TILE = static_cast<uint64_t>(kBS) * 4 * scan_rows<uint32_t>(n);
    const uint64_t tiles = (n + TILE - 1) / TILE;
    *count = static_cast<uint32_t>((256 + tiles * 16) / sizeof(uint64_t));
    return static_cast<uint64_t*>(scr);
 }
 int scan_u32_cleared(uint32_t* x, uint64_t n, void* scr, size_t bytes, hipStream_t s) {
-   if (reinterpret_cast<uintptr_t>(x) % 16) return HN_EINVAL; // the words were counted for 16-row tiles
+   if (reinterpret_cast<uintptr_t>(x) % 16) return HN_EINVAL; // the words were counted for aligned tiles
    return run_scan<uint32_t>(x, x, n, scr, bytes, s, true);
 }
 

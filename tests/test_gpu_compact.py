@@ -151,3 +151,24 @@ def test_compaction_tile_sizes(gpu, bits, n):
     assert L.hn_copy_if_flags(x.data_ptr(), flags.data_ptr(), n, bits // 4, out.data_ptr(), cnt.data_ptr(),
                               sc.data_ptr(), sb, None) == 0
     assert int(cnt) == m and torch.equal(out[:m], x[keep])
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("d", [-16385, -1, 0, 1, 70000])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_scan_tile_sizes(gpu, bits, d, shift):
+    """Around the size (8 MiB) at which the scan's tile changes, aligned and
+    not: the exclusive prefix sums modulo the element's size."""
+    from hashinator_amd import _lib
+    L = _lib.load()
+    n = (8 << 20) // (bits // 8) + d
+    dt = torch.int32 if bits == 32 else torch.int64
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    x = torch.randint(-(1 << 31), 1 << 31, (n + shift,), dtype=torch.int64, device="cuda", generator=g).to(dt)[shift:]
+    out = torch.empty(n + shift, dtype=dt, device="cuda")[shift:]
+    sb = int(L.hn_compact_scratch_bytes(n))
+    sc = torch.empty(sb, dtype=torch.uint8, device="cuda")
+    assert getattr(L, f"hn_exclusive_scan_u{bits}")(x.data_ptr(), out.data_ptr(), n, sc.data_ptr(), sb, None) == 0
+    ref = torch.cumsum(x.cpu().to(torch.int64), 0) - x.cpu().to(torch.int64)
+    assert torch.equal(out.cpu(), ref.to(dt) if bits == 64 else ((ref + (1 << 31)) % (1 << 32) - (1 << 31)).to(dt))
