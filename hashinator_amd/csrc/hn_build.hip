@@ -248,10 +248,12 @@ __device__ __forceinline__ Slot<K> part_pair(const PartIn<K>& in, uint64_t e) {
    return s;
 }
 
-// A table's EMPTY and TOMBSTONE slots are left out; a batch's keys are not looked at.
+// A table's EMPTY and TOMBSTONE slots are left out, and a batch's EMPTY keys
+// (a padded batch's: the probing insert finds such a key in the first EMPTY
+// slot and places nothing).
 template <typename K, int SRC>
 __device__ __forceinline__ bool part_live(const PartIn<K>& in, uint64_t e, K key) {
-   return (SRC == SRC_GROW && e >= in.n_table) || (key != empty_key<K>() && key != tomb_key<K>());
+   return key != empty_key<K>() && (key != tomb_key<K>() || (SRC == SRC_GROW && e >= in.n_table));
 }
 
 template <typename K>
@@ -1640,8 +1642,8 @@ struct MergeRegion {
    __device__ __forceinline__ void vals(const Slot<K>* ob, const Slot<K>* S, uint64_t mask, K* vv) const {
       each(ob, S, mask, [&](int k, const Slot<K>& s) { vv[k] = s.val; });
    }
-   // Home offsets of the loaded keys; false in a thread whose old key does
-   // not belong to the region.
+   // Home offsets of the loaded keys, EMPTY ones (a padded batch's too) left
+   // out; false in a thread whose old key does not belong to the region.
    __device__ __forceinline__ bool homes(const K* kk, uint64_t rb, int sp, uint64_t R, uint32_t* uu) const {
       const uint64_t mask = (1ull << sp) - 1;
       bool ok = true;
@@ -1649,7 +1651,7 @@ struct MergeRegion {
       for (int k = 0; k < kMergeIPT; ++k) {
          const uint32_t e = threadIdx.x + k * kRegionBS;
          uu[k] = kAbsent;
-         if (e < m && (e >= Lo || kk[k] != empty_key<K>())) {
+         if (e < m && kk[k] != empty_key<K>()) {
             const uint64_t hr = (fib_home(kk[k], sp) - rb) & mask;
             if (hr >= R || (e < Lo && kk[k] == tomb_key<K>()))
                ok = false;

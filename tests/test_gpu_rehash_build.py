@@ -237,3 +237,25 @@ def test_map_insert_near_full(gpu, bits, lf, frac):
     exp.update(zip(again.tolist(), vals.tolist()))
     rows = live_pairs(hm.host_buckets(), bits)
     assert np.array_equal(rows, np.array(sorted(exp.items()), dtype=NDT[bits]))
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("sp,old,n,grows", [(12, 1500, 1700, True), (12, 3300, 500, False), (12, 2000, 1100, False)])
+def test_map_insert_padded_with_empty_keys(gpu, bits, sp, old, n, grows):
+    """A batch padded with the EMPTY key: as in the probing insert, the padding
+    takes no slot, makes no hole and is not counted, whether the insert grows
+    the map, merges into a nearly full one or merges a large batch."""
+    keys = keyset(old + n, bits, seed=sp)
+    hm = Hashmap(sp, bits, build_min_keys=1)
+    hm.insert(keys[:old], keys[:old], targetLF=1.0)
+    b = np.full(n + n // 8, EMPTY[bits], dtype=NDT[bits])
+    at = np.sort(np.random.default_rng(n).choice(b.size, n, replace=False))
+    b[at] = keys[old:]
+    hm.insert(b, b, targetLF=0.5 if grows else 1.0)
+    assert (hm.getSizePower() > sp) == grows and hm.peek_status() == 0
+    img = hm.host_buckets()
+    assert hm.size() == keys.size
+    assert np.array_equal(live_pairs(img, bits)[:, 0], np.sort(keys))
+    assert reachable_all(img, bits, hm.getSizePower())
+    _, _, hit = hm.retrieve(keys)
+    assert bool(hit.all())
