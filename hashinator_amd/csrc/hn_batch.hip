@@ -274,7 +274,8 @@ struct MapState {
    uint32_t listed;    // clean: keys in the map's scratch slice, to be placed by k_map_clean_end
    uint32_t max_probe; // clean: longest probe of the keys placed by the regions
    uint32_t displaced; // clean: a live key stood away from its home slot
-   uint32_t pad[3];
+   uint32_t placed;    // clean: keys placed by the regions and their borders
+   uint32_t pad[2];
 };
 constexpr uint32_t kSpillCap = 248; // with the state, 1 KiB a map
 
@@ -636,8 +637,8 @@ __global__ __launch_bounds__(kRgBS) void k_boundary_insert(BatchArgs<K> a, Batch
          uint32_t mm, em;
          window_bits<K>(L.key, pos, kRgWin, key, &mm, &em);
          const uint32_t w = pos & ~3u;
-         if (mm) {
-            if (pos >= kRgHalf) put(w + __ffs(mm) - 1, idx); // one before its region's end was set there
+         if (mm) { // (clean: a second copy of the key, dropped)
+            if (!CLEAN && pos >= kRgHalf) put(w + __ffs(mm) - 1, idx); // one before its region's end was set there
             return true;
          }
          if (em) {
@@ -689,7 +690,8 @@ __global__ __launch_bounds__(kRgBS) void k_boundary_insert(BatchArgs<K> a, Batch
       }
       if (threadIdx.x == 0) {
          if (L.flag) __hip_atomic_fetch_or(&st->spilled, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-         if constexpr (CLEAN) { // fill does not change
+         if constexpr (CLEAN) {
+            if (L.n) atomic_add_relaxed(&st->placed, static_cast<uint32_t>(L.n));
             if (L.max_probe) atomic_max_relaxed(&st->max_probe, L.max_probe);
          } else {
             if (L.n) atomic_add_relaxed(&M.info->fill, static_cast<uint64_t>(L.n));
@@ -1022,7 +1024,10 @@ __global__ __launch_bounds__(kRgBS) __attribute__((amdgpu_waves_per_eu(4))) void
 
 // Clean on one region: the live keys standing in it whose home lies in it are
 // placed again in an LDS image that starts empty (read from the table, which
-// does not change meanwhile), then the image is written over the region.
+// does not change meanwhile), then the image is written over the region.  Of a
+// key that stands there twice (inserted before an EMPTY slot that
+// reset_to_empty has left on the way to its old copy) one copy is placed, as
+// when the lifted keys are inserted again, so the keys placed are counted.
 // Keys of other regions standing here, and keys that run past the region's
 // end, go to the map's scratch slice (at most its live keys), from which
 // k_boundary_insert and k_map_clean_end place them.  The Info is not changed
@@ -1045,7 +1050,7 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
       MapState* const st = &map_state(sc, a.n_maps)[mi];
       for (uint32_t i = threadIdx.x; i < R; i += kRgBS) L.key[i] = kEmpty;
       __syncthreads();
-      uint32_t max_probe = 0;
+      uint32_t max_probe = 0, placed = 0;
       bool displaced = false;
       lds_probe<K>(
           L, SlotKeys<K>{b, R}, sp,
@@ -1061,10 +1066,12 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
              uint32_t mm, em;
              window_bits<K>(L.key, pos, W, key, &mm, &em);
              const uint32_t w = pos & ~3u;
+             if (mm) return true;
              if (em) {
                 const uint32_t at = w + __ffs(em) - 1;
-                if (lds_cas(&L.key[at], kEmpty, key) != kEmpty) return false;
+                if (lds_cas(&L.key[at], kEmpty, key) != kEmpty) return false; // look again
                 L.val[at] = static_cast<K>(idx);
+                ++placed;
                 const uint32_t pr = off + (at - pos) + 1;
                 max_probe = pr > max_probe ? pr : max_probe;
                 return true;
@@ -1082,8 +1089,10 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
              return false; // the region's keys fit: they came from its slots
           });
       max_probe = wave_max(max_probe);
+      placed = wave_sum(placed);
       const bool wd = __ballot(displaced) != 0;
       if (__lane_id() == 0) {
+         if (placed) atomicAdd(&L.n, static_cast<unsigned long long>(placed));
          if (max_probe) atomicMax(&L.max_probe, max_probe);
          if (wd) L.flag = 1;
       }
@@ -1106,6 +1115,7 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
          if (i < R) b[i] = s[e];
       }
       if (threadIdx.x == 0) {
+         if (L.n) atomic_add_relaxed(&st->placed, static_cast<uint32_t>(L.n));
          if (L.max_probe) atomic_max_relaxed(&st->max_probe, L.max_probe);
          if (L.flag) __hip_atomic_store(&st->displaced, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
@@ -1117,7 +1127,7 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
 // then the Info.
 template <typename K>
 __global__ __launch_bounds__(kRgBS) void k_map_clean_end(BatchArgs<K> a, BatchScratch* sc) {
-   __shared__ uint32_t s_max, s_failed;
+   __shared__ uint32_t s_max, s_failed, s_placed;
    for (uint32_t m = blockIdx.x; m < a.n_maps; m += gridDim.x) {
       const hn_batch_map M = a.maps[m];
       hn_info* info = M.info;
@@ -1131,6 +1141,7 @@ __global__ __launch_bounds__(kRgBS) void k_map_clean_end(BatchArgs<K> a, BatchSc
       if (threadIdx.x == 0) {
          s_max = st.max_probe;
          s_failed = 0;
+         s_placed = st.placed;
       }
       __syncthreads();
       InsertCounters c;
@@ -1139,8 +1150,10 @@ __global__ __launch_bounds__(kRgBS) void k_map_clean_end(BatchArgs<K> a, BatchSc
          insert_one<K>(static_cast<Slot<K>*>(M.buckets), sp, list[i].key, list[i].val, c);
       if (c.max_probe) atomicMax(&s_max, static_cast<uint32_t>(c.max_probe));
       if (c.failed) atomicOr(&s_failed, 1u);
+      if (c.placed) atomicAdd(&s_placed, static_cast<uint32_t>(c.placed));
       __syncthreads();
       if (threadIdx.x == 0) {
+         info->fill = s_placed;
          info->tombstone_counter = 0;
          const uint64_t o = next_overflow(s_max, kBucketOverflow);
          info->current_max_bucket_overflow = o > kBucketOverflow ? o : kBucketOverflow;

@@ -322,3 +322,55 @@ def test_batch_regions_full_and_short_scratch(gpu):
     torch.cuda.synchronize()
     assert bm.info(1).err == 1 and bm.info(1).tombstone_counter == 4000
     assert np.array_equal(before, bm.buckets(1))
+
+
+def plant_copies(img, sp, key_bits, per_map, rng):
+    """Second copies of live keys behind EMPTY slots, as an insert leaves them in a table that
+    reset_to_empty has made holes in; half of them across a region's end where the map has several.
+    Returns the number planted."""
+    from tests.helpers import EMPTY, TOMB
+    n, one = 1 << sp, 13 if key_bits == 32 else 12
+    keys = img[:, 0]
+    empty = np.flatnonzero(keys == EMPTY[key_bits])
+    ends = (np.arange(1, max(1, n >> one)) << one) - 1
+    last = np.searchsorted(empty, ends, side="right") - 1  # the last EMPTY slot before each region's end
+    at = np.concatenate([last, rng.permutation(empty.size - 2)[:per_map]])
+    planted = 0
+    for j in at:
+        e, e2 = int(empty[j]), int(empty[j + 1])
+        if e == 0 or keys[e - 1] >= TOMB[key_bits] or keys[e2] != EMPTY[key_bits]:
+            continue
+        img[e2] = img[e - 1]
+        planted += 1
+    return planted
+
+
+@pytest.mark.parametrize("key_bits", [32, 64])
+def test_batch_clean_keeps_one_copy_of_a_key(gpu, key_bits):
+    """clean_tombstones lifts out the keys away from home and inserts them again, so of a key
+    that stands in the table twice one copy is left, and the fill counts it once."""
+    one = 13 if key_bits == 32 else 12
+    sps = [one + 2, one + 1, one, 10, 6]
+    ins = [W.unique_keys(int(0.6 * (1 << sp)), key_bits, 50 + m) for m, sp in enumerate(sps)]
+    ers = [k[: k.size // 3] for k in ins]
+    bm = BatchedMaps(sps, ins, ins, [k[:0] for k in ins], ers, key_bits=key_bits)
+    bm.init()
+    bm.run(_lib.HN_BATCH_INSERT | _lib.HN_BATCH_ERASE)
+    torch.cuda.synchronize()
+    rng = np.random.default_rng(3)
+    infos = bm.infos.cpu().numpy()
+    arena = bm.arena.cpu().numpy().view(ins[0].dtype)
+    for m, sp in enumerate(sps):
+        lo = int(bm.slot_off[m])
+        infos[m, 1] += plant_copies(arena[lo:lo + (1 << sp)], sp, key_bits, ins[m].size // 8, rng)
+    assert (infos[:, 1] > bm.infos.cpu().numpy()[:, 1]).all()  # there are copies in every map
+    bm.arena.copy_(torch.from_numpy(arena.view(np.int32 if key_bits == 32 else np.int64)))
+    bm.infos.copy_(torch.from_numpy(infos))
+    bm.run(_lib.HN_BATCH_CLEAN)
+    torch.cuda.synchronize()
+    for m, sp in enumerate(sps):
+        left = np.sort(ins[m][ins[m].size // 3:])
+        img, info = bm.buckets(m), bm.info(m)
+        assert np.array_equal(live_pairs(img, key_bits), np.stack([left, left], axis=1)), m
+        assert (info.fill, info.tombstone_counter, info.err) == (left.size, 0, 0), m
+        assert reachable_all(img, key_bits, sp), m
