@@ -75,20 +75,40 @@ __device__ __forceinline__ void insert_publish(hn_info* info) {
 }
 
 // An insert of at most kSmallInsert keys.  Into a table of one region (64 KiB
-// of slots, known on the device only) and at least a 64th of its slots,
-// workgroup 0 runs it with the table in LDS, where a probe chain does not wait
-// for global memory at every step (900 u64 keys into 2^10 slots: k_insert
-// 32.8 us, here 21.6); otherwise as k_insert.  Up to kSoloInsert keys take one
+// of slots, known on the device only), workgroup 0 runs it with the table in
+// LDS where the probe chains are long enough to pay for the table's way in
+// (lds_insert_pays); otherwise as k_insert.  Up to kSoloInsert keys take one
 // workgroup, which finishes the Info too: a launch less (200 keys into 2^18
 // slots 19.1 -> 13.0 us; more keys want more CUs, whose address translations
 // run side by side: 10^3 keys on one workgroup took 21 us, on eight 14).
 constexpr uint64_t kSmallInsert = 8192, kSoloInsert = 256;
+// Direct and LDS, us a call, from a 64th of the slots on.  Tables of up to 16
+// KiB always (2^10 u32 slots: 64 keys at load .1 8.5 and 8.8, at .6 13.1 and
+// 10.4, 896 into an empty one 46 and 35).  Larger ones by the load over and
+// after the insert where one workgroup runs it (64 keys into 2^12 u64 slots
+// empty 7.4 and 10.8, at load .6 15.1 and 14.9, at .85 44 and 38).  Several
+// workgroups must agree whatever the fill is when each starts, so by the sizes
+// alone: tables of 32 KiB (512 into 2^12 u32 slots empty 11.5 and 14.2, at
+// load .6 24 and 24, 1,024 at .7 99 and 77), and of 64 KiB from a quarter of
+// the slots on in 64 bits (2^12: 1,024 into an empty one 13 and 16, at .7 110
+// and 93) and three quarters in 32 (2^13: 2,048 into an empty one 13 and 19, at
+// .6 46 and 44).
+template <typename K>
+__device__ __forceinline__ bool lds_insert_pays(const hn_info* info, int sp, uint64_t len, int solo) {
+   constexpr int kLog = kRegionLogB<K>;
+   const uint64_t R = 1ull << sp;
+   if (sp > kLog || len * 64 < R) return false;
+   if (sp <= kLog - 2) return true;
+   if (!solo) return sp < kLog || len * 4 >= (sizeof(K) == 8 ? R : R * 3);
+   const uint64_t used = info->fill + info->tombstone_counter;
+   return (2 * used + len) * 8 >= R * 9 || (used + len) * 4 >= R * 3;
+}
 template <typename K, int G, int SRC>
 __global__ __launch_bounds__(kRgBS) void k_insert_small(InsertArgs<K> a, int solo) {
    __shared__ RegionMem<K> L;
    const int sp = a.info->size_power;
    const bool sp_ok = sp >= 1 && sp <= max_size_power<K>();
-   if (!(sp_ok && sp <= kRegionLogB<K> && a.len * 64 >= 1ull << sp)) {
+   if (!(sp_ok && lds_insert_pays<K>(a.info, sp, a.len, solo))) {
       InsertCounters c;
       c.failed = sp_ok ? 0 : 1;
       const uint64_t gstride = static_cast<uint64_t>(gridDim.x) * (blockDim.x / G);

@@ -65,3 +65,22 @@ def reachable_all(img, bits, sp):
 
 def next_overflow(x, w=64):
     return x if x % w == 0 else x + (w - x % w)
+
+
+def race(a, b, before=lambda: None, reps=25):
+    """Median GPU microseconds of calls a and b, timed in turn; ``before`` runs untimed before each."""
+    import torch
+
+    t = ([], [])
+    for r in range(reps + 3):
+        for fn, ts in ((a, t[0]), (b, t[1])):
+            before()
+            torch.cuda.synchronize()
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            fn()
+            e1.record()
+            torch.cuda.synchronize()
+            if r >= 3:
+                ts.append(e0.elapsed_time(e1) * 1e3)
+    return float(np.median(t[0])), float(np.median(t[1]))

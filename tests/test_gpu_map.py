@@ -521,3 +521,42 @@ def test_small_insert_sizes(gpu, bits, form, shift):
         torch.cuda.synchronize()
         check_insert_invariants(hm, model, bits)
         assert hm.info().reserved0 == 0 and hm.info().reserved1 == 0
+
+
+@pytest.mark.parametrize("bits,below,lf,n", [(32, 0, 0.0, 128), (32, 0, 0.0, 512), (32, 0, 0.0, 2048), (32, 0, 0.1, 4096),
+                                             (32, 0, 0.0, 6200), (32, 0, 0.65, 256), (64, 0, 0.0, 256), (64, 0, 0.3, 512),
+                                             (64, 0, 0.3, 1024), (64, 0, 0.65, 200), (32, 1, 0.3, 300), (64, 1, 0.0, 100)])
+def test_small_insert_takes_the_faster_way(gpu, bits, below, lf, n):
+    """Keys into a table of one region, or half of one: the live set is the oracle's, and
+    the default is no slower than the group kernel asked for by its shape."""
+    from hashinator_amd import _lib
+    from tests.helpers import race
+    L = _lib.load()
+    sp = (13 if bits == 32 else 12) - below
+    old = keyset(int(lf * (1 << sp)), bits, seed=sp)
+    keys = keyset(n, bits, seed=sp, start=old.size + 2)
+    model = fresh_model(sp, bits)
+    if old.size:
+        model.insert(old, old)
+    hm = Hashmap(sp, bits, auto_reorder=0, auto_build=0)
+    upload(hm, model)
+    b0, i0 = hm.buckets.clone(), hm._info.clone()
+    dk = torch.from_numpy(keys.view(np.int32 if bits == 32 else np.int64)).cuda()
+    p = lambda t: C.c_void_p(t.data_ptr())
+    group = hn_tune(4, 1024, 0, 0)
+
+    def put(tune):
+        assert getattr(L, f"hn_insert_u{bits}")(p(dk), p(dk), p(hm.buckets), p(hm._info), n,
+                                                C.c_void_p(torch.cuda.current_stream().cuda_stream), tune) == 0
+
+    def back():
+        hm.buckets.copy_(b0)
+        hm._info.copy_(i0)
+
+    default, asked = race(lambda: put(None), lambda: put(C.byref(group)), back)
+    assert default <= 1.2 * asked, (default, asked)
+    back()
+    put(None)
+    torch.cuda.synchronize()
+    model.insert(keys, keys)
+    check_insert_invariants(hm, model, bits)
