@@ -241,16 +241,18 @@ class Hashmap:
         return to_numpy(self.buckets, self.kb).reshape(-1, 2)
 
     # ----------------------------------------------------------- accelerated API
-    def _grow_for(self, k, v, n, pairs, targetLF, stream) -> bool:
-        """Auto-grow before an insert (hashinator.h:1329-1332).  True when the
-        batch is in the table already: growing a map of many keys by a batch
-        that the reorder pass would follow is one build of both (hn_grow_*).
-        An empty map that the build will fill is not rehashed."""
+    def _grow_for(self, k, v, n, pairs, targetLF, stream):
+        """Auto-grow before an insert (hashinator.h:1329-1332).  True first
+        when the batch is in the table already: growing a map of many keys by a
+        batch that the reorder pass would follow is one build of both
+        (hn_grow_*).  An empty map that the build will fill is not rehashed.
+        Second the map's Info where it was read and still holds (a map that
+        does not grow), for the rest of the insert."""
         i = self.info()
         fill = i.fill
         needed = math.ceil(math.log2((fill + n) * (1.0 / targetLF)))
         if needed <= self._sp:
-            return False
+            return False, i
         N = 1 << needed
         if fill == 0 and needed <= 32 and self._builds(n, N) and \
                 getattr(self._L, f"hn_build_scratch_bytes_{self._sfx}")(needed, n):
@@ -263,12 +265,12 @@ class Hashmap:
             finally:
                 if not built:  # no memory for its scratch, say
                     check(self._fn("table_init")(_ptr(self.buckets), N, _stream(stream)), "hn_table_init")
-            return built
+            return built, None
         if self.auto_build and self.auto_reorder and fill >= self.build_min_keys and n >= self.auto_reorder * N:
             if self._grow(k, v, n, pairs, needed, stream):
-                return True
+                return True, None
         self.resize(needed, targets.device, stream)
-        return False
+        return False, None
 
     def _grow(self, k, v, n, pairs, new_sp, stream) -> bool:
         sb = 0 if new_sp > 32 else getattr(self._L, f"hn_grow_scratch_bytes_{self._sfx}")(self._sp, new_sp, n)
@@ -313,11 +315,12 @@ class Hashmap:
         if n == 0:
             self._info.view(torch.int32)[8] = status.success
             return
-        if self._grow_for(k, None if vals is None else v, n, vals is None, targetLF, stream):
+        done, i = self._grow_for(k, None if vals is None else v, n, vals is None, targetLF, stream)
+        if done:
             return
         if self._try_build(k, None if vals is None else v, n, vals is None, stream):
             return
-        if self._try_merge(k, None if vals is None else v, n, vals is None, stream):
+        if self._try_merge(k, None if vals is None else v, n, vals is None, stream, i):
             return
         if vals is None:
             rc = self._fn("insert_pairs")(_ptr(k), _ptr(self.buckets), _ptr(self._info), n, _stream(stream), self._tune())
@@ -353,7 +356,7 @@ class Hashmap:
         del scratch
         return self.info().err == status.success
 
-    def _try_merge(self, k, v, n, pairs, stream) -> bool:
+    def _try_merge(self, k, v, n, pairs, stream, i=None) -> bool:
         """Large insert into a table that holds keys: hn_merge_* writes the
         insert + reorder image into a fresh bucket array, which then replaces
         the old one.  Where the merge itself declines (keys crowding one
@@ -373,7 +376,8 @@ class Hashmap:
         small = n < self.merge_min * N
         if small and not (self.auto_reorder and n >= self.auto_reorder * N):
             return False
-        i = self.info()
+        if i is None:
+            i = self.info()
         if i.fill == 0 or i.tombstone_counter != 0:
             return False
         ordered = bool(i.reserved1 & _lib.HN_INFO_ORDERED)
@@ -446,11 +450,12 @@ class Hashmap:
         if n == 0:
             self._info.view(torch.int32)[8] = status.success
             return
-        if self._grow_for(k, None, n, False, targetLF, stream):
+        done, i = self._grow_for(k, None, n, False, targetLF, stream)
+        if done:
             return
         if self._try_build(k, None, n, False, stream):
             return
-        if self._try_merge(k, None, n, False, stream):
+        if self._try_merge(k, None, n, False, stream, i):
             return
         check(self._fn("insert_index")(_ptr(k), _ptr(self.buckets), _ptr(self._info), n, _stream(stream),
                                        self._tune()), "insertIndex")

@@ -259,3 +259,19 @@ def test_map_insert_padded_with_empty_keys(gpu, bits, sp, old, n, grows):
     assert reachable_all(img, bits, hm.getSizePower())
     _, _, hit = hm.retrieve(keys)
     assert bool(hit.all())
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_map_insert_reads_the_info_once(gpu, bits):
+    """An insert of a sixteenth of the slots and more that neither grows the map nor is built
+    or merged reads the Info back once, for its size."""
+    sp = 14
+    keys = keyset(6000, bits, seed=9)
+    hm = Hashmap(sp, bits, build_min_keys=1, auto_build=0)
+    hm.insert(keys[:4000], keys[:4000], targetLF=1.0)
+    reads, info = [], hm.info
+    hm.info = lambda: reads.append(1) or info()
+    hm.insert(keys[4000:], keys[4000:], targetLF=1.0)
+    assert len(reads) == 1
+    assert hm.size() == 6000 and hm.ordered()
+    assert np.array_equal(live_pairs(hm.host_buckets(), bits)[:, 0], np.sort(keys))
