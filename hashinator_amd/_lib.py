@@ -88,6 +88,8 @@ SIGNATURES = {
     "hn_insert_index_u64": (I, [P, P, P, S, P, TUNE]),
     "hn_insert_pairs_u32": (I, [P, P, P, S, P, TUNE]),
     "hn_insert_pairs_u64": (I, [P, P, P, S, P, TUNE]),
+    "hn_insert_look_u32": (I, [P, S, S, P, P, P, P]),
+    "hn_insert_look_u64": (I, [P, S, S, P, P, P, P]),
     "hn_retrieve_u32": (I, [P, P, P, P, P, S, P, TUNE]),
     "hn_retrieve_u64": (I, [P, P, P, P, P, S, P, TUNE]),
     "hn_retrieve_zero_u32": (I, [P, P, P, P, P, S, P, TUNE]),

@@ -172,6 +172,57 @@ __global__ void k_insert_finish(hn_info* info, const uint64_t* expected_fill) {
    info->reserved1 = 0;
 }
 
+// The Info and, of kLookKeys keys at equal distances in a batch, how many the
+// table does not hold: what the choice between a merge and a probing insert
+// needs, in one read-back with the Info.  Eight lanes a key, whose windows
+// start at its home slot; a chain of a few loads, so one workgroup.
+constexpr uint32_t kLookKeys = 128;
+template <typename K>
+__global__ __launch_bounds__(kLookKeys * 8) void k_insert_look(const char* keys, uint64_t stride, uint64_t len,
+                                                               const Slot<K>* b, const hn_info* info,
+                                                               hn_insert_look* out) {
+   __shared__ uint32_t absent_s;
+   if (threadIdx.x == 0) absent_s = 0;
+   __syncthreads();
+   const hn_info i = *info;
+   const int sp = i.size_power;
+   const bool run = sp >= 1 && sp <= max_size_power<K>() && (i.reserved1 & kInfoOrdered) && i.tombstone_counter == 0;
+   const uint32_t m = len < kLookKeys ? static_cast<uint32_t>(len) : kLookKeys;
+   const uint32_t g = threadIdx.x / 8, gl = threadIdx.x & 7u;
+   const int gbase = __lane_id() & ~7;
+   const uint32_t mask = slot_mask32(sp);
+   const uint64_t nsl = static_cast<uint64_t>(mask) + 1;
+   const uint64_t bound = i.current_max_bucket_overflow < nsl ? i.current_max_bucket_overflow : nsl;
+   const bool mine = run && g < m;
+   K key = 0;
+   uint32_t home = 0;
+   if (mine) {
+      key = *reinterpret_cast<const K*>(keys + g * (len / m) * stride);
+      home = home_slot(key, sp);
+   }
+   bool active = mine, found = false;
+   for (uint64_t off = 0; __ballot(active); off += 8) {
+      const uint64_t p = off + gl;
+      const uint32_t slot = (home + static_cast<uint32_t>(p)) & mask;
+      K k = empty_key<K>();
+      if (active && p < bound) k = b[slot].key;
+      const bool stop = k == empty_key<K>() || ((slot - home_slot(k, sp)) & mask) < p; // Robin Hood order
+      const uint32_t hit = group_bits32<8>(__ballot(active && k == key), gbase);
+      const uint32_t end = group_bits32<8>(__ballot(stop), gbase);
+      if (active && (hit | end)) {
+         found = hit && (!end || __ffs(hit) < __ffs(end));
+         active = false;
+      }
+   }
+   if (mine && gl == 0 && !found) atomicAdd(&absent_s, 1u);
+   __syncthreads();
+   if (threadIdx.x == 0) {
+      out->info = i;
+      out->sampled = run ? m : 0;
+      out->absent = absent_s;
+   }
+}
+
 // A size power that no table has: nothing is found, and a caller that left its
 // values to the kernel gets its zeros all the same.
 template <typename K, bool PAIRS, int MODE>
@@ -581,6 +632,15 @@ int insert_pairs(const void* pairs, void* buckets, hn_info* info, size_t len, hi
 }
 
 template <typename K>
+int insert_look(const void* keys, size_t stride, size_t len, const void* buckets, const hn_info* info,
+                hn_insert_look* out, hipStream_t s) {
+   if (!buckets || !info || !out || (len && (!keys || stride < sizeof(K)))) return HN_EINVAL;
+   hipLaunchKernelGGL(k_insert_look<K>, dim3(1), dim3(kLookKeys * 8), 0, s, static_cast<const char*>(keys), stride, len,
+                      static_cast<const Slot<K>*>(buckets), info, out);
+   return static_cast<int>(hipGetLastError());
+}
+
+template <typename K>
 int retrieve_soa(const K* keys, K* vals, uint8_t* hit, const void* buckets, const hn_info* info, size_t len,
                  hipStream_t s, const hn_tune* t, bool zero) {
    if (!buckets || !info || (len && (!keys || !vals))) return HN_EINVAL;
@@ -822,6 +882,14 @@ int hn_insert_pairs_u32(const void* p, void* b, hn_info* i, size_t n, hn_stream_
 }
 int hn_insert_pairs_u64(const void* p, void* b, hn_info* i, size_t n, hn_stream_t s, const hn_tune* t) {
    return insert_pairs<uint64_t>(p, b, i, n, s, t);
+}
+int hn_insert_look_u32(const void* k, size_t stride, size_t n, const void* b, const hn_info* i, hn_insert_look* out,
+                       hn_stream_t s) {
+   return insert_look<uint32_t>(k, stride, n, b, i, out, s);
+}
+int hn_insert_look_u64(const void* k, size_t stride, size_t n, const void* b, const hn_info* i, hn_insert_look* out,
+                       hn_stream_t s) {
+   return insert_look<uint64_t>(k, stride, n, b, i, out, s);
 }
 int hn_retrieve_u32(const uint32_t* k, uint32_t* v, uint8_t* h, const void* b, const hn_info* i, size_t n,
                     hn_stream_t s, const hn_tune* t) {

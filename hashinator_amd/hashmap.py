@@ -246,13 +246,13 @@ class Hashmap:
         when the batch is in the table already: growing a map of many keys by a
         batch that the reorder pass would follow is one build of both
         (hn_grow_*).  An empty map that the build will fill is not rehashed.
-        Second the map's Info where it was read and still holds (a map that
-        does not grow), for the rest of the insert."""
-        i = self.info()
+        Second what _look has read, for the rest of the insert, where it still
+        holds (a map that does not grow)."""
+        look = i, _ = self._look(k, n, pairs, stream)
         fill = i.fill
         needed = math.ceil(math.log2((fill + n) * (1.0 / targetLF)))
         if needed <= self._sp:
-            return False, i
+            return False, look
         N = 1 << needed
         if fill == 0 and needed <= 32 and self._builds(n, N) and \
                 getattr(self._L, f"hn_build_scratch_bytes_{self._sfx}")(needed, n):
@@ -271,6 +271,25 @@ class Hashmap:
                 return True, None
         self.resize(needed, targets.device, stream)
         return False, None
+
+    def _may_merge_small(self, n) -> bool:
+        """Sizes of an insert that _try_merge takes if the map ends nearly full."""
+        N = self.bucket_count()
+        return bool(self.auto_reorder) and max(self.auto_reorder * N, self.build_min_keys) <= n < self.merge_min * N \
+            and n < N and self._sp <= 30
+
+    def _look(self, k, n, pairs, stream):
+        """The map's Info and, for an insert that may be merged though it is
+        small, about what share of its keys the map does not hold (hn_insert_look_*:
+        128 of them looked up, in the one read-back that the Info takes anyway)."""
+        if not self._may_merge_small(n):
+            return self.info(), 0.0
+        out = torch.empty(7, dtype=torch.int64, pin_memory=True)
+        check(self._fn("insert_look")(_ptr(k), k.element_size() * (2 if pairs else 1), n, _ptr(self.buckets),
+                                      _ptr(self._info), _ptr(out), _stream(stream)), "insert")
+        self._sync(stream)
+        raw = out.numpy()
+        return hn_info.from_buffer_copy(raw[:5].tobytes()), float(raw[6]) / max(1, int(raw[5]))
 
     def _grow(self, k, v, n, pairs, new_sp, stream) -> bool:
         sb = 0 if new_sp > 32 else getattr(self._L, f"hn_grow_scratch_bytes_{self._sfx}")(self._sp, new_sp, n)
@@ -315,12 +334,12 @@ class Hashmap:
         if n == 0:
             self._info.view(torch.int32)[8] = status.success
             return
-        done, i = self._grow_for(k, None if vals is None else v, n, vals is None, targetLF, stream)
+        done, look = self._grow_for(k, None if vals is None else v, n, vals is None, targetLF, stream)
         if done:
             return
         if self._try_build(k, None if vals is None else v, n, vals is None, stream):
             return
-        if self._try_merge(k, None if vals is None else v, n, vals is None, stream, i):
+        if self._try_merge(k, None if vals is None else v, n, vals is None, stream, look):
             return
         if vals is None:
             rc = self._fn("insert_pairs")(_ptr(k), _ptr(self.buckets), _ptr(self._info), n, _stream(stream), self._tune())
@@ -356,7 +375,7 @@ class Hashmap:
         del scratch
         return self.info().err == status.success
 
-    def _try_merge(self, k, v, n, pairs, stream, i=None) -> bool:
+    def _try_merge(self, k, v, n, pairs, stream, look=None) -> bool:
         """Large insert into a table that holds keys: hn_merge_* writes the
         insert + reorder image into a fresh bucket array, which then replaces
         the old one.  Where the merge itself declines (keys crowding one
@@ -364,24 +383,25 @@ class Hashmap:
         new array instead, so the insert is complete either way.
 
         Smaller inserts that the reorder pass would follow take it too where
-        the map ends at least 87% full and is ordered already: the probing
-        insert's chains grow with the load, the merge does not (one MI355X,
-        insert + reorder against merge + copy, a sixteenth of the slots
-        inserted up to load 0.9: 2^26 u64 slots 1.73 and 1.44 ms, 2^22 0.23
-        and 0.17; up to 0.85: 1.26 and 1.44, 0.15 and 0.17).  The image is
-        copied back, so that the bucket array stays the one that it was."""
+        the map ends at least 87% full, is ordered already and does not hold
+        most of the batch's keys: the probing insert's chains for
+        new keys grow with the load, its updates and the merge do not.  One
+        MI355X, insert + reorder against merge + copy, a sixteenth of 2^26 u64
+        slots: new keys up to load .82 1.18 and 1.52 ms, .88 1.76 and 1.54, .94
+        3.33 and 1.54, updates at .82 0.77 and 2.10, at .88 0.80 and 2.12; u32
+        new 1.06 and 1.14, 1.42 and 1.14, 3.02 and 1.16, updates 0.73 and 1.68,
+        0.75 and 1.68.  The image is copied back, so that the bucket array
+        stays the one that it was."""
         N = self.bucket_count()
-        if not self.merge_min or n < self.build_min_keys or n >= N or self._sp > 30:
+        small = self._may_merge_small(n)
+        if not small and (not self.merge_min or n < max(self.merge_min * N, self.build_min_keys) or n >= N or
+                          self._sp > 30):
             return False
-        small = n < self.merge_min * N
-        if small and not (self.auto_reorder and n >= self.auto_reorder * N):
-            return False
-        if i is None:
-            i = self.info()
+        i, new = look or self._look(k, n, pairs, stream)
         if i.fill == 0 or i.tombstone_counter != 0:
             return False
         ordered = bool(i.reserved1 & _lib.HN_INFO_ORDERED)
-        if small and not (ordered and i.fill + n >= 0.87 * N):
+        if small and not (ordered and new >= 0.5 and i.fill + new * n >= 0.87 * N):
             return False
         if not ordered:
             if n < self.merge_min * N * 4 / 3:
@@ -450,12 +470,12 @@ class Hashmap:
         if n == 0:
             self._info.view(torch.int32)[8] = status.success
             return
-        done, i = self._grow_for(k, None, n, False, targetLF, stream)
+        done, look = self._grow_for(k, None, n, False, targetLF, stream)
         if done:
             return
         if self._try_build(k, None, n, False, stream):
             return
-        if self._try_merge(k, None, n, False, stream, i):
+        if self._try_merge(k, None, n, False, stream, look):
             return
         check(self._fn("insert_index")(_ptr(k), _ptr(self.buckets), _ptr(self._info), n, _stream(stream),
                                        self._tune()), "insertIndex")

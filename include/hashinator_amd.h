@@ -146,6 +146,21 @@ HN_API int hn_insert_pairs_u32(const void* pairs, void* buckets, hn_info* info, 
 HN_API int hn_insert_pairs_u64(const void* pairs, void* buckets, hn_info* info, size_t len, hn_stream_t s,
                         const hn_tune* t);
 
+/* What an insert of these keys would meet, before it (an addition): the Info,
+ * and of up to 128 of the keys, taken at equal distances, how many the table
+ * does not hold.  Keys are looked up in a table with HN_INFO_ORDERED and no
+ * TOMBSTONEs only (sampled = 0 otherwise).  `key_stride`: bytes from one key
+ * to the next (the element size of a key list, or of a list of pairs).  `out`
+ * is device or pinned host memory; nothing else is written. */
+typedef struct hn_insert_look {
+   hn_info info;
+   uint64_t sampled, absent;
+} hn_insert_look;
+HN_API int hn_insert_look_u32(const void* keys, size_t key_stride, size_t len, const void* buckets, const hn_info* info,
+                              hn_insert_look* out, hn_stream_t s);
+HN_API int hn_insert_look_u64(const void* keys, size_t key_stride, size_t len, const void* buckets, const hn_info* info,
+                              hn_insert_look* out, hn_stream_t s);
+
 /* ---------------------------------------------------------------- retrieve */
 
 /* Hasher::retrieve(keys, vals, ...) (hashers.h:111-119) -> retrieve_kernel
