@@ -263,21 +263,26 @@ struct BatchScratch {
    uint64_t items;      // regions of all maps
    uint64_t n_big;      // maps without regions
    uint64_t pad[3];
-   // followed by unit_start[n_maps + 1], item_start[n_maps + 1], MapState[n_maps], kSpillCap indices per map
+   // followed by unit_start[n_maps + 1], item_start[n_maps + 1], MapState[n_maps], the spill lists
 };
 static_assert(sizeof(BatchScratch) == 64, "header of hn_batch_scratch_bytes");
 
 // What the region kernels leave for the per-map kernels.
 struct MapState {
+   uint32_t list;      // a map of several regions: its spill list, if below spill_lists(n_maps)
    uint32_t spilled;   // 1: an insert ran past its region's end; 2: k_boundary_insert left some keys
-   uint32_t n_spill;   // such keys; the first kSpillCap are listed by index
+   uint32_t n_spill;   // such keys; the first ones are listed by index
    uint32_t listed;    // clean: keys in the map's scratch slice, to be placed by k_map_clean_end
    uint32_t max_probe; // clean: longest probe of the keys placed by the regions
    uint32_t displaced; // clean: a live key stood away from its home slot
    uint32_t placed;    // clean: keys placed by the regions and their borders
-   uint32_t pad[2];
 };
-constexpr uint32_t kSpillCap = 248; // with the state, 1 KiB a map
+// Indices in a spill list.  Only maps of several regions can spill, and only
+// the first kSpillLists of them have a list (a list a map made a batch of a
+// million maps of one region take 1 GB of workspace; now 44 MB): without one,
+// or when it is full, k_boundary_insert looks through all of the map's keys.
+constexpr uint32_t kSpillCap = 248, kSpillLists = 4096;
+__host__ __device__ inline uint32_t spill_lists(uint32_t n_maps) { return n_maps < kSpillLists ? n_maps : kSpillLists; }
 
 __host__ __device__ inline uint64_t* unit_start(BatchScratch* sc) { return reinterpret_cast<uint64_t*>(sc + 1); }
 __host__ __device__ inline uint64_t* item_start(BatchScratch* sc, uint32_t n_maps) {
@@ -286,13 +291,19 @@ __host__ __device__ inline uint64_t* item_start(BatchScratch* sc, uint32_t n_map
 __host__ __device__ inline MapState* map_state(BatchScratch* sc, uint32_t n_maps) {
    return reinterpret_cast<MapState*>(item_start(sc, n_maps) + n_maps + 1);
 }
-__host__ __device__ inline uint32_t* spill_list(BatchScratch* sc, uint32_t n_maps, uint64_t map) {
-   return reinterpret_cast<uint32_t*>(map_state(sc, n_maps) + n_maps) + map * kSpillCap;
-}
+// A map's spill list and how many indices it holds.
+struct SpillList {
+   uint32_t* idx;
+   uint32_t cap;
+   __device__ SpillList(BatchScratch* sc, uint32_t n_maps, const MapState& st)
+       : idx(reinterpret_cast<uint32_t*>(map_state(sc, n_maps) + n_maps) + static_cast<uint64_t>(st.list) * kSpillCap),
+         cap(st.list < spill_lists(n_maps) ? kSpillCap : 0) {}
+};
 
 size_t batch_scratch_bytes(uint32_t n_maps) {
    const size_t b = sizeof(BatchScratch) + (static_cast<size_t>(n_maps) + 1) * 2 * sizeof(uint64_t) +
-                    static_cast<size_t>(n_maps) * (sizeof(MapState) + kSpillCap * sizeof(uint32_t));
+                    static_cast<size_t>(n_maps) * sizeof(MapState) +
+                    static_cast<size_t>(spill_lists(n_maps)) * kSpillCap * sizeof(uint32_t);
    return (b + 255) & ~static_cast<size_t>(255);
 }
 
@@ -328,7 +339,7 @@ __global__ __launch_bounds__(1024) void k_batch_prep(const hn_batch_map* maps, u
    uint64_t* us = unit_start(sc);
    uint64_t* is = item_start(sc, n_maps);
    MapState* st = map_state(sc, n_maps);
-   uint64_t units = 0, items = 0, big = 0;
+   uint64_t units = 0, items = 0, big = 0, several = 0;
    for (uint64_t base = 0; base < n_maps; base += 1024) {
       const uint64_t m = base + threadIdx.x;
       uint64_t u = 0, r = 0;
@@ -336,19 +347,23 @@ __global__ __launch_bounds__(1024) void k_batch_prep(const hn_batch_map* maps, u
          const hn_batch_map M = maps[m];
          r = regions ? batch_regions<K>(M, M.info->size_power, ops) : 0;
          u = r ? 0 : (M.qry_len + kBatchUnit - 1) / kBatchUnit;
-         st[m] = MapState{};
       }
       uint64_t tu, ti, tb;
       const uint64_t xu = block_excl_scan(u, wsum, &tu);
       const uint64_t xi = block_excl_scan(r, wsum, &ti);
-      block_excl_scan(m < n_maps && r == 0 ? 1 : 0, wsum, &tb);
+      // maps without regions, and (high half) those of several
+      const uint64_t xb = block_excl_scan(m < n_maps && r == 0 ? 1 : static_cast<uint64_t>(r > 1) << 32, wsum, &tb);
       if (m < n_maps) {
          us[m] = units + xu;
          is[m] = items + xi;
+         MapState z{};
+         z.list = static_cast<uint32_t>(several + (xb >> 32));
+         st[m] = z;
       }
       units += tu;
       items += ti;
-      big += tb;
+      big += tb & 0xFFFFFFFFull;
+      several += tb >> 32;
    }
    if (threadIdx.x == 0) {
       us[n_maps] = units;
@@ -469,6 +484,8 @@ __global__ __launch_bounds__(kRgBS) void k_region_insert(BatchArgs<K> a, BatchSc
       const int rlog = sp < kRegionLogB<K> ? sp : kRegionLogB<K>;
       const uint32_t R = 1u << rlog, W = R < kRgWin ? R : kRgWin;
       const uint64_t nreg = 1ull << (sp - rlog);
+      MapState* const st = &map_state(sc, a.n_maps)[mi];
+      const SpillList spill(sc, a.n_maps, *st);
       Slot<K>* b = static_cast<Slot<K>*>(M.buckets) + (r << rlog);
       for (uint32_t i = threadIdx.x; i < R; i += kRgBS) {
          const Slot<K> s = b[i];
@@ -485,18 +502,18 @@ __global__ __launch_bounds__(kRgBS) void k_region_insert(BatchArgs<K> a, BatchSc
           [&](uint32_t home) { return home & (R - 1); },
           [&](K key, uint32_t idx, uint32_t& pos, uint32_t& off) -> bool {
              uint32_t at;
-             const InsertStep st = lds_insert_step<K>(L, R, W, key, idx, pos, off, &at);
-             if (st == STEP_PLACED) {
+             const InsertStep did = lds_insert_step<K>(L, R, W, key, idx, pos, off, &at);
+             if (did == STEP_PLACED) {
                 ++placed;
                 const uint32_t pr = off + (at - pos) + 1;
                 max_probe = pr > max_probe ? pr : max_probe;
              }
-             if (st != STEP_NEXT) return st != STEP_AGAIN;
+             if (did != STEP_NEXT) return did != STEP_AGAIN;
              if (pos == R) {
                 if (nreg > 1) { // k_boundary_insert's
                    spilled = true;
-                   const uint32_t n = atomic_add_relaxed(&map_state(sc, a.n_maps)[mi].n_spill, 1u);
-                   if (n < kSpillCap) spill_list(sc, a.n_maps, mi)[n] = idx;
+                   const uint32_t n = atomic_add_relaxed(&st->n_spill, 1u);
+                   if (n < spill.cap) spill.idx[n] = idx;
                    return true;
                 }
                 pos = 0;
@@ -527,8 +544,7 @@ __global__ __launch_bounds__(kRgBS) void k_region_insert(BatchArgs<K> a, BatchSc
             atomic_max_relaxed(&M.info->current_max_bucket_overflow,
                                next_overflow(L.max_probe, kBucketOverflow));
          if (L.flag & 1u)
-            __hip_atomic_fetch_or(&map_state(sc, a.n_maps)[mi].spilled, 1u, __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_or(&st->spilled, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
          if (L.flag & 2u)
             __hip_atomic_fetch_or(&M.info->reserved1, kInfoFail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
@@ -664,11 +680,11 @@ __global__ __launch_bounds__(kRgBS) void k_boundary_insert(BatchArgs<K> a, Batch
       };
       auto place = [&](uint32_t home) { return home - lo; };
       const Slot<K>* const list = CLEAN ? a.clean_scratch + M.scratch_off : nullptr;
+      const SpillList spill(sc, a.n_maps, *st);
       if constexpr (CLEAN)
          lds_probe<K>(L, SlotKeys<K>{list, st->listed}, sp, take, place, step);
-      else if (st->n_spill <= kSpillCap)
-         lds_probe<K>(L, PickedKeys<K>{a.ins_keys + M.ins_off, spill_list(sc, a.n_maps, mi), st->n_spill}, sp, take,
-                      place, step);
+      else if (st->n_spill <= spill.cap)
+         lds_probe<K>(L, PickedKeys<K>{a.ins_keys + M.ins_off, spill.idx, st->n_spill}, sp, take, place, step);
       else
          lds_probe<K>(L, KeyList<K>(a.ins_keys + M.ins_off, static_cast<uint32_t>(M.ins_len)), sp, take, place, step);
       placed = wave_sum(placed);

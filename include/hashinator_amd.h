@@ -491,9 +491,12 @@ typedef struct hn_batch_map {
 
 enum { HN_BATCH_INSERT = 1, HN_BATCH_RETRIEVE = 2, HN_BATCH_ERASE = 4, HN_BATCH_CLEAN = 8 };
 
-/* Device scratch of hn_batch_run for a batch of n_maps maps: the tickets and,
- * per map, its first retrieve unit, its first region and what its regions
- * leave for the map (about 1 KiB per map). */
+/* Device scratch of hn_batch_run for a batch of n_maps maps: the tickets, per
+ * map its first retrieve unit, its first region and what its regions leave for
+ * the map (44 bytes), and lists of up to 4 MB for maps of several regions.
+ * hn_batch_run_* is not told the size of the buffer that it is given, so ask
+ * this function, of the library that runs, for it: the layout is that
+ * library's own and not a sum of the above. */
 HN_API size_t hn_batch_scratch_bytes(uint32_t n_maps);
 
 /* Fresh tables ({EMPTYBUCKET, 0}) and Info(sps[m]) for all maps, one launch.

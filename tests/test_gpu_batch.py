@@ -374,3 +374,26 @@ def test_batch_clean_keeps_one_copy_of_a_key(gpu, key_bits):
         assert np.array_equal(live_pairs(img, key_bits), np.stack([left, left], axis=1)), m
         assert (info.fill, info.tombstone_counter, info.err) == (left.size, 0, 0), m
         assert reachable_all(img, key_bits, sp), m
+
+
+def test_batch_more_maps_than_spill_lists(gpu):
+    """4,130 maps of two regions whose keys crowd the regions' ends: the last ones have no list for
+    the keys that run past an end, and are found among all of the map's."""
+    key_bits, sp, n_maps = 64, 13, 4130
+    pool = W.unique_keys(1 << 17, key_bits, 8)
+    home = O.fibhash(pool, np.full(pool.size, sp), key_bits) & ((1 << sp) - 1)
+    pool = pool[(home & 4095) >= 4096 - 350]
+    ins = [pool[(37 * m) % 1000:][:900] for m in range(n_maps)]
+    none = [pool[:0]] * n_maps
+    bm = BatchedMaps([sp] * n_maps, ins, ins, [k[:200] for k in ins], none, key_bits=key_bits)
+    bm.init()
+    bm.run(_lib.HN_BATCH_INSERT | _lib.HN_BATCH_RETRIEVE)
+    torch.cuda.synchronize()
+    infos = bm.infos.cpu().numpy()
+    assert (infos[:, 1] == 900).all() and (infos[:, 4] & 0xFFFFFFFF == 0).all()
+    assert bool(bm.qry_hit.bool().all())
+    for m in [0, 4095, *range(4096, n_maps)]:
+        img = bm.buckets(m)
+        k = np.sort(ins[m])
+        assert np.array_equal(live_pairs(img, key_bits), np.stack([k, k], axis=1)), m
+        assert reachable_all(img, key_bits, sp), m
