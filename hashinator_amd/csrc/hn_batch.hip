@@ -247,22 +247,23 @@ __global__ void k_zero_u64(uint64_t* p) { *p = 0; }
 
 // ---------------------------------------------------------- retrieve phase
 //
-// The retrieve phase runs on its own, one key per lane (lane_lookup): every
-// map's queries are cut into units of kBatchUnit, numbered map after map
-// (map m owns units [unit_start[m], unit_start[m+1]), so units come in the
-// caller's map order, largest maps first), and a wave takes the next unit by
-// a 64-bit ticket.  No unit is empty and no ticket is wasted.  Results per
+// The queries of maps without regions, and of those with regions whose lists
+// are long (by_units), run on their own, one key per lane (lane_lookup): they
+// are cut into units of kBatchUnit, numbered map after map (map m owns units
+// [unit_start[m], unit_start[m+1]), so units come in the caller's map order,
+// largest maps first), and dealt to the waves in turn: units are alike, a
+// ticket for each wave and unit took 16 ns apiece (53 us of any call), and with
+// units of 4,096 the last one alone took 130.  No unit is empty.  Results per
 // map are those of the plain retrieve: maps are independent, and the phases
 // still run insert -> retrieve -> erase -> clean for each of them.
-constexpr uint64_t kBatchUnit = 4096;
+constexpr uint64_t kBatchUnit = 1024;
 
 struct BatchScratch {
-   uint64_t ticket;     // map ticket of k_batch
-   uint64_t qry_ticket; // unit ticket of the retrieve phase
-   uint64_t units;      // units of all maps
-   uint64_t items;      // regions of all maps
-   uint64_t n_big;      // maps without regions
-   uint64_t pad[3];
+   uint64_t ticket; // map ticket of k_batch
+   uint64_t units;  // retrieve units of all maps
+   uint64_t items;  // regions of all maps
+   uint64_t n_big;  // maps without regions
+   uint64_t pad[4];
    // followed by unit_start[n_maps + 1], item_start[n_maps + 1], MapState[n_maps], the spill lists
 };
 static_assert(sizeof(BatchScratch) == 64, "header of hn_batch_scratch_bytes");
@@ -307,63 +308,92 @@ size_t batch_scratch_bytes(uint32_t n_maps) {
    return (b + 255) & ~static_cast<size_t>(255);
 }
 
-// Block-wide exclusive prefix of one value per thread (1,024 threads);
-// *total receives the sum.  wsum: one word per wave.
-__device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t* wsum, uint64_t* total) {
+// Block-wide exclusive prefixes of N values per thread (1,024 threads, sums
+// below 2^32); total receives the sums.  wsum: one entry per wave.
+template <int N>
+__device__ __forceinline__ void block_excl_scan(uint32_t (&v)[N], uint32_t (*wsum)[N], uint32_t (&total)[N]) {
    const int lane = __lane_id(), w = threadIdx.x / kWave;
-   uint64_t x = v;
-   for (int o = 1; o < kWave; o <<= 1) {
-      const uint64_t y = __shfl_up(x, o, kWave);
-      if (lane >= o) x += y;
-   }
-   if (lane == kWave - 1) wsum[w] = x;
-   __syncthreads();
-   uint64_t off = 0, sum = 0;
-   for (int i = 0; i < 1024 / kWave; ++i) {
-      if (i < w) off += wsum[i];
-      sum += wsum[i];
+   static_assert(1024 / kWave == 16, "a row of 16 lanes scans the waves' sums");
+#pragma unroll
+   for (int k = 0; k < N; ++k) {
+      const uint32_t x = wave_incl_add(v[k]);
+      if (lane == kWave - 1) wsum[w][k] = x;
+      v[k] = x - v[k];
    }
    __syncthreads();
-   *total = sum;
-   return off + x - v;
+#pragma unroll
+   for (int k = 0; k < N; ++k) {
+      const uint32_t mine = wsum[lane & 15][k];
+      int x = static_cast<int>(mine);
+      x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false); // row_shr:1, 2, 4, 8
+      x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+      x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+      x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+      total[k] = static_cast<uint32_t>(__shfl(x, 15, kWave));
+      v[k] += static_cast<uint32_t>(__shfl(x, w, kWave) - __shfl(static_cast<int>(mine), w, kWave));
+   }
+   __syncthreads();
 }
 
-// Over the maps, exclusive prefix sums of the retrieve units (maps without
-// regions, or every map when `regions` is 0) and of the regions; the tickets
-// and the maps' states start at 0.  One workgroup of 1,024 threads, 1,024
-// maps per step.
+// Whether a map's queries are looked up by units, although it has regions.
+// Each of its regions' workgroups reads the whole list (0.43 ns a query) and
+// looks up its own share (2.2 ns each) on the CU that it has; the units go over
+// the whole device, but wait for memory, and for clustered keys' long probes.
+// So by units: lists that a region takes long for, over 30 us where it is alone,
+// over 100 where the regions of as many such maps as the call has would give
+// every CU one; and maps of more than 32 regions, whose reading
+// costs more than the lookups.  By regions and by units, us a call: one u32 map
+// of 2^13 slots, 8,192 queries 45 and 46, 2^22 9,480 and 75; 100 such maps,
+// 30,011 each 97 and 64; 256, 8,192 each 55 and 67, 32,768 each 122 and 143; one
+// of 2^16 slots with 65,536 73 and 46, 64 with 78,643 ids of a grid each 130 and
+// 296; one of 2^20 with 262,144 144 and 54; one u64 map of 2^22 slots, 2^24
+// queries 19,300 and 449.
+constexpr uint64_t kRegionsByUnits = 32, kRegionsFill = 256;
+__device__ __forceinline__ bool by_units(uint64_t nq, uint64_t regions, uint32_t n_maps) {
+   const uint64_t wgs = n_maps * regions, limit_ns = 30000 + 70000 * (wgs < kRegionsFill ? wgs : kRegionsFill) / kRegionsFill;
+   return regions == 0 || regions > kRegionsByUnits || nq * (430 * regions + 2200) > 1000 * limit_ns * regions;
+}
+
+// Over the maps, exclusive prefix sums of the retrieve units (maps that are
+// looked up by units; every map when `regions` is 0) and of the regions; the
+// maps' states start at 0.  One workgroup of 1,024 threads, 1,024 maps per
+// step.
 template <typename K>
 __global__ __launch_bounds__(1024) void k_batch_prep(const hn_batch_map* maps, uint32_t n_maps, uint32_t ops,
                                                      int regions, BatchScratch* sc) {
-   __shared__ uint64_t wsum[1024 / kWave];
+   __shared__ uint32_t wsum[1024 / kWave][4];
    uint64_t* us = unit_start(sc);
    uint64_t* is = item_start(sc, n_maps);
    MapState* st = map_state(sc, n_maps);
-   uint64_t units = 0, items = 0, big = 0, several = 0;
+   constexpr int kLow = 22; // a step's units in two parts, whose sums stay below 2^32
+   uint64_t units = 0, items = 0;
+   uint32_t several = 0, big = 0;
    for (uint64_t base = 0; base < n_maps; base += 1024) {
       const uint64_t m = base + threadIdx.x;
-      uint64_t u = 0, r = 0;
+      uint64_t u = 0;
+      uint32_t r = 0;
       if (m < n_maps) {
          const hn_batch_map M = maps[m];
+         const uint64_t nq = (ops & HN_BATCH_RETRIEVE) ? M.qry_len : 0;
          r = regions ? batch_regions<K>(M, M.info->size_power, ops) : 0;
-         u = r ? 0 : (M.qry_len + kBatchUnit - 1) / kBatchUnit;
+         if (by_units(nq, r, n_maps)) u = (nq + kBatchUnit - 1) / kBatchUnit;
       }
-      uint64_t tu, ti, tb;
-      const uint64_t xu = block_excl_scan(u, wsum, &tu);
-      const uint64_t xi = block_excl_scan(r, wsum, &ti);
-      // maps without regions, and (high half) those of several
-      const uint64_t xb = block_excl_scan(m < n_maps && r == 0 ? 1 : static_cast<uint64_t>(r > 1) << 32, wsum, &tb);
+      // units, regions (at most 2^20 a step), and maps of several regions and of none
+      uint32_t v[4] = {static_cast<uint32_t>(u & ((1u << kLow) - 1)), static_cast<uint32_t>(u >> kLow), r,
+                       (r > 1 ? 1u : 0u) | (m < n_maps && r == 0 ? 1u << 16 : 0u)};
+      uint32_t total[4];
+      block_excl_scan<4>(v, wsum, total);
       if (m < n_maps) {
-         us[m] = units + xu;
-         is[m] = items + xi;
+         us[m] = units + v[0] + (static_cast<uint64_t>(v[1]) << kLow);
+         is[m] = items + v[2];
          MapState z{};
-         z.list = static_cast<uint32_t>(several + (xb >> 32));
+         z.list = several + (v[3] & 0xFFFFu);
          st[m] = z;
       }
-      units += tu;
-      items += ti;
-      big += tb & 0xFFFFFFFFull;
-      several += tb >> 32;
+      units += total[0] + (static_cast<uint64_t>(total[1]) << kLow);
+      items += total[2];
+      several += total[3] & 0xFFFFu;
+      big += total[3] >> 16;
    }
    if (threadIdx.x == 0) {
       us[n_maps] = units;
@@ -371,21 +401,7 @@ __global__ __launch_bounds__(1024) void k_batch_prep(const hn_batch_map* maps, u
       sc->units = units;
       sc->items = items;
       sc->n_big = big;
-      sc->qry_ticket = 0;
    }
-}
-
-// The next work unit of a wave.  Lane 0 draws one ticket and readfirstlane
-// hands it to the wave as a scalar, so the unit -- and every branch on it --
-// is wave-uniform by construction and each wave takes exactly one ticket per
-// unit.  Must be called with the whole wave active (lane 0 is then the first
-// active lane).
-__device__ __forceinline__ uint64_t next_unit(uint64_t* ticket) {
-   uint64_t t = 0;
-   if (__lane_id() == 0) t = __hip_atomic_fetch_add(ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-   const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(t));
-   const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(t >> 32));
-   return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
 template <typename K>
@@ -394,9 +410,7 @@ __global__ __launch_bounds__(kWave) void k_batch_retrieve_lane(BatchArgs<K> a, B
    const uint64_t units = sc->units;
    if (units == 0) return; // every map has regions
    const uint64_t* us = unit_start(sc);
-   for (;;) {
-      const uint64_t u = next_unit(&sc->qry_ticket);
-      if (u >= units) break;
+   for (uint64_t u = blockIdx.x; u < units; u += gridDim.x) {
       // the map holding unit u: us[lo] <= u < us[hi] throughout, so map lo has units
       uint32_t lo = 0, hi = a.n_maps;
       while (hi - lo > 1) {
@@ -868,7 +882,8 @@ __global__ __launch_bounds__(kRgBS) __attribute__((amdgpu_waves_per_eu(4))) void
    uint64_t mi, r64, item = blockIdx.x;
    while (next_region(L, sc, a.n_maps, &item, &mi, &r64)) {
       const hn_batch_map M = a.maps[mi];
-      const uint32_t nq = (a.ops & HN_BATCH_RETRIEVE) ? static_cast<uint32_t>(M.qry_len) : 0;
+      const uint64_t* const us = unit_start(sc) + mi;
+      const uint32_t nq = (a.ops & HN_BATCH_RETRIEVE) && us[0] == us[1] ? static_cast<uint32_t>(M.qry_len) : 0;
       const uint32_t ne = (a.ops & HN_BATCH_ERASE) ? static_cast<uint32_t>(M.ers_len) : 0;
       if (nq == 0 && ne == 0) continue;
       const int sp = M.info->size_power;

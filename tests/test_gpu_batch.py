@@ -397,3 +397,58 @@ def test_batch_more_maps_than_spill_lists(gpu):
         k = np.sort(ins[m])
         assert np.array_equal(live_pairs(img, key_bits), np.stack([k, k], axis=1)), m
         assert reachable_all(img, key_bits, sp), m
+
+
+def scratch_words(bm):
+    """ticket, retrieve units, regions and maps without regions, as the call's set-up left them."""
+    return bm.scratch[:32].cpu().numpy().view(np.uint64)
+
+
+@pytest.mark.parametrize("key_bits", [32, 64])
+# maps, size power below a one-region map's (negative: above), queries each, whether they go by units
+@pytest.mark.parametrize("n_maps,below,nq,units", [(1, 0, 1 << 21, True), (8, 1, 1 << 18, True), (1, 0, 4000, False),
+                                                   (1, 1, 30_011, True), (3, -3, 1 << 19, True), (1, -9, 70_001, True),
+                                                   (300, 2, 20_000, False), (16, -2, 5000, False), (100, 0, 30_011, True)])
+def test_batch_long_query_lists(gpu, key_bits, n_maps, below, nq, units):
+    """Query lists much longer than the table go over the whole device in units, those of a size
+    with it stay with its regions; the results are the oracle's either way, and a call is not much
+    slower than the lookups by units alone, which asking for a launch shape gives."""
+    from tests.helpers import race
+    sp = (13 if key_bits == 32 else 12) - below
+    n = int(0.55 * (1 << sp))
+    rng = np.random.default_rng(nq)
+    ins = [W.unique_keys(n, key_bits, 40 + m) for m in range(n_maps)]
+    pool = [np.concatenate([k, W.unique_keys(n, key_bits, 40 + m, start=n + 2)]) for m, k in enumerate(ins)]
+    qry = [p[rng.integers(0, p.size, nq - m)] for m, p in enumerate(pool)]
+    wl = ([sp] * n_maps, ins, [(k ^ k.dtype.type(0x33)).astype(k.dtype) for k in ins], qry, [k[: n // 7] for k in ins])
+    bm = BatchedMaps(*wl, key_bits=key_bits)
+    bm.init()
+    bm.run(_lib.HN_BATCH_INSERT)
+    shape = hn_tune(4, 512, 0, 0)
+    default, asked = race(lambda: bm.run(_lib.HN_BATCH_RETRIEVE), lambda: bm.run(_lib.HN_BATCH_RETRIEVE, shape), reps=9)
+    assert default <= 1.5 * asked, (default, asked)
+    bm.qry_vals.zero_()
+    bm.qry_hit.zero_()
+    bm.run(_lib.HN_BATCH_RETRIEVE | _lib.HN_BATCH_ERASE)
+    torch.cuda.synchronize()
+    assert (int(scratch_words(bm)[1]) > 0) == units
+    check_bulk(bm, wl, key_bits, _lib.HN_BATCH_INSERT | _lib.HN_BATCH_RETRIEVE | _lib.HN_BATCH_ERASE)
+
+
+def test_batch_query_units_beside_regions(gpu):
+    """Maps of every way in one call: one region and several, a few queries and a great many, none at
+    all, and a map that is not cut into regions."""
+    key_bits, rng = 32, np.random.default_rng(12)
+    sps = [16, 13, 13, 12, 10, 8, 3, 1, 15, 13]
+    nqs = [300_000, 1_000_000, 9000, 0, 200_000, 1, 700, 3, 20_000, 64]
+    ins = [W.unique_keys(max(1, int(0.6 * (1 << sp))), key_bits, 70 + m) for m, sp in enumerate(sps)]
+    qry = [np.concatenate([k, W.unique_keys(k.size + 8, key_bits, 70 + m, start=k.size + 2)])[rng.integers(0, 2 * k.size + 8, q)]
+           for m, (k, q) in enumerate(zip(ins, nqs))]
+    wl = (sps, ins, ins, qry, [rng.choice(k, k.size // 4, replace=False) for k in ins])
+    bm = BatchedMaps(*wl, key_bits=key_bits)
+    for ops in (_lib.HN_BATCH_ALL, _lib.HN_BATCH_INSERT | _lib.HN_BATCH_RETRIEVE):
+        bm.init()
+        bm.qry_vals.zero_()
+        bm.run(ops)
+        torch.cuda.synchronize()
+        check_against_oracle(bm, wl, key_bits, ops)
