@@ -1,10 +1,10 @@
-"""Many independent maps: the one-launch batched path and the per-map path.
+"""Many independent maps: the batched path and the per-map path.
 
 ``BatchedMaps`` lays out a set of maps (sizes 2^sp each) and their per-map
 inputs in device memory and runs, for every map, insert -> retrieve -> erase
 -> clean_tombstones either
 
-* batched: one persistent launch (``hn_batch_run_*``), graph-capturable, or
+* batched: a few launches for all maps (``hn_batch_run_*``), graph-capturable, or
 * per map: the plain C-ABI calls, one launch (or a few) per map per operation,
   which is how the reference's API is used (hashers.h:46-163).
 
@@ -103,7 +103,7 @@ class BatchedMaps:
                                                            self._s(stream)), "hn_batch_init")
 
     def run(self, ops=_lib.HN_BATCH_ALL, tune: hn_tune | None = None, stream=None):
-        """All requested phases on every map in one persistent launch."""
+        """All requested phases on every map, in a few launches whatever their number."""
         check(getattr(self.L, f"hn_batch_run_{self.sfx}")(
             _p(self.descs), self.n, ops, _p(self.ins_keys), _p(self.ins_vals), _p(self.qry_keys),
             _p(self.qry_vals), _p(self.qry_hit), _p(self.ers_keys), _p(self.clean_scratch), _p(self.scratch),

@@ -1,4 +1,4 @@
-// hn_batch.hip -- many independent maps in a few persistent launches.
+// hn_batch.hip -- many independent maps in a few launches.
 //
 // No counterpart kernel in the reference (its API is one launch per map per
 // operation, hashers.h:46-163); the per-map semantics are the reference's:
@@ -17,17 +17,23 @@
 // factor 0.6, velocity-grid ids: 4.99 ms, two launches of 2.16 ms among them;
 // by regions 1.04 ms: insert 0.32 + 0.08, lookups 0.35, clean 0.15 + 0.05 ms.
 // 4,096 such maps: 10.3 -> 4.2 ms; one u64 map of 2^20 slots: 13.8 -> 1.3
-// ms).  Maps of more than kMaxRegions regions, maps that a call barely
-// touches, and calls with explicit tuning take the paths below:
+// ms).  What is few keys for its map goes another way (map_ways): the insert
+// and the erase by one workgroup that probes the table where it stands
+// (k_batch_group), lookups one key per lane (k_batch_retrieve_lane), as do
+// query lists much longer than the table.  A small call is launches only, so
+// the set-up (batch_prep) is a workgroup of the first of them, and an insert
+// is 4 launches, lookups and erases 3 (one map of 2^13 slots, 16 keys updated
+// 38 us by 6 launches and 19 us by 4; one workgroup in 2 launches 15).
 //
-// Insert, and erase + clean: one workgroup owns one map at a time and runs
-// the phases on it back to back, separated by workgroup barriers with
-// workgroup-scope fences (no other workgroup touches the map during the
-// launch); maps are handed out by an atomic ticket in the order the caller
-// lists them (largest first balances the grid).  Retrieve runs between the
-// two as its own launch, one key per lane over units of every map's queries
-// (k_batch_retrieve_lane).  The probe loops are the single-map ones
-// (hn_probe.hpp), so a map's results are those of the plain calls.
+// Maps of more than kMaxRegions regions, maps that a call barely touches, and
+// calls with explicit tuning: one workgroup owns one map at a time and runs
+// insert, and erase + clean, on it back to back, separated by workgroup
+// barriers with workgroup-scope fences (no other workgroup touches the map
+// during the launch).  With tuning, maps are handed out by an atomic ticket in
+// the order the caller lists them (largest first balances the grid).  Retrieve
+// runs between the two, one key per lane over units of every map's queries.
+// The probe loops are the single-map ones (hn_probe.hpp), so a map's results
+// are those of the plain calls.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -53,31 +59,100 @@ struct BatchArgs {
    const K* ers_keys;
    Slot<K>* clean_scratch;
    uint64_t* ticket;
-   uint32_t req;          // the call's phases (ops is the launch's)
-   const uint64_t* n_big; // if set, the launch serves only the maps without regions, this many
+   uint32_t req; // the call's phases (ops is the launch's)
 };
 
 // ------------------------------------------------------------ regions
 //
 constexpr uint64_t kMaxRegions = 1024;
+// Whether a map's queries are looked up by units, although it has regions.
+// Each of its regions' workgroups reads the whole list (0.43 ns a query) and
+// looks up its own share (2.2 ns each) on the CU that it has; the units go over
+// the whole device, but wait for memory, and for clustered keys' long probes.
+// So by units: lists that a region takes long for, over 30 us where it is alone,
+// over 100 where the regions of as many such maps as the call has would give
+// every CU one; and maps of more than 32 regions, whose reading
+// costs more than the lookups.  By regions and by units, us a call: one u32 map
+// of 2^13 slots, 8,192 queries 45 and 46, 2^22 9,480 and 75; 100 such maps,
+// 30,011 each 97 and 64; 256, 8,192 each 55 and 67, 32,768 each 122 and 143; one
+// of 2^16 slots with 65,536 73 and 46, 64 with 78,643 ids of a grid each 130 and
+// 296; one of 2^20 with 262,144 144 and 54; one u64 map of 2^22 slots, 2^24
+// queries 19,300 and 449.
+constexpr uint64_t kRegionsByUnits = 32, kRegionsFill = 256;
+__device__ __forceinline__ bool by_units(uint64_t nq, uint64_t regions, uint32_t n_maps) {
+   const uint64_t wgs = n_maps * regions, limit_ns = 30000 + 70000 * (wgs < kRegionsFill ? wgs : kRegionsFill) / kRegionsFill;
+   return regions == 0 || regions > kRegionsByUnits || nq * (430 * regions + 2200) > 1000 * limit_ns * regions;
+}
 
-// Regions of a map, or 0 when it takes the one-workgroup path: a size power
-// out of range; more than kMaxRegions regions (every region reads the map's
-// whole key lists, so the reads grow with the square of the map: a u64 map of
-// 1,024 regions at load factor 0.6 takes 13.9 ms, one of 256 1.3 ms, against
-// 54 and 13.8 ms for one workgroup per map); lists
-// too long for 32-bit indices; or several regions and fewer keys than a
-// sixteenth of the slots, where loading the table costs more than probing it.
+// How a map's phases run: by its regions, or else by one workgroup (insert,
+// erase, clean) and by units (retrieve).
+enum : uint32_t { kWayIns = 1, kWayQry = 2, kWayErs = 4, kWayClean = 8 };
+
+// The map's regions, or 0: a size power out of range; more than kMaxRegions of
+// them (every region reads the map's whole key lists, so the reads grow with the
+// square of the map: a u64 map of 1,024 regions at load factor 0.6 takes 13.9
+// ms, one of 256 1.3 ms, against 54 and 13.8 ms for one workgroup per map); or
+// lists too long for 32-bit indices.
 template <typename K>
-__device__ __forceinline__ uint32_t batch_regions(const hn_batch_map& M, int sp, uint32_t ops) {
+__device__ __forceinline__ uint32_t map_regions(const hn_batch_map& M, int sp, uint32_t ops) {
    if (sp < 1 || sp > max_size_power<K>()) return 0;
+   const uint64_t nreg = sp <= kRegionLogB<K> ? 1 : 1ull << (sp - kRegionLogB<K>);
+   const uint64_t longest = ((ops & HN_BATCH_INSERT) ? M.ins_len : 0) | ((ops & HN_BATCH_RETRIEVE) ? M.qry_len : 0) |
+                            ((ops & HN_BATCH_ERASE) ? M.ers_len : 0);
+   return nreg > kMaxRegions || (longest >> 31) ? 0 : static_cast<uint32_t>(nreg);
+}
+// A map of several regions goes by them unless its lists hold fewer keys than a
+// sixteenth of the slots, where loading the table costs more than probing it.
+__device__ __forceinline__ bool several_pay(const hn_batch_map& M, uint32_t nreg, uint64_t n, uint32_t ops, uint32_t n_maps) {
+   const uint64_t nq = (ops & HN_BATCH_RETRIEVE) && !by_units(M.qry_len, nreg, n_maps) ? M.qry_len : 0;
+   const uint64_t keys = ((ops & HN_BATCH_INSERT) ? M.ins_len : 0) + nq + ((ops & HN_BATCH_ERASE) ? M.ers_len : 0);
+   return (ops & HN_BATCH_CLEAN) || keys * 16 >= n;
+}
+// Whether a map is inserted into by regions.  A map of one region is above an
+// eighth of its slots; up to there, its one workgroup probes the table where it
+// stands (4,096 u32 maps of 2^13 slots, 16 keys each 56 us, through LDS 188,
+// 1,024 of their keys updated 179 and 245; 1,024 maps, a quarter of the slots
+// into empty ones 117 and 62), unless TOMBSTONEs make the probes long (a table
+// full of them: 24 ms and 0.2).  By what an insert does not change, so that two
+// workgroups that ask agree.
+template <typename K>
+__device__ __forceinline__ bool ins_by_regions(const hn_batch_map& M, const hn_info* info, int sp, uint32_t ops,
+                                               uint32_t n_maps) {
+   const uint32_t nreg = map_regions<K>(M, sp, ops);
+   if (!(ops & HN_BATCH_INSERT) || nreg == 0 || M.ins_len == 0) return false;
    const uint64_t n = 1ull << sp;
-   const uint64_t nreg = sp <= kRegionLogB<K> ? 1 : n >> kRegionLogB<K>;
-   const uint64_t ni = (ops & HN_BATCH_INSERT) ? M.ins_len : 0, nq = (ops & HN_BATCH_RETRIEVE) ? M.qry_len : 0,
-                  ne = (ops & HN_BATCH_ERASE) ? M.ers_len : 0;
-   if (nreg > kMaxRegions || ((ni | nq | ne) >> 31)) return 0;
-   if (nreg > 1 && !(ops & HN_BATCH_CLEAN) && (ni + nq + ne) * 16 < n) return 0;
-   return static_cast<uint32_t>(nreg);
+   return nreg > 1 ? several_pay(M, nreg, n, ops, n_maps) : M.ins_len * 8 > n || info->tombstone_counter * 4 >= n;
+}
+// All of a map's ways, decided once a call (batch_prep).  The keys of a map of
+// one region are looked up and erased where the table stands while they are few,
+// since indexing the region costs more than their probes, and by the region as
+// the probes get long.  Measured at u32, so / by the region:
+// - lookups, from 512 queries on or seven eighths of the slots taken: 256 maps
+//   of 2^12 slots, 128 queries, load factor 0.6 23 and 27 us, 0.9 74 and 29,
+//   4,096 maps 53 and 147, 129 and 152, 512 queries at 0.6 80 and 155 but one
+//   map of 2^10 27 and 24; fewer than 2^10 slots 62 and 113 also at 0.9;
+// - erases, from a tenth of the slots on in the largest two sizes and a quarter
+//   in others (256 maps of 2^13 slots, 0.6: a sixteenth 29 and 36 us, a quarter
+//   55 and 37), where five eighths are taken from a 64th on (0.8: 49 and 36; of
+//   2^10 slots 35 and 26; 4 keys each of 4,096 maps of 2^8 83 and 105);
+// - both where nearly all are: a table full of TOMBSTONEs is probed slot by slot.
+template <typename K>
+__device__ __forceinline__ uint32_t map_ways(const hn_batch_map& M, const hn_info* info, int sp, uint32_t ops,
+                                             uint32_t n_maps) {
+   const uint32_t nreg = map_regions<K>(M, sp, ops);
+   if (nreg == 0) return 0;
+   const uint64_t n = 1ull << sp, nq = (ops & HN_BATCH_RETRIEVE) ? M.qry_len : 0, ne = (ops & HN_BATCH_ERASE) ? M.ers_len : 0;
+   bool qry = nq && !by_units(nq, nreg, n_maps), ers = ne != 0;
+   if (nreg > 1) {
+      if (!several_pay(M, nreg, n, ops, n_maps)) return 0;
+   } else {
+      const uint64_t used = info->fill + info->tombstone_counter + ((ops & HN_BATCH_INSERT) ? M.ins_len : 0);
+      const bool full = used * 16 >= n * 15;
+      qry = qry && (nq >= 512 || full || (sp >= 10 && used * 8 >= n * 7));
+      ers = ers && (ne * (sp + 1 >= kRegionLogB<K> ? 10 : 4) >= n || full || (used * 8 >= n * 5 && ne >= 16 && ne * 64 >= n));
+   }
+   return (ins_by_regions<K>(M, info, sp, ops, n_maps) ? kWayIns : 0u) | (qry ? kWayQry : 0u) | (ers ? kWayErs : 0u) |
+          ((ops & HN_BATCH_CLEAN) ? kWayClean : 0u);
 }
 
 __device__ __forceinline__ void phase_barrier() {
@@ -86,160 +161,152 @@ __device__ __forceinline__ void phase_barrier() {
    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// One workgroup runs `ops` on one map.
+struct GroupMem {
+   unsigned long long placed, max, erased, lifted;
+   int failed;
+};
 template <typename K, int G>
-__global__ __launch_bounds__(1024) void k_batch(BatchArgs<K> a) {
-   __shared__ uint64_t s_map;
-   __shared__ unsigned long long s_placed, s_max, s_erased, s_lifted;
-   __shared__ int s_failed;
+__device__ __forceinline__ void map_phases(const BatchArgs<K>& a, const hn_batch_map& M, uint32_t ops, GroupMem& S) {
    const uint64_t groups = blockDim.x / G;
    const uint64_t g = threadIdx.x / G;
    const int lane = __lane_id();
-   if (a.n_big && *a.n_big == 0) return; // every map has regions
-
-   auto reset_shared = [&]() {
-      s_placed = 0;
-      s_max = 0;
-      s_erased = 0;
-      s_lifted = 0;
-      s_failed = 0;
-   };
+   hn_info* info = M.info;
+   Slot<K>* b = static_cast<Slot<K>*>(M.buckets);
+   const int sp = info->size_power;
+   const bool sp_ok = sp >= 1 && sp <= max_size_power<K>();
+   const uint64_t nsl = sp_ok ? (1ull << sp) : 0;
    auto fold_insert = [&](const InsertCounters& c) {
       const uint64_t p = wave_sum(c.placed);
       const uint64_t m = wave_max(c.max_probe);
       const int f = wave_max(c.failed);
       if (lane == 0) {
-         if (p) atomicAdd(&s_placed, static_cast<unsigned long long>(p));
-         if (m) atomicMax(&s_max, static_cast<unsigned long long>(m));
-         if (f) atomicOr(&s_failed, 1);
+         if (p) atomicAdd(&S.placed, static_cast<unsigned long long>(p));
+         if (m) atomicMax(&S.max, static_cast<unsigned long long>(m));
+         if (f) atomicOr(&S.failed, 1);
       }
    };
-
-   for (;;) {
-      if (threadIdx.x == 0) {
-         s_map = __hip_atomic_fetch_add(a.ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-         reset_shared();
+   if (threadIdx.x == 0) S = GroupMem{0, 0, 0, 0, 0};
+   __syncthreads();
+   if (ops & HN_BATCH_INSERT) {
+      InsertCounters c;
+      if (sp_ok) {
+         InsertArgs<K> ia{a.ins_keys + M.ins_off, a.ins_vals + M.ins_off, nullptr, b, info, M.ins_len,
+                          nullptr, nullptr, nullptr};
+         insert_range<K, G, SRC_SOA>(ia, sp, M.ins_len, g, groups, c);
       }
+      fold_insert(c);
       __syncthreads();
-      const uint64_t mi = s_map;
-      if (mi >= a.n_maps) break;
-      const hn_batch_map M = a.maps[mi];
-      hn_info* info = M.info;
-      Slot<K>* b = static_cast<Slot<K>*>(M.buckets);
-      const int sp = info->size_power;
-      const bool sp_ok = sp >= 1 && sp <= max_size_power<K>();
-      const uint64_t nsl = sp_ok ? (1ull << sp) : 0;
-      if (a.n_big && batch_regions<K>(M, sp, a.req)) {
-         __syncthreads(); // s_map is rewritten by thread 0 next
-         continue;
+      if (threadIdx.x == 0) {
+         info->fill += S.placed;
+         if (S.max) {
+            const uint64_t o = next_overflow(S.max, kBucketOverflow);
+            if (o > info->current_max_bucket_overflow) info->current_max_bucket_overflow = o;
+         }
+         info->err = (S.failed || !sp_ok) ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
+         info->reserved1 = 0; // inserts do not keep Robin Hood order
+         S.placed = 0;
+         S.max = 0;
+         S.failed = 0;
       }
-
-      if (a.ops & HN_BATCH_INSERT) {
+      phase_barrier();
+   }
+   if ((ops & HN_BATCH_RETRIEVE) && sp_ok) {
+      LookupArgs<K> la{a.qry_keys + M.qry_off, a.qry_vals + M.qry_off, nullptr,
+                       a.qry_hit ? a.qry_hit + M.qry_off : nullptr, b, info, M.qry_len, false};
+      lookup_range<K, G, false, LK_RETRIEVE>(la, sp, info->current_max_bucket_overflow, M.qry_len, g, groups,
+                                             (info->reserved1 & kInfoOrdered) != 0);
+      phase_barrier();
+   }
+   if ((ops & HN_BATCH_ERASE) && sp_ok) {
+      LookupArgs<K> la{a.ers_keys + M.ers_off, nullptr, nullptr, nullptr, b, info, M.ers_len, false};
+      const uint64_t e =
+          wave_sum(lookup_range<K, G, false, LK_ERASE>(la, sp, info->current_max_bucket_overflow, M.ers_len, g, groups,
+                                                       (info->reserved1 & kInfoOrdered) != 0));
+      if (lane == 0 && e) atomicAdd(&S.erased, static_cast<unsigned long long>(e));
+      __syncthreads();
+      if (threadIdx.x == 0) {
+         info->tombstone_counter += S.erased;
+         info->fill -= S.erased;
+      }
+      phase_barrier();
+   }
+   if ((ops & HN_BATCH_CLEAN) && sp_ok && info->tombstone_counter > 0) {
+      if (info->fill > M.scratch_cap) {
+         // not enough scratch to lift the displaced elements out: leave the map as it is
+         if (threadIdx.x == 0) info->err = HN_STATUS_FAIL;
+      } else {
+         // TOMBSTONE -> EMPTY; live elements away from home are lifted into scratch (one region: the map)
+         Slot<K>* out = a.clean_scratch + M.scratch_off;
+         const uint64_t mask = nsl - 1;
+         for (uint64_t base = 0; base < nsl; base += blockDim.x) {
+            const uint64_t i = base + threadIdx.x;
+            bool take = false;
+            Slot<K> s{};
+            if (i < nsl) {
+               s = b[i];
+               if (s.key == tomb_key<K>()) {
+                  Slot<K> e = s;
+                  e.key = empty_key<K>();
+                  b[i] = e;
+               } else if (s.key != empty_key<K>() && (fib_home(s.key, sp) & mask) != i) {
+                  take = true;
+               }
+            }
+            const uint64_t m = __ballot(take);
+            if (m) {
+               unsigned long long wb = 0;
+               const int leader = first_bit(m);
+               if (lane == leader) wb = atomicAdd(&S.lifted, static_cast<unsigned long long>(__popcll(m)));
+               wb = __shfl(wb, leader, kWave);
+               if (take) {
+                  out[wb + __popcll(m & ((1ull << lane) - 1ull))] = s;
+                  Slot<K> e = s;
+                  e.key = empty_key<K>();
+                  b[i] = e;
+               }
+            }
+         }
+         phase_barrier();
+         const uint64_t lifted = S.lifted;
+         if (threadIdx.x == 0) {
+            info->tombstone_counter = 0;
+            info->current_max_bucket_overflow = kBucketOverflow;
+            info->fill -= lifted;
+            info->reserved1 = 0; // the reinsertion does not keep Robin Hood order
+         }
+         phase_barrier();
          InsertCounters c;
-         if (sp_ok) {
-            InsertArgs<K> ia{a.ins_keys + M.ins_off, a.ins_vals + M.ins_off, nullptr, b, info, M.ins_len,
-                             nullptr, nullptr, nullptr};
-            insert_range<K, G, SRC_SOA>(ia, sp, M.ins_len, g, groups, c);
+         if (lifted) {
+            InsertArgs<K> ia{nullptr, nullptr, out, b, info, lifted, nullptr, nullptr, nullptr};
+            insert_range<K, G, SRC_PAIRS>(ia, sp, lifted, g, groups, c);
          }
          fold_insert(c);
          __syncthreads();
          if (threadIdx.x == 0) {
-            info->fill += s_placed;
-            if (s_max) {
-               const uint64_t o = next_overflow(s_max, kBucketOverflow);
+            info->fill += S.placed;
+            if (S.max) {
+               const uint64_t o = next_overflow(S.max, kBucketOverflow);
                if (o > info->current_max_bucket_overflow) info->current_max_bucket_overflow = o;
             }
-            info->err = (s_failed || !sp_ok) ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
-            info->reserved1 = 0; // inserts do not keep Robin Hood order
-            s_placed = 0;
-            s_max = 0;
-            s_failed = 0;
+            if (lifted) info->err = S.failed ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
          }
-         phase_barrier();
       }
-      if ((a.ops & HN_BATCH_RETRIEVE) && sp_ok) {
-         LookupArgs<K> la{a.qry_keys + M.qry_off, a.qry_vals + M.qry_off, nullptr,
-                          a.qry_hit ? a.qry_hit + M.qry_off : nullptr, b, info, M.qry_len, false};
-         lookup_range<K, G, false, LK_RETRIEVE>(la, sp, info->current_max_bucket_overflow, M.qry_len, g, groups,
-                                                (info->reserved1 & kInfoOrdered) != 0);
-         phase_barrier();
-      }
-      if ((a.ops & HN_BATCH_ERASE) && sp_ok) {
-         LookupArgs<K> la{a.ers_keys + M.ers_off, nullptr, nullptr, nullptr, b, info, M.ers_len, false};
-         const uint64_t e =
-             wave_sum(lookup_range<K, G, false, LK_ERASE>(la, sp, info->current_max_bucket_overflow, M.ers_len, g, groups,
-                                                          (info->reserved1 & kInfoOrdered) != 0));
-         if (lane == 0 && e) atomicAdd(&s_erased, static_cast<unsigned long long>(e));
-         __syncthreads();
-         if (threadIdx.x == 0) {
-            info->tombstone_counter += s_erased;
-            info->fill -= s_erased;
-         }
-         phase_barrier();
-      }
-      if ((a.ops & HN_BATCH_CLEAN) && sp_ok && info->tombstone_counter > 0) {
-         if (info->fill > M.scratch_cap) {
-            // not enough scratch to lift the displaced elements out: leave the map as it is
-            if (threadIdx.x == 0) info->err = HN_STATUS_FAIL;
-         } else {
-            // TOMBSTONE -> EMPTY; live elements away from home are lifted into scratch (one region: the map)
-            Slot<K>* out = a.clean_scratch + M.scratch_off;
-            const uint64_t mask = nsl - 1;
-            for (uint64_t base = 0; base < nsl; base += blockDim.x) {
-               const uint64_t i = base + threadIdx.x;
-               bool take = false;
-               Slot<K> s{};
-               if (i < nsl) {
-                  s = b[i];
-                  if (s.key == tomb_key<K>()) {
-                     Slot<K> e = s;
-                     e.key = empty_key<K>();
-                     b[i] = e;
-                  } else if (s.key != empty_key<K>() && (fib_home(s.key, sp) & mask) != i) {
-                     take = true;
-                  }
-               }
-               const uint64_t m = __ballot(take);
-               if (m) {
-                  unsigned long long wb = 0;
-                  const int leader = first_bit(m);
-                  if (lane == leader) wb = atomicAdd(&s_lifted, static_cast<unsigned long long>(__popcll(m)));
-                  wb = __shfl(wb, leader, kWave);
-                  if (take) {
-                     out[wb + __popcll(m & ((1ull << lane) - 1ull))] = s;
-                     Slot<K> e = s;
-                     e.key = empty_key<K>();
-                     b[i] = e;
-                  }
-               }
-            }
-            phase_barrier();
-            const uint64_t lifted = s_lifted;
-            if (threadIdx.x == 0) {
-               info->tombstone_counter = 0;
-               info->current_max_bucket_overflow = kBucketOverflow;
-               info->fill -= lifted;
-               info->reserved1 = 0; // the reinsertion does not keep Robin Hood order
-            }
-            phase_barrier();
-            InsertCounters c;
-            if (lifted) {
-               InsertArgs<K> ia{nullptr, nullptr, out, b, info, lifted, nullptr, nullptr, nullptr};
-               insert_range<K, G, SRC_PAIRS>(ia, sp, lifted, g, groups, c);
-            }
-            fold_insert(c);
-            __syncthreads();
-            if (threadIdx.x == 0) {
-               info->fill += s_placed;
-               if (s_max) {
-                  const uint64_t o = next_overflow(s_max, kBucketOverflow);
-                  if (o > info->current_max_bucket_overflow) info->current_max_bucket_overflow = o;
-               }
-               if (lifted) info->err = s_failed ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
-            }
-         }
-         phase_barrier();
-      }
-      __syncthreads(); // s_map is rewritten by thread 0 next
+      phase_barrier();
+   }
+   __syncthreads(); // S is set again by thread 0 next
+}
+
+template <typename K, int G>
+__global__ __launch_bounds__(1024) void k_batch(BatchArgs<K> a) {
+   __shared__ uint64_t s_map;
+   __shared__ GroupMem S;
+   for (;;) {
+      if (threadIdx.x == 0) s_map = __hip_atomic_fetch_add(a.ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      const uint64_t mi = s_map;
+      if (mi >= a.n_maps) break;
+      map_phases<K, G>(a, a.maps[mi], a.ops, S);
    }
 }
 
@@ -259,17 +326,32 @@ __global__ void k_zero_u64(uint64_t* p) { *p = 0; }
 constexpr uint64_t kBatchUnit = 1024;
 
 struct BatchScratch {
-   uint64_t ticket; // map ticket of k_batch
-   uint64_t units;  // retrieve units of all maps
-   uint64_t items;  // regions of all maps
-   uint64_t n_big;  // maps without regions
+   uint64_t ticket;  // map ticket of k_batch
+   uint64_t units;   // retrieve units of all maps
+   uint64_t items;   // regions of all maps
+   uint32_t several; // maps of several regions
+   uint32_t any;     // kAny*: what there is to do for whole launches
    uint64_t pad[4];
    // followed by unit_start[n_maps + 1], item_start[n_maps + 1], MapState[n_maps], the spill lists
 };
 static_assert(sizeof(BatchScratch) == 64, "header of hn_batch_scratch_bytes");
+enum : uint32_t {
+   kAnyIns = 1,     // a map is inserted into by regions
+   kAnyLook = 2,    // a map is looked up, or erased from, by regions
+   kAnyGroup = 4,   // a map is erased from, or cleaned, by one workgroup
+   kAnySpill = 8,   // an insert ran past its region's end
+   kAnyLeft = 16,   // k_boundary_insert left some of those
+   kAnyListed = 32, // clean: a map of several regions has listed keys
+};
+// Read first: 2,280 regions' atomics on the one word took 35 us.
+__device__ __forceinline__ void set_any(BatchScratch* sc, uint32_t bits) {
+   if (!(__hip_atomic_load(&sc->any, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bits))
+      __hip_atomic_fetch_or(&sc->any, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // What the region kernels leave for the per-map kernels.
 struct MapState {
+   uint32_t ways;      // kWay*
    uint32_t list;      // a map of several regions: its spill list, if below spill_lists(n_maps)
    uint32_t spilled;   // 1: an insert ran past its region's end; 2: k_boundary_insert left some keys
    uint32_t n_spill;   // such keys; the first ones are listed by index
@@ -280,7 +362,7 @@ struct MapState {
 };
 // Indices in a spill list.  Only maps of several regions can spill, and only
 // the first kSpillLists of them have a list (a list a map made a batch of a
-// million maps of one region take 1 GB of workspace; now 44 MB): without one,
+// million maps of one region take 1 GB of workspace; now 48 MB): without one,
 // or when it is full, k_boundary_insert looks through all of the map's keys.
 constexpr uint32_t kSpillCap = 248, kSpillLists = 4096;
 __host__ __device__ inline uint32_t spill_lists(uint32_t n_maps) { return n_maps < kSpillLists ? n_maps : kSpillLists; }
@@ -308,12 +390,12 @@ size_t batch_scratch_bytes(uint32_t n_maps) {
    return (b + 255) & ~static_cast<size_t>(255);
 }
 
-// Block-wide exclusive prefixes of N values per thread (1,024 threads, sums
+// Block-wide exclusive prefixes of N values per thread (kRgBS threads, sums
 // below 2^32); total receives the sums.  wsum: one entry per wave.
 template <int N>
 __device__ __forceinline__ void block_excl_scan(uint32_t (&v)[N], uint32_t (*wsum)[N], uint32_t (&total)[N]) {
    const int lane = __lane_id(), w = threadIdx.x / kWave;
-   static_assert(1024 / kWave == 16, "a row of 16 lanes scans the waves' sums");
+   static_assert(kRgWaves <= 16, "a row of 16 lanes scans the waves' sums");
 #pragma unroll
    for (int k = 0; k < N; ++k) {
       const uint32_t x = wave_incl_add(v[k]);
@@ -323,7 +405,7 @@ __device__ __forceinline__ void block_excl_scan(uint32_t (&v)[N], uint32_t (*wsu
    __syncthreads();
 #pragma unroll
    for (int k = 0; k < N; ++k) {
-      const uint32_t mine = wsum[lane & 15][k];
+      const uint32_t mine = (lane & 15) < kRgWaves ? wsum[lane & 15][k] : 0;
       int x = static_cast<int>(mine);
       x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false); // row_shr:1, 2, 4, 8
       x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
@@ -335,72 +417,93 @@ __device__ __forceinline__ void block_excl_scan(uint32_t (&v)[N], uint32_t (*wsu
    __syncthreads();
 }
 
-// Whether a map's queries are looked up by units, although it has regions.
-// Each of its regions' workgroups reads the whole list (0.43 ns a query) and
-// looks up its own share (2.2 ns each) on the CU that it has; the units go over
-// the whole device, but wait for memory, and for clustered keys' long probes.
-// So by units: lists that a region takes long for, over 30 us where it is alone,
-// over 100 where the regions of as many such maps as the call has would give
-// every CU one; and maps of more than 32 regions, whose reading
-// costs more than the lookups.  By regions and by units, us a call: one u32 map
-// of 2^13 slots, 8,192 queries 45 and 46, 2^22 9,480 and 75; 100 such maps,
-// 30,011 each 97 and 64; 256, 8,192 each 55 and 67, 32,768 each 122 and 143; one
-// of 2^16 slots with 65,536 73 and 46, 64 with 78,643 ids of a grid each 130 and
-// 296; one of 2^20 with 262,144 144 and 54; one u64 map of 2^22 slots, 2^24
-// queries 19,300 and 449.
-constexpr uint64_t kRegionsByUnits = 32, kRegionsFill = 256;
-__device__ __forceinline__ bool by_units(uint64_t nq, uint64_t regions, uint32_t n_maps) {
-   const uint64_t wgs = n_maps * regions, limit_ns = 30000 + 70000 * (wgs < kRegionsFill ? wgs : kRegionsFill) / kRegionsFill;
-   return regions == 0 || regions > kRegionsByUnits || nq * (430 * regions + 2200) > 1000 * limit_ns * regions;
-}
-
-// Over the maps, exclusive prefix sums of the retrieve units (maps that are
-// looked up by units; every map when `regions` is 0) and of the regions; the
-// maps' states start at 0.  One workgroup of 1,024 threads, 1,024 maps per
-// step.
+// A call's set-up, by one workgroup of kRgBS threads, as many maps per step:
+// exclusive prefix sums over the maps of the retrieve units (every map's when
+// `regions` is 0) and of the regions; the maps' states; err of the maps that
+// are inserted into by regions, to be set to FAIL by a region that fails.
 template <typename K>
-__global__ __launch_bounds__(1024) void k_batch_prep(const hn_batch_map* maps, uint32_t n_maps, uint32_t ops,
-                                                     int regions, BatchScratch* sc) {
-   __shared__ uint32_t wsum[1024 / kWave][4];
+__device__ __forceinline__ void batch_prep(const BatchArgs<K>& a, int regions, BatchScratch* sc) {
+   __shared__ uint32_t wsum[kRgWaves][4];
+   __shared__ uint32_t any_s;
+   const uint32_t n_maps = a.n_maps;
    uint64_t* us = unit_start(sc);
    uint64_t* is = item_start(sc, n_maps);
    MapState* st = map_state(sc, n_maps);
    constexpr int kLow = 22; // a step's units in two parts, whose sums stay below 2^32
    uint64_t units = 0, items = 0;
-   uint32_t several = 0, big = 0;
-   for (uint64_t base = 0; base < n_maps; base += 1024) {
+   uint32_t several = 0;
+   if (threadIdx.x == 0) any_s = 0;
+   for (uint64_t base = 0; base < n_maps; base += kRgBS) {
       const uint64_t m = base + threadIdx.x;
       uint64_t u = 0;
-      uint32_t r = 0;
+      uint32_t ways = 0, nreg = 0;
+      bool group = false;
       if (m < n_maps) {
-         const hn_batch_map M = maps[m];
-         const uint64_t nq = (ops & HN_BATCH_RETRIEVE) ? M.qry_len : 0;
-         r = regions ? batch_regions<K>(M, M.info->size_power, ops) : 0;
-         if (by_units(nq, r, n_maps)) u = (nq + kBatchUnit - 1) / kBatchUnit;
+         const hn_batch_map M = a.maps[m];
+         if (regions) {
+            const int sp = M.info->size_power;
+            ways = map_ways<K>(M, M.info, sp, a.req, n_maps);
+            nreg = ways ? map_regions<K>(M, sp, a.req) : 0;
+         }
+         if ((a.req & HN_BATCH_RETRIEVE) && !(ways & kWayQry)) u = (M.qry_len + kBatchUnit - 1) / kBatchUnit;
+         group = ((a.req & HN_BATCH_ERASE) && !(ways & kWayErs) && M.ers_len) ||
+                 ((a.req & HN_BATCH_CLEAN) && !(ways & kWayClean));
+         if (ways & kWayIns) {
+            M.info->err = HN_STATUS_SUCCESS;
+            M.info->reserved1 = 0; // inserts do not keep Robin Hood order
+         }
       }
-      // units, regions (at most 2^20 a step), and maps of several regions and of none
-      uint32_t v[4] = {static_cast<uint32_t>(u & ((1u << kLow) - 1)), static_cast<uint32_t>(u >> kLow), r,
-                       (r > 1 ? 1u : 0u) | (m < n_maps && r == 0 ? 1u << 16 : 0u)};
+      uint32_t v[4] = {static_cast<uint32_t>(u & ((1u << kLow) - 1)), static_cast<uint32_t>(u >> kLow), nreg,
+                       nreg > 1 ? 1u : 0u};
       uint32_t total[4];
       block_excl_scan<4>(v, wsum, total);
+      const uint32_t any = (__ballot(ways & kWayIns) ? kAnyIns : 0u) |
+                           (__ballot(ways & (kWayQry | kWayErs)) ? kAnyLook : 0u) | (__ballot(group) ? kAnyGroup : 0u);
+      if (__lane_id() == 0 && any) atomicOr(&any_s, any);
       if (m < n_maps) {
          us[m] = units + v[0] + (static_cast<uint64_t>(v[1]) << kLow);
          is[m] = items + v[2];
          MapState z{};
-         z.list = several + (v[3] & 0xFFFFu);
+         z.ways = ways;
+         z.list = several + v[3];
          st[m] = z;
       }
       units += total[0] + (static_cast<uint64_t>(total[1]) << kLow);
       items += total[2];
-      several += total[3] & 0xFFFFu;
-      big += total[3] >> 16;
+      several += total[3];
    }
+   __syncthreads();
    if (threadIdx.x == 0) {
       us[n_maps] = units;
       is[n_maps] = items;
       sc->units = units;
       sc->items = items;
-      sc->n_big = big;
+      sc->several = several;
+      sc->any = any_s;
+   }
+}
+
+// The phases that do not run by regions, a workgroup per map.  With `prep` the
+// call's set-up runs beside an insert phase, in workgroup 0 (both are mostly a
+// few waits for memory, and a launch is another 4 us).
+template <typename K>
+__global__ __launch_bounds__(kRgBS) void k_batch_group(BatchArgs<K> a, BatchScratch* sc, int prep, int regions) {
+   __shared__ GroupMem S;
+   if (prep && blockIdx.x == 0) {
+      batch_prep<K>(a, regions, sc);
+      return;
+   }
+   if (!prep && !(sc->any & kAnyGroup)) return;
+   for (uint64_t m = blockIdx.x - prep; m < a.n_maps; m += gridDim.x - prep) {
+      const hn_batch_map M = a.maps[m];
+      uint32_t ops;
+      if (prep) {
+         ops = ins_by_regions<K>(M, M.info, M.info->size_power, a.req, a.n_maps) ? 0 : a.ops;
+      } else {
+         const uint32_t ways = map_state(sc, a.n_maps)[m].ways;
+         ops = ((ways & kWayErs) || !M.ers_len ? 0 : a.ops & HN_BATCH_ERASE) | ((ways & kWayClean) ? 0 : a.ops & HN_BATCH_CLEAN);
+      }
+      if (ops) map_phases<K, default_probe_width<K>(OP_INSERT)>(a, M, ops, S);
    }
 }
 
@@ -408,7 +511,7 @@ template <typename K>
 __global__ __launch_bounds__(kWave) void k_batch_retrieve_lane(BatchArgs<K> a, BatchScratch* sc) {
    __shared__ LaneLds<K, LK_RETRIEVE> L;
    const uint64_t units = sc->units;
-   if (units == 0) return; // every map has regions
+   if (units == 0) return;
    const uint64_t* us = unit_start(sc);
    for (uint64_t u = blockIdx.x; u < units; u += gridDim.x) {
       // the map holding unit u: us[lo] <= u < us[hi] throughout, so map lo has units
@@ -483,6 +586,11 @@ __device__ __forceinline__ bool next_region(Mem& L, BatchScratch* sc, uint32_t n
    return true;
 }
 
+// err = FAIL, whatever other workgroups do to it (SUCCESS is 0).
+__device__ __forceinline__ void set_fail(hn_info* info) {
+   __hip_atomic_fetch_or(&info->err, HN_STATUS_FAIL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Insert phase on one region.  Bound by LDS probing and by the lists a region
 // has to read; the table passes through LDS once each way.  While keys are
 // placed a slot holds its value's index in the list, so that no probe waits
@@ -490,15 +598,16 @@ __device__ __forceinline__ bool next_region(Mem& L, BatchScratch* sc, uint32_t n
 template <typename K>
 __global__ __launch_bounds__(kRgBS) void k_region_insert(BatchArgs<K> a, BatchScratch* sc) {
    __shared__ RegionMem<K> L;
+   if (!(sc->any & kAnyIns)) return;
    uint64_t mi, r, item = blockIdx.x;
    while (next_region(L, sc, a.n_maps, &item, &mi, &r)) {
+      MapState* const st = &map_state(sc, a.n_maps)[mi];
+      if (!(st->ways & kWayIns)) continue;
       const hn_batch_map M = a.maps[mi];
-      if (M.ins_len == 0) continue;
       const int sp = M.info->size_power;
       const int rlog = sp < kRegionLogB<K> ? sp : kRegionLogB<K>;
       const uint32_t R = 1u << rlog, W = R < kRgWin ? R : kRgWin;
       const uint64_t nreg = 1ull << (sp - rlog);
-      MapState* const st = &map_state(sc, a.n_maps)[mi];
       const SpillList spill(sc, a.n_maps, *st);
       Slot<K>* b = static_cast<Slot<K>*>(M.buckets) + (r << rlog);
       for (uint32_t i = threadIdx.x; i < R; i += kRgBS) {
@@ -557,10 +666,11 @@ __global__ __launch_bounds__(kRgBS) void k_region_insert(BatchArgs<K> a, BatchSc
          if (L.max_probe)
             atomic_max_relaxed(&M.info->current_max_bucket_overflow,
                                next_overflow(L.max_probe, kBucketOverflow));
-         if (L.flag & 1u)
+         if (L.flag & 1u) {
             __hip_atomic_fetch_or(&st->spilled, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-         if (L.flag & 2u)
-            __hip_atomic_fetch_or(&M.info->reserved1, kInfoFail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            set_any(sc, kAnySpill);
+         }
+         if (L.flag & 2u) set_fail(M.info);
       }
    }
 }
@@ -619,6 +729,7 @@ __global__ __launch_bounds__(kRgBS) void k_boundary_insert(BatchArgs<K> a, Batch
    constexpr K kEmpty = empty_key<K>();
    constexpr uint32_t kSpan = 2 * kRgHalf;
    static_assert(kSpan <= RegionMem<K>::kSlots, "the window fits a region's arrays; windows are disjoint");
+   if (!(sc->any & (CLEAN ? kAnyListed : kAnySpill))) return;
    uint64_t mi, r, item = blockIdx.x;
    while (next_region(L, sc, a.n_maps, &item, &mi, &r)) {
       MapState* const st = &map_state(sc, a.n_maps)[mi];
@@ -648,7 +759,10 @@ __global__ __launch_bounds__(kRgBS) void k_boundary_insert(BatchArgs<K> a, Batch
       } else {
          if (tail == kRgHalf) continue; // the region's last slot is EMPTY
          if (tail == 0) {               // the run may reach back further
-            if (threadIdx.x == 0) __hip_atomic_fetch_or(&st->spilled, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (threadIdx.x == 0) {
+               __hip_atomic_fetch_or(&st->spilled, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+               set_any(sc, kAnyLeft);
+            }
             continue;
          }
       }
@@ -719,7 +833,10 @@ __global__ __launch_bounds__(kRgBS) void k_boundary_insert(BatchArgs<K> a, Batch
          b[(lo + i) & mask] = s;
       }
       if (threadIdx.x == 0) {
-         if (L.flag) __hip_atomic_fetch_or(&st->spilled, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+         if (L.flag) {
+            __hip_atomic_fetch_or(&st->spilled, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            set_any(sc, kAnyLeft);
+         }
          if constexpr (CLEAN) {
             if (L.n) atomic_add_relaxed(&st->placed, static_cast<uint32_t>(L.n));
             if (L.max_probe) atomic_max_relaxed(&st->max_probe, L.max_probe);
@@ -732,51 +849,49 @@ __global__ __launch_bounds__(kRgBS) void k_boundary_insert(BatchArgs<K> a, Batch
    }
 }
 
-// After k_region_insert and k_boundary_insert, one workgroup per map: the
-// keys that k_boundary_insert left (every key with a home in a region's last
-// run of occupied slots is tried in global memory), then err.
+// After k_region_insert and k_boundary_insert, a workgroup per map: the keys
+// that k_boundary_insert left (every key with a home in a region's last run of
+// occupied slots is tried in global memory).
 template <typename K>
 __global__ __launch_bounds__(kRgBS) void k_map_insert_end(BatchArgs<K> a, BatchScratch* sc) {
    __shared__ uint64_t tail[kMaxRegions]; // first slot of each region's last run of occupied slots
+   if (!(sc->any & kAnyLeft)) return;
    for (uint32_t m = blockIdx.x; m < a.n_maps; m += gridDim.x) {
+      MapState* const st = &map_state(sc, a.n_maps)[m];
+      if (!(st->spilled & 2u)) continue;
       const hn_batch_map M = a.maps[m];
-      hn_info* info = M.info;
-      const int sp = info->size_power;
-      const uint32_t nreg = batch_regions<K>(M, sp, a.req);
-      if (nreg == 0) continue;
-      if (map_state(sc, a.n_maps)[m].spilled & 2u) {
-         const int rlog = kRegionLogB<K>;
-         const uint64_t R = 1ull << rlog;
-         Slot<K>* b = static_cast<Slot<K>*>(M.buckets);
-         const int lane = __lane_id();
-         for (uint32_t r = threadIdx.x / kWave; r < nreg; r += kRgWaves) {
-            const uint64_t base = static_cast<uint64_t>(r) << rlog;
-            uint64_t first = base;
-            for (uint64_t o = R; o > 0; o -= kWave) {
-               const uint64_t e = __ballot(b[base + o - kWave + lane].key == empty_key<K>());
-               if (e) {
-                  first = base + o - __clzll(static_cast<long long>(e));
-                  break;
-               }
+      const int sp = M.info->size_power, rlog = kRegionLogB<K>; // only maps of several regions spill
+      const uint32_t nreg = 1u << (sp - rlog);
+      const uint64_t R = 1ull << rlog;
+      Slot<K>* b = static_cast<Slot<K>*>(M.buckets);
+      const int lane = __lane_id();
+      for (uint32_t r = threadIdx.x / kWave; r < nreg; r += kRgWaves) {
+         const uint64_t base = static_cast<uint64_t>(r) << rlog;
+         uint64_t first = base;
+         for (uint64_t o = R; o > 0; o -= kWave) {
+            const uint64_t e = __ballot(b[base + o - kWave + lane].key == empty_key<K>());
+            if (e) {
+               first = base + o - __clzll(static_cast<long long>(e));
+               break;
             }
-            if (lane == 0) tail[r] = first;
          }
-         __syncthreads();
-         InsertCounters c;
-         for (uint64_t i = threadIdx.x; i < M.ins_len; i += kRgBS) {
-            const K key = a.ins_keys[M.ins_off + i];
-            const uint64_t home = home_slot(key, sp);
-            if (home >= tail[home >> rlog]) insert_one<K>(b, sp, key, a.ins_vals[M.ins_off + i], c);
-         }
-         insert_fold(info, c.placed, c.max_probe, c.failed);
-         phase_barrier();
+         if (lane == 0) tail[r] = first;
       }
-      if (threadIdx.x == 0) {
-         const int32_t f = __hip_atomic_load(&info->reserved1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kInfoFail;
-         info->err = f ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
-         info->reserved1 = 0; // inserts do not keep Robin Hood order
+      __syncthreads();
+      InsertCounters c;
+      for (uint64_t i = threadIdx.x; i < M.ins_len; i += kRgBS) {
+         const K key = a.ins_keys[M.ins_off + i];
+         const uint64_t home = home_slot(key, sp);
+         if (home >= tail[home >> rlog]) insert_one<K>(b, sp, key, a.ins_vals[M.ins_off + i], c);
       }
-      __syncthreads(); // tail is rewritten for the next map
+      const uint64_t placed = wave_sum(c.placed), max_probe = wave_max(c.max_probe);
+      if (lane == 0) {
+         if (placed) atomic_add_relaxed(&M.info->fill, placed);
+         if (max_probe) atomic_max_relaxed(&M.info->current_max_bucket_overflow, next_overflow(max_probe, kBucketOverflow));
+      }
+      if (__ballot(c.failed) && lane == 0) set_fail(M.info);
+      __syncthreads(); // tail is rewritten for the next map; the state has been read
+      if (threadIdx.x == 0) st->spilled = 0; // the clean's from here
    }
 }
 
@@ -879,14 +994,15 @@ __global__ __launch_bounds__(kRgBS) __attribute__((amdgpu_waves_per_eu(4))) void
    constexpr K kTomb = tomb_key<K>();
    constexpr int E = static_cast<int>((IndexMem<K>::kHeld + kRgBS - 1) / kRgBS); // held slots per thread
    const int lane = __lane_id(), wave = threadIdx.x / kWave;
+   if (!(sc->any & kAnyLook)) return;
    uint64_t mi, r64, item = blockIdx.x;
    while (next_region(L, sc, a.n_maps, &item, &mi, &r64)) {
+      const uint32_t ways = map_state(sc, a.n_maps)[mi].ways;
+      if (!(ways & (kWayQry | kWayErs))) continue;
       const hn_batch_map M = a.maps[mi];
-      const uint64_t* const us = unit_start(sc) + mi;
-      const uint32_t nq = (a.ops & HN_BATCH_RETRIEVE) && us[0] == us[1] ? static_cast<uint32_t>(M.qry_len) : 0;
-      const uint32_t ne = (a.ops & HN_BATCH_ERASE) ? static_cast<uint32_t>(M.ers_len) : 0;
-      if (nq == 0 && ne == 0) continue;
       const int sp = M.info->size_power;
+      const uint32_t nq = (ways & kWayQry) ? static_cast<uint32_t>(M.qry_len) : 0;
+      const uint32_t ne = (ways & kWayErs) ? static_cast<uint32_t>(M.ers_len) : 0;
       const int rlog = sp < kRegionLogB<K> ? sp : kRegionLogB<K>;
       const uint32_t r = static_cast<uint32_t>(r64), R = 1u << rlog, mask = slot_mask32(sp), first = r << rlog;
       const uint64_t nreg = 1ull << (sp - rlog);
@@ -1053,6 +1169,17 @@ __global__ __launch_bounds__(kRgBS) __attribute__((amdgpu_waves_per_eu(4))) void
    }
 }
 
+// A cleaned map's Info, by one thread.
+__device__ __forceinline__ void clean_info(hn_info* info, uint64_t placed, uint32_t max_probe, bool displaced,
+                                           bool failed) {
+   const uint64_t o = next_overflow(max_probe, kBucketOverflow);
+   info->fill = placed;
+   info->tombstone_counter = 0;
+   info->current_max_bucket_overflow = o > kBucketOverflow ? o : kBucketOverflow;
+   info->reserved1 = 0; // the keys are not placed in Robin Hood order
+   if (displaced) info->err = failed ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
+}
+
 // Clean on one region: the live keys standing in it whose home lies in it are
 // placed again in an LDS image that starts empty (read from the table, which
 // does not change meanwhile), then the image is written over the region.  Of a
@@ -1061,8 +1188,8 @@ __global__ __launch_bounds__(kRgBS) __attribute__((amdgpu_waves_per_eu(4))) void
 // when the lifted keys are inserted again, so the keys placed are counted.
 // Keys of other regions standing here, and keys that run past the region's
 // end, go to the map's scratch slice (at most its live keys), from which
-// k_boundary_insert and k_map_clean_end place them.  The Info is not changed
-// here.
+// k_boundary_insert and k_map_clean_end place them.  The Info of a map of
+// several regions is not changed here.
 template <typename K>
 __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScratch* sc) {
    __shared__ RegionMem<K> L;
@@ -1071,8 +1198,12 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
    uint64_t mi, r, item = blockIdx.x;
    while (next_region(L, sc, a.n_maps, &item, &mi, &r)) {
       const hn_batch_map M = a.maps[mi];
-      if (M.info->tombstone_counter == 0 || M.info->fill > M.scratch_cap) continue;
+      if (M.info->tombstone_counter == 0) continue;
       const int sp = M.info->size_power;
+      if (M.info->fill > M.scratch_cap) { // not enough scratch: the map is left as it is
+         if (sp <= kRegionLogB<K> && threadIdx.x == 0) M.info->err = HN_STATUS_FAIL;
+         continue;
+      }
       const int rlog = sp < kRegionLogB<K> ? sp : kRegionLogB<K>;
       const uint32_t R = 1u << rlog, W = R < kRgWin ? R : kRgWin, first = static_cast<uint32_t>(r << rlog);
       const uint64_t nreg = 1ull << (sp - rlog);
@@ -1102,7 +1233,6 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
                 const uint32_t at = w + __ffs(em) - 1;
                 if (lds_cas(&L.key[at], kEmpty, key) != kEmpty) return false; // look again
                 L.val[at] = static_cast<K>(idx);
-                ++placed;
                 const uint32_t pr = off + (at - pos) + 1;
                 max_probe = pr > max_probe ? pr : max_probe;
                 return true;
@@ -1120,10 +1250,8 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
              return false; // the region's keys fit: they came from its slots
           });
       max_probe = wave_max(max_probe);
-      placed = wave_sum(placed);
       const bool wd = __ballot(displaced) != 0;
       if (__lane_id() == 0) {
-         if (placed) atomicAdd(&L.n, static_cast<unsigned long long>(placed));
          if (max_probe) atomicMax(&L.max_probe, max_probe);
          if (wd) L.flag = 1;
       }
@@ -1137,8 +1265,11 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
          if (i < R) {
             s[e].key = L.key[i];
             if (s[e].key != kEmpty) s[e].val = b[static_cast<uint32_t>(L.val[i])].val;
+            placed += s[e].key != kEmpty;
          }
       }
+      placed = wave_sum(placed);
+      if (__lane_id() == 0) atomicAdd(&L.n, static_cast<unsigned long long>(placed));
       __syncthreads(); // every value is read before the region is written
 #pragma unroll
       for (int e = 0; e < E; ++e) {
@@ -1146,29 +1277,36 @@ __global__ __launch_bounds__(kRgBS) void k_region_clean(BatchArgs<K> a, BatchScr
          if (i < R) b[i] = s[e];
       }
       if (threadIdx.x == 0) {
-         if (L.n) atomic_add_relaxed(&st->placed, static_cast<uint32_t>(L.n));
-         if (L.max_probe) atomic_max_relaxed(&st->max_probe, L.max_probe);
-         if (L.flag) __hip_atomic_store(&st->displaced, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+         if (nreg == 1) {
+            clean_info(M.info, L.n, L.max_probe, L.flag != 0, false);
+         } else {
+            if (L.n) atomic_add_relaxed(&st->placed, static_cast<uint32_t>(L.n));
+            if (L.max_probe) atomic_max_relaxed(&st->max_probe, L.max_probe);
+            if (L.flag) __hip_atomic_store(&st->displaced, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // some key of the map has been listed by now, by this region or another
+            if (__hip_atomic_load(&st->listed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) set_any(sc, kAnyListed);
+         }
       }
    }
 }
 
-// After k_region_clean and k_boundary_insert, one workgroup per map: the
-// listed keys, if some were left (those already placed find themselves),
+// After k_region_clean and k_boundary_insert, a workgroup per map of several
+// regions: the listed keys, if some were left (those already placed find themselves),
 // then the Info.
 template <typename K>
 __global__ __launch_bounds__(kRgBS) void k_map_clean_end(BatchArgs<K> a, BatchScratch* sc) {
    __shared__ uint32_t s_max, s_failed, s_placed;
+   if (sc->several == 0) return;
    for (uint32_t m = blockIdx.x; m < a.n_maps; m += gridDim.x) {
       const hn_batch_map M = a.maps[m];
       hn_info* info = M.info;
       const int sp = info->size_power;
-      if (batch_regions<K>(M, sp, a.req) == 0 || info->tombstone_counter == 0) continue;
+      const MapState st = map_state(sc, a.n_maps)[m];
+      if (sp <= kRegionLogB<K> || !(st.ways & kWayClean) || info->tombstone_counter == 0) continue;
       if (info->fill > M.scratch_cap) { // not enough scratch: the map is left as it is
          if (threadIdx.x == 0) info->err = HN_STATUS_FAIL;
          continue;
       }
-      const MapState st = map_state(sc, a.n_maps)[m];
       if (threadIdx.x == 0) {
          s_max = st.max_probe;
          s_failed = 0;
@@ -1183,14 +1321,7 @@ __global__ __launch_bounds__(kRgBS) void k_map_clean_end(BatchArgs<K> a, BatchSc
       if (c.failed) atomicOr(&s_failed, 1u);
       if (c.placed) atomicAdd(&s_placed, static_cast<uint32_t>(c.placed));
       __syncthreads();
-      if (threadIdx.x == 0) {
-         info->fill = s_placed;
-         info->tombstone_counter = 0;
-         const uint64_t o = next_overflow(s_max, kBucketOverflow);
-         info->current_max_bucket_overflow = o > kBucketOverflow ? o : kBucketOverflow;
-         info->reserved1 = 0; // the keys are not placed in Robin Hood order
-         if (st.displaced) info->err = s_failed ? HN_STATUS_FAIL : HN_STATUS_SUCCESS;
-      }
+      if (threadIdx.x == 0) clean_info(info, s_placed, s_max, st.displaced != 0, s_failed != 0);
       __syncthreads(); // s_max is rewritten for the next map
    }
 }
@@ -1248,54 +1379,58 @@ int batch_run(const hn_batch_map* maps, uint32_t n_maps, uint32_t ops, const K* 
    if ((ops & HN_BATCH_CLEAN) && !clean_scratch) return HN_EINVAL;
    if (n_maps == 0) return 0;
    const int G = (t && t->probe_width) ? t->probe_width : default_probe_width<K>(OP_INSERT);
-   const int bs = (t && t->block_size) ? t->block_size : 512;
+   const int bs = (t && t->block_size) ? t->block_size : kRgBS;
    if (G < 1 || G > 64 || (G & (G - 1)) || bs < 64 || bs > 1024 || (bs % 64)) return HN_EINVAL;
    uint32_t blocks = (t && t->grid_blocks > 0) ? static_cast<uint32_t>(t->grid_blocks)
                                                : static_cast<uint32_t>(cu_count()) * (2048 / bs);
    if (blocks > n_maps) blocks = n_maps;
-   BatchKernel<K> k = pick_batch<K>(G);
    BatchScratch* sc = static_cast<BatchScratch*>(scratch);
-   uint64_t* ticket = &sc->ticket;
-   // Launch tuning asks for the one-workgroup-per-map kernel at that shape.
-   const bool regions = !(t && (t->probe_width || t->block_size || t->grid_blocks));
-   BatchArgs<K> a{maps, n_maps, ops, ik, iv, qk, qv, qh, ek, static_cast<Slot<K>*>(clean_scratch), ticket, ops,
-                  regions ? &sc->n_big : nullptr};
-   const uint32_t rg_blocks = static_cast<uint32_t>(cu_count()) * 2; // two regions' LDS per CU
-   const uint32_t map_blocks = std::min<uint32_t>(n_maps, rg_blocks);
-   if (regions || (ops & HN_BATCH_RETRIEVE))
-      hipLaunchKernelGGL(k_batch_prep<K>, dim3(1), dim3(1024), 0, s, maps, n_maps, ops, regions ? 1 : 0, sc);
-   // insert; retrieve (one key per lane, its own launch); erase and clean
-   if (ops & HN_BATCH_INSERT) {
-      a.ops = HN_BATCH_INSERT;
-      hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, ticket);
-      hipLaunchKernelGGL(k, dim3(blocks), dim3(bs), 0, s, a);
-      if (regions) {
-         hipLaunchKernelGGL(k_region_insert<K>, dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
-         hipLaunchKernelGGL((k_boundary_insert<K, false>), dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
-         hipLaunchKernelGGL(k_map_insert_end<K>, dim3(map_blocks), dim3(kRgBS), 0, s, a, sc);
-      }
-   }
-   if (ops & HN_BATCH_RETRIEVE) {
+   BatchArgs<K> a{maps, n_maps, ops, ik, iv, qk, qv, qh, ek, static_cast<Slot<K>*>(clean_scratch), &sc->ticket, ops};
+   auto retrieve_units = [&]() {
       static std::atomic<int> occ{0};
       const int per_cu = resident_blocks_per_cu(k_batch_retrieve_lane<K>, kWave, occ);
-      a.ops = HN_BATCH_RETRIEVE;
       hipLaunchKernelGGL(k_batch_retrieve_lane<K>, dim3(static_cast<uint32_t>(cu_count()) * per_cu), dim3(kWave), 0, s,
                          a, sc);
+   };
+   const uint32_t late = ops & (HN_BATCH_ERASE | HN_BATCH_CLEAN);
+   if (t && (t->probe_width || t->block_size || t->grid_blocks)) {
+      // Launch tuning asks for the one-workgroup-per-map kernel at that shape.
+      BatchKernel<K> k = pick_batch<K>(G);
+      auto group = [&](uint32_t phases) {
+         a.ops = phases;
+         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, &sc->ticket);
+         hipLaunchKernelGGL(k, dim3(blocks), dim3(bs), 0, s, a);
+      };
+      if (ops & HN_BATCH_INSERT) group(HN_BATCH_INSERT);
+      if (ops & HN_BATCH_RETRIEVE) {
+         a.ops = 0;
+         hipLaunchKernelGGL(k_batch_group<K>, dim3(1), dim3(kRgBS), 0, s, a, sc, 1, 0);
+         retrieve_units();
+      }
+      if (late) group(late);
+      return static_cast<int>(hipGetLastError());
    }
-   if (regions && (ops & (HN_BATCH_RETRIEVE | HN_BATCH_ERASE))) {
-      a.ops = ops & (HN_BATCH_RETRIEVE | HN_BATCH_ERASE);
-      hipLaunchKernelGGL(k_region_lookup<K>, dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
+   const dim3 rg(static_cast<uint32_t>(cu_count()) * 2); // two regions' LDS per CU
+   const dim3 per_map(std::min<uint32_t>(n_maps, rg.x)), bd(kRgBS);
+   const uint32_t groups = std::min<uint32_t>(n_maps, 65535);
+   // The set-up, and beside it the inserts that do not run by regions.
+   a.ops = ops & HN_BATCH_INSERT;
+   hipLaunchKernelGGL(k_batch_group<K>, dim3(1 + (a.ops ? groups : 0)), bd, 0, s, a, sc, 1, 1);
+   if (ops & HN_BATCH_INSERT) {
+      hipLaunchKernelGGL(k_region_insert<K>, rg, bd, 0, s, a, sc);
+      hipLaunchKernelGGL((k_boundary_insert<K, false>), rg, bd, 0, s, a, sc);
+      hipLaunchKernelGGL(k_map_insert_end<K>, per_map, bd, 0, s, a, sc);
    }
-   if (ops & (HN_BATCH_ERASE | HN_BATCH_CLEAN)) {
-      a.ops = ops & (HN_BATCH_ERASE | HN_BATCH_CLEAN);
-      hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, s, ticket);
-      hipLaunchKernelGGL(k, dim3(blocks), dim3(bs), 0, s, a);
+   if (ops & HN_BATCH_RETRIEVE) retrieve_units();
+   if (ops & (HN_BATCH_RETRIEVE | HN_BATCH_ERASE)) hipLaunchKernelGGL(k_region_lookup<K>, rg, bd, 0, s, a, sc);
+   if (late) {
+      a.ops = late;
+      hipLaunchKernelGGL(k_batch_group<K>, dim3(groups), bd, 0, s, a, sc, 0, 1);
    }
-   if (regions && (ops & HN_BATCH_CLEAN)) {
-      a.ops = HN_BATCH_CLEAN;
-      hipLaunchKernelGGL(k_region_clean<K>, dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
-      hipLaunchKernelGGL((k_boundary_insert<K, true>), dim3(rg_blocks), dim3(kRgBS), 0, s, a, sc);
-      hipLaunchKernelGGL(k_map_clean_end<K>, dim3(map_blocks), dim3(kRgBS), 0, s, a, sc);
+   if (ops & HN_BATCH_CLEAN) {
+      hipLaunchKernelGGL(k_region_clean<K>, rg, bd, 0, s, a, sc);
+      hipLaunchKernelGGL((k_boundary_insert<K, true>), rg, bd, 0, s, a, sc);
+      hipLaunchKernelGGL(k_map_clean_end<K>, per_map, bd, 0, s, a, sc);
    }
    return static_cast<int>(hipGetLastError());
 }

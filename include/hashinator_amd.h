@@ -474,12 +474,12 @@ HN_API int hn_exclusive_scan_u64(const uint64_t* in, uint64_t* out, size_t n, vo
  * (hashers.h:46-65), retrieve (111-119), erase (132-142), clean_tombstones
  * (hashinator.h:1261-1315) -- with the single-map semantics above; maps are
  * taken in array order (list the largest first).  By default a workgroup runs
- * a phase on one 64-KiB region of a map's slots in LDS; maps of more than 1,024
- * regions, maps of several regions that a call without clean barely touches,
- * and calls with launch tuning take one workgroup per map for insert and for
- * erase + clean, and one key per lane for retrieve in between.  Persistent
- * launches plus small set-up kernels (graph-capturable: no host
- * synchronisation, no allocation, no memset). */
+ * a phase on one 64-KiB region of a map's slots in LDS; lists that are short for
+ * their map, maps of more than 1,024 regions and calls with launch tuning take
+ * one workgroup per map for insert and for erase + clean, and one key per lane
+ * for retrieve in between, as do query lists much longer than the map.  A few
+ * launches, the set-up among them (graph-capturable: no host synchronisation,
+ * no allocation, no memset). */
 typedef struct hn_batch_map {
    void* buckets;        /* 2^size_power slots; size_power is read from *info */
    hn_info* info;
@@ -493,7 +493,7 @@ enum { HN_BATCH_INSERT = 1, HN_BATCH_RETRIEVE = 2, HN_BATCH_ERASE = 4, HN_BATCH_
 
 /* Device scratch of hn_batch_run for a batch of n_maps maps: the tickets, per
  * map its first retrieve unit, its first region and what its regions leave for
- * the map (44 bytes), and lists of up to 4 MB for maps of several regions.
+ * the map (48 bytes), and lists of up to 4 MB for maps of several regions.
  * hn_batch_run_* is not told the size of the buffer that it is given, so ask
  * this function, of the library that runs, for it: the layout is that
  * library's own and not a sum of the above. */

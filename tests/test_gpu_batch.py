@@ -452,3 +452,89 @@ def test_batch_query_units_beside_regions(gpu):
         bm.run(ops)
         torch.cuda.synchronize()
         check_against_oracle(bm, wl, key_bits, ops)
+
+
+@pytest.mark.parametrize("key_bits", [32, 64])
+# maps, size power below a one-region map's, keys of each phase, load factor, the phases
+@pytest.mark.parametrize("n_maps,below,k,lf,ops", [
+    (1, 0, 16, 0.6, 1), (1, 5, 4, 0.6, 1), (2000, 0, 16, 0.6, 1), (2000, 3, 16, 0.3, 2), (2000, 0, 4, 0.6, 4), (1, 0, 16, 0.6, 15),
+    (300, 1, 64, 0.6, 7), (40, 2, 600, 0.5, 7), (64, 1, 2, 0.89, 6), (64, 2, 40, 0.7, 6), (5, 10, 3, 0.5, 15), (30, -1, 100, 0.6, 7)])
+def test_batch_few_keys(gpu, key_bits, n_maps, below, k, lf, ops):
+    """Lists much shorter than the tables: the oracle's results, and not much slower than one
+    workgroup for each map, which asking for a launch shape gives (8 us are two launches)."""
+    from tests.helpers import race
+    sp = (13 if key_bits == 32 else 12) - below
+    n = max(k, int(lf * (1 << sp)))
+    base = [W.unique_keys(n, key_bits, 200 + m % 37) for m in range(n_maps)]
+    rng = np.random.default_rng(k)
+    vals = [(b ^ b.dtype.type(0x51)).astype(b.dtype) for b in base]
+    table = BatchedMaps([sp] * n_maps, base, vals, [b[:0] for b in base], [b[:0] for b in base], key_bits=key_bits)
+    table.init()
+    table.run(_lib.HN_BATCH_INSERT)
+    upd = [rng.choice(b, k, replace=False) for b in base]
+    qry = [np.concatenate([rng.choice(b, k - k // 3), W.unique_keys(k // 3, key_bits, 200 + m % 37, start=n + 5)])
+           for m, b in enumerate(base)]
+    ers = [rng.choice(b, k, replace=False) for b in base]
+    bm = BatchedMaps([sp] * n_maps, upd, upd, qry, ers, key_bits=key_bits)
+    desc = bm.descs.cpu().numpy().view(np.uint64).reshape(n_maps, 10).copy()  # clean: room for the keys already there
+    desc[:, 8], desc[:, 9] = bm.slot_off[bm.order], 1 << sp
+    bm.clean_scratch = torch.empty_like(bm.arena)
+    bm.descs.copy_(torch.from_numpy(desc.view(np.uint8).reshape(-1)))
+
+    def before():
+        bm.arena.copy_(table.arena)
+        bm.infos.copy_(table.infos)
+    shape = hn_tune(4, 512, 0, 0)
+    default, asked = race(lambda: bm.run(ops), lambda: bm.run(ops, shape), before, reps=9)
+    assert default <= 1.3 * asked + 8, (default, asked)
+    before()
+    bm.qry_vals.zero_()
+    bm.qry_hit.zero_()
+    bm.run(ops)
+    torch.cuda.synchronize()
+    if ops & _lib.HN_BATCH_INSERT:
+        for b, v, u in zip(base, vals, upd):
+            v[np.isin(b, u)] = b[np.isin(b, u)]
+    check_bulk(bm, ([sp] * n_maps, base, vals, qry, ers), key_bits, ops | _lib.HN_BATCH_INSERT)
+
+
+@pytest.mark.parametrize("key_bits", [32, 64])
+@pytest.mark.parametrize("below,k", [(0, 1), (0, 30), (5, 3)])
+def test_batch_few_keys_among_tombstones(gpu, key_bits, below, k):
+    """A few keys into, of and out of tables whose slots are nearly all TOMBSTONEs, which every probe
+    runs through."""
+    from tests.helpers import race
+    sp, n_maps = (13 if key_bits == 32 else 12) - below, 40
+    n = int(0.97 * (1 << sp))
+    pool = [W.unique_keys(n + 2 * k, key_bits, 300 + m) for m in range(n_maps)]
+    none = [p[:0] for p in pool]
+    table = BatchedMaps([sp] * n_maps, [p[:n] for p in pool], [p[:n] for p in pool], none, [p[5:n] for p in pool], key_bits=key_bits)
+    table.init()
+    table.run(_lib.HN_BATCH_INSERT | _lib.HN_BATCH_ERASE)
+    new, qry = [p[n:n + k] for p in pool], [p[n - 3:] for p in pool]
+    ers = [np.concatenate([p[:1], p[n:n + k // 2], p[n + k:]]) for p in pool]
+    bm = BatchedMaps([sp] * n_maps, new, new, qry, ers, key_bits=key_bits)
+
+    def before():
+        bm.arena.copy_(table.arena)
+        bm.infos.copy_(table.infos)
+    ops = _lib.HN_BATCH_INSERT | _lib.HN_BATCH_RETRIEVE | _lib.HN_BATCH_ERASE
+    default, asked = race(lambda: bm.run(ops), lambda: bm.run(ops, hn_tune(4, 512, 0, 0)), before, reps=3)
+    assert default <= 1.3 * asked + 8, (default, asked)
+    before()
+    bm.run(ops)
+    torch.cuda.synchronize()
+    for m, p in enumerate(pool):
+        model = O.GpuModel(sp, key_bits)
+        model.insert(p[:n], p[:n])
+        model.erase(p[5:n])
+        model.insert(new[m], new[m])
+        ev, eh = model.retrieve(qry[m])
+        model.erase(ers[m])
+        v, h = bm.results(m)
+        assert np.array_equal(h, eh) and np.array_equal(v[h], ev[eh]), m
+        img, info = bm.buckets(m), bm.info(m)
+        assert np.array_equal(live_pairs(img, key_bits), live_pairs(model.b, key_bits)), m
+        assert np.array_equal(occupancy(img, key_bits), occupancy(model.b, key_bits)), m
+        assert (info.fill, info.tombstone_counter, info.err) == (model.info.fill, model.info.tombstones, 0), m
+        assert reachable_all(img, key_bits, sp), m

@@ -136,8 +136,8 @@ def test_output_tensors_are_checked_before_a_launch():
 
 def test_batch_workspace_of_many_maps():
     """The batched call's workspace: bytes per map in the tens, and room for the
-    layout (64 + 44 per map) whatever their number."""
+    layout (64 + 48 per map) whatever their number."""
     need = _lib.load().hn_batch_scratch_bytes
     assert need(1_000_000) <= 64 << 20
     for n in (0, 1, 7, 4096, 4097, 100_000):
-        assert 64 + 44 * n <= need(n) <= 44 * n + (4 << 20) + 512
+        assert 64 + 48 * n <= need(n) <= 48 * n + (4 << 20) + 512
