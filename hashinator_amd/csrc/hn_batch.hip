@@ -127,14 +127,20 @@ __device__ __forceinline__ bool ins_by_regions(const hn_batch_map& M, const hn_i
 // one region are looked up and erased where the table stands while they are few,
 // since indexing the region costs more than their probes, and by the region as
 // the probes get long.  Measured at u32, so / by the region:
-// - lookups, from 512 queries on or seven eighths of the slots taken: 256 maps
-//   of 2^12 slots, 128 queries, load factor 0.6 23 and 27 us, 0.9 74 and 29,
-//   4,096 maps 53 and 147, 129 and 152, 512 queries at 0.6 80 and 155 but one
-//   map of 2^10 27 and 24; fewer than 2^10 slots 62 and 113 also at 0.9;
-// - erases, from a tenth of the slots on in the largest two sizes and a quarter
-//   in others (256 maps of 2^13 slots, 0.6: a sixteenth 29 and 36 us, a quarter
-//   55 and 37), where five eighths are taken from a 64th on (0.8: 49 and 36; of
-//   2^10 slots 35 and 26; 4 keys each of 4,096 maps of 2^8 83 and 105);
+// - lookups, from 512 queries or as many as slots on, and where seven eighths of
+//   the slots are taken: 256 maps of 2^12 slots, 128 queries, load factor 0.6 23
+//   and 27 us, 0.9 74 and 29, 4,096 maps 53 and 147, 129 and 152, 512 queries at
+//   0.6 80 and 155 but one map of 2^10 27 and 24; fewer than 2^10 slots 62 and
+//   113 also at 0.9;
+// - erases, from a tenth of the slots on (256 maps of 2^13 slots, 0.6: a
+//   sixteenth 29 and 36 us, a quarter 55 and 37), where five eighths are taken
+//   from a 64th on (0.8: 49 and 36; of 2^10 slots 35 and 26; 4 keys each of 4,096
+//   maps of 2^8 83 and 105);
+// The lines lie lower than lists like these alone would have them (4,096 maps of
+// 2^8, an eighth erased at 0.6: 99 and 110 us), since among larger maps both
+// ways run and each waits for its last map (1,024 maps of 2^8..2^16 slots, all
+// phases: a quarter of the slots of small maps as the line 1,108 us, a tenth
+// 1,081).
 // - both where nearly all are: a table full of TOMBSTONEs is probed slot by slot.
 template <typename K>
 __device__ __forceinline__ uint32_t map_ways(const hn_batch_map& M, const hn_info* info, int sp, uint32_t ops,
@@ -148,8 +154,8 @@ __device__ __forceinline__ uint32_t map_ways(const hn_batch_map& M, const hn_inf
    } else {
       const uint64_t used = info->fill + info->tombstone_counter + ((ops & HN_BATCH_INSERT) ? M.ins_len : 0);
       const bool full = used * 16 >= n * 15;
-      qry = qry && (nq >= 512 || full || (sp >= 10 && used * 8 >= n * 7));
-      ers = ers && (ne * (sp + 1 >= kRegionLogB<K> ? 10 : 4) >= n || full || (used * 8 >= n * 5 && ne >= 16 && ne * 64 >= n));
+      qry = qry && (nq >= 512 || nq >= n || full || (sp >= 10 && used * 8 >= n * 7));
+      ers = ers && (ne * 10 >= n || full || (used * 8 >= n * 5 && ne >= 16 && ne * 64 >= n));
    }
    return (ins_by_regions<K>(M, info, sp, ops, n_maps) ? kWayIns : 0u) | (qry ? kWayQry : 0u) | (ers ? kWayErs : 0u) |
           ((ops & HN_BATCH_CLEAN) ? kWayClean : 0u);
