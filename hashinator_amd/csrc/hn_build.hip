@@ -431,7 +431,6 @@ __global__ __launch_bounds__(BS) void k_part_scatter(PartIn<K> in, uint64_t n_in
       if (start && blockIdx.x == 0) {
          start[d] = o;
          if (d == D - 1) start[D] = FILTER ? h->n : n;
-         lb.word[d] = 0;
          lb.mark[d] = 0;
       }
    }
@@ -585,7 +584,7 @@ __host__ __device__ __forceinline__ RegionSum compose(RegionSum first, RegionSum
 // A region's carry function in one 64-bit word: a <= keys in the region
 // < 2^24; b + R in [0, 2^24).
 __device__ __forceinline__ uint64_t pack_sum(RegionSum g, int64_t R) {
-   return (1ull << 63) | (static_cast<uint64_t>(g.b + R) << 24) | static_cast<uint64_t>(g.a);
+   return (static_cast<uint64_t>(g.b + R) << 24) | static_cast<uint64_t>(g.a);
 }
 __device__ __forceinline__ RegionSum unpack_sum(uint64_t w, int64_t R) {
    RegionSum g;
@@ -602,7 +601,8 @@ __device__ __forceinline__ RegionSum load_sum(const RegionLB& lb, uint64_t r, in
 // does), start[NR] = n: a binary search per region over the sorted array.
 // Neighbouring lanes search neighbouring regions and share the upper levels
 // of their searches in cache; the array itself is not streamed.  The same
-// launch clears the region bookkeeping of the placing step.
+// launch clears the regions' marks; their sums are written by the placing step
+// before any kernel reads them.
 template <typename K>
 __global__ __launch_bounds__(256) void k_region_starts(const Slot<K>* S, uint64_t* start, RegionLB lb, uint64_t NR,
                                                        int sp, int rlog, BuildHeader* h) {
@@ -617,10 +617,7 @@ __global__ __launch_bounds__(256) void k_region_starts(const Slot<K>* S, uint64_
          else hi = mid;
       }
       start[r] = lo;
-      if (r < NR) {
-         lb.word[r] = 0;
-         lb.mark[r] = 0;
-      }
+      if (r < NR) lb.mark[r] = 0;
    }
 }
 
@@ -1528,7 +1525,6 @@ int grow(const void* keys, const void* vals, const void* pairs, const void* old_
                 static_cast<const Slot<K>*>(old_b), nt};
    return build_core<K>(P, BUILD_GROW, SRC_GROW, in, nt + len, new_b, info, scratch, s);
 }
-
 
 // ------------------------------------------------------------------ merge insert
 //

@@ -45,10 +45,11 @@ namespace compact {
 // 0.35; whole u64 pairs 0.63 -> 0.67, their registers leaving one workgroup
 // on a CU (in the caches they gain too: 2^23 pairs 48 -> 43 us, 2^24
 // 93 -> 94).  From kLargeMin elements on: below, the larger tiles are too few
-// for the CUs (u32 pairs: 2^21 18.0 -> 20.0 us, 2^22 24.5 -> 23.2).  (Workgroups that take tile after tile, with the next tile's
-// elements loaded or not while the current one waits for its prefix, were
-// slower than one workgroup per tile, two on a CU: 0.65 to 0.72 ms and 0.57
-// at best for the u64 keys.)
+// for the CUs (u32 pairs: 2^21 18.0 -> 20.0 us, 2^22 24.5 -> 23.2).
+// Workgroups that take tile after tile, with the next tile's elements loaded
+// or not while the current one waits for its prefix, were slower than one
+// workgroup per tile, two on a CU: 0.65 to 0.72 ms and 0.57 at best for the
+// u64 keys.
 constexpr int kThreads = 1024;
 constexpr int kWaveSize = 64;
 constexpr int kWaves = kThreads / kWaveSize;
