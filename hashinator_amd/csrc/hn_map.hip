@@ -282,10 +282,14 @@ __global__ __launch_bounds__(lane_block(MODE)) void k_lookup_lane(LookupArgs<K> 
          const int wv = threadIdx.x / kWave;
          // Waves on a CU, where the grid is the automatic one: 16 for a table in
          // the L2s, 8 for one in the last-level cache, 12 beyond, where more only
-         // queue for the memory (u64 queries, 8 / 12 / 16 / 20 waves: 2^26 of 2^18
-         // slots 1.66 / 1.24 / 1.07 / 1.06 ms; 12 million of 2^24 319 / 326 / 331 /
-         // 333 us; 30 million of 2^26 1.195 / 1.126 / 1.122 / 1.133 ms).  The size
-         // is known on the device only: the waves over that number end at once.
+         // queue for the memory.  At load .9, 8 million queries and up to as many
+         // erases, 8 / 12 / 16 waves, us: 16 MiB u64 queries 219 / - / 208, u32
+         // 187 / - / 168; 32 MiB 240 / - / 249, u32 196 / - / 199; 64 MiB 262 / 270
+         // / 270, erases 66 / 73 / 76, u32 queries 206 / 214 / 215, erases 100 / 101
+         // / 105; 256 MiB 279 / 290 / 288, erases 217 / 214 / 211, u32 220 / 228 /
+         // 231, erases 363 / 374 / 373; 1 GiB 337 / 316 / 313, erases 475 each, u32
+         // of 512 MiB 233 / 224 / 227, erases 369 / 387 / 388.  The size is known on
+         // the device only: the waves over that number end at once.
          const uint64_t bytes = sizeof(Slot<K>) << sp;
          const uint64_t per_cu = bytes <= 1ull << 25 ? 16 : bytes <= 1ull << 28 ? 8 : 12;
          uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * kWaves;

@@ -394,9 +394,11 @@ __device__ __forceinline__ uint64_t lookup_range(const LookupArgs<K>& a, const i
 // memory.  Measured, 2^26 queries, half of them present, u64 and u32 at load
 // .9, staged -> here: 2^18 slots (in L2) 1.58 -> 1.03 ms and 1.93 -> 0.88;
 // 2^24 2.18 -> 2.20 and 2.40 -> 1.71; 2^28 2.97 -> 2.97 and 2.94 -> 2.12.
-// The bound is now the rate of 128-byte requests, 1.56 (u64) and 1.28 (u32)
-// a query here: random ones reach 98 G/s in L2 and 55 G/s beyond, and these
-// make 101 and 97 G/s in 2^18 slots, 48 and 50 in 2^24.
+// The bound is now the rate of requests to L2, counted (TCP_TCC_READ_REQ)
+// 1.67 (u64) and 1.33 (u32) a query, the keys' among them: of 2^18 slots that
+// makes 96 and 92 G/s, and the calibration kernel's random 128-byte reads of a
+// buffer as large (4 and 2 MiB) 94 and 92; of 2^24 slots 54 and 56 G/s, where
+// it makes 55 and 56 (256 and 128 MiB).
 //
 // The Robin Hood stop is tested on the window's LAST slot only: in an
 // ordered table the stop predicate is monotone along a cluster (homes never

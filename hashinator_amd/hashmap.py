@@ -133,20 +133,29 @@ class Hashmap:
         this fraction of the bucket count into an empty table takes the bulk
         path (hn_build_*: partition + per-region sort, no probing), which
         writes the reordered image directly; 0 turns it off.
-        ``build_min_keys``: and holds at least this many keys -- the build's
-        dozen small launches take about 0.09 ms however few the keys, so
-        below about 2^17 keys at low load factors the probing insert and
-        reorder are faster (one MI355X, u32: 0.088 against 0.090 ms at
-        131,072 keys and LF 0.5, 0.10 against 0.19 ms at 235,929 keys and LF
-        0.9, 0.10 against 0.26 ms at 524,288 keys and LF 0.5).  Growing a
-        map of at least this many keys rehashes it by the build too.
+        ``build_min_keys``: and holds at least this many keys -- a build call
+        takes about 0.125 ms however few the keys, the probing insert and
+        reorder from 0.06 by keys and load.  One MI355X, whole call, probing
+        against build, us: 117,964 keys to LF 0.9 u32 168 and 133, u64 181 and
+        132, 58,982 of them 131 and 131, 124 and 135; 786,432 to 0.75 144 and
+        144, 153 and 151; to LF 0.5 131,072 86 and 124, 90 and 127, 1,048,576
+        138 and 174, 146 and 180.  So 2^17 is the crossover of a table that
+        ends nearly full; at half load up to 2^20 keys the build costs 0.04 ms
+        more and is still taken.  Growing a map of at least this many keys
+        rehashes it by the build too.
         ``merge_min``: an insert of at least this fraction of the bucket count
         (and of ``build_min_keys``) into a table that holds keys and no
         tombstones takes the merge (hn_merge_*), which writes the insert +
         reorder image into a fresh bucket array; the merge reads and writes
-        the whole table, so it pays from about a quarter of the table (one
-        MI355X, a quarter of 2^26 u64 slots up to load 0.5: 1.32 ms against
-        1.54), sooner only where the table is nearly full (see _try_merge).
+        the whole table, so it pays from about a quarter of the table of new
+        keys, sooner only where the table is nearly full (see _try_merge).
+        One MI355X, whole call, insert + reorder against merge, into a table
+        of load 0.3: 2^26 u64 slots, an eighth 1.01 and 1.15 ms, three
+        sixteenths 1.32 and 1.28, a quarter 1.58 and 1.39, u32 0.88 and 0.93,
+        1.13 and 1.01, 1.32 and 1.09; a quarter of 2^24 u64 0.54 and 0.45,
+        u32 0.40 and 0.39, of 2^22 0.18 and 0.23, 0.17 and 0.21 (into load 0.6
+        0.27 and 0.24, 0.28 and 0.22).  Updates alone are faster probed (a
+        quarter of 2^26 u64 1.24 and 1.99 ms).
         A table not in Robin Hood order is reordered first when the batch is
         at least 4/3 of this fraction.  0 turns it off."""
         if key_bits not in (32, 64):
@@ -387,11 +396,11 @@ class Hashmap:
         most of the batch's keys: the probing insert's chains for
         new keys grow with the load, its updates and the merge do not.  One
         MI355X, insert + reorder against merge + copy, a sixteenth of 2^26 u64
-        slots: new keys up to load .82 1.18 and 1.52 ms, .88 1.76 and 1.54, .94
-        3.33 and 1.54, updates at .82 0.77 and 2.10, at .88 0.80 and 2.12; u32
-        new 1.06 and 1.14, 1.42 and 1.14, 3.02 and 1.16, updates 0.73 and 1.68,
-        0.75 and 1.68.  The image is copied back, so that the bucket array
-        stays the one that it was."""
+        slots: new keys up to load .82 1.16 and 1.52 ms, .88 1.51 and 1.49, .91
+        2.05 and 1.51, .94 3.14 and 1.53, updates at .82 0.76 and 2.06, at .88
+        0.80 and 2.09; u32 new 1.03 and 1.10, 1.39 and 1.12, 1.80 and 1.11, 2.84
+        and 1.12, updates 0.72 and 1.64, 0.75 and 1.66.  The image is copied
+        back, so that the bucket array stays the one that it was."""
         N = self.bucket_count()
         small = self._may_merge_small(n)
         if not small and (not self.merge_min or n < max(self.merge_min * N, self.build_min_keys) or n >= N or
