@@ -88,18 +88,18 @@ constexpr uint64_t kSmallInsert = 8192, kSoloInsert = 256;
 // after the insert where one workgroup runs it (64 keys into 2^12 u64 slots
 // empty 7.4 and 10.8, at load .6 15.1 and 14.9, at .85 44 and 38).  Several
 // workgroups must agree whatever the fill is when each starts, so by the sizes
-// alone: tables of 32 KiB (512 into 2^12 u32 slots empty 11.5 and 14.2, at
-// load .6 24 and 24, 1,024 at .7 99 and 77), and of 64 KiB from a quarter of
-// the slots on in 64 bits (2^12: 1,024 into an empty one 13 and 16, at .7 110
-// and 93) and three quarters in 32 (2^13: 2,048 into an empty one 13 and 19, at
-// .6 46 and 44).
+// alone: from a quarter of the slots on, into tables of 32 KiB (512 into 2^12
+// u32 slots empty 11.0 and 14.1, at load .6 24 and 24, 1,024 at .7 99 and 77)
+// and of 64 KiB in 64 bits (2^12: 1,024 into an empty one 13 and 16, at .7 110
+// and 93); not in 32 (2^13: 2,048 into an empty one 13 and 19, at .6 46 and 44,
+// 6,200 into an empty one 29 and 36, at .1 48 and 55, at .2 163 and 150).
 template <typename K>
 __device__ __forceinline__ bool lds_insert_pays(const hn_info* info, int sp, uint64_t len, int solo) {
    constexpr int kLog = kRegionLogB<K>;
    const uint64_t R = 1ull << sp;
    if (sp > kLog || len * 64 < R) return false;
    if (sp <= kLog - 2) return true;
-   if (!solo) return sp < kLog || len * 4 >= (sizeof(K) == 8 ? R : R * 3);
+   if (!solo) return len * 4 >= R && (sp < kLog || sizeof(K) == 8);
    const uint64_t used = info->fill + info->tombstone_counter;
    return (2 * used + len) * 8 >= R * 9 || (used + len) * 4 >= R * 3;
 }
