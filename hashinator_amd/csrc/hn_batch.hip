@@ -62,9 +62,9 @@ struct BatchArgs {
    uint32_t req; // the call's phases (ops is the launch's)
 };
 
-// ------------------------------------------------------------ regions
-//
+// ------------------------------------------------------- ways of a map
 constexpr uint64_t kMaxRegions = 1024;
+
 // Whether a map's queries are looked up by units, although it has regions.
 // Each of its regions' workgroups reads the whole list (0.43 ns a query) and
 // looks up its own share (2.2 ns each) on the CU that it has; the units go over
@@ -80,7 +80,8 @@ constexpr uint64_t kMaxRegions = 1024;
 // queries 19,300 and 449.
 constexpr uint64_t kRegionsByUnits = 32, kRegionsFill = 256;
 __device__ __forceinline__ bool by_units(uint64_t nq, uint64_t regions, uint32_t n_maps) {
-   const uint64_t wgs = n_maps * regions, limit_ns = 30000 + 70000 * (wgs < kRegionsFill ? wgs : kRegionsFill) / kRegionsFill;
+   const uint64_t wgs = n_maps * regions;
+   const uint64_t limit_ns = 30000 + 70000 * (wgs < kRegionsFill ? wgs : kRegionsFill) / kRegionsFill;
    return regions == 0 || regions > kRegionsByUnits || nq * (430 * regions + 2200) > 1000 * limit_ns * regions;
 }
 
@@ -103,7 +104,8 @@ __device__ __forceinline__ uint32_t map_regions(const hn_batch_map& M, int sp, u
 }
 // A map of several regions goes by them unless its lists hold fewer keys than a
 // sixteenth of the slots, where loading the table costs more than probing it.
-__device__ __forceinline__ bool several_pay(const hn_batch_map& M, uint32_t nreg, uint64_t n, uint32_t ops, uint32_t n_maps) {
+__device__ __forceinline__ bool several_pay(const hn_batch_map& M, uint32_t nreg, uint64_t n, uint32_t ops,
+                                            uint32_t n_maps) {
    const uint64_t nq = (ops & HN_BATCH_RETRIEVE) && !by_units(M.qry_len, nreg, n_maps) ? M.qry_len : 0;
    const uint64_t keys = ((ops & HN_BATCH_INSERT) ? M.ins_len : 0) + nq + ((ops & HN_BATCH_ERASE) ? M.ers_len : 0);
    return (ops & HN_BATCH_CLEAN) || keys * 16 >= n;
@@ -136,18 +138,19 @@ __device__ __forceinline__ bool ins_by_regions(const hn_batch_map& M, const hn_i
 //   sixteenth 29 and 36 us, a quarter 55 and 37), where five eighths are taken
 //   from a 64th on (0.8: 49 and 36; of 2^10 slots 35 and 26; 4 keys each of 4,096
 //   maps of 2^8 83 and 105);
+// - both where nearly all are: a table full of TOMBSTONEs is probed slot by slot.
 // The lines lie lower than lists like these alone would have them (4,096 maps of
 // 2^8, an eighth erased at 0.6: 99 and 110 us), since among larger maps both
 // ways run and each waits for its last map (1,024 maps of 2^8..2^16 slots, all
 // phases: a quarter of the slots of small maps as the line 1,108 us, a tenth
 // 1,081).
-// - both where nearly all are: a table full of TOMBSTONEs is probed slot by slot.
 template <typename K>
 __device__ __forceinline__ uint32_t map_ways(const hn_batch_map& M, const hn_info* info, int sp, uint32_t ops,
                                              uint32_t n_maps) {
    const uint32_t nreg = map_regions<K>(M, sp, ops);
    if (nreg == 0) return 0;
-   const uint64_t n = 1ull << sp, nq = (ops & HN_BATCH_RETRIEVE) ? M.qry_len : 0, ne = (ops & HN_BATCH_ERASE) ? M.ers_len : 0;
+   const uint64_t n = 1ull << sp, nq = (ops & HN_BATCH_RETRIEVE) ? M.qry_len : 0;
+   const uint64_t ne = (ops & HN_BATCH_ERASE) ? M.ers_len : 0;
    bool qry = nq && !by_units(nq, nreg, n_maps), ers = ne != 0;
    if (nreg > 1) {
       if (!several_pay(M, nreg, n, ops, n_maps)) return 0;
@@ -507,7 +510,8 @@ __global__ __launch_bounds__(kRgBS) void k_batch_group(BatchArgs<K> a, BatchScra
          ops = ins_by_regions<K>(M, M.info, M.info->size_power, a.req, a.n_maps) ? 0 : a.ops;
       } else {
          const uint32_t ways = map_state(sc, a.n_maps)[m].ways;
-         ops = ((ways & kWayErs) || !M.ers_len ? 0 : a.ops & HN_BATCH_ERASE) | ((ways & kWayClean) ? 0 : a.ops & HN_BATCH_CLEAN);
+         ops = ((ways & kWayErs) || !M.ers_len ? 0 : a.ops & HN_BATCH_ERASE) |
+               ((ways & kWayClean) ? 0 : a.ops & HN_BATCH_CLEAN);
       }
       if (ops) map_phases<K, default_probe_width<K>(OP_INSERT)>(a, M, ops, S);
    }
